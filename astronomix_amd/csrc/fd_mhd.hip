@@ -7,11 +7,12 @@
 //   k_prep     positivity floors of the carried stage state and the
 //              face-to-centre B with its energy correction
 //              (_enforce_positivity.py:21-59, _constrained_transport.py:160-198)
-//   k_weno<d>  interface fluxes along d: the cells of a tile are staged in LDS
-//              with their flux and wave speeds; each thread builds the
-//              interface eigen-system once and runs the 7 characteristic
-//              WENO-5 reconstructions (_weno.py:111-324, _eigen.py:116-911);
-//              also emits the CT modified fluxes (_constrained_transport.py:81-102)
+//   k_weno     interface fluxes along x, y and z in one launch: the cells of a
+//              tile are staged in LDS with their flux and wave speeds; each
+//              thread builds the interface eigen-system once and runs the 7
+//              characteristic WENO-5 reconstructions (_weno.py:111-324,
+//              _eigen.py:116-911); also emits the CT modified fluxes
+//              (_constrained_transport.py:81-102)
 //   k_ct_edge  edge EMFs by 4th-order interpolation (_constrained_transport.py:107-131)
 //   k_ct_avg   point values to averages (_interpolate.py:38-62)
 //   k_face     6th-order curl of the EMFs + SSPRK combine of the face fields
@@ -38,7 +39,7 @@ constexpr int TP = 8;    // waves per WENO block
 constexpr int NTH = TP * TBZ;
 
 struct Phys {
-  float gamma, gm1, inv_gm1, rhomin, pgmin;
+  float gamma, gm1, inv_gm1, rhomin, pgmin, inv_rhomin;
   int positivity;
 };
 
@@ -77,45 +78,11 @@ __device__ __forceinline__ unsigned nb(const Grid& g, const Pos& p, int axis, in
 
 __device__ __forceinline__ float dss(float x) { return fsqrt(fmaxf(x, 1e-12f)); }
 
-// component permutation of the direction's frame (the reference's swaps of
-// (m_x, m_d) and (B_x, B_d)); an involution
-__device__ __forceinline__ int perm(int dir, int v) {
-  if (dir == 1) {
-    const int t[8] = {0, 2, 1, 3, 4, 6, 5, 7};
-    return t[v];
-  }
-  if (dir == 2) {
-    const int t[8] = {0, 3, 2, 1, 4, 7, 6, 5};
-    return t[v];
-  }
-  return v;
-}
+// Rows of a direction's frame in the state's numbering (the reference's swaps
+// of (m_x, m_d) and (B_x, B_d)); an involution.
+constexpr int FRAME[3][8] = {{0, 1, 2, 3, 4, 5, 6, 7}, {0, 2, 1, 3, 4, 6, 5, 7}, {0, 3, 2, 1, 4, 7, 6, 5}};
 
-// _mhd_flux_x of one cell in the direction's frame (_fluxes.py:20-69)
-__device__ __forceinline__ void cell_flux(const float* q, float* f, const Phys& ph) {
-  float rho = q[0];
-  const float ri = frcp(rho);
-  const float vx = q[1] * ri, vy = q[2] * ri, vz = q[3] * ri;
-  const float Bx = q[5], By = q[6], Bz = q[7];
-  const float u2 = (vx * vx + vy * vy) + vz * vz;
-  const float b2 = (Bx * Bx + By * By) + Bz * Bz;
-  float p = ph.gm1 * ((q[4] - (0.5f * rho) * u2) - 0.5f * b2);
-  if (ph.positivity) {
-    rho = fmaxf(rho, ph.rhomin);
-    p = fmaxf(p, ph.pgmin);
-  }
-  const float Pt = p + 0.5f * b2;
-  const float vB = (vx * Bx + vy * By) + vz * Bz;
-  const float E = (p * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2;
-  f[0] = rho * vx;
-  f[1] = ((rho * (vx * vx)) + Pt) - Bx * Bx;
-  f[2] = ((rho * vx) * vy) - Bx * By;
-  f[3] = ((rho * vx) * vz) - Bx * Bz;
-  f[4] = (E + Pt) * vx - vB * Bx;
-  f[5] = 0.f;
-  f[6] = By * vx - Bx * vy;
-  f[7] = Bz * vx - Bx * vz;
-}
+__device__ __forceinline__ int perm(int dir, int v) { return FRAME[dir][v]; }
 
 // cell floors of the building-block routines (_eigen.py:62-74 / 148-160)
 struct Cell {
@@ -154,363 +121,412 @@ __device__ __forceinline__ void cell_speeds(const float* q, float* sp, const Phy
   sp[3] = dss(fmaxf(0.f, 0.5f * (s - droot)));
 }
 
-// interface eigen-system building blocks (_eigen.py:116-337)
+// LDS fields of a staged cell, in the direction's frame.
+enum { C_Q = 0, C_F = 8, C_VX = 15, C_CF = 16, C_CA = 17, C_CS = 18, C_VY = 19, C_VZ = 20, C_H = 21, NFIELD = 22 };
+
+// One cell of the window: conserved rows u, its flux (_fluxes.py:20-69; rows
+// 0-4, 6, 7 -- the normal field's flux is 0), v_x and the fast, Alfven and slow
+// speeds (_eigen.py:27-114; the 7 eigenvalues are v_x -/+ these and v_x), and
+// what the interface averages need of it (_eigen.py:148-190).
+__device__ __forceinline__ void stage_cell(const float* u, const Phys& ph, float* o) {
+  const float rho = u[0], ri = frcp(rho);
+  const float vx = u[1] * ri, vy = u[2] * ri, vz = u[3] * ri;
+  const float Bx = u[5], By = u[6], Bz = u[7];
+  const float u2 = (vx * vx + vy * vy) + vz * vz;
+  const float b2 = (Bx * Bx + By * By) + Bz * Bz;
+  const float pc = ph.gm1 * ((u[4] - (0.5f * rho) * u2) - 0.5f * b2);
+  float fr = rho, fp = pc;
+  if (ph.positivity) {
+    fr = fmaxf(rho, ph.rhomin);
+    fp = fmaxf(pc, ph.pgmin);
+  }
+  const float Pt = fp + 0.5f * b2;
+  const float vB = (vx * Bx + vy * By) + vz * Bz;
+  const float E = (fp * ph.inv_gm1 + (0.5f * fr) * u2) + 0.5f * b2;
+#pragma unroll
+  for (int v = 0; v < 8; ++v) o[C_Q + v] = u[v];
+  o[C_F + 0] = fr * vx;
+  o[C_F + 1] = ((fr * (vx * vx)) + Pt) - Bx * Bx;
+  o[C_F + 2] = ((fr * vx) * vy) - Bx * By;
+  o[C_F + 3] = ((fr * vx) * vz) - Bx * Bz;
+  o[C_F + 4] = (E + Pt) * vx - vB * Bx;
+  o[C_F + 5] = By * vx - Bx * vy;
+  o[C_F + 6] = Bz * vx - Bx * vz;
+  // the eigen-system's own floors (_eigen.py:62-74, 148-160)
+  const bool low = rho < ph.rhomin;
+  const float ra = low ? ph.rhomin : rho, rinv = low ? ph.inv_rhomin : ri;
+  const float pe = pc < ph.pgmin ? ph.pgmin : pc;
+  (void)ra;
+  const float cs2 = fmaxf(0.f, ph.gamma * fabsf(pe * rinv));
+  const float s = b2 * rinv + cs2;
+  const float bx2 = (Bx * Bx) * rinv;
+  const float droot = dss(s * s - (4.f * bx2) * cs2);
+  o[C_VX] = vx;
+  o[C_CF] = dss(0.5f * (s + droot));
+  o[C_CA] = dss(bx2);
+  o[C_CS] = dss(0.5f * (s - droot));
+  o[C_VY] = vy;
+  o[C_VZ] = vz;
+  o[C_H] = (u[4] + pe) * rinv;
+}
+
+// Coefficients of the characteristic fields at one interface
+// (_eigen.py:116-337), the projections and the columns taken apart into the
+// combinations that the fast, slow, Alfven and entropy fields share. The
+// degeneracy signs of the reference (multiplying a field's row and column
+// alike) drop out of row, odd WENO function and column together.
 struct EB {
-  float sqrt_rho, rsr, vx, vy, vz, v2, by, bz, bty, btz, sgn_bx, sgn_bt, cs, cs2, cs2inv, cf, csl, af, as, gam0, gam1,
-      gam2;
-  bool cs_ge_ca;
+  float vx, vy, vz, hv2, by, bz, bty, btz, btv;
+  float a1, a2, b1, b2;  // fast / slow weight of W and of T
+  float c1, c2;          // fast (slow) weight of N and slow (fast) weight of S, sign of B_x apart
+  float sgn, al, k3, e0;
+  float af, as, cf, csl, p1, p2, z1, z2, rsr;
 };
 
-__device__ __forceinline__ EB interface_blocks(const float* qa, const float* qb, const Phys& ph) {
-  const Cell a = floored(qa, ph), b = floored(qb, ph);
-  const float Ha = (a.E + a.p) * frcp(a.rho), Hb = (b.E + b.p) * frcp(b.rho);
+__device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
+
+__device__ __forceinline__ EB interface_blocks(const float* A, const float* B, const Phys& ph) {
   EB e;
-  const float rho = 0.5f * (a.rho + b.rho);
-  e.vx = 0.5f * (a.vx + b.vx);
-  e.vy = 0.5f * (a.vy + b.vy);
-  e.vz = 0.5f * (a.vz + b.vz);
-  const float bx = 0.5f * (qa[5] + qb[5]);
-  e.by = 0.5f * (qa[6] + qb[6]);
-  e.bz = 0.5f * (qa[7] + qb[7]);
-  const float H = 0.5f * (Ha + Hb);
-  e.v2 = (e.vx * e.vx + e.vy * e.vy) + e.vz * e.vz;
-  const float bsq = (bx * bx + e.by * e.by) + e.bz * e.bz;
+  const float ra = A[0] < ph.rhomin ? ph.rhomin : A[0], rb = B[0] < ph.rhomin ? ph.rhomin : B[0];
+  const float rho = 0.5f * (ra + rb);
+  e.vx = 0.5f * (A[1] + B[1]);
+  e.vy = 0.5f * (A[2] + B[2]);
+  e.vz = 0.5f * (A[3] + B[3]);
+  const float H = 0.5f * (A[4] + B[4]);
+  const float bx = 0.5f * (A[5] + B[5]);
+  e.by = 0.5f * (A[6] + B[6]);
+  e.bz = 0.5f * (A[7] + B[7]);
+  const float v2 = (e.vx * e.vx + e.vy * e.vy) + e.vz * e.vz;
+  e.hv2 = 0.5f * v2;
+  const float bt2 = e.by * e.by + e.bz * e.bz;
   const float ri = frcp(rho);
-  const float b2r = bsq * ri;
+  const float b2r = (bx * bx + bt2) * ri;
   const float bx2r = (bx * bx) * ri;
-  e.cs2 = ph.gm1 * (H - 0.5f * (e.v2 + b2r));
-  e.cs = dss(fmaxf(0.f, e.cs2));
-  const float s = b2r + e.cs2;
-  const float droot = dss(fmaxf(0.f, s * s - (4.f * bx2r) * e.cs2));
-  e.cf = dss(fmaxf(0.f, 0.5f * (s + droot)));
-  const float ca = dss(fmaxf(0.f, bx2r));
-  e.csl = dss(fmaxf(0.f, 0.5f * (s - droot)));
-  float bt2 = e.by * e.by + e.bz * e.bz;
-  e.sgn_bx = bx >= 0.f ? 1.f : -1.f;
-  bt2 = fmaxf(bt2, 1e-12f);
-  const float rbt = frcp(dss(bt2));
+  const float cs2 = ph.gm1 * (H - 0.5f * (v2 + b2r));
+  const float cs = dss(cs2);
+  const float s = b2r + cs2;
+  const float droot = dss(s * s - (4.f * bx2r) * cs2);
+  const float cf2 = fmaxf(0.5f * (s + droot), 1e-12f), cl2 = fmaxf(0.5f * (s - droot), 1e-12f);
+  e.cf = fsqrt(cf2);
+  e.csl = fsqrt(cl2);
+  e.sgn = bx >= 0.f ? 1.f : -1.f;
+  const float rbt = frsq(fmaxf(bt2, 1e-12f));
   e.bty = e.by * rbt;
   e.btz = e.bz * rbt;
-  const float denom = fmaxf(e.cf * e.cf - e.csl * e.csl, 1e-12f);
-  const float rd = frcp(dss(denom));
-  e.af = dss(fmaxf(0.f, e.cs2 - e.csl * e.csl)) * rd;
-  e.as = dss(fmaxf(0.f, e.cf * e.cf - e.cs2)) * rd;
-  e.sqrt_rho = dss(rho);
-  e.rsr = frcp(e.sqrt_rho);
-  e.gam0 = 1.f - ph.gamma;
-  e.gam1 = 0.5f * ph.gm1;
-  e.gam2 = (ph.gamma - 2.f) * ph.inv_gm1;
-  e.cs2inv = e.cs2 > 0.f ? frcp(e.cs2) : 0.f;
-  e.sgn_bt = e.by != 0.f ? (e.by >= 0.f ? 1.f : -1.f) : (e.bz >= 0.f ? 1.f : -1.f);
-  e.cs_ge_ca = e.cs >= ca;
+  const float rd = frsq(fmaxf(cf2 - cl2, 1e-12f));
+  e.af = dss(cs2 - cl2) * rd;
+  e.as = dss(cf2 - cs2) * rd;
+  const float rc = fmaxf(rho, 1e-12f);
+  e.rsr = frsq(rc);
+  const float sqrt_rho = rc * e.rsr;
+  const float ci = cs2 > 0.f ? frcp(cs2) : 0.f;
+  // rows carry 1/2 of the eigenvectors' normalisation and 1/2 of the flux splitting
+  const float k = 0.25f * ci, g0 = -ph.gm1;
+  const float gk = g0 * k, tk = (cs * sqrt_rho) * k;
+  e.a1 = e.af * gk;
+  e.a2 = e.as * gk;
+  e.b1 = e.as * tk;
+  e.b2 = -(e.af * tk);
+  e.c1 = (e.af * e.cf) * k;
+  e.c2 = (e.as * e.csl) * k;
+  e.al = (0.25f * e.sgn) * sqrt_rho;
+  e.k3 = (-0.5f * g0) * ci;
+  e.e0 = cs2 > 0.f ? 0.5f : 0.f;
+  e.btv = e.bty * e.vy + e.btz * e.vz;
+  const float gam2 = (ph.gamma - 2.f) * ph.inv_gm1;
+  e.p1 = e.af * (cf2 - gam2 * cs2);
+  e.p2 = e.as * (cl2 - gam2 * cs2);
+  const float cr = cs * e.rsr;
+  e.z1 = cr * e.as;
+  e.z2 = cr * e.af;
   return e;
 }
 
-// _eigen_L_row (_eigen.py:625-911): the 7 entries (rows 0,1,2,3,4,6,7 of the
-// conserved vector; the B_x entry is 0)
-template <int S>
-__device__ __forceinline__ void L_row(const EB& e, float* L) {
-  const float btv = e.bty * e.vy + e.btz * e.vz;
-  if (S == 0 || S == 6) {
-    const float sg = S == 0 ? 1.f : -1.f;  // fast -: +cf terms; fast +: -cf terms
-    L[0] = e.af * (e.gam1 * e.v2 + sg * (e.cf * e.vx)) - sg * (((e.as * e.csl) * btv) * e.sgn_bx);
-    L[1] = e.af * (e.gam0 * e.vx - sg * e.cf);
-    L[2] = (e.gam0 * e.af) * e.vy + sg * (((e.as * e.csl) * e.bty) * e.sgn_bx);
-    L[3] = (e.gam0 * e.af) * e.vz + sg * (((e.as * e.csl) * e.btz) * e.sgn_bx);
-    L[6] = (e.gam0 * e.af) * e.by + ((e.cs * e.as) * e.bty) * e.sqrt_rho;
-    L[7] = (e.gam0 * e.af) * e.bz + ((e.cs * e.as) * e.btz) * e.sqrt_rho;
-    L[4] = -e.gam0 * e.af;
-    const float f = e.cs_ge_ca ? 1.f : e.sgn_bt;
-#pragma unroll
-    for (int v = 0; v < 8; ++v) L[v] = ((0.5f * L[v]) * e.cs2inv) * f;
-  } else if (S == 1 || S == 5) {
-    const float sg = S == 1 ? 1.f : -1.f;
-    L[0] = 0.5f * (e.btz * e.vy - e.bty * e.vz);
-    L[1] = 0.f;
-    L[2] = 0.5f * -e.btz;
-    L[3] = 0.5f * e.bty;
-    L[4] = 0.f;
-    L[6] = 0.5f * ((sg * -e.btz * e.sgn_bx) * e.sqrt_rho);
-    L[7] = 0.5f * ((sg * e.bty * e.sgn_bx) * e.sqrt_rho);
-  } else if (S == 2) {
-    L[0] = e.as * (e.gam1 * e.v2 + e.csl * e.vx) + ((e.af * e.cf) * btv) * e.sgn_bx;
-    L[1] = (e.gam0 * e.as) * e.vx - e.as * e.csl;
-    L[2] = (e.gam0 * e.as) * e.vy - ((e.af * e.cf) * e.bty) * e.sgn_bx;
-    L[3] = (e.gam0 * e.as) * e.vz - ((e.af * e.cf) * e.btz) * e.sgn_bx;
-    L[6] = (e.gam0 * e.as) * e.by - ((e.cs * e.af) * e.bty) * e.sqrt_rho;
-    L[7] = (e.gam0 * e.as) * e.bz - ((e.cs * e.af) * e.btz) * e.sqrt_rho;
-    L[4] = -e.gam0 * e.as;
-    const float f = e.cs_ge_ca ? e.sgn_bt : 1.f;
-#pragma unroll
-    for (int v = 0; v < 8; ++v) L[v] = ((0.5f * L[v]) * e.cs2inv) * f;
-  } else if (S == 3) {
-    const float k = (-e.gam0) * e.cs2inv;
-    L[0] = (-e.cs2 * frcp(e.gam0) - 0.5f * e.v2) * k;
-    L[1] = e.vx * k;
-    L[2] = e.vy * k;
-    L[3] = e.vz * k;
-    L[6] = e.by * k;
-    L[7] = e.bz * k;
-    L[4] = -1.f * k;
-  } else {  // S == 4
-    L[0] = e.as * (e.gam1 * e.v2 - e.csl * e.vx) - ((e.af * e.cf) * btv) * e.sgn_bx;
-    L[1] = e.as * (e.gam0 * e.vx + e.csl);
-    L[2] = (e.gam0 * e.as) * e.vy + ((e.af * e.cf) * e.bty) * e.sgn_bx;
-    L[3] = (e.gam0 * e.as) * e.vz + ((e.af * e.cf) * e.btz) * e.sgn_bx;
-    L[6] = (e.gam0 * e.as) * e.by - ((e.cs * e.af) * e.bty) * e.sqrt_rho;
-    L[7] = (e.gam0 * e.as) * e.bz - ((e.cs * e.af) * e.btz) * e.sqrt_rho;
-    L[4] = -e.gam0 * e.as;
-    const float f = e.cs_ge_ca ? e.sgn_bt : 1.f;
-#pragma unroll
-    for (int v = 0; v < 8; ++v) L[v] = ((0.5f * L[v]) * e.cs2inv) * f;
-  }
+// u (rows 0, 1, 2, 3, 4, 6, 7 of the conserved vector) on the 7 characteristic
+// fields, order of _eigen.py: fast-, Alfven-, slow-, entropy, slow+, Alfven+, fast+
+// (_eigen_L_row, _eigen.py:625-911), times 1/2.
+__device__ __forceinline__ void project(const EB& e, const float* u, float* m) {
+  float W = -(e.hv2 * u[0]) - u[4];
+  W = e.vx * u[1] + W;
+  W = e.vy * u[2] + W;
+  W = e.vz * u[3] + W;
+  W = e.by * u[5] + W;
+  W = e.bz * u[6] + W;
+  const float T = e.bty * u[5] + e.btz * u[6];
+  const float A2 = e.bty * u[6] - e.btz * u[5];
+  const float N = e.vx * u[0] - u[1];
+  const float p2 = e.vy * u[0] - u[2], p3 = e.vz * u[0] - u[3];
+  const float S = e.sgn * (e.bty * p2 + e.btz * p3);
+  const float A1 = 0.25f * (e.btz * p2 - e.bty * p3);
+  const float fs = e.a1 * W + e.b1 * T, fa = e.c1 * N - e.c2 * S;
+  const float ss = e.a2 * W + e.b2 * T, sa = e.c2 * N + e.c1 * S;
+  m[0] = fs + fa;
+  m[6] = fs - fa;
+  m[2] = ss + sa;
+  m[4] = ss - sa;
+  m[3] = e.k3 * W + e.e0 * u[0];
+  m[1] = e.al * A2 + A1;
+  m[5] = A1 - e.al * A2;
 }
 
-// _eigen_R_col (_eigen.py:340-622): rows 0,1,2,3,4,6,7 (B_x row is 0)
-template <int S>
-__device__ __forceinline__ void R_col(const EB& e, float* R) {
-  const float btv = e.bty * e.vy + e.btz * e.vz;
-  if (S == 0 || S == 6) {
-    const float sg = S == 0 ? -1.f : 1.f;  // fast -: vx - cf; fast +: vx + cf
-    R[0] = e.af;
-    R[1] = e.af * (e.vx + sg * e.cf);
-    R[2] = e.af * e.vy - sg * (((e.as * e.csl) * e.bty) * e.sgn_bx);
-    R[3] = e.af * e.vz - sg * (((e.as * e.csl) * e.btz) * e.sgn_bx);
-    R[6] = ((e.cs * e.as) * e.bty) * e.rsr;
-    R[7] = ((e.cs * e.as) * e.btz) * e.rsr;
-    R[4] = e.af * (((e.cf * e.cf + sg * (e.cf * e.vx)) + 0.5f * e.v2) - e.gam2 * e.cs2) - sg * (((e.as * e.csl) * btv) * e.sgn_bx);
-    if (!e.cs_ge_ca) {
-#pragma unroll
-      for (int v = 0; v < 8; ++v) R[v] *= e.sgn_bt;
-    }
-  } else if (S == 1 || S == 5) {
-    const float sg = S == 1 ? 1.f : -1.f;
-    R[0] = 0.f;
-    R[1] = 0.f;
-    R[2] = -e.btz;
-    R[3] = e.bty;
-    R[6] = (sg * -e.btz * e.sgn_bx) * e.rsr;
-    R[7] = (sg * e.bty * e.sgn_bx) * e.rsr;
-    R[4] = e.bty * e.vz - e.btz * e.vy;
-  } else if (S == 2 || S == 4) {
-    const float sg = S == 2 ? -1.f : 1.f;
-    R[0] = e.as;
-    R[1] = e.as * (e.vx + sg * e.csl);
-    R[2] = e.as * e.vy + sg * (((e.af * e.cf) * e.bty) * e.sgn_bx);
-    R[3] = e.as * e.vz + sg * (((e.af * e.cf) * e.btz) * e.sgn_bx);
-    R[6] = ((-e.cs * e.af) * e.bty) * e.rsr;
-    R[7] = ((-e.cs * e.af) * e.btz) * e.rsr;
-    R[4] = e.as * (((e.csl * e.csl + sg * (e.csl * e.vx)) + 0.5f * e.v2) - e.gam2 * e.cs2) + sg * (((e.af * e.cf) * btv) * e.sgn_bx);
-    if (e.cs_ge_ca) {
-#pragma unroll
-      for (int v = 0; v < 8; ++v) R[v] *= e.sgn_bt;
-    }
-  } else {  // S == 3
-    R[0] = 1.f;
-    R[1] = e.vx;
-    R[2] = e.vy;
-    R[3] = e.vz;
-    R[4] = 0.5f * e.v2;
-    R[6] = 0.f;
-    R[7] = 0.f;
+// 6 times the WENO interpolant with Jiang-Shu weights (_weno.py:185-205). The
+// indicators are taken over 13 (the weights do not change, the floor of their
+// sum does by 169). SAFE: one reciprocal per weight, for any finite indicator.
+// Otherwise the weights share one reciprocal of their common denominator,
+// whose products hold for indicators up to PHI_MAX; `top` collects the largest
+// indicator, and the caller repeats the interface the SAFE way above it.
+constexpr float PHI_MAX = 1e8f;
+
+template <bool SAFE>
+__device__ __forceinline__ float weno_phi6(float a, float b, float c, float d, float& top) {
+  const float eps = 1e-8f / 13.f, r3 = 3.f / 13.f, lim = 169e-14f;
+  const float x = a - b, y = b - c, z = c - d;
+  const float t0 = x - 2.f * b, t1 = b + c, t2 = 2.f * c + z;
+  const float e0 = x * x + ((r3 * t0) * t0 + eps);
+  const float e1 = y * y + ((r3 * t1) * t1 + eps);
+  const float e2 = z * z + ((r3 * t2) * t2 + eps);
+  float w0, w2;
+  if (SAFE) {
+    const float a0 = frcp(e0 * e0) * (1.f / 169.f), a1 = frcp(e1 * e1) * (6.f / 169.f), a2 = frcp(e2 * e2) * (3.f / 169.f);
+    const float rs = frcp(fmaxf((a0 + a1) + a2, 1e-14f));
+    w0 = a0 * rs;
+    w2 = a2 * rs;
+  } else {
+    top = fmaxf(fmaxf(top, e0), fmaxf(e1, e2));
+    const float s0 = e0 * e0, s1 = e1 * e1, s2 = e2 * e2;
+    const float n0 = s1 * s2, q = 3.f * s0;
+    const float n2 = q * s1, n1 = q * s2;  // n1: half of it
+    const float sum = 2.f * n1 + (n0 + n2);
+    const float r = frcp(fmaxf(sum, (lim * s0) * n0));
+    w0 = n0 * r;
+    w2 = n2 * r;
   }
+  return (2.f * w0) * (x - y) + (w2 - 0.5f) * (y - z);
 }
 
-// WENO interpolant with Jiang-Shu weights (_weno.py:185-205)
-__device__ __forceinline__ float weno_phi(float a, float b, float c, float d) {
-  const float eps = 1e-8f;
-  const float t0 = a - 3.f * b, t2 = 3.f * c - d;
-  const float IS0 = 13.f * ((a - b) * (a - b)) + 3.f * (t0 * t0);
-  const float IS1 = 13.f * ((b - c) * (b - c)) + 3.f * ((b + c) * (b + c));
-  const float IS2 = 13.f * ((c - d) * (c - d)) + 3.f * (t2 * t2);
-  const float e0 = eps + IS0, e1 = eps + IS1, e2 = eps + IS2;
-  const float a0 = frcp(e0 * e0);
-  const float a1 = 6.f * frcp(e1 * e1);
-  const float a2 = 3.f * frcp(e2 * e2);
-  const float rs = frcp(fmaxf((a0 + a1) + a2, 1e-14f));
-  const float w0 = a0 * rs, w2 = a2 * rs;
-  return (w0 * ((a - 2.f * b) + c)) * (1.f / 3.f) + ((w2 - 0.5f) * ((b - 2.f * c) + d)) * (1.f / 6.f);
-}
+struct WenoDir {
+  const float* u[8];  // frame rows of the stage state: density and momenta after the
+                      // floors, E and B after update_cell_center_fields
+  float* F[7];        // interface flux (cell i -> face i+1/2), frame rows 0-4, 6, 7
+  float* mod[2];      // CT modified fluxes of frame rows 6 and 7
+};
 
 struct WenoArgs {
-  const float* q[4];   // rho, m_x, m_y, m_z of the stage state (after floors)
-  const float* qt[4];  // E, B_x, B_y, B_z after update_cell_center_fields
-  float* F[8];         // interface flux along the direction (cell i -> face i+1/2)
-  float* modA;         // CT modified flux of the tangential B component in frame row 6
-  float* modB;         // ... in frame row 7
+  WenoDir d[3];
+  unsigned first[4];  // first block of each direction, and the number of blocks
+  int zin;            // interfaces of a z block
+  unsigned mzp, mz;   // ceil(2^20 / (nz + 5)), ceil(2^20 / nz): quotients below 1024
+  unsigned ntx, nty;  // tiles of TP positions along x and y
   Grid g;
   Phys ph;
 };
 
-// Cells staged per block: direction x / y: (TP + 5) positions x 64 lanes;
-// direction z: TP rows x (64 + 5) positions.
-template <int DIR>
-struct Tile {
-  static constexpr int NCELL = DIR < 2 ? (TP + 5) * TBZ : TP * (TBZ + 5);
-};
+constexpr int NCELL = (TP + 5) * TBZ;  // staged cells of a block
 
-// LDS index of window cell k (0..5 = i-2 .. i+3) of thread (w, l)
-template <int DIR>
-__device__ __forceinline__ int win(int w, int l, int k) {
-  return DIR < 2 ? (w + k) * TBZ + l : w * (TBZ + 5) + l + k;
-}
+__device__ __forceinline__ unsigned small_div(unsigned x, unsigned m) { return (x * m) >> 20; }
 
-// characteristic mode S of the WENO-5 flux at one interface (_weno.py:134-235)
-template <int DIR, int S>
-__device__ __forceinline__ void weno_mode(const EB& e, const float (*sQ)[Tile<DIR>::NCELL],
-                                          const float (*sF)[Tile<DIR>::NCELL], const float (*sS)[Tile<DIR>::NCELL],
-                                          int w, int l, float* out) {
-  float L[8], R[8];
-  L_row<S>(e, L);
-  R_col<S>(e, R);
-  float sk[6], qk[6], amx = 0.f;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    const int c = win<DIR>(w, l, k);
-    float a = 0.f, b = 0.f;
+// The 7 characteristic WENO-5 fluxes of one interface added to the linear part
+// (_weno.py:134-235). s: the staged cells, c: LDS index of cell i-2, ws: index
+// step between window cells. Returns the largest smoothness indicator.
+template <bool SAFE>
+__device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, int ws, const Phys& ph, float* out) {
+  float A[8], B[8];
+  {
+    const int i = c + 2 * ws, j = c + 3 * ws;
+    constexpr int f[8] = {C_Q, C_VX, C_VY, C_VZ, C_H, C_Q + 5, C_Q + 6, C_Q + 7};
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      if (v == 5) continue;
-      a += L[v] * sF[v][c];
-      b += L[v] * sQ[v][c];
+      A[v] = s[f[v]][i];
+      B[v] = s[f[v]][j];
     }
-    sk[k] = a;
-    qk[k] = b;
-    const float vx = sS[0][c];
-    float lam;
-    if (S == 0) lam = vx - sS[1][c];
-    else if (S == 1) lam = vx - sS[2][c];
-    else if (S == 2) lam = vx - sS[3][c];
-    else if (S == 3) lam = vx;
-    else if (S == 4) lam = vx + sS[3][c];
-    else if (S == 5) lam = vx + sS[2][c];
-    else lam = vx + sS[1][c];
-    amx = fmaxf(amx, fabsf(lam));
   }
-  float d[5], dq[5];
+  const EB e = interface_blocks(A, B, ph);
+  float df[5][7], dq[5][7];  // characteristic differences of the flux and of the state
+  {
+    float t[5][7];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    d[k] = sk[k + 1] - sk[k];
-    dq[k] = qk[k + 1] - qk[k];
-  }
-  const float ap = 0.5f * (d[0] + amx * dq[0]), bp = 0.5f * (d[1] + amx * dq[1]);
-  const float cp = 0.5f * (d[2] + amx * dq[2]), dp = 0.5f * (d[3] + amx * dq[3]);
-  const float am = 0.5f * (d[4] - amx * dq[4]), bm = 0.5f * (d[3] - amx * dq[3]);
-  const float cm = 0.5f * (d[2] - amx * dq[2]), dm = 0.5f * (d[1] - amx * dq[1]);
-  const float Fs = -weno_phi(ap, bp, cp, dp) + weno_phi(am, bm, cm, dm);
+    for (int v = 0; v < 7; ++v) {
+      float w[6];
 #pragma unroll
-  for (int v = 0; v < 8; ++v) {
-    if (v == 5) continue;
-    out[v] = out[v] + R[v] * Fs;
+      for (int k = 0; k < 6; ++k) w[k] = s[C_F + v][c + k * ws];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) t[k][v] = w[k + 1] - w[k];
+      out[v] = (1.0f / 12.0f) * (((-w[1] + 7.f * w[2]) + 7.f * w[3]) - w[4]);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) project(e, t[k], df[k]);
+#pragma unroll
+    for (int v = 0; v < 7; ++v) {
+      float w[6];
+      const int row = v < 5 ? v : v + 1;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) w[k] = s[C_Q + row][c + k * ws];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) t[k][v] = w[k + 1] - w[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) project(e, t[k], dq[k]);
   }
+  // largest |eigenvalue| of each field over the window
+  float am[7];
+#pragma unroll
+  for (int m = 0; m < 7; ++m) am[m] = 0.f;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const int i = c + k * ws;
+    const float vx = s[C_VX][i];
+    am[3] = fmaxf(am[3], fabsf(vx));
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const float sp = s[C_CF + m][i];
+      am[m] = fmaxf(am[m], fabsf(vx - sp));
+      am[6 - m] = fmaxf(am[6 - m], fabsf(vx + sp));
+    }
+  }
+  // C_CF, C_CA, C_CS are the speeds of fields (0, 6), (1, 5), (2, 4)
+  float fs[7], top = 0.f;
+#pragma unroll
+  for (int m = 0; m < 7; ++m) {
+    const float x = am[m];
+    const float up = weno_phi6<SAFE>(df[0][m] + x * dq[0][m], df[1][m] + x * dq[1][m], df[2][m] + x * dq[2][m],
+                                     df[3][m] + x * dq[3][m], top);
+    const float dn = weno_phi6<SAFE>(df[4][m] - x * dq[4][m], df[3][m] - x * dq[3][m], df[2][m] - x * dq[2][m],
+                                     df[1][m] - x * dq[1][m], top);
+    fs[m] = (dn - up) * (1.f / 6.f);
+  }
+  // the columns (_eigen_R_col, _eigen.py:340-622) on the shared combinations
+  const float p = fs[0] + fs[6], q = fs[6] - fs[0], ps = fs[2] + fs[4], qs = fs[4] - fs[2];
+  const float pa = fs[1] + fs[5], qa = (fs[1] - fs[5]) * (e.sgn * e.rsr);
+  const float G = (e.af * p + e.as * ps) + fs[3];
+  const float afq = e.af * e.cf, asq = e.as * e.csl;
+  const float X = afq * q + asq * qs;
+  const float Y = e.sgn * (afq * qs - asq * q);
+  const float T2 = e.bty * Y - e.btz * pa, T3 = e.btz * Y + e.bty * pa;
+  const float Z = e.z1 * p - e.z2 * ps;
+  out[0] += G;
+  out[1] += e.vx * G + X;
+  out[2] += e.vy * G + T2;
+  out[3] += e.vz * G + T3;
+  out[4] += (((e.hv2 * G + e.vx * X) + e.vy * T2) + e.vz * T3) + (e.p1 * p + e.p2 * ps);
+  out[5] += e.bty * Z - e.btz * qa;
+  out[6] += e.btz * Z + e.bty * qa;
+  return top;
 }
 
-// Interface fluxes along DIR (_weno_flux_x/_y/_z): one face per thread.
-template <int DIR>
-__global__ __launch_bounds__(NTH) void k_weno(const WenoArgs a) {
-  constexpr int NC = Tile<DIR>::NCELL;
-  __shared__ float sQ[8][NC];
-  __shared__ float sF[8][NC];
-  __shared__ float sS[4][NC];
+// Interface fluxes along the three directions (_weno_flux_x/_y/_z), one
+// interface per thread. A block stages the cells of its window in LDS with
+// their flux, speeds and enthalpy (each thread's own work), then every thread
+// computes one interface from 6 staged cells.
+//   x, y: TP positions along the direction (+ 5 halo cells) times 64 lanes that
+//         run along the flattened plane of the other two axes, so that no lane
+//         is idle whatever nz is;
+//   z:    a range of `zin` interfaces in linear order; each row piece in it is
+//         staged with its own 5 halo cells (wrapped in its row).
+//
+// Bound by VALU issue: about 1300 instructions an interface, 14 WENO functions
+// of 38 among them. What keeps them few: differences of the window are
+// projected rather than its cells (10 vectors, not 12, and the flux's
+// cancellation happens before the products); the rows and columns of the seven
+// fields share their sums (34 operations a vector instead of 45, and no row is
+// ever formed); the three weights of a WENO function share one quarter-rate
+// reciprocal. LDS holds 22 fields of a cell (73 KB a block, two blocks of 8
+// waves on a CU), each read once per interface; 119 VGPRs, 4 waves a SIMD.
+// 256^3, three directions: 3554 -> 1923 us; 101^3: 305 -> 137 us, where 64
+// lanes along z of 101 cells had also left a fifth of the lanes idle; 32^3:
+// 32 -> 12 us, three launches in one.
+__global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_weno(const WenoArgs a) {
+  __shared__ float s[NFIELD][NCELL];
   const Grid g = a.g;
   const Phys ph = a.ph;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int nbz = (g.nz + TBZ - 1) / TBZ;
-  int bid = blockIdx.x;
-  const int bz = bid % nbz;
-  bid /= nbz;
-  int x0, y0;
-  if (DIR == 0) {  // tile: TP x-positions, fixed y
-    y0 = bid % g.ny;
-    x0 = (bid / g.ny) * TP;
-  } else {         // tile: TP y-positions (or rows), fixed x
-    const int nby = (g.ny + TP - 1) / TP;
-    y0 = (bid % nby) * TP;
-    x0 = bid / nby;
-  }
-  const int z0 = bz * TBZ;
-  // stage the cells of the tile (frame of DIR) with their flux and speeds
-  for (int c = tid; c < NC; c += NTH) {
-    int x, y, z;
-    if (DIR == 0) {
-      x = wrapi(x0 - 2 + c / TBZ, g.nx);
-      y = y0;
-      z = wrapi(z0 + c % TBZ, g.nz);
-    } else if (DIR == 1) {
-      x = x0;
-      y = wrapi(y0 - 2 + c / TBZ, g.ny);
-      z = wrapi(z0 + c % TBZ, g.nz);
-    } else {
-      x = x0;
-      y = wrapi(y0 + c / (TBZ + 5), g.ny);
-      z = wrapi(z0 - 2 + c % (TBZ + 5), g.nz);
+  unsigned bid = blockIdx.x;
+  const int dir = bid < a.first[1] ? 0 : (bid < a.first[2] ? 1 : 2);
+  bid -= a.first[dir];
+  const WenoDir& D = a.d[dir];
+  int ws, c0;            // window: LDS index of cell i-2 and the step to the next
+  unsigned gc;           // this thread's interface (its left cell)
+  bool live;
+  if (dir < 2) {
+    const unsigned nt = dir == 0 ? a.ntx : a.nty;
+    const unsigned tile = bid % nt, pb = bid / nt;
+    const unsigned np = dir == 0 ? (unsigned)g.sx : (unsigned)g.nx * (unsigned)g.nz;
+    const int n = dir == 0 ? g.nx : g.ny;
+    const unsigned st = dir == 0 ? (unsigned)g.sx : (unsigned)g.nz;
+    const unsigned pl = pb * TBZ + l, p = pl < np ? pl : np - 1;
+    unsigned base = p;
+    if (dir == 1) {
+      const unsigned x = p / (unsigned)g.nz;
+      base = x * (unsigned)g.sx + (p - x * (unsigned)g.nz);
     }
-    const long gc = cell(g, x, y, z);
-    const float u[8] = {a.q[0][gc], a.q[1][gc], a.q[2][gc], a.q[3][gc], a.qt[0][gc], a.qt[1][gc], a.qt[2][gc], a.qt[3][gc]};
-    float r[8], f[8], sp[4];
+    const int i0 = (int)tile * TP;
+    for (int r = w; r < TP + 5; r += TP) {
+      const unsigned gi = base + (unsigned)wrapi(i0 - 2 + r, n) * st;
+      float u[8], o[NFIELD];
 #pragma unroll
-    for (int v = 0; v < 8; ++v) r[v] = u[perm(DIR, v)];
-    cell_flux(r, f, ph);
-    cell_speeds(r, sp, ph);
+      for (int v = 0; v < 8; ++v) u[v] = D.u[v][gi];
+      stage_cell(u, ph, o);
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      sQ[v][c] = r[v];
-      sF[v][c] = f[v];
+      for (int v = 0; v < NFIELD; ++v) s[v][r * TBZ + l] = o[v];
     }
+    ws = TBZ;
+    c0 = w * TBZ + l;
+    gc = base + (unsigned)(i0 + w) * st;
+    live = pl < np && i0 + w < n;
+  } else {
+    const unsigned nz = (unsigned)g.nz, nc = (unsigned)g.nc, nrow = nc / nz;
+    const unsigned start = bid * (unsigned)a.zin;
+    const unsigned row0 = start / nz, z0 = start - row0 * nz, len0 = nz - z0;
+    const unsigned left = nc - start < (unsigned)a.zin ? nc - start : (unsigned)a.zin;
+    // pieces: the rest of row0, then whole rows, the last one cut
+    const unsigned pieces = left <= len0 ? 1 : 1 + (left - len0 + nz - 1) / nz;
+    const unsigned ncell = left + 5 * pieces;
+    for (unsigned c = tid; c < ncell; c += NTH) {
+      const unsigned c1 = c - (len0 + 5);
+      const unsigned j = c < len0 + 5 ? 0 : 1 + small_div(c1, a.mzp);
+      const unsigned at = j == 0 ? c : c1 - (j - 1) * (nz + 5);
+      const int z = wrapi((int)((j == 0 ? z0 : 0) + at) - 2, (int)nz);
+      const unsigned r = row0 + j < nrow ? row0 + j : nrow - 1;
+      const unsigned gi = r * nz + (unsigned)z;
+      float u[8], o[NFIELD];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sS[v][c] = sp[v];
+      for (int v = 0; v < 8; ++v) u[v] = D.u[v][gi];
+      stage_cell(u, ph, o);
+#pragma unroll
+      for (int v = 0; v < NFIELD; ++v) s[v][c] = o[v];
+    }
+    const unsigned t = (unsigned)tid;
+    const unsigned j = t < len0 ? 0 : 1 + small_div(t - len0, a.mz);
+    ws = 1;
+    c0 = (int)(t + 5 * j);
+    gc = start + t;
+    live = t < left;
   }
   __syncthreads();
-  int xi, yi, zi;
-  if (DIR == 0) {
-    xi = x0 + w;
-    yi = y0;
-  } else {
-    xi = x0;
-    yi = y0 + w;
+  if (!live) return;
+  float out[7];
+  const float top = interface_flux<false>(s, c0, ws, ph, out);
+  if (!(top < PHI_MAX)) {
+    // opaque to the compiler, which otherwise keeps the first pass's 70
+    // projections in registers for this one
+    asm volatile("" : "+v"(c0));
+    interface_flux<true>(s, c0, ws, ph, out);
   }
-  zi = z0 + l;
-  if (xi >= g.nx || yi >= g.ny || zi >= g.nz) return;
-  float qa[8], qb[8];
-  const int c2 = win<DIR>(w, l, 2), c3 = win<DIR>(w, l, 3);
 #pragma unroll
-  for (int v = 0; v < 8; ++v) {
-    qa[v] = sQ[v][c2];
-    qb[v] = sQ[v][c3];
-  }
-  const EB e = interface_blocks(qa, qb, ph);
-  float out[8];
-  {
-    const int c1 = win<DIR>(w, l, 1), c4 = win<DIR>(w, l, 4);
-#pragma unroll
-    for (int v = 0; v < 8; ++v)
-      out[v] = (1.0f / 12.0f) * (((-sF[v][c1] + 7.f * sF[v][c2]) + 7.f * sF[v][c3]) - sF[v][c4]);
-  }
-  weno_mode<DIR, 0>(e, sQ, sF, sS, w, l, out);
-  weno_mode<DIR, 1>(e, sQ, sF, sS, w, l, out);
-  weno_mode<DIR, 2>(e, sQ, sF, sS, w, l, out);
-  weno_mode<DIR, 3>(e, sQ, sF, sS, w, l, out);
-  weno_mode<DIR, 4>(e, sQ, sF, sS, w, l, out);
-  weno_mode<DIR, 5>(e, sQ, sF, sS, w, l, out);
-  weno_mode<DIR, 6>(e, sQ, sF, sS, w, l, out);
-  const long gc = cell(g, xi, yi, zi);
-#pragma unroll
-  for (int v = 0; v < 8; ++v) a.F[perm(DIR, v)][gc] = out[v];
+  for (int v = 0; v < 7; ++v) D.F[v][gc] = out[v];
   // CT modified fluxes: frame rows 6 / 7 plus c2f(B_d) c2f(v_t) (_constrained_transport.py:81-102)
   float bn[4], v2[4], v3[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int c = win<DIR>(w, l, k + 1);
-    const float ri = frcp(sQ[0][c]);
-    bn[k] = sQ[5][c];
-    v2[k] = sQ[2][c] * ri;
-    v3[k] = sQ[3][c] * ri;
+    const int c = c0 + (k + 1) * ws;
+    bn[k] = s[C_Q + 5][c];
+    v2[k] = s[C_VY][c];
+    v3[k] = s[C_VZ][c];
   }
   const float bf = (((-bn[0] + 9.f * bn[1]) + 9.f * bn[2]) - bn[3]) * (1.f / 16.f);
   const float v2f = (((-v2[0] + 9.f * v2[1]) + 9.f * v2[2]) - v2[3]) * (1.f / 16.f);
   const float v3f = (((-v3[0] + 9.f * v3[1]) + 9.f * v3[2]) - v3[3]) * (1.f / 16.f);
-  a.modA[gc] = out[6] + bf * v2f;
-  a.modB[gc] = out[7] + bf * v3f;
+  D.mod[0][gc] = out[5] + bf * v2f;
+  D.mod[1][gc] = out[6] + bf * v3f;
 }
 
 // ---------------------------------------------------------------- stencils
@@ -663,9 +679,7 @@ __global__ void k_face(const FaceArgs a) {
 }
 
 struct QupdArgs {
-  const float* Fx[8];
-  const float* Fy[8];
-  const float* Fz[8];
+  const float* F[3][8];  // interface fluxes of the state's rows (none for the normal field)
   const float* q0[8];
   float* qc[8];
   float* qf[8];
@@ -685,7 +699,10 @@ __global__ void k_qupd(const QupdArgs a) {
     const unsigned xm = nb(g, P, 0, -1), ym = nb(g, P, 1, -1), zm = nb(g, P, 2, -1);
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const float rhs = (-dtdx) * (((a.Fx[v][c] - a.Fx[v][xm]) + (a.Fy[v][c] - a.Fy[v][ym])) + (a.Fz[v][c] - a.Fz[v][zm]));
+      float div = v == 5 ? 0.f : a.F[0][v][c] - a.F[0][v][xm];
+      if (v != 6) div += a.F[1][v][c] - a.F[1][v][ym];
+      if (v != 7) div += a.F[2][v][c] - a.F[2][v][zm];
+      const float rhs = (-dtdx) * div;
       if (a.k.final_stage) {
         a.qf[v][c] = a.qf[v][c] + rhs;
       } else {
@@ -869,7 +886,7 @@ struct amx_fd_ctx {
   float dx, inv_dx;
   float* ws;
   // buffer offsets (fields of nc floats)
-  float *Q0[8], *QC[8], *QF[8], *QT[4], *FX[8], *FY[8], *FZ[8], *MOD[6], *OM[3], *OMB[3], *BC[3], *BF[3];
+  float *Q0[8], *QC[8], *QF[8], *QT[4], *F[3][7], *MOD[6], *OM[3], *OMB[3], *BC[3], *BF[3];
   Ctl* ctl;
   Ctl* hctl;
   int timing;
@@ -885,7 +902,7 @@ struct amx_fd_ctx {
 
 namespace {
 
-constexpr int FD_FIELDS = 8 * 3 + 4 + 8 * 3 + 6 + 3 + 3 + 3 + 3;  // 70
+constexpr int FD_FIELDS = 8 * 3 + 4 + 7 * 3 + 6 + 3 + 3 + 3 + 3;  // 67
 
 amx_status fd_validate(const amx_fd_config* c) {
   if (!c) return amx_fail(AMX_ERR_INVALID, "null config%s");
@@ -935,26 +952,34 @@ void fd_tresolve(amx_fd_ctx* c) {
   c->ev_used = 0;
 }
 
-template <int DIR>
-hipError_t launch_weno(amx_fd_ctx* c, float* const* F, float* modA, float* modB, hipStream_t st) {
+// All three directions in one launch: a small grid's blocks share the chip.
+hipError_t launch_weno(amx_fd_ctx* c, hipStream_t st) {
+  const Grid& g = c->g;
   WenoArgs a;
-  for (int v = 0; v < 4; ++v) {
-    a.q[v] = c->QC[v];
-    a.qt[v] = c->QT[v];
+  for (int d = 0; d < 3; ++d) {
+    for (int v = 0; v < 8; ++v) {
+      const int r = FRAME[d][v];
+      a.d[d].u[v] = r < 4 ? c->QC[r] : c->QT[r - 4];
+    }
+    for (int v = 0; v < 7; ++v) a.d[d].F[v] = c->F[d][v];
+    a.d[d].mod[0] = c->MOD[2 * d];
+    a.d[d].mod[1] = c->MOD[2 * d + 1];
   }
-  for (int v = 0; v < 8; ++v) a.F[v] = F[v];
-  a.modA = modA;
-  a.modB = modB;
-  a.g = c->g;
+  auto up = [](long n, long m) { return (unsigned)((n + m - 1) / m); };
+  a.ntx = up(g.nx, TP);
+  a.nty = up(g.ny, TP);
+  // short rows: fewer interfaces per z block, so that their halo cells fit
+  a.zin = g.nz >= 12 ? NTH : NTH / 2;
+  a.mz = up(1 << 20, g.nz);
+  a.mzp = up(1 << 20, g.nz + 5);
+  a.first[0] = 0;
+  a.first[1] = up(g.sx, TBZ) * a.ntx;
+  a.first[2] = a.first[1] + up((long)g.nx * g.nz, TBZ) * a.nty;
+  a.first[3] = a.first[2] + up(g.nc, a.zin);
+  a.g = g;
   a.ph = c->ph;
-  const int nbz = (c->g.nz + TBZ - 1) / TBZ;
-  long nb;
-  if (DIR == 0)
-    nb = (long)nbz * c->g.ny * ((c->g.nx + TP - 1) / TP);
-  else
-    nb = (long)nbz * c->g.nx * ((c->g.ny + TP - 1) / TP);
   const int e = fd_tbegin(c, st);
-  hipLaunchKernelGGL(k_weno<DIR>, dim3((unsigned)nb), dim3(NTH), 0, st, a);
+  hipLaunchKernelGGL(k_weno, dim3(a.first[3]), dim3(NTH), 0, st, a);
   fd_tend(c, st, e);
   return hipGetLastError();
 }
@@ -1004,9 +1029,7 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     pa.floors = (s < 4) && c->ph.positivity;
     hipLaunchKernelGGL(k_prep, grid, blk, 0, st, pa);
     AMX_HIPCHK(hipGetLastError());
-    AMX_HIPCHK(launch_weno<0>(c, c->FX, c->MOD[0], c->MOD[1], st));
-    AMX_HIPCHK(launch_weno<1>(c, c->FY, c->MOD[2], c->MOD[3], st));
-    AMX_HIPCHK(launch_weno<2>(c, c->FZ, c->MOD[4], c->MOD[5], st));
+    AMX_HIPCHK(launch_weno(c, st));
     EdgeArgs ea;
     ea.fyx = c->MOD[0];
     ea.fzx = c->MOD[1];
@@ -1041,9 +1064,10 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     AMX_HIPCHK(hipGetLastError());
     QupdArgs qa;
     for (int v = 0; v < 8; ++v) {
-      qa.Fx[v] = c->FX[v];
-      qa.Fy[v] = c->FY[v];
-      qa.Fz[v] = c->FZ[v];
+      for (int d = 0; d < 3; ++d) {
+        const int f = FRAME[d][v];  // frame rows 0-4, 6, 7 are stored
+        qa.F[d][v] = f == 5 ? nullptr : c->F[d][f < 5 ? f : f - 1];
+      }
       qa.q0[v] = c->Q0[v];
       qa.qc[v] = c->QC[v];
       qa.qf[v] = c->QF[v];
@@ -1094,6 +1118,7 @@ extern "C" amx_status amx_fd_create(const amx_fd_config* cfg, amx_fd_ctx** out) 
   c->ph.inv_gm1 = 1.0f / c->ph.gm1;
   c->ph.rhomin = cfg->minimum_density;
   c->ph.pgmin = cfg->minimum_pressure;
+  c->ph.inv_rhomin = 1.0f / cfg->minimum_density;
   c->ph.positivity = cfg->enforce_positivity ? 1 : 0;
   c->dx = (float)cfg->grid_spacing;
   c->inv_dx = (float)(1.0 / cfg->grid_spacing);
@@ -1113,9 +1138,7 @@ extern "C" amx_status amx_fd_create(const amx_fd_config* cfg, amx_fd_ctx** out) 
   take(c->QC, 8);
   take(c->QF, 8);
   take(c->QT, 4);
-  take(c->FX, 8);
-  take(c->FY, 8);
-  take(c->FZ, 8);
+  for (int d = 0; d < 3; ++d) take(c->F[d], 7);
   take(c->MOD, 6);
   take(c->OM, 3);
   take(c->OMB, 3);

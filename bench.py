@@ -78,14 +78,14 @@ def cpu_baseline(n: int, steps: int, start=None, first_step: int = 0):
     }
 
 
-# FD (WENO-5 + CT + SSPRK(5,4)), per cell of one k_weno launch: reads
-# rho, m (4) + E, B after the centre update (4), writes the 8 interface fluxes
-# and the 2 CT modified fluxes -> 18 fields = 72 B.
-WENO_BYTES_PER_CELL = 72.0
+# FD (WENO-5 + CT + SSPRK(5,4)), per cell of one k_weno launch (all three
+# directions): each direction reads rho, m (4) + E, B after the centre update
+# (4) and writes 7 interface fluxes and the 2 CT modified fluxes -> 51 fields.
+WENO_BYTES_PER_CELL = 204.0
 # Whole FD step, per cell (fields read + written once per pass):
-#   init R11 W22; per stage: prep R12(+2 floors) W4(+2), 3 x weno 18, ct_edge R6 W3,
-#   ct_avg R3 W3, face R9 W6 (final R6 W3), qupd R48 W16 (final R32 W8); finish R11 W11
-FD_STEP_FIELDS = 33 + 4 * (20 + 54 + 9 + 6 + 15 + 64) + (16 + 54 + 9 + 6 + 9 + 40) + 22
+#   init R11 W22; per stage: prep R12(+2 floors) W4(+2), weno 51, ct_edge R6 W3,
+#   ct_avg R3 W3, face R9 W6 (final R6 W3), qupd R45 W16 (final R29 W8); finish R11 W11
+FD_STEP_FIELDS = 33 + 4 * (20 + 51 + 9 + 6 + 15 + 61) + (16 + 51 + 9 + 6 + 9 + 37) + 22
 
 
 def cpu_baseline_fd(n: int, steps: int):
