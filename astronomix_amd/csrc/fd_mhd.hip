@@ -4,9 +4,7 @@
 //
 // Passes of one right-hand-side evaluation (all direction-specific; the
 // reference's transposes become index arithmetic):
-//   k_prep     positivity floors of the carried stage state and the
-//              face-to-centre B with its energy correction
-//              (_enforce_positivity.py:21-59, _constrained_transport.py:160-198)
+//   k_first    conserved rows of the state as the first stage's input
 //   k_weno     interface fluxes along x, y and z in one launch: the cells of a
 //              tile are staged in LDS with their flux and wave speeds; each
 //              thread builds the interface eigen-system once and runs the 7
@@ -16,8 +14,12 @@
 //   k_ct_edge  edge EMFs by 4th-order interpolation (_constrained_transport.py:107-131)
 //   k_ct_avg   point values to averages (_interpolate.py:38-62)
 //   k_face     6th-order curl of the EMFs + SSPRK combine of the face fields
-//   k_qupd     flux divergence + SSPRK combine of the conserved state
-//              (_ssprk.py:224-228, 300-311)
+//   k_combine  flux divergence + SSPRK combine of the conserved state
+//              (_ssprk.py:224-228, 300-311), then the next stage's input:
+//              positivity floors and the face-to-centre B with its energy
+//              correction (_enforce_positivity.py:21-59,
+//              _constrained_transport.py:160-198); after the last stage the
+//              primitive state
 // Boundaries are periodic.
 
 #include <hip/hip_runtime.h>
@@ -51,17 +53,25 @@ struct Grid {
 
 __device__ __forceinline__ long cell(const Grid& g, int x, int y, int z) { return (long)x * g.sx + (long)y * g.sy + z; }
 
-// Cell index with its coordinates: computed once per cell with 32-bit
-// arithmetic (grids have < 2^30 cells), so that stencil neighbours need no
-// division.
+// Byte offset of a cell in a field, with its coordinates: one division per
+// cell in 32-bit arithmetic (grids have < 2^30 cells), none for its stencil
+// neighbours, and loads with a scalar base and a 32-bit offset.
 struct Pos {
-  unsigned c;
+  unsigned o;
   int x, y, z;
 };
 
+__device__ __forceinline__ float ld(const float* p, unsigned o) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + o);
+}
+
+__device__ __forceinline__ void st(float* p, unsigned o, float v) {
+  *reinterpret_cast<float*>(reinterpret_cast<char*>(p) + o) = v;
+}
+
 __device__ __forceinline__ Pos pos_of(const Grid& g, unsigned c) {
   Pos p;
-  p.c = c;
+  p.o = 4u * c;
   const unsigned t = c / (unsigned)g.nz;
   p.z = (int)(c - t * (unsigned)g.nz);
   p.x = (int)(t / (unsigned)g.ny);
@@ -69,11 +79,13 @@ __device__ __forceinline__ Pos pos_of(const Grid& g, unsigned c) {
   return p;
 }
 
-// neighbour of p along axis by s (periodic)
+// neighbour of p along axis by s (periodic, |s| <= the axis's cells)
 __device__ __forceinline__ unsigned nb(const Grid& g, const Pos& p, int axis, int s) {
-  if (axis == 2) return p.c - p.z + wrapi(p.z + s, g.nz);
-  if (axis == 1) return p.c + (unsigned)((wrapi(p.y + s, g.ny) - p.y) * g.nz);
-  return p.c + (unsigned)((wrapi(p.x + s, g.nx) - p.x)) * (unsigned)g.sx;
+  const int i = axis == 0 ? p.x : (axis == 1 ? p.y : p.z), n = axis == 0 ? g.nx : (axis == 1 ? g.ny : g.nz);
+  const unsigned step = 4u * (axis == 0 ? (unsigned)g.sx : (axis == 1 ? (unsigned)g.sy : 1u));
+  const bool out = s < 0 ? i + s < 0 : i + s >= n;
+  const unsigned in = (unsigned)s * step, wrapped = (unsigned)(s < 0 ? s + n : s - n) * step;
+  return p.o + (out ? wrapped : in);
 }
 
 __device__ __forceinline__ float dss(float x) { return fsqrt(fmaxf(x, 1e-12f)); }
@@ -463,7 +475,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       const unsigned gi = base + (unsigned)wrapi(i0 - 2 + r, n) * st;
       float u[8], o[NFIELD];
 #pragma unroll
-      for (int v = 0; v < 8; ++v) u[v] = D.u[v][gi];
+      for (int v = 0; v < 8; ++v) u[v] = ld(D.u[v], 4u * gi);
       stage_cell(u, ph, o);
 #pragma unroll
       for (int v = 0; v < NFIELD; ++v) s[v][r * TBZ + l] = o[v];
@@ -489,7 +501,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       const unsigned gi = r * nz + (unsigned)z;
       float u[8], o[NFIELD];
 #pragma unroll
-      for (int v = 0; v < 8; ++v) u[v] = D.u[v][gi];
+      for (int v = 0; v < 8; ++v) u[v] = ld(D.u[v], 4u * gi);
       stage_cell(u, ph, o);
 #pragma unroll
       for (int v = 0; v < NFIELD; ++v) s[v][c] = o[v];
@@ -512,7 +524,7 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     interface_flux<true>(s, c0, ws, ph, out);
   }
 #pragma unroll
-  for (int v = 0; v < 7; ++v) D.F[v][gc] = out[v];
+  for (int v = 0; v < 7; ++v) st(D.F[v], 4u * gc, out[v]);
   // CT modified fluxes: frame rows 6 / 7 plus c2f(B_d) c2f(v_t) (_constrained_transport.py:81-102)
   float bn[4], v2[4], v3[4];
 #pragma unroll
@@ -525,74 +537,101 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   const float bf = (((-bn[0] + 9.f * bn[1]) + 9.f * bn[2]) - bn[3]) * (1.f / 16.f);
   const float v2f = (((-v2[0] + 9.f * v2[1]) + 9.f * v2[2]) - v2[3]) * (1.f / 16.f);
   const float v3f = (((-v3[0] + 9.f * v3[1]) + 9.f * v3[2]) - v3[3]) * (1.f / 16.f);
-  D.mod[0][gc] = out[5] + bf * v2f;
-  D.mod[1][gc] = out[6] + bf * v3f;
+  st(D.mod[0], 4u * gc, out[5] + bf * v2f);
+  st(D.mod[1], 4u * gc, out[6] + bf * v3f);
 }
 
 // ---------------------------------------------------------------- stencils
 __device__ __forceinline__ float c2f(const Grid& g, const float* a, const Pos& p, int ax) {
-  return (((-a[nb(g, p, ax, -1)] + 9.f * a[p.c]) + 9.f * a[nb(g, p, ax, 1)]) - a[nb(g, p, ax, 2)]) * (1.f / 16.f);
+  return (((-ld(a, nb(g, p, ax, -1)) + 9.f * ld(a, p.o)) + 9.f * ld(a, nb(g, p, ax, 1))) - ld(a, nb(g, p, ax, 2))) * (1.f / 16.f);
 }
 
 __device__ __forceinline__ float f2c(const Grid& g, const float* f, const Pos& p, int ax) {
-  return (((((3.f * f[nb(g, p, ax, -3)] - 25.f * f[nb(g, p, ax, -2)]) + 150.f * f[nb(g, p, ax, -1)]) + 150.f * f[p.c]) -
-           25.f * f[nb(g, p, ax, 1)]) +
-          3.f * f[nb(g, p, ax, 2)]) *
+  return (((((3.f * ld(f, nb(g, p, ax, -3)) - 25.f * ld(f, nb(g, p, ax, -2))) + 150.f * ld(f, nb(g, p, ax, -1))) + 150.f * ld(f, p.o)) -
+           25.f * ld(f, nb(g, p, ax, 1))) +
+          3.f * ld(f, nb(g, p, ax, 2))) *
          (1.f / 256.f);
 }
 
 __device__ __forceinline__ float d6(const Grid& g, const float* f, const Pos& p, int ax) {
   const float c1 = 75.f / 64.f, c2 = -25.f / 384.f, c3 = 3.f / 640.f;
-  return (c1 * (f[p.c] - f[nb(g, p, ax, -1)]) + c2 * (f[nb(g, p, ax, 1)] - f[nb(g, p, ax, -2)])) +
-         c3 * (f[nb(g, p, ax, 2)] - f[nb(g, p, ax, -3)]);
+  return (c1 * (ld(f, p.o) - ld(f, nb(g, p, ax, -1))) + c2 * (ld(f, nb(g, p, ax, 1)) - ld(f, nb(g, p, ax, -2)))) +
+         c3 * (ld(f, nb(g, p, ax, 2)) - ld(f, nb(g, p, ax, -3)));
 }
 
 __device__ __forceinline__ float p2a(const Grid& g, const float* q, const Pos& p, int A, int B) {
-  const float sa = ((q[nb(g, p, A, -1)] - 2.f * q[p.c]) + q[nb(g, p, A, 1)]) * (1.f / 24.f);
-  const float sb = ((q[nb(g, p, B, -1)] - 2.f * q[p.c]) + q[nb(g, p, B, 1)]) * (1.f / 24.f);
-  return (q[p.c] + sa) + sb;
+  const float sa = ((ld(q, nb(g, p, A, -1)) - 2.f * ld(q, p.o)) + ld(q, nb(g, p, A, 1))) * (1.f / 24.f);
+  const float sb = ((ld(q, nb(g, p, B, -1)) - 2.f * ld(q, p.o)) + ld(q, nb(g, p, B, 1))) * (1.f / 24.f);
+  return (ld(q, p.o) + sa) + sb;
 }
 
 #define FD_LOOP(g)                                                                     \
   for (unsigned c = blockIdx.x * blockDim.x + threadIdx.x; c < (unsigned)(g).nc; \
        c += gridDim.x * blockDim.x)
 
-// _enforce_positivity on the stage state (in place, optional) and
-// update_cell_center_fields into qt = (E, B_x, B_y, B_z)
-struct PrepArgs {
-  float* q[8];
-  const float* b[3];
+// Conserved rows of a primitive state (_equations.py:65-101).
+__device__ __forceinline__ void conserved(const float* const* w, unsigned o, const Phys& ph, float* q) {
+  const float rho = ld(w[0], o);
+  const float vx = ld(w[1], o), vy = ld(w[2], o), vz = ld(w[3], o);
+  const float Bx = ld(w[5], o), By = ld(w[6], o), Bz = ld(w[7], o);
+  const float u2 = (vx * vx + vy * vy) + vz * vz;
+  const float b2 = (Bx * Bx + By * By) + Bz * Bz;
+  q[0] = rho;
+  q[1] = rho * vx;
+  q[2] = rho * vy;
+  q[3] = rho * vz;
+  q[4] = (ld(w[4], o) * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2;
+  q[5] = Bx;
+  q[6] = By;
+  q[7] = Bz;
+}
+
+// _enforce_positivity of conserved rows with the field energy b2/2 (_enforce_positivity.py:21-59)
+__device__ __forceinline__ void floor_state(float& rho, float& E, const float* m, float b2, const Phys& ph) {
+  rho = fmaxf(rho, ph.rhomin);
+  const float ri = frcp(rho);
+  const float vx = m[0] * ri, vy = m[1] * ri, vz = m[2] * ri;
+  const float v2 = (vx * vx + vy * vy) + vz * vz;
+  const float p = fmaxf(ph.gm1 * ((E - (0.5f * rho) * v2) - 0.5f * b2), ph.pgmin);
+  E = (p * ph.inv_gm1 + (0.5f * rho) * v2) + 0.5f * b2;
+}
+
+// cell-centred B of the faces (update_cell_center_fields)
+__device__ __forceinline__ void centre_field(const Grid& g, const float* const* b, const Pos& P, float* B) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) B[i] = f2c(g, b[i], P, i);
+}
+
+// The first stage's input: the primitive state (11 rows) as conserved rows with
+// the floors, and update_cell_center_fields into qt = (E, B_x, B_y, B_z).
+// Only what k_weno reads is written: the stage combines take q0 and b0 from the
+// state itself, which stays as it is until the last of them. Bound by memory
+// (R11 W8): with the copies of q0 in three buffers and a pass of its own for
+// the floors it moved 49 fields.
+struct FirstArgs {
+  const float* w[11];
+  float* q[4];
   float* qt[4];
   Grid g;
   Phys ph;
-  int floors;
 };
 
-__global__ void k_prep(const PrepArgs a) {
+__global__ void k_first(const FirstArgs a) {
   const Grid g = a.g;
   const Phys ph = a.ph;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    (void)P;
-    float rho = a.q[0][c], E = a.q[4][c];
-    const float Bx = a.q[5][c], By = a.q[6][c], Bz = a.q[7][c];
-    const float b2 = (Bx * Bx + By * By) + Bz * Bz;
-    if (a.floors) {
-      rho = fmaxf(rho, ph.rhomin);
-      const float ri = frcp(rho);
-      const float vx = a.q[1][c] * ri, vy = a.q[2][c] * ri, vz = a.q[3][c] * ri;
-      const float v2 = (vx * vx + vy * vy) + vz * vz;
-      const float p = fmaxf(ph.gm1 * ((E - (0.5f * rho) * v2) - 0.5f * b2), ph.pgmin);
-      E = (p * ph.inv_gm1 + (0.5f * rho) * v2) + 0.5f * b2;
-      a.q[0][c] = rho;
-      a.q[4][c] = E;
-    }
-    const float X = f2c(g, a.b[0], P, 0), Y = f2c(g, a.b[1], P, 1), Z = f2c(g, a.b[2], P, 2);
-    const float nb2 = (X * X + Y * Y) + Z * Z;
-    a.qt[0][c] = E + 0.5f * (nb2 - b2);
-    a.qt[1][c] = X;
-    a.qt[2][c] = Y;
-    a.qt[3][c] = Z;
+    float q[8], B[3];
+    conserved(a.w, P.o, ph, q);
+    const float b2 = (q[5] * q[5] + q[6] * q[6]) + q[7] * q[7];
+    if (ph.positivity) floor_state(q[0], q[4], q + 1, b2, ph);
+    centre_field(g, a.w + 8, P, B);
+    const float nb2 = (B[0] * B[0] + B[1] * B[1]) + B[2] * B[2];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) st(a.q[v], P.o, q[v]);
+    st(a.qt[0], P.o, q[4] + 0.5f * (nb2 - b2));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) st(a.qt[1 + i], P.o, B[i]);
   }
 }
 
@@ -612,10 +651,9 @@ __global__ void k_ct_edge(const EdgeArgs a) {
   const Grid g = a.g;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    (void)P;
-    a.O[2][c] = c2f(g, a.fxy, P, 0) - c2f(g, a.fyx, P, 1);
-    a.O[0][c] = c2f(g, a.fyz, P, 1) - c2f(g, a.fzy, P, 2);
-    a.O[1][c] = c2f(g, a.fzx, P, 2) - c2f(g, a.fxz, P, 0);
+    st(a.O[2], P.o, c2f(g, a.fxy, P, 0) - c2f(g, a.fyx, P, 1));
+    st(a.O[0], P.o, c2f(g, a.fyz, P, 1) - c2f(g, a.fzy, P, 2));
+    st(a.O[1], P.o, c2f(g, a.fzx, P, 2) - c2f(g, a.fxz, P, 0));
   }
 }
 
@@ -629,18 +667,21 @@ __global__ void k_ct_avg(const AvgArgs a) {
   const Grid g = a.g;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    (void)P;
-    a.Ob[2][c] = p2a(g, a.O[2], P, 0, 1);
-    a.Ob[0][c] = p2a(g, a.O[0], P, 1, 2);
-    a.Ob[1][c] = p2a(g, a.O[1], P, 0, 2);
+    st(a.Ob[2], P.o, p2a(g, a.O[2], P, 0, 1));
+    st(a.Ob[0], P.o, p2a(g, a.O[0], P, 1, 2));
+    st(a.Ob[1], P.o, p2a(g, a.O[1], P, 0, 2));
   }
 }
 
 // SSPRK(5,4) coefficients (_ssprk.py:247-272)
 struct Coef {
   float k1, k2, k3, ff;  // q0 weight, dt weight, current weight, final-state weight
-  int final_stage;
 };
+
+// What a stage reads and writes of the carried buffers: the first stage has
+// k3 = ff = 0; the second is the first to accumulate into the final state
+// (seeded with ff0 q0, _ssprk.py:321-324); the last adds to it only.
+enum { ST_FIRST = 0, ST_SECOND = 1, ST_MID = 2, ST_LAST = 3 };
 
 struct FaceArgs {
   const float* Ob[3];
@@ -648,164 +689,130 @@ struct FaceArgs {
   float* bc[3];
   float* bf[3];
   const float* dtp;
-  float inv_dx;
+  float inv_dx, ff0;
   Coef k;
   Grid g;
 };
 
 // 6th-order curl of the averaged EMFs and the stage combine of the faces
+template <int ST>
 __global__ void k_face(const FaceArgs a) {
   const Grid g = a.g;
   const float dtdx = (a.k.k2 * (*a.dtp)) * a.inv_dx;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    (void)P;
     const float r[3] = {(-dtdx) * d6(g, a.Ob[2], P, 1) + dtdx * d6(g, a.Ob[1], P, 2),
                         (-dtdx) * d6(g, a.Ob[0], P, 2) + dtdx * d6(g, a.Ob[2], P, 0),
                         (-dtdx) * d6(g, a.Ob[1], P, 0) + dtdx * d6(g, a.Ob[0], P, 1)};
+    // every load before the first store, which the compiler may not move them past
+    float bn[3], bf[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      if (a.k.final_stage) {
-        a.bf[i][c] = a.bf[i][c] + r[i];
-      } else {
-        // a zero weight skips its buffer (the first stage: k3 = ff = 0)
-        const float bn = a.k.k3 != 0.f ? (a.k.k1 * a.b0[i][c] + a.k.k3 * a.bc[i][c]) + r[i]
-                                       : __fmul_rn(a.k.k1, a.b0[i][c]) + r[i];
-        a.bc[i][c] = bn;
-        if (a.k.ff != 0.f) a.bf[i][c] = a.bf[i][c] + bn * a.k.ff;
+      bf[i] = ST >= ST_MID ? ld(a.bf[i], P.o) : 0.f;
+      if (ST == ST_LAST) {
+        bf[i] = bf[i] + r[i];
+        continue;
       }
+      const float b0 = ld(a.b0[i], P.o);
+      bn[i] = ST == ST_FIRST ? __fmul_rn(a.k.k1, b0) + r[i] : (a.k.k1 * b0 + a.k.k3 * ld(a.bc[i], P.o)) + r[i];
+      if (ST == ST_SECOND) bf[i] = __fmul_rn(a.ff0, b0);
+      bf[i] = bf[i] + bn[i] * a.k.ff;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      if (ST != ST_LAST) st(a.bc[i], P.o, bn[i]);
+      if (ST != ST_FIRST) st(a.bf[i], P.o, bf[i]);
     }
   }
 }
 
-struct QupdArgs {
+struct CombineArgs {
   const float* F[3][8];  // interface fluxes of the state's rows (none for the normal field)
-  const float* q0[8];
+  float* w[11];          // the state at the step's start; the last stage writes it
   float* qc[8];
   float* qf[8];
+  const float* b[3];     // the stage's new faces
+  float* qt[4];
   const float* dtp;
-  float inv_dx;
+  float inv_dx, ff0;
+  int floors;            // of the next stage's input
   Coef k;
   Grid g;
+  Phys ph;
 };
 
-// flux divergence (_ssprk.py:224-228) and the stage combine (_ssprk.py:300-311)
-__global__ void k_qupd(const QupdArgs a) {
+// Flux divergence (_ssprk.py:224-228), the stage combine (_ssprk.py:300-311) and
+// the next stage's input in one pass: floors and update_cell_center_fields; after
+// the last stage the final field update, floors (_ssprk.py:336-347) and the
+// conserved -> primitive map with the faces appended (_evolve_state.py:63-71).
+// Bound by memory: R21 fluxes + 3 faces + 8 to 24 carried rows, W12 to 20 (last
+// stage R32 W11). As a pass of its own each, the combine, the floors with the
+// field update, the start and the end of a step moved 461 fields a step instead
+// of 302.
+template <int ST>
+__global__ void k_combine(const CombineArgs a) {
   const Grid g = a.g;
+  const Phys ph = a.ph;
   const float dtdx = (a.k.k2 * (*a.dtp)) * a.inv_dx;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    (void)P;
     const unsigned xm = nb(g, P, 0, -1), ym = nb(g, P, 1, -1), zm = nb(g, P, 2, -1);
+    // every load before the first store, which the compiler may not move them past
+    float q0[8], q[8], qf[8], B[3];
+    if (ST != ST_LAST) conserved(a.w, P.o, ph, q0);
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      float div = v == 5 ? 0.f : a.F[0][v][c] - a.F[0][v][xm];
-      if (v != 6) div += a.F[1][v][c] - a.F[1][v][ym];
-      if (v != 7) div += a.F[2][v][c] - a.F[2][v][zm];
+      float div = v == 5 ? 0.f : ld(a.F[0][v], P.o) - ld(a.F[0][v], xm);
+      if (v != 6) div += ld(a.F[1][v], P.o) - ld(a.F[1][v], ym);
+      if (v != 7) div += ld(a.F[2][v], P.o) - ld(a.F[2][v], zm);
       const float rhs = (-dtdx) * div;
-      if (a.k.final_stage) {
-        a.qf[v][c] = a.qf[v][c] + rhs;
-      } else {
-        // a zero weight skips its buffer (the first stage: k3 = ff = 0)
-        const float qn = a.k.k3 != 0.f ? (a.k.k1 * a.q0[v][c] + a.k.k3 * a.qc[v][c]) + rhs
-                                       : __fmul_rn(a.k.k1, a.q0[v][c]) + rhs;
-        a.qc[v][c] = qn;
-        if (a.k.ff != 0.f) a.qf[v][c] = a.qf[v][c] + qn * a.k.ff;
+      qf[v] = ST >= ST_MID ? ld(a.qf[v], P.o) : 0.f;
+      if (ST == ST_LAST) {
+        q[v] = qf[v] + rhs;
+        continue;
+      }
+      q[v] = ST == ST_FIRST ? __fmul_rn(a.k.k1, q0[v]) + rhs : (a.k.k1 * q0[v] + a.k.k3 * ld(a.qc[v], P.o)) + rhs;
+      if (ST == ST_SECOND) qf[v] = __fmul_rn(a.ff0, q0[v]);
+      qf[v] = qf[v] + q[v] * a.k.ff;
+    }
+    centre_field(g, a.b, P, B);
+    const float ob2 = (q[5] * q[5] + q[6] * q[6]) + q[7] * q[7];
+    const float nb2 = (B[0] * B[0] + B[1] * B[1]) + B[2] * B[2];
+    if (ST != ST_LAST) {
+      if (a.floors) floor_state(q[0], q[4], q + 1, ob2, ph);
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        st(a.qc[v], P.o, q[v]);
+        if (ST != ST_FIRST) st(a.qf[v], P.o, qf[v]);
+      }
+      st(a.qt[0], P.o, q[4] + 0.5f * (nb2 - ob2));
+#pragma unroll
+      for (int i = 0; i < 3; ++i) st(a.qt[1 + i], P.o, B[i]);
+    } else {
+      float rho = q[0], E = q[4] + 0.5f * (nb2 - ob2);
+      if (ph.positivity) floor_state(rho, E, q + 1, nb2, ph);
+      const float ri = frcp(rho);
+      const float ux = q[1] * ri, uy = q[2] * ri, uz = q[3] * ri;
+      const float u2 = (ux * ux + uy * uy) + uz * uz;
+      float p = ph.gm1 * ((E - (0.5f * rho) * u2) - 0.5f * nb2);
+      if (ph.positivity) {
+        rho = fmaxf(rho, ph.rhomin);
+        p = fmaxf(p, ph.pgmin);
+      }
+      float bf[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) bf[i] = ld(a.b[i], P.o);
+      st(a.w[0], P.o, rho);
+      st(a.w[1], P.o, ux);
+      st(a.w[2], P.o, uy);
+      st(a.w[3], P.o, uz);
+      st(a.w[4], P.o, p);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        st(a.w[5 + i], P.o, B[i]);
+        st(a.w[8 + i], P.o, bf[i]);
       }
     }
-  }
-}
-
-// primitive (11 rows) -> conserved stage buffers (_equations.py:65-101) and
-// the SSPRK accumulators seeded with ff0 * (q0, b0) (_ssprk.py:321-324)
-struct InitArgs {
-  const float* w[11];
-  float* q0[8];
-  float* qc[8];
-  float* qf[8];
-  float* bc[3];
-  float* bf[3];
-  float ff0;
-  Grid g;
-  Phys ph;
-};
-
-__global__ void k_init(const InitArgs a) {
-  const Grid g = a.g;
-  const Phys ph = a.ph;
-  FD_LOOP(g) {
-    const Pos P = pos_of(g, c);
-    (void)P;
-    const float rho = a.w[0][c];
-    const float vx = a.w[1][c], vy = a.w[2][c], vz = a.w[3][c];
-    const float Bx = a.w[5][c], By = a.w[6][c], Bz = a.w[7][c];
-    const float u2 = (vx * vx + vy * vy) + vz * vz;
-    const float b2 = (Bx * Bx + By * By) + Bz * Bz;
-    const float q[8] = {rho, rho * vx, rho * vy, rho * vz, (a.w[4][c] * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2, Bx, By, Bz};
-#pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      a.q0[v][c] = q[v];
-      a.qc[v][c] = q[v];
-      a.qf[v][c] = a.ff0 * q[v];
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const float b = a.w[8 + i][c];
-      a.bc[i][c] = b;
-      a.bf[i][c] = a.ff0 * b;
-    }
-  }
-}
-
-// final update_cell_center_fields + positivity (_ssprk.py:336-347), then
-// conserved -> primitive with floors and the faces appended (_evolve_state.py:63-71)
-struct FinishArgs {
-  const float* qf[8];
-  const float* bf[3];
-  float* w[11];
-  Grid g;
-  Phys ph;
-};
-
-__global__ void k_finish(const FinishArgs a) {
-  const Grid g = a.g;
-  const Phys ph = a.ph;
-  FD_LOOP(g) {
-    const Pos P = pos_of(g, c);
-    (void)P;
-    float rho = a.qf[0][c], E = a.qf[4][c];
-    const float m[3] = {a.qf[1][c], a.qf[2][c], a.qf[3][c]};
-    const float ob2 = (a.qf[5][c] * a.qf[5][c] + a.qf[6][c] * a.qf[6][c]) + a.qf[7][c] * a.qf[7][c];
-    const float X = f2c(g, a.bf[0], P, 0), Y = f2c(g, a.bf[1], P, 1), Z = f2c(g, a.bf[2], P, 2);
-    const float b2 = (X * X + Y * Y) + Z * Z;
-    E = E + 0.5f * (b2 - ob2);
-    if (ph.positivity) {
-      rho = fmaxf(rho, ph.rhomin);
-      const float ri = frcp(rho);
-      const float v2 = ((m[0] * ri) * (m[0] * ri) + (m[1] * ri) * (m[1] * ri)) + (m[2] * ri) * (m[2] * ri);
-      const float p = fmaxf(ph.gm1 * ((E - (0.5f * rho) * v2) - 0.5f * b2), ph.pgmin);
-      E = (p * ph.inv_gm1 + (0.5f * rho) * v2) + 0.5f * b2;
-    }
-    const float ri = frcp(rho);
-    const float ux = m[0] * ri, uy = m[1] * ri, uz = m[2] * ri;
-    const float u2 = (ux * ux + uy * uy) + uz * uz;
-    float p = ph.gm1 * ((E - (0.5f * rho) * u2) - 0.5f * b2);
-    float r = rho;
-    if (ph.positivity) {
-      r = fmaxf(r, ph.rhomin);
-      p = fmaxf(p, ph.pgmin);
-    }
-    a.w[0][c] = r;
-    a.w[1][c] = ux;
-    a.w[2][c] = uy;
-    a.w[3][c] = uz;
-    a.w[4][c] = p;
-    a.w[5][c] = X;
-    a.w[6][c] = Y;
-    a.w[7][c] = Z;
-    a.w[8][c] = a.bf[0][c];
-    a.w[9][c] = a.bf[1][c];
-    a.w[10][c] = a.bf[2][c];
   }
 }
 
@@ -886,7 +893,7 @@ struct amx_fd_ctx {
   float dx, inv_dx;
   float* ws;
   // buffer offsets (fields of nc floats)
-  float *Q0[8], *QC[8], *QF[8], *QT[4], *F[3][7], *MOD[6], *OM[3], *OMB[3], *BC[3], *BF[3];
+  float *QC[8], *QF[8], *QT[4], *F[3][7], *MOD[6], *OM[3], *OMB[3], *BC[3], *BF[3];
   Ctl* ctl;
   Ctl* hctl;
   int timing;
@@ -902,7 +909,7 @@ struct amx_fd_ctx {
 
 namespace {
 
-constexpr int FD_FIELDS = 8 * 3 + 4 + 7 * 3 + 6 + 3 + 3 + 3 + 3;  // 67
+constexpr int FD_FIELDS = 8 * 2 + 4 + 7 * 3 + 6 + 3 + 3 + 3 + 3;  // 59
 
 amx_status fd_validate(const amx_fd_config* c) {
   if (!c) return amx_fail(AMX_ERR_INVALID, "null config%s");
@@ -996,21 +1003,15 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
   float* w[11];
   for (int v = 0; v < 11; ++v) w[v] = state + (long)v * nc;
   const dim3 grid = fd_grid(c), blk(256);
-  InitArgs ia;
+  FirstArgs ia;
   for (int v = 0; v < 11; ++v) ia.w[v] = w[v];
-  for (int v = 0; v < 8; ++v) {
-    ia.q0[v] = c->Q0[v];
-    ia.qc[v] = c->QC[v];
-    ia.qf[v] = c->QF[v];
+  for (int v = 0; v < 4; ++v) {
+    ia.q[v] = c->QC[v];
+    ia.qt[v] = c->QT[v];
   }
-  for (int i = 0; i < 3; ++i) {
-    ia.bc[i] = c->BC[i];
-    ia.bf[i] = c->BF[i];
-  }
-  ia.ff0 = FF[0];
   ia.g = c->g;
   ia.ph = c->ph;
-  hipLaunchKernelGGL(k_init, grid, blk, 0, st, ia);
+  hipLaunchKernelGGL(k_first, grid, blk, 0, st, ia);
   AMX_HIPCHK(hipGetLastError());
   const float* dtp = &c->ctl->dt;
   for (int s = 0; s < 5; ++s) {
@@ -1019,16 +1020,6 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     k.k2 = K2[s];
     k.k3 = K3[s];
     k.ff = s < 4 ? FF[s + 1] : 0.f;
-    k.final_stage = s == 4;
-    PrepArgs pa;
-    for (int v = 0; v < 8; ++v) pa.q[v] = c->QC[v];
-    for (int i = 0; i < 3; ++i) pa.b[i] = c->BC[i];
-    for (int v = 0; v < 4; ++v) pa.qt[v] = c->QT[v];
-    pa.g = c->g;
-    pa.ph = c->ph;
-    pa.floors = (s < 4) && c->ph.positivity;
-    hipLaunchKernelGGL(k_prep, grid, blk, 0, st, pa);
-    AMX_HIPCHK(hipGetLastError());
     AMX_HIPCHK(launch_weno(c, st));
     EdgeArgs ea;
     ea.fyx = c->MOD[0];
@@ -1058,35 +1049,37 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     }
     fa.dtp = dtp;
     fa.inv_dx = c->inv_dx;
+    fa.ff0 = FF[0];
     fa.k = k;
     fa.g = c->g;
-    hipLaunchKernelGGL(k_face, grid, blk, 0, st, fa);
-    AMX_HIPCHK(hipGetLastError());
-    QupdArgs qa;
+    CombineArgs qa;
     for (int v = 0; v < 8; ++v) {
       for (int d = 0; d < 3; ++d) {
         const int f = FRAME[d][v];  // frame rows 0-4, 6, 7 are stored
         qa.F[d][v] = f == 5 ? nullptr : c->F[d][f < 5 ? f : f - 1];
       }
-      qa.q0[v] = c->Q0[v];
       qa.qc[v] = c->QC[v];
       qa.qf[v] = c->QF[v];
     }
+    for (int v = 0; v < 11; ++v) qa.w[v] = w[v];
+    for (int v = 0; v < 4; ++v) qa.qt[v] = c->QT[v];
+    for (int i = 0; i < 3; ++i) qa.b[i] = s == 4 ? c->BF[i] : c->BC[i];
     qa.dtp = dtp;
     qa.inv_dx = c->inv_dx;
+    qa.ff0 = FF[0];
+    qa.floors = s + 1 < 4 && c->ph.positivity;  // the last stage's input has none (_ssprk.py:333-335)
     qa.k = k;
     qa.g = c->g;
-    hipLaunchKernelGGL(k_qupd, grid, blk, 0, st, qa);
+    qa.ph = c->ph;
+    const int kind = s == 0 ? ST_FIRST : (s == 1 ? ST_SECOND : (s < 4 ? ST_MID : ST_LAST));
+    static void (*const face[])(FaceArgs) = {k_face<ST_FIRST>, k_face<ST_SECOND>, k_face<ST_MID>, k_face<ST_LAST>};
+    static void (*const combine[])(CombineArgs) = {k_combine<ST_FIRST>, k_combine<ST_SECOND>, k_combine<ST_MID>,
+                                                   k_combine<ST_LAST>};
+    hipLaunchKernelGGL(face[kind], grid, blk, 0, st, fa);
+    AMX_HIPCHK(hipGetLastError());
+    hipLaunchKernelGGL(combine[kind], grid, blk, 0, st, qa);
     AMX_HIPCHK(hipGetLastError());
   }
-  FinishArgs fa;
-  for (int v = 0; v < 8; ++v) fa.qf[v] = c->QF[v];
-  for (int i = 0; i < 3; ++i) fa.bf[i] = c->BF[i];
-  for (int v = 0; v < 11; ++v) fa.w[v] = w[v];
-  fa.g = c->g;
-  fa.ph = c->ph;
-  hipLaunchKernelGGL(k_finish, grid, blk, 0, st, fa);
-  AMX_HIPCHK(hipGetLastError());
   return AMX_OK;
 }
 
@@ -1134,7 +1127,6 @@ extern "C" amx_status amx_fd_create(const amx_fd_config* cfg, amx_fd_ctx** out) 
       p += nc;
     }
   };
-  take(c->Q0, 8);
   take(c->QC, 8);
   take(c->QF, 8);
   take(c->QT, 4);
@@ -1186,14 +1178,12 @@ __global__ void k_cfl(const CflArgs a) {
   const Phys ph = a.ph;
   float mx[3] = {0.f, 0.f, 0.f};
   FD_LOOP(g) {
-    const Pos P = pos_of(g, c);
-    (void)P;
-    const float rho = a.w[0][c];
-    const float vx = a.w[1][c], vy = a.w[2][c], vz = a.w[3][c];
-    const float Bx = a.w[5][c], By = a.w[6][c], Bz = a.w[7][c];
+    const float rho = ld(a.w[0], 4u * c);
+    const float vx = ld(a.w[1], 4u * c), vy = ld(a.w[2], 4u * c), vz = ld(a.w[3], 4u * c);
+    const float Bx = ld(a.w[5], 4u * c), By = ld(a.w[6], 4u * c), Bz = ld(a.w[7], 4u * c);
     const float u2 = (vx * vx + vy * vy) + vz * vz;
     const float b2 = (Bx * Bx + By * By) + Bz * Bz;
-    const float u[8] = {rho, rho * vx, rho * vy, rho * vz, (a.w[4][c] * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2, Bx, By, Bz};
+    const float u[8] = {rho, rho * vx, rho * vy, rho * vz, (ld(a.w[4], 4u * c) * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2, Bx, By, Bz};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       float r[8], sp[4];
@@ -1410,13 +1400,20 @@ struct C2fArgs {
   Grid g;
 };
 
+// Cell indices here, not byte offsets: this entry point takes grids of 2^30
+// cells and more, whose byte offsets do not fit in 32 bits.
 __global__ void k_interface_fields(const C2fArgs a) {
   const Grid g = a.g;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    (void)P;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) a.b[d][c] = c2f(g, a.B[d], P, d);
+    for (int d = 0; d < 3; ++d) {
+      const float* B = a.B[d];
+      const int i = d == 0 ? P.x : (d == 1 ? P.y : P.z), n = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
+      const unsigned sd = d == 0 ? (unsigned)g.sx : (d == 1 ? (unsigned)g.sy : 1u);
+      auto at = [&](int s) { return B[c + (unsigned)(wrapi(i + s, n) - i) * sd]; };
+      a.b[d][c] = (((-at(-1) + 9.f * B[c]) + 9.f * at(1)) - at(2)) * (1.f / 16.f);
+    }
   }
 }
 

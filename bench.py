@@ -82,10 +82,11 @@ def cpu_baseline(n: int, steps: int, start=None, first_step: int = 0):
 # directions): each direction reads rho, m (4) + E, B after the centre update
 # (4) and writes 7 interface fluxes and the 2 CT modified fluxes -> 51 fields.
 WENO_BYTES_PER_CELL = 204.0
-# Whole FD step, per cell (fields read + written once per pass):
-#   init R11 W22; per stage: prep R12(+2 floors) W4(+2), weno 51, ct_edge R6 W3,
-#   ct_avg R3 W3, face R9 W6 (final R6 W3), qupd R45 W16 (final R29 W8); finish R11 W11
-FD_STEP_FIELDS = 33 + 4 * (20 + 51 + 9 + 6 + 15 + 61) + (16 + 51 + 9 + 6 + 9 + 37) + 22
+# Whole FD step, per cell (fields read + written once per pass): first R11 W8;
+#   per stage: weno 51, ct_edge R6 W3, ct_avg R3 W3; face R6 W3, R9 W6, 2 x R12 W6,
+#   R6 W3; combine (21 fluxes, 3 faces and the carried rows) R32 W12, R40 W20,
+#   2 x R48 W20, R32 W11
+FD_STEP_FIELDS = 19 + 5 * (51 + 9 + 6) + (9 + 15 + 2 * 18 + 9) + (44 + 60 + 2 * 68 + 43)
 
 
 def cpu_baseline_fd(n: int, steps: int):
