@@ -2190,23 +2190,38 @@ void free_ctx(amx_fv_ctx* c) {
   delete c;
 }
 
-// Planes per block of the 3D pair kernel along x. A block loads its chunk plus
-// the 4 planes that the two iterates' x stencils reach past it, and one block
-// fills a CU, so a launch runs in rounds of (CU count) blocks. The pick is the
-// chunk length (>= 8 planes) whose in-order list schedule of `blocks_per_chunk`
-// x chunks blocks onto the CUs, a block costing its loaded planes, ends
-// first; past 16 rounds the tail is ignored. At 256^3 on 256 CUs this is 32
-// planes: 768 blocks, three full rounds (0.435 ms per launch against 0.468 ms
-// for 16-plane chunks in six rounds, 0.52 ms for 64-plane chunks in two).
-int pick_mag_chunk(long blocks_per_chunk, int nx) {
+int device_cus() {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  if (nx <= 8) return nx;
+  return cus;
+}
+
+// Planes per block of the 3D pair kernel along x. A block loads its chunk plus
+// the 4 planes that the two iterates' x stencils reach past it, and one block
+// fills a CU, so a launch runs in rounds of (CU count) blocks. The pick is the
+// chunk length whose in-order list schedule of `blocks_per_chunk` x chunks
+// blocks onto the CUs, a block costing its loaded planes, ends first; past 16
+// rounds the tail is ignored. At 256^3 on 256 CUs this is 32 planes: 768
+// blocks, three full rounds (0.435 ms per launch against 0.468 ms for 16-plane
+// chunks in six rounds, 0.52 ms for 64-plane chunks in two). Grids of few
+// tiles need short chunks to reach every CU: at 32^3, 1 plane 15.5 us against
+// 30.1 at 8; 64^3, 2 planes 17.9 against 30.2; 80^3, 5 planes 24.2 against 30.4.
+int pick_mag_chunk(long blocks_per_chunk, int nx) {
+  int cus = device_cus();
   if (cus > 1024) cus = 1024;
-  int best = 8, prev = -1;
+  int best = nx, prev = -1;
   double best_t = 0.0;
+  // short chunks: full rounds of equal blocks
+  for (int lx = 1; lx < 8 && lx <= nx; ++lx) {
+    const long blocks = blocks_per_chunk * ((nx + lx - 1) / lx);
+    const double t = (double)((blocks + cus - 1) / cus) * (lx + 4.0);
+    if (best_t == 0.0 || t < best_t) {
+      best_t = t;
+      best = lx;
+    }
+  }
   double fin_buf[1024];  // the CUs' finish times (no heap use: the allocation-free entry point calls this)
   double* const fin = fin_buf;
   for (int want = 1; want <= (nx + 7) / 8; ++want) {
@@ -2231,6 +2246,30 @@ int pick_mag_chunk(long blocks_per_chunk, int nx) {
       }
       t = *std::max_element(fin, fin + cus);
     }
+    if (best_t == 0.0 || t < best_t) {
+      best_t = t;
+      best = lx;
+    }
+  }
+  return best;
+}
+
+// Planes per block of the 3D stage kernels along x, for grids that make fewer
+// blocks than fill the chip several times over. Two blocks share a CU and are
+// VALU-bound there: measured, a block spends 1.65 us a plane alone and 2.55 us
+// beside another, 3 planes of it for its chunk's start. The pick is the chunk
+// whose rounds of (2 x CUs) blocks end first. Per launch, mean of the four
+// stages, against chunks of 8: 32^3 9.5 / 21.1 us (1 plane), 64^3 14.4 / 21.8
+// (3), 96^3 25.8 / 30.4 (6), 128^3 42.0 / 46.3 (10), 144^3 66.1 / 74.9 (18);
+// within 3 % of the best chunk of a sweep over 1-32 at 13 grids of 24^3-192^3.
+int pick_stage_chunk(long tiles, int nx) {
+  const long cus = device_cus();
+  int best = nx;
+  double best_t = 0.0;
+  for (int lx = 1; lx <= nx && lx <= 32; ++lx) {
+    const long blocks = tiles * ((nx + lx - 1) / lx);
+    const long rounds = blocks / (2 * cus), rest = blocks % (2 * cus);
+    const double t = (lx + 3.0) * (2.55 * rounds + (rest > cus ? 2.55 : (rest > 0 ? 1.65 : 0.0)));
     if (best_t == 0.0 || t < best_t) {
       best_t = t;
       best = lx;
@@ -2271,21 +2310,21 @@ void init_geometry(amx_fv_ctx* c, const amx_fv_config* cfg, int cap, int own_sta
   c->nta_mag = (c->na + TA_MAG - 1) / TA_MAG;
   c->ntb_mag = (c->nb + TB_MAG - 1) / TB_MAG;
   if (cfg->dim == 3) {
-    // planes per block along x for the stage kernels: about `blocks` blocks,
-    // the chunk the multiple of 4 planes (the kernels' x-march unroll) nearest
-    // to that, at least 8 (the kernels reload 4 planes at each chunk start, so
-    // longer chunks save traffic). Measured at 256^3 (148 tiles): 20 planes
-    // 1.718 ms per step, 16: 1.753, 24 and 30: 1.73, 28: 1.80, 36: 1.85.
-    auto pick = [&](long tiles, const char* env, long blocks) {
-      int lx = env_int(env, 0);
-      if (lx <= 0) {
-        const long target = (tiles * cfg->nx + blocks / 2) / blocks;
-        lx = (int)(((target + 2) / 4) * 4);
-        if (lx < 8) lx = 8;
-      }
-      return lx > cfg->nx ? cfg->nx : lx;
-    };
-    c->lx = pick((long)c->ntb * c->nta, "AMX_LX", 1900);
+    // planes per block along x for the stage kernels: about 1900 blocks, the
+    // chunk the multiple of 4 planes (the kernels' x-march unroll) nearest to
+    // that (the kernels reload 4 planes at each chunk start, so longer chunks
+    // save traffic). Measured at 256^3 (148 tiles): 20 planes 1.718 ms per
+    // step, 16: 1.753, 24 and 30: 1.73, 28: 1.80, 36: 1.85. Grids whose chunk
+    // would be 8 planes or less (up to about 190^3) are short of blocks
+    // instead: pick_stage_chunk.
+    const long tiles = (long)c->ntb * c->nta;
+    c->lx = env_int("AMX_LX", 0);
+    if (c->lx <= 0) {
+      const long target = (tiles * cfg->nx + 950) / 1900;
+      c->lx = (int)(((target + 2) / 4) * 4);
+      if (c->lx <= 8) c->lx = pick_stage_chunk(tiles, cfg->nx);
+    }
+    if (c->lx > cfg->nx) c->lx = cfg->nx;
     c->lx_mag = env_int("AMX_LX_MAG", 0);
     // one simulation's blocks: pools run partly filled as often as full
     if (c->lx_mag <= 0) c->lx_mag = pick_mag_chunk((long)c->ntb_mag * c->nta_mag, cfg->nx);
