@@ -832,6 +832,7 @@ struct StepParams {
   float tp = 0.f;
 };
 
+// One wavefront, a lane per partial slot; the scalars are the same in every lane.
 // dt = min(C dx / (lx + ly + lz), dt_max) (_timestep_estimator.py(FD):89-90),
 // or t_end / num_timesteps; clamp to t_end - t (time_integration.py:667-678)
 __global__ void k_step_begin(Ctl* c, StepParams p) {
@@ -855,8 +856,7 @@ __global__ void k_step_begin(Ctl* c, StepParams p) {
     dt = rem < dt ? rem : dt;
   }
   c->dt = dt;
-  for (int d = 0; d < 3; ++d)
-    for (int i = 0; i < NSLOT; ++i) c->cflp[d][i] = 0u;
+  for (int d = 0; d < 3; ++d) c->cflp[d][threadIdx.x] = 0u;
 }
 
 __global__ void k_set_dt(Ctl* c, const float* dtp) { c->dt = *dtp; }
@@ -870,8 +870,7 @@ __global__ void k_reset(Ctl* c) {
   c->dt = 0.f;
   c->t = 0.f;
   c->steps = 0;
-  for (int d = 0; d < 3; ++d)
-    for (int i = 0; i < NSLOT; ++i) c->cflp[d][i] = 0u;
+  for (int d = 0; d < 3; ++d) c->cflp[d][threadIdx.x] = 0u;
 }
 
 __global__ void k_dt_out(const Ctl* c, float* out) { *out = c->dt; }
@@ -1142,7 +1141,7 @@ extern "C" amx_status amx_fd_create(const amx_fd_config* cfg, amx_fd_ctx** out) 
     delete c;
     return amx_fail(AMX_ERR_NOMEM, "control allocation failed%s");
   }
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(1), 0, 0, c->ctl);
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(NSLOT), 0, 0, c->ctl);
   if (hipDeviceSynchronize() != hipSuccess) return amx_fail(AMX_ERR_HIP, "init sync failed%s");
   *out = c;
   return AMX_OK;
@@ -1238,10 +1237,10 @@ StepParams fd_params(const amx_fd_ctx* c, const amx_fv_run* run, int use_cfl) {
 extern "C" amx_status amx_fd_cfl_dt(amx_fd_ctx* c, const float* state, float* d_dt, void* stream) {
   if (!c || !state || !d_dt) return amx_fail(AMX_ERR_INVALID, "null argument%s");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(1), 0, st, c->ctl);
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl);
   AMX_HIPCHK(hipGetLastError());
   AMX_HIPCHK(fd_cfl(c, state, st));
-  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, st, c->ctl, fd_params(c, nullptr, 1));
+  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, fd_params(c, nullptr, 1));
   hipLaunchKernelGGL(k_dt_out, dim3(1), dim3(1), 0, st, (const Ctl*)c->ctl, d_dt);
   AMX_HIPCHK(hipGetLastError());
   return AMX_OK;
@@ -1281,7 +1280,7 @@ amx_diag_desc fd_diag_desc(const amx_fd_ctx* c, double box_size) {
 // snapshot rows of time_integration.py:539-610, 736-745 when snp is given.
 amx_status fd_loop(amx_fd_ctx* c, float* state, const amx_fv_run* run, amx::snap::Driver* snp, amx_fv_stats* stats,
                    hipStream_t st) {
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(1), 0, st, c->ctl);
+  hipLaunchKernelGGL(k_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl);
   AMX_HIPCHK(hipGetLastError());
   StepParams sp = fd_params(c, run, 1);
   // the end-time clamp is off with snapshot time points (time_integration.py:677)
@@ -1302,7 +1301,7 @@ amx_status fd_loop(amx_fd_ctx* c, float* state, const amx_fv_run* run, amx::snap
       if (sp.clamp_tp) sp.tp = snp->clamp_target();
     }
     if (!run->fixed_timestep) AMX_HIPCHK(fd_cfl(c, state, st));
-    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, st, c->ctl, sp);
+    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
     AMX_HIPCHK(hipGetLastError());
     if (c->hook && c->hook(c->hook_user, state, &c->ctl->dt, steps, st) != 0)
       return amx_fail(AMX_ERR_INVALID, "the step hook stopped the run%s");

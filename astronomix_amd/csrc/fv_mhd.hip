@@ -1659,7 +1659,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   }
 }
 
-// Final launch index of the fixed point of each running slot (one thread per
+// Final launch index of the fixed point of each running slot (one wavefront per
 // slot) from its last executed pair, recorded in ctl->iters: the stage
 // kernels after the sub-step read the iterate of that launch. spec: the call
 // is queued before the host has seen the residuals; if the reference's loop
@@ -1767,7 +1767,7 @@ struct StepParams {
 __device__ __forceinline__ void cfl_reduce(Ctl* c, int dim) {
   for (int k = 0; k < dim; ++k) {
     c->cfl[k] = slots_max(c->cflp[k]);
-    for (int i = 0; i < NSLOT; ++i) c->cflp[k][i] = 0u;
+    c->cflp[k][threadIdx.x] = 0u;
   }
 }
 
@@ -1778,17 +1778,19 @@ __device__ __forceinline__ float cfl_dt_from(const Ctl* c, float C, float dx, in
 }
 
 __device__ __forceinline__ void fixed_point_reset(Ctl* c) {
-  for (int i = 0; i < NSLOT; ++i) c->resp[0][i] = c->resp[1][i] = 0u;
+  c->resp[0][threadIdx.x] = c->resp[1][threadIdx.x] = 0u;
   c->iters = 0;
   c->done = 0;
 }
 
 __device__ __forceinline__ void zero_cflp(Ctl* c) {
-  for (int k = 0; k < 3; ++k)
-    for (int i = 0; i < NSLOT; ++i) c->cflp[k][i] = 0u;
+  for (int k = 0; k < 3; ++k) c->cflp[k][threadIdx.x] = 0u;
 }
 
-// One thread per slot (slot = blockIdx.x): the step's dt, and whether the
+// The control kernels: one wavefront per simulation (slot = blockIdx.x), a lane
+// per partial slot; the scalars are the same in every lane, which all write them.
+//
+// The step's dt, and whether the
 // slot runs this step (live and not yet at t_end / num_timesteps).
 __device__ void step_begin(Ctl* c, const StepParams& p) {
   if (p.batch_first) {
@@ -1905,10 +1907,8 @@ __global__ void k_slot_reset(Ctl* ctl, int slot0, float t_end, int live, int fre
   c->t = 0.f;
   c->steps = 0;
   for (int i = 0; i < 4; ++i) c->cfl[i] = 0u;
-  for (int k = 0; k < 3; ++k)
-    for (int i = 0; i < NSLOT; ++i) c->cflp[k][i] = 0u;
-  for (int k = 0; k < NRES; ++k)
-    for (int i = 0; i < NSLOT; ++i) c->resp[k][i] = 0u;
+  zero_cflp(c);
+  for (int k = 0; k < NRES; ++k) c->resp[k][threadIdx.x] = 0u;
   c->iters = 0;
   c->done = 0;
   c->live = live;
@@ -2383,7 +2383,7 @@ amx_status make_ctx(const amx_fv_config* cfg, int cap, int own_state, amx_fv_ctx
     return fail(AMX_ERR_HIP, "parameter upload failed%s");
   }
   // single simulation: slot 0 is live from the start; pool slots start empty
-  hipLaunchKernelGGL(k_slot_reset, dim3(cap), dim3(1), 0, 0, c->ctl, 0, 0.f, own_state ? 0 : 1, 1);
+  hipLaunchKernelGGL(k_slot_reset, dim3(cap), dim3(NSLOT), 0, 0, c->ctl, 0, 0.f, own_state ? 0 : 1, 1);
   if (hipDeviceSynchronize() != hipSuccess) {
     free_ctx(c);
     return fail(AMX_ERR_HIP, "init sync failed%s");
@@ -2756,7 +2756,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   // the final iterate, where it is the first of a pair that did not store it
   const int rq = c->skip_mask && (regen || !spec);
   if (rq) HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
-  hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(1), 0, st, c->ctl, c->cfg.fixed_point_tol,
+  hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(NSLOT), 0, st, c->ctl, c->cfg.fixed_point_tol,
                      c->cfg.max_fixed_point_iterations, spec, c->skip_mask, rq);
   HIPCHK(hipGetLastError());
   StageArgs b1 = stage_base(c, 0.5f);
@@ -2902,10 +2902,10 @@ extern "C" amx_status amx_fv_cfl_dt(amx_fv_ctx* c, const float* state, float* d_
   if (!c || !state || !d_dt) return fail(AMX_ERR_INVALID, "null argument%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_zero_cfl, dim3(1), dim3(1), 0, st, c->ctl);
+  hipLaunchKernelGGL(k_zero_cfl, dim3(1), dim3(NSLOT), 0, st, c->ctl);
   HIPCHK(hipGetLastError());
   HIPCHK(launch_cfl(c, state, 0, 1, st));
-  hipLaunchKernelGGL(k_cfl_out, dim3(1), dim3(1), 0, st, c->ctl, c->cfg.C_cfl, c->dx, c->cfg.dim, d_dt);
+  hipLaunchKernelGGL(k_cfl_out, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->cfg.C_cfl, c->dx, c->cfg.dim, d_dt);
   HIPCHK(hipGetLastError());
   return AMX_OK;
 }
@@ -2915,7 +2915,7 @@ extern "C" amx_status amx_fv_evolve_state(amx_fv_ctx* c, float* state, const flo
   if (!c || !state || !d_dt) return fail(AMX_ERR_INVALID, "null argument%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, st, c->ctl, d_dt);
+  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(NSLOT), 0, st, c->ctl, d_dt);
   HIPCHK(hipGetLastError());
   int K = 0;
   amx_status s = do_step(c, state, st, 0, &K);
@@ -3034,7 +3034,7 @@ extern "C" amx_status amx_fv_evolve_state_noalloc(const amx_fv_config* cfg, floa
   Ctl hctl;
   c.hctl = &hctl;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_noalloc_begin, dim3(1), dim3(1), 0, st, c.ctl, c.dph,
+  hipLaunchKernelGGL(k_noalloc_begin, dim3(1), dim3(NSLOT), 0, st, c.ctl, c.dph,
                      make_phys(cfg->gamma, cfg->grid_spacing), d_dt);
   HIPCHK(hipGetLastError());
   const Bufs b = bufs(&c, state);
@@ -3100,7 +3100,7 @@ hipError_t copy_b_home(amx_fv_ctx* c, const Bufs& bl, hipStream_t st, int gate) 
 // snapshot driver, rows are taken as in time_integration.py:539-610, 736-745.
 amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Driver* snp, amx_fv_stats* stats,
                    hipStream_t st) {
-  hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(1), 0, st, c->ctl, 0, run->t_end, 1, 0);
+  hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, run->t_end, 1, 0);
   HIPCHK(hipGetLastError());
   // Without snapshot rows or a step hook nothing reads the state's B rows
   // between steps: the final B of each step stays in its iterate set (the
@@ -3149,16 +3149,16 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       long n = BATCH;
       if (run->max_steps >= 0 && run->max_steps - steps < n) n = run->max_steps - steps;
       if (run->fixed_timestep && run->num_timesteps - steps < n) n = run->num_timesteps - steps;
-      hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, st, c->ctl, sp);
+      hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
       HIPCHK(hipGetLastError());
       for (long i = 0; i < n; ++i) {
         amx_status s = do_step(c, state, st, !run->fixed_timestep, nullptr);
         if (s != AMX_OK) return s;
         // this step's end and the next one's beginning
         if (i + 1 < n)
-          hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(1), 0, st, c->ctl, 0, sp);
+          hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, sp);
         else
-          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, st, c->ctl, 0);
+          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0);
         HIPCHK(hipGetLastError());
       }
       HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cflp), hipMemcpyDeviceToHost, st));
@@ -3178,7 +3178,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       int klast = 0;
       StepParams spi = sp;
       spi.batch_first = 1;
-      hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, st, c->ctl, spi);
+      hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, spi);
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
       for (long i = 0; i < n; ++i) {
@@ -3188,9 +3188,9 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
         if (s != AMX_OK) return s;
         // this step's end and the next one's beginning
         if (i + 1 < n)
-          hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(1), 0, st, c->ctl, c->keep_b, spi);
+          hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b, spi);
         else
-          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, st, c->ctl, c->keep_b);
+          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
         HIPCHK(hipGetLastError());
       }
       // the loop's last batch: B goes home behind it, unless a step stalled
@@ -3215,7 +3215,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
         fixed_point_settled(c, 1, &K);
         s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 0);
         if (s != AMX_OK) return s;
-        hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, st, c->ctl, c->keep_b);
+        hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cfl), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
@@ -3234,14 +3234,14 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       sp.clamp_tp = snp->clamp();
       if (sp.clamp_tp) sp.tp = snp->clamp_target();
     }
-    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(1), 0, st, c->ctl, sp);
+    hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
     HIPCHK(hipGetLastError());
     if (c->hook && c->hook(c->hook_user, state, &c->ctl[0].dt, steps, st) != 0)
       return fail(AMX_ERR_INVALID, "the step hook stopped the run%s");
     int K = 0;
     amx_status s = do_step(c, state, st, !run->fixed_timestep, &K);
     if (s != AMX_OK) return s;
-    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, st, c->ctl, c->keep_b);
+    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
     HIPCHK(hipGetLastError());
     if (!c->cfg.mhd) {
       // hydro steps have no fixed-point readback: read dt here
@@ -3577,7 +3577,7 @@ extern "C" amx_status amx_fv_adjoint_step(amx_fv_ctx* c, const float* state, con
     }
   }
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, st, c->ctl, d_dt);
+  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(NSLOT), 0, st, c->ctl, d_dt);
   HIPCHK(hipGetLastError());
   if (c->cfg.mhd)
     return dim == 3 ? adjoint_step_mhd<3>(c, state, lam_out, lam_in, st) : adjoint_step_mhd<2>(c, state, lam_out, lam_in, st);
@@ -3684,7 +3684,7 @@ extern "C" amx_status amx_fv_pool_load(amx_fv_pool* p, int slot, const float* st
   HIPCHK(hipStreamSynchronize(st));  // the pinned parameter mirror is rewritten below
   c->hph[slot] = make_phys(gamma, c->cfg.grid_spacing);
   HIPCHK(hipMemcpyAsync(c->dph + slot, c->hph + slot, sizeof(Phys), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(1), 0, st, c->ctl, slot, t_end, 1, 1);
+  hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl, slot, t_end, 1, 1);
   HIPCHK(hipGetLastError());
   if (!c->sp.fixed) HIPCHK(launch_cfl(c, c->mem, slot, 1, st));
   c->live[slot] = 1;
@@ -3695,7 +3695,7 @@ extern "C" amx_status amx_fv_pool_load(amx_fv_pool* p, int slot, const float* st
 extern "C" amx_status amx_fv_pool_release(amx_fv_pool* p, int slot, void* stream) {
   amx_status s = pool_slot_check(p, slot);
   if (s != AMX_OK) return s;
-  hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(1), 0, (hipStream_t)stream, p->c->ctl, slot, 0.f, 0, 1);
+  hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(NSLOT), 0, (hipStream_t)stream, p->c->ctl, slot, 0.f, 0, 1);
   HIPCHK(hipGetLastError());
   p->c->live[slot] = 0;
   p->c->fresh[slot] = 0;
@@ -3763,7 +3763,7 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
     amx_status bs = replay_or_capture(c, st, &bx, bx != nullptr, [&]() -> amx_status {
       StepParams spi = c->sp;
       spi.batch_first = 1;
-      hipLaunchKernelGGL(k_step_begin, dim3(span), dim3(1), 0, st, c->ctl, spi);
+      hipLaunchKernelGGL(k_step_begin, dim3(span), dim3(NSLOT), 0, st, c->ctl, spi);
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
       for (int i = 0; i < nb; ++i) {
@@ -3774,9 +3774,9 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
         if (r != AMX_OK) return r;
         // this step's end and the next one's beginning
         if (i + 1 < nb)
-          hipLaunchKernelGGL(k_step_end_begin, dim3(span), dim3(1), 0, st, c->ctl, c->keep_b, spi);
+          hipLaunchKernelGGL(k_step_end_begin, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b, spi);
         else
-          hipLaunchKernelGGL(k_step_end, dim3(span), dim3(1), 0, st, c->ctl, c->keep_b);
+          hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
         HIPCHK(hipGetLastError());
       }
       return AMX_OK;
@@ -3794,7 +3794,7 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
   auto it = c->g_launch.find(key);
   hipGraphExec_t x = it == c->g_launch.end() ? nullptr : it->second;
   amx_status s = replay_or_capture(c, st, &x, x != nullptr, [&]() -> amx_status {
-    hipLaunchKernelGGL(k_step_begin, dim3(span), dim3(1), 0, st, c->ctl, c->sp);
+    hipLaunchKernelGGL(k_step_begin, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->sp);
     HIPCHK(hipGetLastError());
     int kl = 0;
     return step_phase1(c, b, span, st, !c->sp.fixed, &kl);
@@ -3838,7 +3838,7 @@ extern "C" amx_status amx_fv_pool_step_finish(amx_fv_pool* p, void* stream) {
       bmax = km > bmax ? km : bmax;
       s = step_phase3(c, b, span, st, !c->sp.fixed, 0);
       if (s != AMX_OK) return s;
-      hipLaunchKernelGGL(k_step_end, dim3(span), dim3(1), 0, st, c->ctl, c->keep_b);
+      hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
       HIPCHK(hipGetLastError());
     }
     if (c->cfg.mhd && bmax > 0) c->last_k = bmax;
@@ -3860,7 +3860,7 @@ extern "C" amx_status amx_fv_pool_step_finish(amx_fv_pool* p, void* stream) {
   amx_status s = replay_or_capture(c, st, &x, x != nullptr, [&]() -> amx_status {
     amx_status r = step_phase3(c, b, span, st, !c->sp.fixed, 0);
     if (r != AMX_OK) return r;
-    hipLaunchKernelGGL(k_step_end, dim3(span), dim3(1), 0, st, c->ctl, c->keep_b);
+    hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
     HIPCHK(hipGetLastError());
     return AMX_OK;
   });
