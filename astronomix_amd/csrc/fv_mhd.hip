@@ -126,11 +126,22 @@ __device__ __forceinline__ float half_slope(float wm, float w0, float wp) {
 // Limiter ids (simulation_config.py:29-34 values).
 enum { LIM_MINMOD = 0, LIM_OSHER = 1, LIM_DOUBLE_MINMOD = 2, LIM_SUPERBEE = 3, LIM_VAN_ALBADA = 4, LIM_VAN_ALBADA_PP = 5 };
 
+// Scale of the gradients the other limiters work on.
+struct GradScale {
+  float inv_dx, half_dx, eps;  // 1 / dx, dx / 2, van Albada's 3 dx
+};
+
+__device__ __forceinline__ GradScale grad_scale(float dx) { return {1.f / dx, 0.5f * dx, 3.f * dx}; }
+
 // The other limiters of _calculate_limited_gradients (limited_gradients.py:49-88,
 // limiters.py:18-64) on the backward / forward gradients b, f, chosen by a
 // block-uniform id; the result is (g dx) / 2 as the reconstruction applies it.
-__device__ __forceinline__ float half_slope_x(float wm, float w0, float wp, int lim, float dx) {
-  const float b = (w0 - wm) / dx, f = (wp - w0) / dx;
+// The gradients take the reciprocal of dx, and the one quotient of a slope that
+// depends on data the hardware reciprocal: three IEEE divisions a slope, of
+// about ten instructions each, made the limiter cost more than the Riemann
+// solver.
+__device__ __forceinline__ float half_slope_x(float wm, float w0, float wp, int lim, const GradScale& gs) {
+  const float b = (w0 - wm) * gs.inv_dx, f = (wp - w0) * gs.inv_dx;
   float g;
   if (lim == LIM_SUPERBEE) {
     // where(a b > 0, minmod(maxmod(a, b), minmod(2a, 2b)), 0): for a, b of one
@@ -139,24 +150,31 @@ __device__ __forceinline__ float half_slope_x(float wm, float w0, float wp, int 
     g = b * f > 0.f ? copysignf(fminf(fmaxf(aa, ab), 2.f * fminf(aa, ab)), b) : 0.f;
   } else if (lim == LIM_DOUBLE_MINMOD) {
     // where(a b > 0, minmod3((a + b) / 2, 2a, 2b), 0)
-    const float m = (b + f) / 2.f;
+    const float m = 0.5f * (b + f);
     g = b * f > 0.f ? copysignf(fminf(fabsf(m), fminf(fabsf(2.f * b), fabsf(2.f * f))), m) : 0.f;
   } else if (lim == LIM_VAN_ALBADA) {
     // ((f^2 + eps) b + (b^2 + eps) f) / (f^2 + b^2 + 2 eps), eps = 3 dx
-    const float eps = 3.f * dx, eps2 = 6.f * dx;
-    g = ((f * f + eps) * b + (b * b + eps) * f) / ((f * f + b * b) + eps2);
+    const float f2 = f * f, b2 = b * b;
+    g = ((f2 + gs.eps) * b + (b2 + gs.eps) * f) * frcp((f2 + b2) + 2.f * gs.eps);
   } else {  // LIM_OSHER: b max(0, min(1.3, f / (b + 1e-11))) where |b| > 1e-11
-    const float r = fabsf(b) > 1e-11f ? f / (b + 1e-11f) : 0.f;
+    const float r = fabsf(b) > 1e-11f ? f * frcp(b + 1e-11f) : 0.f;
     g = fmaxf(0.f, fminf(1.3f, r)) * b;
   }
-  return (g * dx) / 2.f;
+  return g * gs.half_dx;
 }
 
+// Limiter forms the stage kernels are instantiated with: minmod; van Albada; any
+// other by its run-time id, and van Albada with the plane factors of
+// VAN_ALBADA_PP. Van Albada has a form of its own because the code of the four
+// limiters side by side in every slope, 65 KB of it in 3D, outgrows the
+// instruction cache, and without the factors' LDS it takes the lagged update.
+enum { LX_MINMOD = 0, LX_VAN_ALBADA = 1, LX_ANY = 2 };
+
 // Limited half slope: minmod in its exact difference form, or another limiter.
-template <bool LIMX>
-__device__ __forceinline__ float slope(float wm, float w0, float wp, int lim, float dx) {
-  if (LIMX) return half_slope_x(wm, w0, wp, lim, dx);
-  return half_slope(wm, w0, wp);
+template <int LIMX>
+__device__ __forceinline__ float slope(float wm, float w0, float wp, int lim, const GradScale& gs) {
+  if (LIMX == LX_MINMOD) return half_slope(wm, w0, wp);
+  return half_slope_x(wm, w0, wp, LIMX == LX_VAN_ALBADA ? (int)LIM_VAN_ALBADA : lim, gs);
 }
 
 // Boundary codes (AMX_BC_*) of the two sides of one axis.
@@ -480,7 +498,7 @@ struct StageArgs {
   int nx, na, nb;        // 3D: (nx, ny, nz); 2D: (1, nx, ny)
   int ntb, nta, ncx, lx;
   float dt_scale;        // 0.5: MHD half step dt/2; 1: hydro step
-  int limiter;           // LIM_* (the kernels instantiated with LIMX read it)
+  int limiter;           // LIM_* (the LX_ANY kernels read it)
   float dxf;             // float(grid_spacing): the limiters' gradient scale
   unsigned char* amg;    // hybrid / AM-HLLC: compression switch per cell of the stage input
   long gstride;          // bytes between consecutive slots' switch arrays
@@ -490,7 +508,7 @@ struct StageArgs {
   float* ppf[7];
   long ppstride;
   float ppq;             // q = 2 / C_cfl with MHD, 1 / C_cfl without
-  int pp;                // the kernels instantiated with LIMX scale their slopes by ppf
+  int pp;                // the LX_ANY kernels scale their slopes by ppf
   // energy-fixed pressure of the magnetic sub-step's output: written by the
   // SRC_MAGFIX stage (when set), read by the W0M == SRC_PFIX Heun centre
   float* pfix;
@@ -510,7 +528,7 @@ struct StageArgs {
 // bnd_index maps them to, with the normal velocity negated at reflective
 // walls (_reflective_*_boundary, boundaries.py:323-357); the flux into the
 // ghost layer at an upper edge is computed from those values like any other.
-template <int DIM, int TA, int SRC, bool HEUN, int W0M, int RS, bool LIMX, bool BCX>
+template <int DIM, int TA, int SRC, bool HEUN, int W0M, int RS, int LIMX, bool BCX>
 __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(AMX_STAGE_WAVES))) void k_stage(const StageArgs a) {
   constexpr int NV = DIM + 2, P = DIM + 1, NT = (TA + 1) * TB, WW = TB + 4;
   constexpr int AXA = DIM == 3 ? 2 : 1;  // velocity row of the plane axis A
@@ -519,10 +537,10 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   constexpr int NFA = (TA + 1) * TB, NF = NFA + TA * (TB + 1);
   static_assert(NFA == NT && NF - NFA <= NT, "flux rounds assume (TA+1)*TB threads");
   static_assert(NH <= NT, "every halo cell of a plane needs its own thread (TA >= 4)");
-  // LAG (3D, limiters without plane factors): the cell update runs one
+  // LAG (3D, forms without plane factors): the cell update runs one
   // plane behind the interface fluxes, and with the plane arrays double
   // buffered one barrier per plane orders both phases
-  constexpr bool LAG = DIM == 3 && !LIMX;
+  constexpr bool LAG = DIM == 3 && LIMX != LX_ANY;
   constexpr int NBUF = LAG ? 2 : 1;
   __shared__ float sW[NBUF][NV][(TA + 4) * WW];
   __shared__ float sFA[NBUF][NV][(TA + 1) * TB];
@@ -531,7 +549,7 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   static_assert(!(AMS && BCX), "the compression switch of ghost cells is not defined here");
   __shared__ unsigned char sG[NBUF][AMS ? (TA + 4) * WW : 1];
   // VAN_ALBADA_PP factors of the plane cells: alpha_A, kappa_A, alpha_B, kappa_B, beta
-  __shared__ float sPF[LIMX ? 5 : 1][LIMX ? (TA + 4) * WW : 1];
+  __shared__ float sPF[LIMX == LX_ANY ? 5 : 1][LIMX == LX_ANY ? (TA + 4) * WW : 1];
 
   const int slot = a.slot0 + blockIdx.y;
   Ctl* const C = a.ctl + slot;
@@ -565,9 +583,9 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   const Phys ph = a.phs[slot];
   const int tid = threadIdx.x, ta = tid / TB, tb = tid % TB;
   const int lim = a.limiter;
-  const float ldx = a.dxf;
+  const GradScale ldx = grad_scale(a.dxf);
   // VAN_ALBADA_PP: slopes scaled by the factor of their cell (reconstruction.py:343-365)
-  const bool pp = LIMX && a.pp;
+  const bool pp = LIMX == LX_ANY && a.pp;
   const float* pfp[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // plane factors, as sPF
   const float* pfx[2] = {nullptr, nullptr};                             // alpha_x, kappa_x (3D)
   if (pp) {
@@ -1086,7 +1104,8 @@ __global__ __launch_bounds__(256) void k_pp_factors(const StageArgs a) {
     for (int k = 0; k < DIM; ++k) Cw[k] = al[k] / sum;
   }
   const float qm2 = a.ppq - 2.f;
-  const float eps = 1e-14f, dx = a.dxf;
+  const float eps = 1e-14f;
+  const GradScale gs = grad_scale(a.dxf);
   // axes of the state: 3D (nx, na, nb) = (x, y, z); 2D (na, nb) = (x, y)
   const int n0 = DIM == 3 ? a.nx : a.na, n1 = DIM == 3 ? a.na : a.nb, n2 = DIM == 3 ? a.nb : 1;
   const unsigned n = (unsigned)n0 * (unsigned)n1 * (unsigned)n2;
@@ -1109,7 +1128,7 @@ __global__ __launch_bounds__(256) void k_pp_factors(const StageArgs a) {
       load_w<DIM, SRC>(src, base + (unsigned)(ii[ax] == 0 ? nn[ax] - 1 : ii[ax] - 1) * ss[ax], wm);
       load_w<DIM, SRC>(src, base + (unsigned)(ii[ax] + 1 == nn[ax] ? 0 : ii[ax] + 1) * ss[ax], wp);
 #pragma unroll
-      for (int v = 0; v < NV; ++v) d[ax][v] = half_slope_x(wm[v], w[v], wp[v], LIM_VAN_ALBADA, dx);
+      for (int v = 0; v < NV; ++v) d[ax][v] = half_slope_x(wm[v], w[v], wp[v], LIM_VAN_ALBADA, gs);
     }
     const float rho = w[0], p = w[P];
     float al[DIM], ka[DIM];
@@ -2422,7 +2441,7 @@ Bufs bufs(const amx_fv_ctx* c, float* state) {
   return b;
 }
 
-template <int DIM, int SRC, bool HEUN, int W0M, bool LIMX, bool BCX>
+template <int DIM, int SRC, bool HEUN, int W0M, int LIMX, bool BCX>
 void launch_stage_rs(const amx_fv_ctx* c, const StageArgs& a, dim3 grid, dim3 block, hipStream_t st) {
 #define AMX_STAGE(RS) hipLaunchKernelGGL((k_stage<DIM, TA_DEF, SRC, HEUN, W0M, RS, LIMX, BCX>), grid, block, 0, st, a)
   switch (c->cfg.riemann) {
@@ -2460,16 +2479,20 @@ hipError_t launch_stage_t(const amx_fv_ctx* c, const StageArgs& a, int nspan, hi
   if (c->cfg.riemann == AMX_HYBRID_HLLC || c->cfg.riemann == AMX_AM_HLLC)
     hipLaunchKernelGGL((k_am_switch<DIM, SRC>), dim3(LF_BLOCKS, nspan), dim3(256), 0, st, a);
   const dim3 grid(c->ntb * c->nta * c->ncx, nspan), block((TA_DEF + 1) * TB);
-  const bool lim = c->cfg.limiter != AMX_MINMOD;
+  const int lim = c->cfg.limiter;
   if (c->bcx) {
-    if (lim)
-      launch_stage_rs<DIM, SRC, HEUN, W0M, true, true>(c, a, grid, block, st);
+    if (lim == AMX_MINMOD)
+      launch_stage_rs<DIM, SRC, HEUN, W0M, LX_MINMOD, true>(c, a, grid, block, st);
+    else if (lim == AMX_VAN_ALBADA)
+      launch_stage_rs<DIM, SRC, HEUN, W0M, LX_VAN_ALBADA, true>(c, a, grid, block, st);
     else
-      launch_stage_rs<DIM, SRC, HEUN, W0M, false, true>(c, a, grid, block, st);
-  } else if (lim) {
-    launch_stage_rs<DIM, SRC, HEUN, W0M, true, false>(c, a, grid, block, st);
+      launch_stage_rs<DIM, SRC, HEUN, W0M, LX_ANY, true>(c, a, grid, block, st);
+  } else if (lim == AMX_MINMOD) {
+    launch_stage_rs<DIM, SRC, HEUN, W0M, LX_MINMOD, false>(c, a, grid, block, st);
+  } else if (lim == AMX_VAN_ALBADA) {
+    launch_stage_rs<DIM, SRC, HEUN, W0M, LX_VAN_ALBADA, false>(c, a, grid, block, st);
   } else {
-    launch_stage_rs<DIM, SRC, HEUN, W0M, false, false>(c, a, grid, block, st);
+    launch_stage_rs<DIM, SRC, HEUN, W0M, LX_ANY, false>(c, a, grid, block, st);
   }
   return hipGetLastError();
 }
