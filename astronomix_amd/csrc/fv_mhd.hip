@@ -3159,7 +3159,23 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // stalled step with the further launches and goes on. Event timing keeps
   // the step-by-step path, which sorts out early-exited launches per step.
   const bool mbatch = c->cfg.mhd && c->keep_b && c->timing == 0;
-  constexpr long BATCH = 16;
+  // A loop with an end time takes about (t_end - t) / dt more steps, from the
+  // last step's dt; the first batch, before any dt is known, has 4. (Sixteen
+  // steps a batch whatever was left: a 20-step run of a 256^2 grid queued 32,
+  // 9 launches of 1-2 us each for a step that did nothing.)
+  constexpr long BATCH = 16, BATCH0 = 4;
+  auto batch_steps = [&](float dt, long left) -> long {
+    long n = BATCH0;
+    if (left < 0 && dt > 0.f) {
+      const float rest = (run->t_end - t) / dt;
+      left = rest < 2.f * BATCH ? (long)ceilf(rest) : 2 * BATCH;
+      if (left < 1) left = 1;
+    }
+    // a tail of up to half a batch joins the batch before it (one readback fewer)
+    if (left >= 0) n = left <= BATCH + BATCH / 2 ? left : BATCH;
+    return n;
+  };
+  float last_dt = 0.f;
   bool b_home = false;  // the final B is in the state's rows and hctl is current
   for (;;) {
     if (run->fixed_timestep) {
@@ -3169,9 +3185,9 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
     }
     if (run->max_steps >= 0 && steps >= run->max_steps) break;
     if (batch) {
-      long n = BATCH;
+      long left = run->fixed_timestep ? run->num_timesteps - steps : -1;
+      long n = batch_steps(last_dt, left);
       if (run->max_steps >= 0 && run->max_steps - steps < n) n = run->max_steps - steps;
-      if (run->fixed_timestep && run->num_timesteps - steps < n) n = run->num_timesteps - steps;
       hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
       HIPCHK(hipGetLastError());
       for (long i = 0; i < n; ++i) {
@@ -3189,15 +3205,16 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       time_resolve(c);
       t = c->hctl[0].t;
       steps = c->hctl[0].steps;
+      last_dt = c->hctl[0].dt;
       continue;
     }
     if (mbatch) {
-      // steps left when the loop has a step bound; a tail of up to half a
-      // batch joins the batch before it (one readback fewer)
+      // steps left when the loop has a step bound
       long left = -1;
       if (run->max_steps >= 0) left = run->max_steps - steps;
       if (run->fixed_timestep && (left < 0 || run->num_timesteps - steps < left)) left = run->num_timesteps - steps;
-      const long n = left >= 0 && left <= BATCH + BATCH / 2 ? left : BATCH;
+      long n = last_dt > 0.f || left < 0 ? batch_steps(last_dt, run->fixed_timestep ? left : -1) : BATCH;
+      if (left >= 0 && (left < n || left <= BATCH + BATCH / 2)) n = left;
       int klast = 0;
       StepParams spi = sp;
       spi.batch_first = 1;
@@ -3216,8 +3233,10 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
           hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
         HIPCHK(hipGetLastError());
       }
-      // the loop's last batch: B goes home behind it, unless a step stalled
-      const bool last = n == left;
+      // the loop's last batch (by its step bound, or as the last dt has it): B
+      // goes home behind it, unless a step stalled; a loop that goes on all the
+      // same takes B0 from the state's rows
+      const bool last = n == left || (last_dt > 0.f && (float)n * last_dt >= run->t_end - t);
       if (last) HIPCHK(copy_b_home(c, bl, st, 1));
       HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st));
       HIPCHK(hipStreamSynchronize(st));
@@ -3245,6 +3264,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       }
       t = c->hctl[0].t;
       steps = c->hctl[0].steps;
+      last_dt = c->hctl[0].dt;
       iters = c->hctl[0].iters_sum;
       kmax = c->hctl[0].iters_max;
       // the next batch queues launches for the largest count of this one
@@ -3779,11 +3799,28 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
     // its speculative launches; the device decides per slot whether they
     // settled the fixed point (a slot whose step stalls does nothing until
     // step_finish has completed that step)
-    const int nb = c->batch;
-    const auto bkey = std::make_tuple(span, lk, nb);
-    auto bit = c->g_batch.find(bkey);
-    hipGraphExec_t bx = bit == c->g_batch.end() ? nullptr : bit->second;
-    amx_status bs = replay_or_capture(c, st, &bx, bx != nullptr, [&]() -> amx_status {
+    // A batch shorter than that when the slots' last status says that none
+    // has so many steps left (steps past a slot's end do nothing, but each is
+    // still 8 launches); it is launched directly, not from a graph of its own.
+    int nb = c->batch;
+    if (hipEventQuery(c->ev_status) == hipSuccess) {
+      long need = 1;
+      for (int i = 0; i < span; ++i) {
+        if (!c->live[i]) continue;
+        if (c->fresh[i]) {
+          need = nb;
+          break;
+        }
+        const Ctl& h = c->hctl[i];
+        const float rest = c->sp.fixed ? (float)(c->sp.num_timesteps - h.steps) : (h.t_end - h.t) / h.dt;
+        const long n = rest < (float)nb ? (long)ceilf(rest) : nb;
+        need = n > need ? n : need;
+      }
+      nb = need < nb ? (int)need : nb;
+    } else {
+      (void)hipGetLastError();  // not ready
+    }
+    auto enqueue = [&]() -> amx_status {
       StepParams spi = c->sp;
       spi.batch_first = 1;
       hipLaunchKernelGGL(k_step_begin, dim3(span), dim3(NSLOT), 0, st, c->ctl, spi);
@@ -3803,9 +3840,18 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
         HIPCHK(hipGetLastError());
       }
       return AMX_OK;
-    });
-    if (bs != AMX_OK) return bs;
-    if (bx) c->g_batch[bkey] = bx;
+    };
+    if (nb < c->batch) {
+      const amx_status bs = enqueue();
+      if (bs != AMX_OK) return bs;
+    } else {
+      const auto bkey = std::make_tuple(span, lk, nb);
+      auto bit = c->g_batch.find(bkey);
+      hipGraphExec_t bx = bit == c->g_batch.end() ? nullptr : bit->second;
+      const amx_status bs = replay_or_capture(c, st, &bx, bx != nullptr, enqueue);
+      if (bs != AMX_OK) return bs;
+      if (bx) c->g_batch[bkey] = bx;
+    }
     c->klast = klast;
     HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl) * span, hipMemcpyDeviceToHost, st));
     HIPCHK(hipEventRecord(c->ev_status, st));
