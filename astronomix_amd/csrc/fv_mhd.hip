@@ -38,6 +38,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <tuple>
 #include <new>
 #include <utility>
@@ -3362,40 +3363,56 @@ extern "C" amx_status amx_fv_time_integration_snapshots(amx_fv_ctx* c, float* st
 
 namespace {
 
+// The separate passes: in 3D, and in 2D with dual numbers (k_adj_tile covers the rest).
 template <int DIM, int AXI>
 void launch_adj_iface(const amx_fv_ctx* c, dim3 grid, dim3 blk, hipStream_t st, const float* Win, const float* NU,
-                      float* con, adj::AdjGeom g, Phys ph, bool duals) {
-  if (c->cfg.riemann == AMX_HLLC && duals)
-    hipLaunchKernelGGL((adj::k_adj_iface<DIM, AXI, AMX_HLLC, true>), grid, blk, 0, st, Win, NU, con, c->ctl, g, ph);
-  else if (c->cfg.riemann == AMX_HLLC)
-    hipLaunchKernelGGL((adj::k_adj_iface<DIM, AXI, AMX_HLLC, false>), grid, blk, 0, st, Win, NU, con, c->ctl, g, ph);
-  else if (duals)
-    hipLaunchKernelGGL((adj::k_adj_iface<DIM, AXI, AMX_HLL, true>), grid, blk, 0, st, Win, NU, con, c->ctl, g, ph);
-  else
-    hipLaunchKernelGGL((adj::k_adj_iface<DIM, AXI, AMX_HLL, false>), grid, blk, 0, st, Win, NU, con, c->ctl, g, ph);
+                      float* con, float dt_scale, adj::AdjGeom g, Phys ph, bool duals) {
+#define AMX_IFACE(RS, DUALS) \
+  hipLaunchKernelGGL((adj::k_adj_iface<DIM, AXI, RS, DUALS>), grid, blk, 0, st, Win, NU, con, c->ctl, dt_scale, g, ph)
+  if (duals) {
+    if (c->cfg.riemann == AMX_HLLC)
+      AMX_IFACE(AMX_HLLC, true);
+    else
+      AMX_IFACE(AMX_HLL, true);
+  } else if constexpr (DIM == 3) {
+    if (c->cfg.riemann == AMX_HLLC)
+      AMX_IFACE(AMX_HLLC, false);
+    else
+      AMX_IFACE(AMX_HLL, false);
+  }
+#undef AMX_IFACE
 }
 
 template <int DIM>
-amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, float* lam_in, hipStream_t st) {
+adj::AdjGeom adj_geom(const amx_fv_ctx* c) {
+  adj::AdjGeom g;
+  g.n[0] = c->cfg.nx;
+  g.n[1] = c->cfg.ny;
+  g.n[2] = DIM == 3 ? c->cfg.nz : 1;
+  g.st[2] = 1;
+  g.st[1] = DIM == 3 ? (unsigned)c->cfg.nz : 1u;
+  g.st[0] = (unsigned)c->cfg.ny * g.st[1];
+  g.nc = c->ncell;
+  return g;
+}
+
+template <bool HEUN>
+hipError_t launch_adj_tile(const amx_fv_ctx* c, const adj::AdjTileArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)(a.nta * a.ntb)), block(adj::ANT);
+  if (c->cfg.riemann == AMX_HLLC)
+    hipLaunchKernelGGL((adj::k_adj_tile<AMX_HLLC, HEUN>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((adj::k_adj_tile<AMX_HLL, HEUN>), grid, block, 0, st, a);
+  return hipGetLastError();
+}
+
+// Reverse mode of one SSP-RK2 gas step of dt_scale times the step size in ctl.
+template <int DIM>
+amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, float* lam_in, float dt_scale,
+                          hipStream_t st) {
   constexpr int NV = DIM + 2;
   const long n = c->ncell;
-  adj::AdjGeom g;
-  if (DIM == 3) {
-    g.n[0] = c->cfg.nx;
-    g.n[1] = c->cfg.ny;
-    g.n[2] = c->cfg.nz;
-    g.st[2] = 1;
-    g.st[1] = c->cfg.nz;
-    g.st[0] = (long)c->cfg.ny * c->cfg.nz;
-  } else {
-    g.n[0] = c->cfg.nx;
-    g.n[1] = c->cfg.ny;
-    g.n[2] = 1;
-    g.st[1] = 1;
-    g.st[0] = c->cfg.ny;
-    g.st[2] = n;
-  }
-  g.nc = n;
+  const adj::AdjGeom g = adj_geom<DIM>(c);
   float* G1 = c->mem;                  // W1 = E(W0) (the context's stage buffer)
   float* G2 = c->adj;                  // W2 = E(W1)
   float* L2 = G2 + (long)NV * n;       // lam of W2
@@ -3403,13 +3420,13 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
   float* L1 = NU + (long)NV * n;       // lam of W1
   float* CON = L1 + (long)NV * n;      // DIM x 4 x NV interface contributions
   // recompute the two stage states with the forward kernel (dt in ctl[0])
-  StageArgs a1 = stage_base(c, 1.0f);
+  StageArgs a1 = stage_base(c, dt_scale);
   for (int v = 0; v < NV; ++v) {
     a1.src[v] = w0 + (long)v * n;
     a1.out[v] = G1 + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a1, 1, st)));
-  StageArgs a2 = stage_base(c, 1.0f);
+  StageArgs a2 = stage_base(c, dt_scale);
   for (int v = 0; v < NV; ++v) {
     a2.src[v] = G1 + (long)v * n;
     a2.out[v] = G2 + (long)v * n;
@@ -3418,6 +3435,30 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
   const Phys ph = c->hph[0];  // the interface kernels read dt from ctl[0]
   // AMX_ADJ_DUAL=1: the flux Jacobians by dual numbers (a cross-check of the reverse sweep)
   const bool duals = env_int("AMX_ADJ_DUAL", 0) != 0;
+  if (DIM == 2 && !duals) {
+    adj::AdjTileArgs t;
+    t.w0 = w0;
+    t.w2 = G2;
+    t.lam_out = lam_out;
+    t.ctl = c->ctl;
+    t.dt_scale = dt_scale;
+    t.nx = c->cfg.nx;
+    t.ny = c->cfg.ny;
+    t.nta = (t.nx + adj::ATA - 1) / adj::ATA;
+    t.ntb = (t.ny + TB - 1) / TB;
+    t.ph = ph;
+    t.win = G1;
+    t.wout = G2;
+    t.lam = nullptr;
+    t.dst = L1;
+    HIPCHK(launch_adj_tile<true>(c, t, st));
+    t.win = w0;
+    t.wout = G1;
+    t.lam = L1;
+    t.dst = lam_in;
+    HIPCHK(launch_adj_tile<false>(c, t, st));
+    return AMX_OK;
+  }
   long blocks = (n + 255) / 256;
   if (blocks > 8192) blocks = 8192;
   const dim3 grid(blocks), blk(256);
@@ -3434,11 +3475,11 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
     for (int ax = 0; ax < DIM; ++ax) {
       float* con = CON + (long)ax * 4 * NV * n;
       if (ax == 0)
-        launch_adj_iface<DIM, 0>(c, grid, blk, st, Win, NU, con, g, ph, duals);
+        launch_adj_iface<DIM, 0>(c, grid, blk, st, Win, NU, con, dt_scale, g, ph, duals);
       else if (ax == 1)
-        launch_adj_iface<DIM, 1>(c, grid, blk, st, Win, NU, con, g, ph, duals);
+        launch_adj_iface<DIM, 1>(c, grid, blk, st, Win, NU, con, dt_scale, g, ph, duals);
       else
-        launch_adj_iface<DIM, 2>(c, grid, blk, st, Win, NU, con, g, ph, duals);
+        launch_adj_iface<DIM, 2>(c, grid, blk, st, Win, NU, con, dt_scale, g, ph, duals);
       HIPCHK(hipGetLastError());
     }
     hipLaunchKernelGGL(adj::k_adj_gather<DIM>, grid, blk, 0, st, Win, NU, CON, dst, stage == 0 ? 1 : 0, g, ph);
@@ -3449,10 +3490,10 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
 
 }  // namespace
 
-// Fields of the MHD reverse mode's workspace before the iterates: state copy
-// (NS), W_B (NV), lam of W_B (NV), lam of W_A (NV), two 6-row cotangents, X
-// and Y (3 + 3), the accumulated cotangents of B0, v0, rho (7).
-long adjm_fixed_fields(const amx_fv_ctx* c) { return (long)c->NS + 3L * c->NV + 12 + 6 + 7; }
+// Fields of the MHD reverse mode's workspace before the iterates: W_A (NV; the
+// gas after the first half), W_B (NV), lam of W_B (NV), lam of W_A (NV), two
+// 6-row cotangents, the accumulated cotangents of B0, v0, rho (7).
+long adjm_fixed_fields(const amx_fv_ctx* c) { return 4L * c->NV + 12 + 7; }
 
 amx_status adjm_reserve(amx_fv_ctx* c, int iters, hipStream_t st) {
   if (c->adjm && iters <= c->adjm_iters) return AMX_OK;
@@ -3473,11 +3514,11 @@ amx_status adjm_reserve(amx_fv_ctx* c, int iters, hipStream_t st) {
 }
 
 // Reverse mode of one MHD step S_A(dt/2) S_B(dt) S_A(dt/2)
-// (evolve_state.py:496-600): the forward pass is recomputed from a copy of
-// the state with the forward kernels (so the stage states, the fixed-point
-// iterates and their count are the forward's own), keeping every iterate;
-// then the second gas half, the magnetic sub-step and the first gas half
-// are reversed (adj::k_adjm_*, adjoint_step_t at dt/2).
+// (evolve_state.py:496-600): the forward pass is recomputed with the forward
+// kernels (so the stage states, the fixed-point iterates and their count are
+// the forward's own), every iterate written to a place of its own; then the
+// second gas half, the magnetic sub-step and the first gas half are reversed
+// (adjoint_step_t at dt/2, adj::k_adjm_back).
 template <int DIM>
 amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_out, float* lam_in,
                             hipStream_t st) {
@@ -3485,122 +3526,101 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
   const long n = c->ncell;
   amx_status r = adjm_reserve(c, 8, st);
   if (r != AMX_OK) return r;
-  HIPCHK(hipMemcpyAsync(c->adjm, state, sizeof(float) * (size_t)c->NS * n, hipMemcpyDeviceToDevice, st));
-  Bufs b = bufs(c, c->adjm);
-  // ---- forward: S_A(dt/2) into S's gas rows (as step_phase1 does)
+  // ---- forward: S_A(dt/2) of the state's gas rows into W_A
+  float* G1 = c->mem;
   StageArgs a1 = stage_base(c, 0.5f);
   for (int v = 0; v < NV; ++v) {
-    a1.src[v] = b.gas[v];
-    a1.out[v] = b.G1 + (long)v * n;
+    a1.src[v] = state + (long)v * n;
+    a1.out[v] = G1 + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a1, 1, st)));
   StageArgs a2 = stage_base(c, 0.5f);
   for (int v = 0; v < NV; ++v) {
-    a2.src[v] = b.G1 + (long)v * n;
-    a2.w0[v] = b.gas[v];
-    a2.out[v] = b.gas[v];
+    a2.src[v] = G1 + (long)v * n;
+    a2.w0[v] = state + (long)v * n;
+    a2.out[v] = c->adjm + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, true, SRC_PLAIN>(c, a2, 1, st)));
-  // ---- forward: the fixed point pair by pair, every iterate kept (launch k's
-  // output at iterate slot k), until the residuals settle it
+  // ---- forward: the fixed point, launch k's output to iterate slot k. The
+  // pairs of the last step's count are queued before the residuals are read.
   c->skip_mask = 0u;
   int F = -1;
-  for (int L = 0; F < 0; L += 2) {
-    r = adjm_reserve(c, L + 2, st);  // may move the workspace: the buffers are taken again
+  for (int L = 0; F < 0;) {
+    const int maxit = c->cfg.max_fixed_point_iterations;
+    int upto = L == 0 ? (c->last_k < 1 ? 1 : c->last_k) : L;
+    if (upto > maxit) upto = maxit;
+    if (upto < L) upto = L;
+    r = adjm_reserve(c, upto + 2, st);  // may move the workspace: the buffers are taken again
     if (r != AMX_OK) return r;
-    b = bufs(c, c->adjm);
+    Bufs b;
+    memset(&b, 0, sizeof(b));
+    for (int v = 0; v < NV; ++v) b.gas[v] = c->adjm + (long)v * n;
+    for (int k = 0; k < 3; ++k) b.B[k] = const_cast<float*>(state) + (long)(NV + k) * n;
     float* IT = c->adjm + adjm_fixed_fields(c) * n;
-    HIPCHK(launch_mag_pair(c, b, L, 1, st, 1, 0));
-    for (int k = L; k <= L + 1; ++k)
-      for (int f = 0; f < 6; ++f)
-        HIPCHK(hipMemcpyAsync(IT + (long)(6 * k + f) * n, b.P[iterate_set(-1, k)][f], sizeof(float) * n,
-                              hipMemcpyDeviceToDevice, st));
+    for (; L <= upto; L += 2) {
+      for (int j = 0; j < 4; ++j)
+        for (int f = 0; f < 6; ++f) b.P[j][f] = IT + (long)f * n;  // sets that the pair does not use
+      for (int k = L > 0 ? L - 1 : 0; k <= L + 1; ++k)
+        for (int f = 0; f < 6; ++f) b.P[iterate_set(-1, k)][f] = IT + (long)(6 * k + f) * n;
+      HIPCHK(launch_mag_pair(c, b, L, 1, st, 1, 0));
+    }
     HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     F = slot_final(c, c->hctl[0]);
   }
-  float* S2 = c->adjm;
-  const Bufs bb = bufs(c, S2);
-  float* WB = S2 + (long)c->NS * n;
+  c->last_k = F;
+  float* WA = c->adjm;
+  float* WB = WA + (long)NV * n;
   float* LWB = WB + (long)NV * n;
   float* LWA = LWB + (long)NV * n;
-  float* LB0 = LWA + (long)NV * n;  // two 6-row cotangents
-  float* LB1 = LB0 + 6L * n;
-  float* XY = LB1 + 6L * n;
-  float* ACC = XY + 6L * n;
+  float* LB[2] = {LWA + (long)NV * n, LWA + (long)(NV + 6) * n};  // 6-row cotangents
+  float* ACC = LB[1] + 6L * n;
   float* IT = ACC + 7L * n;
-  adj::AdjGeom g;
-  if (DIM == 3) {
-    g.n[0] = c->cfg.nx;
-    g.n[1] = c->cfg.ny;
-    g.n[2] = c->cfg.nz;
-    g.st[2] = 1;
-    g.st[1] = c->cfg.nz;
-    g.st[0] = (long)c->cfg.ny * c->cfg.nz;
-  } else {
-    g.n[0] = c->cfg.nx;
-    g.n[1] = c->cfg.ny;
-    g.n[2] = 1;
-    g.st[1] = 1;
-    g.st[0] = c->cfg.ny;
-    g.st[2] = n;
-  }
-  g.nc = n;
+  const adj::AdjGeom g = adj_geom<DIM>(c);
   long blocks = (n + 255) / 256;
   if (blocks > 8192) blocks = 8192;
   const dim3 grid(blocks), blk(256);
-  hipLaunchKernelGGL(adj::k_adjm_wb<DIM>, grid, blk, 0, st, bb.gas[0], IT + 6L * F * n, WB, g);
+  hipLaunchKernelGGL(adj::k_adjm_wb<DIM>, grid, blk, 0, st, WA, IT + 6L * F * n, WB, g);
   HIPCHK(hipGetLastError());
   // ---- reverse: second gas half (dt/2) from lam_out's gas rows
-  hipLaunchKernelGGL(adj::k_scale_dt, dim3(1), dim3(1), 0, st, c->ctl, 0.5f);
-  HIPCHK(hipGetLastError());
-  amx_status s = adjoint_step_t<DIM>(c, WB, lam_out, LWB, st);
+  amx_status s = adjoint_step_t<DIM>(c, WB, lam_out, LWB, 0.5f, st);
   if (s != AMX_OK) return s;
-  hipLaunchKernelGGL(adj::k_scale_dt, dim3(1), dim3(1), 0, st, c->ctl, 2.0f);
-  HIPCHK(hipGetLastError());
-  // ---- reverse: the magnetic sub-step, launch F down to 0
-  hipLaunchKernelGGL(adj::k_adjm_init<DIM>, grid, blk, 0, st, lam_out + (long)NV * n, LWB, LB0, ACC, g);
-  HIPCHK(hipGetLastError());
+  // ---- reverse: the magnetic sub-step, launch F down to 0, from the final
+  // iterate's cotangent (B rows of lam_out; v rows of lam of W_B)
   adj::MagAdjArgs m;
   memset(&m, 0, sizeof(m));
   for (int k = 0; k < 3; ++k) {
-    m.B0[k] = bb.B[k];
-    m.v0[k] = k < DIM ? bb.gas[1 + k] : nullptr;
+    m.B0[k] = state + (long)(NV + k) * n;
+    m.v0[k] = k < DIM ? WA + (long)(1 + k) * n : nullptr;
+    m.lB[k] = lam_out + (long)(NV + k) * n;
+    m.lv[k] = k < DIM ? LWB + (long)(1 + k) * n : nullptr;
   }
-  m.rho = bb.gas[0];
-  m.X = XY;
-  m.Y = XY + 3L * n;
+  m.rho = WA;
   m.acc = ACC;
+  m.lam_wb = LWB;
+  m.lam_wa = LWA;
+  m.lam_in_B = lam_in + (long)NV * n;
   m.ctl = c->ctl;
   m.inv_dx = c->hph[0].inv_dx;
   m.euler = c->cfg.magnetic_integrator == AMX_IMPLICIT_EULER;
   m.g = g;
-  float* lcur = LB0;
-  float* lnext = LB1;
   for (int j = F; j >= 0; --j) {
+    m.start = j == F;
     m.first = j == 0;
     for (int k = 0; k < 3; ++k) {
-      m.Bj[k] = j == 0 ? bb.B[k] : IT + (long)(6 * (j - 1) + k) * n;
+      m.Bj[k] = j == 0 ? m.B0[k] : IT + (long)(6 * (j - 1) + k) * n;
       m.vj[k] = j == 0 ? m.v0[k] : IT + (long)(6 * (j - 1) + 3 + k) * n;
     }
-    m.lB = lcur;
-    m.lBn = lnext;
-    hipLaunchKernelGGL(adj::k_adjm_xy<DIM>, grid, blk, 0, st, m);
-    HIPCHK(hipGetLastError());
+    m.lBn = LB[j & 1];
     hipLaunchKernelGGL(adj::k_adjm_back<DIM>, grid, blk, 0, st, m);
     HIPCHK(hipGetLastError());
-    std::swap(lcur, lnext);
+    for (int k = 0; k < 3; ++k) {
+      m.lB[k] = LB[j & 1] + (long)k * n;
+      m.lv[k] = LB[j & 1] + (long)(3 + k) * n;
+    }
   }
-  hipLaunchKernelGGL(adj::k_adjm_final<DIM>, grid, blk, 0, st, LWB, lcur, ACC, LWA, lam_in + (long)NV * n, g);
-  HIPCHK(hipGetLastError());
   // ---- reverse: first gas half (dt/2) at the step's input state
-  hipLaunchKernelGGL(adj::k_scale_dt, dim3(1), dim3(1), 0, st, c->ctl, 0.5f);
-  HIPCHK(hipGetLastError());
-  s = adjoint_step_t<DIM>(c, state, LWA, lam_in, st);
-  if (s != AMX_OK) return s;
-  hipLaunchKernelGGL(adj::k_scale_dt, dim3(1), dim3(1), 0, st, c->ctl, 2.0f);
-  HIPCHK(hipGetLastError());
-  return AMX_OK;
+  return adjoint_step_t<DIM>(c, state, LWA, lam_in, 0.5f, st);
 }
 
 extern "C" amx_status amx_fv_adjoint_step(amx_fv_ctx* c, const float* state, const float* d_dt, const float* lam_out,
@@ -3624,7 +3644,8 @@ extern "C" amx_status amx_fv_adjoint_step(amx_fv_ctx* c, const float* state, con
   HIPCHK(hipGetLastError());
   if (c->cfg.mhd)
     return dim == 3 ? adjoint_step_mhd<3>(c, state, lam_out, lam_in, st) : adjoint_step_mhd<2>(c, state, lam_out, lam_in, st);
-  return dim == 3 ? adjoint_step_t<3>(c, state, lam_out, lam_in, st) : adjoint_step_t<2>(c, state, lam_out, lam_in, st);
+  return dim == 3 ? adjoint_step_t<3>(c, state, lam_out, lam_in, 1.0f, st)
+                  : adjoint_step_t<2>(c, state, lam_out, lam_in, 1.0f, st);
 }
 
 // ============================================================================
