@@ -161,6 +161,8 @@ SIGNATURES = {
     "amx_fv_set_timing": (ctypes.c_int, [_P, ctypes.c_int]),
     "amx_fv_get_timing": (ctypes.c_int, [_P, ctypes.POINTER(AmxFvTiming)]),
     "amx_fv_set_physics": (ctypes.c_int, [_P, ctypes.c_float, ctypes.c_float]),
+    "amx_fv_time_integration_recorded": (ctypes.c_int, [_P, _P, ctypes.POINTER(AmxFvRun), _P, ctypes.c_long, _P,
+                                                        ctypes.c_long, ctypes.POINTER(AmxFvStats), _P]),
     "amx_fv_adjoint_step": (ctypes.c_int, [_P, _P, _P, _P, _P, _P]),
     "amx_fv_pool_slot_bytes": (ctypes.c_int, [ctypes.POINTER(AmxFvConfig), ctypes.POINTER(ctypes.c_size_t)]),
     "amx_fv_pool_create": (ctypes.c_int, [ctypes.POINTER(AmxFvConfig), ctypes.POINTER(AmxFvRun), ctypes.c_int,
@@ -307,6 +309,17 @@ class FvContext:
         st = AmxFvStats()
         check(self.lib.amx_fv_time_integration(self.handle, ctypes.c_void_p(state.data_ptr()), ctypes.byref(run),
                                                ctypes.byref(st), self._stream(stream)), "amx_fv_time_integration")
+        return st
+
+    def time_integration_recorded(self, state, run: AmxFvRun, inputs, dts, stream=None) -> AmxFvStats:
+        """time_integration that records the step sizes into `dts` and the
+        first steps' input states into `inputs` (a stack of states)."""
+        st = AmxFvStats()
+        check(self.lib.amx_fv_time_integration_recorded(
+            self.handle, ctypes.c_void_p(state.data_ptr()), ctypes.byref(run),
+            ctypes.c_void_p(inputs.data_ptr()) if inputs.shape[0] else None, int(inputs.shape[0]),
+            ctypes.c_void_p(dts.data_ptr()), int(dts.shape[0]), ctypes.byref(st), self._stream(stream)),
+            "amx_fv_time_integration_recorded")
         return st
 
     def time_integration_snapshots(self, state, run: AmxFvRun, snapshots: "SnapshotRun", stream=None) -> AmxFvStats:

@@ -1,9 +1,12 @@
 """Reverse mode of the finite-volume step loop (hydro and MHD).
 
-``rollout`` is a ``torch.autograd.Function``: forward runs the step loop with
-the HIP kernels (``amx_fv_evolve_state``) and keeps a checkpoint every
-``checkpoint_every`` steps; backward walks the segments from the last one,
-recomputes each segment's step inputs from its checkpoint and applies the
+``rollout`` is a ``torch.autograd.Function``: forward runs the device step
+loop, which records the step sizes and, for a run of up to
+``checkpoint_every`` steps that fits ``RECORD_BYTES``, every step's input
+(``amx_fv_time_integration_recorded``); a longer run is made once more with
+``amx_fv_evolve_state`` and a checkpoint every ``checkpoint_every`` steps.
+Backward walks the segments from the last one, takes each segment's step
+inputs from the record or recomputes them from its checkpoint, and applies the
 hand-written reverse-mode kernels (``amx_fv_adjoint_step``) step by step.
 Step sizes are recorded in the forward pass and held constant, as the
 reference stop_gradients dt (time_integration.py:632-655); with
@@ -30,19 +33,54 @@ from astronomix_amd._finite_volume import boundary_codes, native_config, require
 from astronomix_amd.option_classes.simulation_config import HLL, HLLC, MINMOD
 
 
+# Device bytes of step inputs that the forward pass keeps: a run whose inputs
+# fit, and that has no more steps than the checkpointed sweep would hold states
+# (its checkpoints and one segment's inputs), is reversed without recomputing.
+RECORD_BYTES = 1 << 30
+
+
 def _function():
     import torch
 
+    def record(state, ctx, run, every):
+        """(final state, dts, the inputs of the steps) of a loop that fits the
+        record; (None, dts, None) of one that does not."""
+        n = int(run.num_timesteps) if run.fixed_timestep else None
+        most = RECORD_BYTES // (state.numel() * 4)
+        if n is not None:
+            if n < 1 or n > most or n > -(-n // every) + every:
+                return None, step_sizes(state, ctx, run.t_end, max(n, 0), bool(run.exact_end_time)), None
+            most = n
+        else:
+            most = min(most, every)
+        inputs = state.new_empty((most,) + tuple(state.shape))
+        cap = n or 1 << 16
+        while True:
+            s = state.clone()
+            dts = state.new_empty((cap,))
+            steps = ctx.time_integration_recorded(s, run, inputs, dts).steps
+            if steps <= cap:
+                break
+            cap = 2 * steps
+        return (s if steps <= most else None), list(dts[:steps].unbind()), (inputs if steps <= most else None)
+
     class Rollout(torch.autograd.Function):
         @staticmethod
-        def forward(fctx, state, ctx, dts, every):
-            s = state.detach().contiguous().clone()
-            ckpts = [s.clone()]
-            for k, dt in enumerate(dts):
-                ctx.evolve_state(s, dt)
-                if (k + 1) % every == 0 and k + 1 < len(dts):
-                    ckpts.append(s.clone())
-            fctx.ctx, fctx.dts, fctx.every, fctx.ckpts = ctx, dts, every, ckpts
+        def forward(fctx, state, ctx, run, every):
+            first = state.detach().contiguous()
+            s, dts, inputs = record(first, ctx, run, every)
+            ckpts = None
+            if inputs is None:
+                # not recorded: step by step, with a checkpoint every `every` steps
+                s = first.clone()
+                ckpts = [s.clone()]
+                for k, dt in enumerate(dts):
+                    ctx.evolve_state(s, dt)
+                    if (k + 1) % every == 0 and k + 1 < len(dts):
+                        ckpts.append(s.clone())
+            if inputs is not None:
+                every = max(1, len(dts))  # one segment
+            fctx.ctx, fctx.dts, fctx.every, fctx.ckpts, fctx.inputs = ctx, dts, every, ckpts, inputs
             return s
 
         @staticmethod
@@ -54,15 +92,18 @@ def _function():
             nseg = (len(dts) + every - 1) // every
             for j in reversed(range(nseg)):
                 lo, hi = j * every, min((j + 1) * every, len(dts))
-                s = fctx.ckpts[j].clone()
-                inputs = []
-                for k in range(lo, hi):
-                    inputs.append(s.clone())
-                    ctx.evolve_state(s, dts[k])
+                if fctx.inputs is not None:
+                    inputs = fctx.inputs
+                else:
+                    s = fctx.ckpts[j].clone()
+                    inputs = []
+                    for k in range(lo, hi):
+                        inputs.append(s.clone())
+                        ctx.evolve_state(s, dts[k])
                 for k in reversed(range(lo, hi)):
                     ctx.adjoint_step(inputs[k - lo], dts[k], lam, lam_in)
                     lam, lam_in = lam_in, lam
-            fctx.ckpts = None
+            fctx.ckpts = fctx.inputs = None
             return lam, None, None, None
 
     return Rollout
@@ -84,9 +125,9 @@ def step_sizes(state, ctx, t_end: float, num_steps: int = None, exact_end: bool 
         out = []
         for _ in range(num_steps):
             dt = min(dt0, np.float32(te - t)) if exact_end else dt0
-            out.append(torch.tensor(dt, dtype=torch.float32, device=state.device))
+            out.append(dt)
             t = np.float32(t + dt)
-        return out
+        return list(torch.from_numpy(np.array(out, dtype=np.float32)).to(state.device).unbind())
     s = state.detach().contiguous().clone()
     dts, t = [], torch.zeros((), dtype=torch.float32, device=state.device)
     d = torch.empty((), dtype=torch.float32, device=state.device)
@@ -120,9 +161,10 @@ def rollout(state, config, params, registered_variables=None, checkpoint_every: 
     if _ROLLOUT is None:
         _ROLLOUT = _function()
     ctx = _native.fv_context(native_config(state.shape, config, params.gamma, params.C_cfl))
-    n = int(config.num_timesteps) if config.fixed_timestep else None
-    dts = step_sizes(state, ctx, float(params.t_end), n, bool(config.exact_end_time))
-    return _ROLLOUT.apply(state, ctx, dts, max(1, int(checkpoint_every)))
+    run = _native.AmxFvRun(t_end=float(params.t_end), fixed_timestep=int(bool(config.fixed_timestep)),
+                           num_timesteps=int(config.num_timesteps), exact_end_time=int(bool(config.exact_end_time)),
+                           max_steps=-1)
+    return _ROLLOUT.apply(state, ctx, run, max(1, int(checkpoint_every)))
 
 
 __all__ = ["rollout", "step_sizes"]

@@ -1693,13 +1693,23 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
 // queues the regeneration when it finishes the step.
 __global__ void k_mag_final(Ctl* ctl, float tol, int max_iter, int spec, unsigned skip_mask, int regen_queued) {
   Ctl* const c = ctl + blockIdx.x;
-  if (!c->run) return;
-  const int L = c->iters - 1;
-  const float r0 = __uint_as_float(slots_max(c->resp[L % NRES]));
-  const float r1 = __uint_as_float(slots_max(c->resp[(L + 1) % NRES]));
+  // everything read is loaded first (as in step_control)
+  const int run = c->run, L = c->iters - 1, kprev = c->kprev, regen_ev = c->regen_ev;
+  unsigned res[NRES];
+#pragma unroll
+  for (int k = 0; k < NRES; ++k) res[k] = c->resp[k][threadIdx.x];
+  if (!run) return;
+  const int i0 = L % NRES, i1 = (L + 1) % NRES;
+  unsigned m0 = 0u, m1 = 0u;
+#pragma unroll
+  for (int k = 0; k < NRES; ++k) {
+    m0 = k == i0 ? res[k] : m0;
+    m1 = k == i1 ? res[k] : m1;
+  }
+  const float r0 = __uint_as_float(wave_max_u(m0)), r1 = __uint_as_float(wave_max_u(m1));
   const int f = pair_final(L, r0, r1, tol, max_iter);
-  const bool unstored = f >= 0 && f == L && L <= 62 && ((skip_mask >> (L >> 1)) & 1u) && L != c->kprev;
-  if (spec && unstored && c->kprev >= 0) c->regen_ev += 1;
+  const bool unstored = f >= 0 && f == L && L <= 62 && ((skip_mask >> (L >> 1)) & 1u) && L != kprev;
+  if (spec && unstored && kprev >= 0) c->regen_ev = regen_ev + 1;
   if ((f < 0 || (unstored && !regen_queued)) && spec) {
     c->held = 1;
     c->stall = 1;
@@ -1784,16 +1794,9 @@ struct StepParams {
 
 // dt = C / sum_a(max_a / dx) (_timestep_estimator.py:128), or t_end/num_timesteps
 // (time_integration.py:667-668); clamp to t_end - t (time_integration.py:677-678).
-__device__ __forceinline__ void cfl_reduce(Ctl* c, int dim) {
-  for (int k = 0; k < dim; ++k) {
-    c->cfl[k] = slots_max(c->cflp[k]);
-    c->cflp[k][threadIdx.x] = 0u;
-  }
-}
-
-__device__ __forceinline__ float cfl_dt_from(const Ctl* c, float C, float dx, int dim) {
-  float s = __uint_as_float(c->cfl[0]) / dx + __uint_as_float(c->cfl[1]) / dx;
-  if (dim == 3) s = s + __uint_as_float(c->cfl[2]) / dx;
+__device__ __forceinline__ float cfl_dt_from(const unsigned* cfl, float C, float dx, int dim) {
+  float s = __uint_as_float(cfl[0]) / dx + __uint_as_float(cfl[1]) / dx;
+  if (dim == 3) s = s + __uint_as_float(cfl[2]) / dx;
   return (C * 1.0f) / s;
 }
 
@@ -1809,33 +1812,62 @@ __device__ __forceinline__ void zero_cflp(Ctl* c) {
 
 // The control kernels: one wavefront per simulation (slot = blockIdx.x), a lane
 // per partial slot; the scalars are the same in every lane, which all write them.
+// Everything they read is loaded before the first store, which the compiler may
+// not move a load past: one memory latency instead of one per value.
 //
-// The step's dt, and whether the
-// slot runs this step (live and not yet at t_end / num_timesteps).
-__device__ void step_begin(Ctl* c, const StepParams& p) {
+// END: the end of a step. keep_b: the final B of the step stays in its iterate
+// set, which holds B0 of the next step (the state's B rows are written once, by
+// k_copy_bset). BEGIN: the next step's dt, and whether the slot runs it (live
+// and not yet at t_end / num_timesteps).
+template <bool END, bool BEGIN>
+__device__ __forceinline__ void step_control(Ctl* c, int keep_b, const StepParams& p) {
+  const int lane = threadIdx.x;
+  const int run = c->run, held = c->held, live = c->live, stall = c->stall, iters = c->iters, bset = c->bset;
+  const int isum = c->iters_sum, imax = c->iters_max, ibmax = c->iters_bmax;
+  const float dt0 = c->dt, t_end = c->t_end;
+  int steps = c->steps;
+  float t = c->t;
+  unsigned m[3] = {0u, 0u, 0u};
+  if (BEGIN) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) m[k] = c->cflp[k][lane];
+  }
+  if (END && run && !held) {  // held: the host finishes the step
+    t = t + dt0;
+    steps += 1;
+    c->t = t;
+    c->steps = steps;
+    c->iters_sum = isum + iters;
+    c->iters_max = iters > imax ? iters : imax;
+    c->iters_bmax = iters > ibmax ? iters : ibmax;
+    if (keep_b) c->bset = iterate_set(bset, iters);
+  }
+  if (!BEGIN) return;
   if (p.batch_first) {
     c->iters_bmax = 0;
     c->regen_ev = 0;
   }
-  if (!c->live) {
-    c->run = 0;
-    return;
-  }
-  c->run = !c->stall && (p.fixed ? (c->steps < p.num_timesteps) : (c->t < c->t_end));
-  if (!c->run) return;
+  const int go = live && !stall && (p.fixed ? (steps < p.num_timesteps) : (t < t_end));
+  c->run = go;
+  if (!go) return;
   float dt;
   if (p.fixed) {
-    dt = c->t_end / (float)p.num_timesteps;
+    dt = t_end / (float)p.num_timesteps;
   } else {
-    cfl_reduce(c, p.dim);
-    dt = cfl_dt_from(c, p.C, p.dx, p.dim);
+    unsigned mx[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) mx[k] = wave_max_u(m[k]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (k < p.dim) c->cfl[k] = mx[k];
+    dt = cfl_dt_from(mx, p.C, p.dx, p.dim);
   }
   if (p.clamp_tp) {
-    const float rem = p.tp - c->t;
+    const float rem = p.tp - t;
     dt = rem < dt ? rem : dt;
   }
   if (p.exact_end) {
-    const float rem = c->t_end - c->t;
+    const float rem = t_end - t;
     dt = rem < dt ? rem : dt;
   }
   c->dt = dt;
@@ -1843,7 +1875,7 @@ __device__ void step_begin(Ctl* c, const StepParams& p) {
   fixed_point_reset(c);
 }
 
-__global__ void k_step_begin(Ctl* ctl, StepParams p) { step_begin(ctl + blockIdx.x, p); }
+__global__ void k_step_begin(Ctl* ctl, StepParams p) { step_control<false, true>(ctl + blockIdx.x, 0, p); }
 
 // dt given by the caller (one step of _evolve_state_fv)
 __global__ void k_set_dt(Ctl* c, const float* dtp) {
@@ -1856,25 +1888,30 @@ __global__ void k_set_dt(Ctl* c, const float* dtp) {
   fixed_point_reset(c);
 }
 
-// keep_b: the final B of the step stays in its iterate set, which holds B0
-// of the next step (the state's B rows are written once, by k_copy_bset).
-__device__ void step_end(Ctl* c, int keep_b) {
-  if (!c->run || c->held) return;  // held: the host finishes the step
-  c->t = c->t + c->dt;
-  c->steps += 1;
-  c->iters_sum += c->iters;
-  c->iters_max = c->iters > c->iters_max ? c->iters : c->iters_max;
-  c->iters_bmax = c->iters > c->iters_bmax ? c->iters : c->iters_bmax;
-  if (keep_b) c->bset = iterate_set(c->bset, c->iters);
-}
-
-__global__ void k_step_end(Ctl* ctl, int keep_b) { step_end(ctl + blockIdx.x, keep_b); }
+__global__ void k_step_end(Ctl* ctl, int keep_b) { step_control<true, false>(ctl + blockIdx.x, keep_b, StepParams()); }
 
 // the end of one queued step and the beginning of the next, in one launch
 __global__ void k_step_end_begin(Ctl* ctl, int keep_b, StepParams p) {
-  Ctl* const c = ctl + blockIdx.x;
-  step_end(c, keep_b);
-  step_begin(c, p);
+  step_control<true, true>(ctl + blockIdx.x, keep_b, p);
+}
+
+// Record of a step loop for the reverse mode, at the start of each step that
+// runs: its dt and its input (n floats), at the step's index.
+struct RecordArgs {
+  const float* state;
+  float* inputs;
+  float* dts;
+  long n, max_inputs, max_dts;
+};
+
+__global__ void k_record(const Ctl* c, RecordArgs a) {
+  if (!c->run) return;
+  const long k = c->steps;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && k < a.max_dts) a.dts[k] = c->dt;
+  if (k >= a.max_inputs) return;
+  float* dst = a.inputs + k * a.n;
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (long)gridDim.x * blockDim.x)
+    dst[i] = a.state[i];
 }
 
 // B of slot 0 from its iterate set into the state's B rows (a loop that kept
@@ -1912,8 +1949,17 @@ __global__ void k_resume(Ctl* ctl) {
 }
 
 __global__ void k_cfl_out(Ctl* c, float C, float dx, int dim, float* out) {
-  cfl_reduce(c, dim);
-  *out = cfl_dt_from(c, C, dx, dim);
+  unsigned m[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) m[k] = c->cflp[k][threadIdx.x];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) m[k] = wave_max_u(m[k]);
+  *out = cfl_dt_from(m, C, dx, dim);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    c->cfl[k] = m[k];
+    c->cflp[k][threadIdx.x] = 0u;
+  }
 }
 
 __global__ void k_zero_cfl(Ctl* c) { zero_cflp(c); }
@@ -3123,7 +3169,7 @@ hipError_t copy_b_home(amx_fv_ctx* c, const Bufs& bl, hipStream_t st, int gate) 
 // The step loop of _time_integration (time_integration.py:629-801); with a
 // snapshot driver, rows are taken as in time_integration.py:539-610, 736-745.
 amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Driver* snp, amx_fv_stats* stats,
-                   hipStream_t st) {
+                   hipStream_t st, const RecordArgs* rec = nullptr) {
   hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, run->t_end, 1, 0);
   HIPCHK(hipGetLastError());
   // Without snapshot rows or a step hook nothing reads the state's B rows
@@ -3133,7 +3179,14 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
     amx_fv_ctx* c;
     ~KeepB() { c->keep_b = 0; }
   } keep_guard{c};
-  c->keep_b = c->cfg.mhd && !snp && !c->hook ? 1 : 0;
+  // (a record takes the whole state of every step)
+  c->keep_b = c->cfg.mhd && !snp && !c->hook && !rec ? 1 : 0;
+  auto record = [&]() -> hipError_t {
+    if (!rec) return hipSuccess;
+    const long blocks = rec->max_inputs > 0 ? (rec->n + 1023) / 1024 : 1;
+    hipLaunchKernelGGL(k_record, dim3(blocks < 4096 ? blocks : 4096), dim3(256), 0, st, c->ctl, *rec);
+    return hipGetLastError();
+  };
   const Bufs bl = bufs(c, state);
   if (!run->fixed_timestep) HIPCHK(launch_cfl(c, state, 0, 1, st));
   StepParams sp;
@@ -3159,7 +3212,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // nothing); the host reads the control block once per batch, finishes a
   // stalled step with the further launches and goes on. Event timing keeps
   // the step-by-step path, which sorts out early-exited launches per step.
-  const bool mbatch = c->cfg.mhd && c->keep_b && c->timing == 0;
+  const bool mbatch = c->cfg.mhd && (c->keep_b || (rec && !c->hook)) && c->timing == 0;
   // A loop with an end time takes about (t_end - t) / dt more steps, from the
   // last step's dt; the first batch, before any dt is known, has 4. (Sixteen
   // steps a batch whatever was left: a 20-step run of a 256^2 grid queued 32,
@@ -3192,6 +3245,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
       HIPCHK(hipGetLastError());
       for (long i = 0; i < n; ++i) {
+        HIPCHK(record());
         amx_status s = do_step(c, state, st, !run->fixed_timestep, nullptr);
         if (s != AMX_OK) return s;
         // this step's end and the next one's beginning
@@ -3223,6 +3277,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
       for (long i = 0; i < n; ++i) {
+        HIPCHK(record());
         amx_status s = step_phase1(c, bl, 1, st, !run->fixed_timestep, &klast);
         if (s != AMX_OK) return s;
         s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 1, c->regen_q);
@@ -3238,7 +3293,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       // goes home behind it, unless a step stalled; a loop that goes on all the
       // same takes B0 from the state's rows
       const bool last = n == left || (last_dt > 0.f && (float)n * last_dt >= run->t_end - t);
-      if (last) HIPCHK(copy_b_home(c, bl, st, 1));
+      if (last && c->keep_b) HIPCHK(copy_b_home(c, bl, st, 1));
       HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st));
       HIPCHK(hipStreamSynchronize(st));
       b_home = last && !c->hctl[0].stall;
@@ -3282,6 +3337,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
     HIPCHK(hipGetLastError());
     if (c->hook && c->hook(c->hook_user, state, &c->ctl[0].dt, steps, st) != 0)
       return fail(AMX_ERR_INVALID, "the step hook stopped the run%s");
+    HIPCHK(record());
     int K = 0;
     amx_status s = do_step(c, state, st, !run->fixed_timestep, &K);
     if (s != AMX_OK) return s;
@@ -3331,6 +3387,18 @@ extern "C" amx_status amx_fv_time_integration(amx_fv_ctx* c, float* state, const
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   if (run->fixed_timestep && run->num_timesteps <= 0) return fail(AMX_ERR_INVALID, "num_timesteps must be positive%s");
   return fv_loop(c, state, run, nullptr, stats, (hipStream_t)stream);
+}
+
+extern "C" amx_status amx_fv_time_integration_recorded(amx_fv_ctx* c, float* state, const amx_fv_run* run,
+                                                       float* inputs, long max_inputs, float* dts, long max_dts,
+                                                       amx_fv_stats* stats, void* stream) {
+  if (!c || !state || !run) return fail(AMX_ERR_INVALID, "null argument%s");
+  if (max_inputs < 0 || max_dts < 0 || (max_inputs && !inputs) || (max_dts && !dts))
+    return fail(AMX_ERR_INVALID, "record arrays missing%s");
+  if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
+  if (run->fixed_timestep && run->num_timesteps <= 0) return fail(AMX_ERR_INVALID, "num_timesteps must be positive%s");
+  const RecordArgs rec = {state, inputs, dts, (long)c->NS * c->ncell, max_inputs, max_dts};
+  return fv_loop(c, state, run, nullptr, stats, (hipStream_t)stream, &rec);
 }
 
 extern "C" amx_status amx_fv_time_integration_snapshots(amx_fv_ctx* c, float* state, const amx_fv_run* run,

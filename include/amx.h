@@ -161,6 +161,15 @@ amx_status amx_fv_evolve_state_noalloc(const amx_fv_config* cfg, float* state, c
 amx_status amx_fv_time_integration(amx_fv_ctx* ctx, float* state, const amx_fv_run* run,
                                    amx_fv_stats* stats, void* stream);
 
+/* The same loop with a record for the reverse mode: dts[k] receives the size
+ * of step k (k < max_dts) and inputs[k] the state it starts from (whole states,
+ * k < max_inputs). Steps past the arrays run unrecorded; stats->steps tells how
+ * many there were. Device arrays; may be NULL with a maximum of 0. The state and
+ * the steps are those of amx_fv_time_integration, bit for bit. */
+amx_status amx_fv_time_integration_recorded(amx_fv_ctx* ctx, float* state, const amx_fv_run* run, float* inputs,
+                                            long max_inputs, float* dts, long max_dts, amx_fv_stats* stats,
+                                            void* stream);
+
 /* Reverse mode of one step: lam_in = (dW_out/dW)^T lam_out where W_out is
  * the state amx_fv_evolve_state makes from `state` with the step size in
  * d_dt, held constant (the reference stop_gradients dt,
