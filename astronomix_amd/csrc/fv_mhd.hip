@@ -554,10 +554,16 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
 
   const int slot = a.slot0 + blockIdx.y;
   Ctl* const C = a.ctl + slot;
-  if (!C->run) return;  // block-uniform: empty or finished slot
-  if (a.gated && C->held) return;  // queued behind a fixed point that needs more launches
+  // all that the block needs of the control block and the physics in one
+  // batch of scalar loads, before the branches that would order them one
+  // after another (at 256^2 a stage launch is a few memory latencies long)
+  const int c_run = C->run, c_held = C->held, c_bset = C->bset, c_iters = C->iters;
+  const float c_dt = C->dt;
+  const Phys ph = a.phs[slot];
+  if (!c_run) return;  // block-uniform: empty or finished slot
+  if (a.gated && c_held) return;  // queued behind a fixed point that needs more launches
   const long so = slot * a.sstride;
-  const int par = iterate_set(C->bset, C->iters);  // set of the fixed point's final iterate
+  const int par = iterate_set(c_bset, c_iters);  // set of the fixed point's final iterate
   const float* src[8];
   const float* w0p[8];
 #pragma unroll
@@ -581,7 +587,6 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   float* outp[5];
 #pragma unroll
   for (int v = 0; v < NV; ++v) outp[v] = a.out[v] + so;
-  const Phys ph = a.phs[slot];
   const int tid = threadIdx.x, ta = tid / TB, tb = tid % TB;
   const int lim = a.limiter;
   const GradScale ldx = grad_scale(a.dxf);
@@ -625,7 +630,7 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   const int gb = BCX ? bnd_index(b0 + tb, a.nb, a.bb, fb) : wrapi(b0 + tb, a.nb);
   const unsigned col = (unsigned)ga * sa + gb;
   const bool active = owner && (a0 + ta < a.na) && (b0 + tb < a.nb);
-  const float coef = ph.inv_dx * (a.dt_scale * C->dt);
+  const float coef = ph.inv_dx * (a.dt_scale * c_dt);
   // plane offset of x index xi (3D), and whether it is a reflective ghost
   auto xplane = [&](int xi, bool& f) -> unsigned {
     f = false;
@@ -953,6 +958,229 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
 #pragma unroll
     for (int k = 0; k < DIM; ++k) {
       const unsigned m = block_max_u<TA + 1>(canon_bits(mx[k]), sred[k]);
+      if (tid == 0 && m) atomicMax(&C->cflp[k][blockIdx.x & (NSLOT - 1)], m);
+    }
+  }
+}
+
+// ---- 2D: both stages of an SSP-RK2 gas step in one launch
+//
+// A 2D stage launch is a chain of latencies (control block, tile, barrier,
+// fluxes, barrier, update) that a grid of up to a few hundred thousand cells
+// does not hide: 4-5 us at 256^2, of which its arithmetic is a tenth. Here a
+// block of 16 waves takes a TA x 64 tile through both stages: the input with
+// four halo cells, the first stage on the tile and the two cells around it that
+// the second stage reads (recomputed by the neighbouring blocks), the second
+// stage and Heun's average on the tile. 1.3 times the interfaces of two
+// launches, half the launches, and the first stage's state never leaves LDS.
+// With minmod it gives the bits of two k_stage launches. Bound by latency still
+// (rk2_rows has the sizes it is taken for, with both sides measured). An MHD
+// step takes it for its first half only: the second half's input is derived
+// from the iterate with the energy fix, whose rounding differs between a stage
+// launch's own cells and its halo cells, and one launch would not reproduce it.
+//
+// The output goes to other rows than the input, whose halo other blocks read.
+// HEUN: the step's result; otherwise the two stage states W1, W2 (the
+// linearisation points of the reverse mode).
+struct Rk2Args {
+  const float* src[4];   // input gas rows
+  float* out[4];         // the step's result, or W1
+  float* out2[4];        // !HEUN: W2
+  Ctl* ctl;
+  const Phys* phs;
+  long sstride;
+  int slot0, want_cfl;
+  // the input and output rows change places with the parity of the slot's step
+  // count (a loop that leaves each step's result where it was written)
+  int swap;
+  int na, nb, nta, ntb;
+  float dt_scale, dxf;
+};
+
+template <int TA, int RS, int LIMX, bool HEUN>
+__global__ __launch_bounds__(1024) void k_rk2(const Rk2Args a) {
+  constexpr int NV = 4, P = 3;
+  constexpr int R0 = TA + 8, W0 = TB + 8;   // input tile
+  constexpr int R1 = TA + 4, W1 = TB + 4;   // first-stage tile (cross shape)
+  // first-stage interfaces: between rows over the tile's columns and, for the
+  // four columns beside it, over the tile's rows; between columns likewise
+  constexpr int FA = (R1 + 1) * TB, FAS = (TA + 1) * 4;
+  constexpr int FB = R1 * (TB + 1), FBS = TA * 4;
+  constexpr int GA = (TA + 1) * TB, GB = TA * (TB + 1);  // second stage
+  constexpr int NS1 = R1 * TB + TA * 4;                  // first-stage cells
+  static_assert(FA + FAS <= 1024 && FB + FBS <= 1024 && GA + GB <= 2048 && NS1 <= 1024, "one round each");
+  __shared__ float s0[NV][R0 * W0];
+  __shared__ float s1[NV][R1 * W1];
+  __shared__ float sA[NV][FA + FAS > GA ? FA + FAS : GA];
+  __shared__ float sB[NV][FB + FBS > GB ? FB + FBS : GB];
+  __shared__ unsigned sred[2][16];
+  const int tid = threadIdx.x, slot = a.slot0 + blockIdx.y;
+  Ctl* const C = a.ctl + slot;
+  const int c_run = C->run, c_steps = C->steps;
+  const float c_dt = C->dt;
+  const Phys ph = a.phs[slot];
+  if (!c_run) return;
+  const long so = slot * a.sstride;
+  const bool swap = a.swap && (c_steps & 1);
+  const float* src[NV];
+  float* out[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    src[v] = a.src[v] + so;
+    out[v] = a.out[v] + so;
+    if (swap) {
+      float* const t = const_cast<float*>(src[v]);
+      src[v] = out[v];
+      out[v] = t;
+    }
+  }
+  const GradScale gs = grad_scale(a.dxf);
+  const int bid = swizzle_block(blockIdx.x, gridDim.x);
+  const int a0 = (bid / a.ntb) * TA, b0 = (bid % a.ntb) * TB;
+  const float coef = ph.inv_dx * (a.dt_scale * c_dt);
+  auto cell = [&](int r, int c) -> unsigned {
+    return (unsigned)wrapi(a0 + r, a.na) * (unsigned)a.nb + (unsigned)wrapi(b0 + c, a.nb);
+  };
+  for (int i = tid; i < R0 * W0; i += 1024) {
+    const int r = i / W0, c = i % W0;
+    const unsigned g = cell(r - 4, c - 4);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) s0[v][i] = ld32(src[v], g);
+  }
+  __syncthreads();
+  // flux through the interface below / left of the cell at offset o of tile s
+  // (row step d), into f[e]
+  auto face = [&](auto axis, const float* s, int st, int o, int d, float* f, int fst, int e) {
+    constexpr int AX = decltype(axis)::value;
+    float wl[NV], wr[NV], fl[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const float q0 = s[v * st + o - 2 * d], q1 = s[v * st + o - d], q2 = s[v * st + o], q3 = s[v * st + o + d];
+      wl[v] = q1 + slope<LIMX>(q0, q1, q2, LIM_VAN_ALBADA, gs);
+      wr[v] = q2 - slope<LIMX>(q1, q2, q3, LIM_VAN_ALBADA, gs);
+    }
+    riemann<2, AX, RS>(wl, wr, fl, ph, 0.f, false);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) f[v * fst + e] = fl[v];
+  };
+  constexpr int SA = sizeof(sA[0]) / sizeof(float), SB = sizeof(sB[0]) / sizeof(float);
+  constexpr std::integral_constant<int, 1> AXA{};
+  constexpr std::integral_constant<int, 2> AXB{};
+  // ---- first stage
+  if (tid < FA + FAS) {
+    int r, c;  // interface between rows r - 1 and r at column c (tile coordinates)
+    if (tid < FA) {
+      r = tid / TB - 2;
+      c = tid % TB;
+    } else {
+      const int j = tid - FA, q = j & 3;
+      r = j >> 2;
+      c = q < 2 ? q - 2 : TB + q - 2;
+    }
+    face(AXA, &s0[0][0], R0 * W0, (r + 4) * W0 + c + 4, W0, &sA[0][0], SA, tid);
+  }
+  if (tid < FB + FBS) {
+    int r, c;  // interface between columns c - 1 and c at row r
+    if (tid < FB) {
+      r = tid / (TB + 1) - 2;
+      c = tid % (TB + 1);
+    } else {
+      const int j = tid - FB, q = j & 3;
+      r = j >> 2;
+      c = q < 2 ? q - 2 : TB + q - 1;
+    }
+    face(AXB, &s0[0][0], R0 * W0, (r + 4) * W0 + c + 4, 1, &sB[0][0], SB, tid);
+  }
+  __syncthreads();
+  if (tid < NS1) {
+    int r, c, ea, da, eb, db;  // the cell; its lower row face and the next, its left face and the next
+    if (tid < R1 * TB) {
+      r = tid / TB - 2;
+      c = tid % TB;
+      ea = (r + 2) * TB + c;
+      da = TB;
+      eb = (r + 2) * (TB + 1) + c;
+      db = 1;
+    } else {
+      const int j = tid - R1 * TB, q = j & 3;
+      r = j >> 2;
+      c = q < 2 ? q - 2 : TB + q - 2;
+      ea = FA + r * 4 + q;
+      da = 4;
+      // left side: faces -2, -1 and the tile's 0; right side: the tile's TB, then TB + 1, TB + 2
+      eb = q == 2 ? (r + 2) * (TB + 1) + TB : FB + r * 4 + (q == 3 ? 2 : q);
+      const int en = q == 1 ? (r + 2) * (TB + 1) : FB + r * 4 + (q == 0 ? 1 : q);
+      db = en - eb;
+    }
+    const int o = (r + 4) * W0 + c + 4;
+    float w[NV], U[NV], n[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) w[v] = s0[v][o];
+    cons<2>(w, U, ph);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) U[v] = U[v] + (sA[v][ea] - sA[v][ea + da]) * coef;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) U[v] = U[v] + (sB[v][eb] - sB[v][eb + db]) * coef;
+    prim<2>(U, n, ph);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) s1[v][(r + 2) * W1 + c + 2] = n[v];
+  }
+  __syncthreads();
+  // ---- second stage
+  for (int e = tid; e < GA + GB; e += 1024) {
+    if (e < GA) {
+      face(AXA, &s1[0][0], R1 * W1, (e / TB + 2) * W1 + e % TB + 2, W1, &sA[0][0], SA, e);
+    } else {
+      const int j = e - GA;
+      face(AXB, &s1[0][0], R1 * W1, (j / (TB + 1) + 2) * W1 + j % (TB + 1) + 2, 1, &sB[0][0], SB, j);
+    }
+  }
+  __syncthreads();
+  float mx[2] = {0.f, 0.f};
+  const int r = tid / TB, c = tid % TB;
+  if (tid < TA * TB && a0 + r < a.na && b0 + c < a.nb) {
+    const unsigned g = cell(r, c);
+    float w[NV], U[NV], n[NV], w0[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      w[v] = s1[v][(r + 2) * W1 + c + 2];
+      w0[v] = s0[v][(r + 4) * W0 + c + 4];
+    }
+    cons<2>(w, U, ph);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) U[v] = U[v] + (sA[v][r * TB + c] - sA[v][(r + 1) * TB + c]) * coef;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) U[v] = U[v] + (sB[v][r * (TB + 1) + c] - sB[v][r * (TB + 1) + c + 1]) * coef;
+    prim<2>(U, n, ph);
+    if (HEUN) {
+      float U0[NV], U2[NV];
+      cons<2>(w0, U0, ph);
+      cons<2>(n, U2, ph);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) U[v] = 0.5f * (U0[v] + U2[v]);
+      prim<2>(U, n, ph);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) st32(out[v], g, n[v]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        st32(out[v], g, w[v]);
+        st32(a.out2[v] + so, g, n[v]);
+      }
+    }
+    if (a.want_cfl) {
+      const float cs = fsqrt(ph.gamma * n[P] * frcp(n[0]));
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float m = fabsf(n[1 + k]) + cs;
+        mx[k] = (m != m || m > mx[k]) ? m : mx[k];
+      }
+    }
+  }
+  if (a.want_cfl) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const unsigned m = block_max_u<16>(canon_bits(mx[k]), sred[k]);
       if (tid == 0 && m) atomicMax(&C->cflp[k][blockIdx.x & (NSLOT - 1)], m);
     }
   }
@@ -1360,7 +1588,16 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   const int tid = threadIdx.x;
   const int slot = a.slot0 + blockIdx.y;
   Ctl* const C = a.ctl + slot;
-  if (!C->run) return;
+  // the control block's scalars in one batch of loads (as in k_stage), and
+  // with them the residuals that a launch after the first looks at
+  const int c_run = C->run, c_done = C->done, c_kprev = C->kprev, c_bset = C->bset, c_iters = C->iters;
+  const float c_dt = C->dt;
+  unsigned prev0 = 0u, prev1 = 0u;
+  if (!a.regen && a.L > 0) {
+    prev0 = C->resp[(a.L - 2) % NRES][tid & 63];
+    prev1 = C->resp[(a.L - 1) % NRES][tid & 63];
+  }
+  if (!c_run) return;
   int L = a.L;
   bool one = a.regen;  // the launch computes its first iterate only
   if (a.regen) {
@@ -1370,17 +1607,17 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
     // previous step's final index), the launch is computed again (the same
     // arithmetic on the same inputs, so bit-identical) and only that iterate
     // is stored. Residuals, counters and flags are left as they are.
-    const int Ll = C->iters - 1;
+    const int Ll = c_iters - 1;
     if (Ll < 0 || Ll > 62) return;
     const float r0 = __uint_as_float(wave_max_u(C->resp[Ll % NRES][tid & 63]));
     const float r1 = __uint_as_float(wave_max_u(C->resp[(Ll + 1) % NRES][tid & 63]));
-    if (pair_final(Ll, r0, r1, a.tol, a.max_iter) != Ll || !((a.skip_mask >> (Ll >> 1)) & 1u) || Ll == C->kprev)
+    if (pair_final(Ll, r0, r1, a.tol, a.max_iter) != Ll || !((a.skip_mask >> (Ll >> 1)) & 1u) || Ll == c_kprev)
       return;
     L = Ll;
   } else if (L > 0) {
-    if (C->done) return;
-    const float r0 = __uint_as_float(wave_max_u(C->resp[(L - 2) % NRES][tid & 63]));
-    const float r1 = __uint_as_float(wave_max_u(C->resp[(L - 1) % NRES][tid & 63]));
+    if (c_done) return;
+    const float r0 = __uint_as_float(wave_max_u(prev0));
+    const float r1 = __uint_as_float(wave_max_u(prev1));
     if (pair_final(L - 2, r0, r1, a.tol, a.max_iter) >= 0) {
       if (blockIdx.x == 0 && tid == 0) C->done = 1;
       return;
@@ -1394,12 +1631,12 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
     C->resp[(L + 2) % NRES][tid] = 0u;
     C->resp[(L + 3) % NRES][tid] = 0u;
   }
-  const bool store1 = a.write_first || one || L == C->kprev;
+  const bool store1 = a.write_first || one || L == c_kprev;
   const long so = slot * a.sstride;
   MagArgs m = a;  // slot-local pointers
   // B0 is in the state's rows or, in a loop that keeps B in the iterate
   // sets, in set bset; launch k writes set iterate_set(bset, k)
-  const int bs = C->bset;
+  const int bs = c_bset;
   const int sin_ = L > 0 ? iterate_set(bs, L - 1) : 0;
   const int so0 = iterate_set(bs, L), so1 = iterate_set(bs, L + 1);
 #pragma unroll
@@ -1466,7 +1703,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
     if (b0 + c == 0 && a.bb.lo != AMX_BC_PERIODIC) put(-1, a.bb.lo, RB);
     if (b0 + c == a.nb - 1 && a.bb.hi != AMX_BC_PERIODIC) put(1, a.bb.hi, RB);
   };
-  const float dt = C->dt;
+  const float dt = c_dt;
   const float idx = a.inv_dx;
   float res0 = 0.f, res1 = 0.f;
   const float* SK[6];
@@ -1895,10 +2132,19 @@ __global__ void k_step_end_begin(Ctl* ctl, int keep_b, StepParams p) {
   step_control<true, true>(ctl + blockIdx.x, keep_b, p);
 }
 
+// n floats from src to dst for every slot that took part in the step (gate), or for all.
+__global__ void k_rows_home(const Ctl* ctl, float* dst, const float* src, long n, long sstride, int gate) {
+  if (gate && !ctl[blockIdx.y].run) return;
+  const long so = blockIdx.y * sstride;
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+    dst[so + i] = src[so + i];
+}
+
 // Record of a step loop for the reverse mode, at the start of each step that
 // runs: its dt and its input (n floats), at the step's index.
 struct RecordArgs {
   const float* state;
+  const float* odd;  // where the state is after an odd number of steps, if elsewhere
   float* inputs;
   float* dts;
   long n, max_inputs, max_dts;
@@ -1911,7 +2157,7 @@ __global__ void k_record(const Ctl* c, RecordArgs a) {
   if (k >= a.max_inputs) return;
   float* dst = a.inputs + k * a.n;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (long)gridDim.x * blockDim.x)
-    dst[i] = a.state[i];
+    dst[i] = (a.odd && (k & 1) ? a.odd : a.state)[i];
 }
 
 // B of slot 0 from its iterate set into the state's B rows (a loop that kept
@@ -2082,6 +2328,8 @@ struct amx_fv_ctx {
   void* snapwork;   // snapshot diagnostics partials (allocated on first use)
   int klast;        // pool: last fixed-point launch of the step in flight
   int keep_b;       // the running loop keeps B in the iterate sets (no per-step copy)
+  int rk2;          // gas steps by k_rk2: its tile rows, or 0 (two stage launches)
+  int rk2_swap;     // the running loop leaves each hydro step's result where k_rk2 wrote it
   int use_graphs;   // pool: replay captured HIP graphs of the step halves
   unsigned skip_mask;  // pairs of the current step queued without storing their first iterate
   int batch;        // pool: steps queued by one step_launch (1: a step in two halves)
@@ -2220,8 +2468,28 @@ amx_status validate(const amx_fv_config* c) {
 // G1 (gas rows) | P0 | P1 | P2 (B, v iterates of the fixed point)
 // G1 (gas rows) | P0 | P1 | P2 (B, v iterate sets) | PF (fixed pressure) | P3
 // (the fourth set: step loops and pools keep B in the sets)
+// Rows of the tiles in which k_rk2 takes this configuration's gas steps, or 0:
+// two stage launches. It covers 2D, the solvers and limiters that need no pass
+// or ghost cells between the stages, and grids that latency bounds. The lines by
+// the number of 8 x 64 tiles, microseconds a step of two stage launches / 4-row
+// / 8-row tiles: hydro 64^2 13.7 / 11.7 / 12.8, 256^2 (128 tiles) 15.4 / 12.6 /
+// 13.3, 384^2 (288) 19.2 / 20.2 / 17.9, 512^2 (512) 20.5 / 24.4 / 19.2, 700^2
+// (968) 29.3 / 40.7 / 29.8; MHD, first half only, 64^2 38.1 / 36.0 / 36.9, 256^2
+// 41.0 / 38.3 / 39.6, 512^2 45.5 / 47.2 / 43.4, 700^2 69.4 / 76.1 / 68.5.
+int rk2_rows(const amx_fv_config* cfg) {
+  if (cfg->dim != 2 || (cfg->riemann != AMX_HLL && cfg->riemann != AMX_HLLC) ||
+      (cfg->limiter != AMX_MINMOD && cfg->limiter != AMX_VAN_ALBADA))
+    return 0;
+  for (int k = 0; k < 4; ++k)
+    if (cfg->boundary[k] != AMX_BC_PERIODIC) return 0;
+  const long tiles = (long)((cfg->nx + 7) / 8) * ((cfg->ny + TB - 1) / TB);
+  if (tiles > 700) return 0;
+  return tiles <= 160 ? 4 : 8;
+}
+
+// (with k_rk2 the gas rows between the halves of an MHD step have rows of their own)
 long ws_fields(const amx_fv_config* cfg, int /*own_state*/) {
-  return (cfg->dim + 2) + (cfg->mhd ? 25 : 0);
+  return (cfg->dim + 2) + (cfg->mhd ? 25 + (rk2_rows(cfg) ? cfg->dim + 2 : 0) : 0);
 }
 long state_fields(const amx_fv_config* cfg) { return (cfg->dim + 2) + (cfg->mhd ? 3 : 0); }
 long cells(const amx_fv_config* cfg) { return (long)cfg->nx * cfg->ny * (cfg->dim == 3 ? cfg->nz : 1); }
@@ -2400,6 +2668,7 @@ void init_geometry(amx_fv_ctx* c, const amx_fv_config* cfg, int cap, int own_sta
   }
   c->ncx = (c->nxm + c->lx - 1) / c->lx;
   c->ncx_mag = (c->nxm + c->lx_mag - 1) / c->lx_mag;
+  c->rk2 = rk2_rows(cfg);
   c->cap = cap;
   c->own_state = own_state;
   const long per_slot = c->ncell * (ws_fields(cfg, own_state) + (own_state ? c->NS : 0));
@@ -2463,6 +2732,7 @@ amx_status make_ctx(const amx_fv_config* cfg, int cap, int own_state, amx_fv_ctx
 // Slot-0 addresses of the state rows and the workspace.
 struct Bufs {
   float* gas[5];
+  float* mid[5];   // gas rows between the two gas halves of an MHD step: the state's, or (k_rk2) rows of their own
   float* B[3];
   float* G1;
   float* P[4][6];  // iterate sets: launch k writes P[iterate_set(bset, k)]
@@ -2479,6 +2749,7 @@ Bufs bufs(const amx_fv_ctx* c, float* state) {
     for (int k = 0; k < 3; ++k) b.B[k] = state + (long)(c->NV + k) * n;
   float* ws = c->own_state ? c->mem + (long)c->NS * n : c->mem;
   b.G1 = ws;
+  for (int v = 0; v < c->NV; ++v) b.mid[v] = c->rk2 && c->cfg.mhd ? ws + (long)(c->NV + 25 + v) * n : b.gas[v];
   if (c->cfg.mhd)
     for (int j = 0; j < 3; ++j)
       for (int k = 0; k < 6; ++k) b.P[j][k] = ws + (long)(c->NV + 6 * j + k) * n;
@@ -2667,6 +2938,60 @@ hipError_t launch_cfl(const amx_fv_ctx* c, const float* state, int slot0, int ns
   return hipGetLastError();
 }
 
+// ---- both stages of a 2D gas step in one launch (k_rk2)
+Rk2Args rk2_base(const amx_fv_ctx* c, float dt_scale) {
+  Rk2Args a;
+  memset(&a, 0, sizeof(a));
+  a.ctl = c->ctl;
+  a.phs = c->dph;
+  a.sstride = c->sstride;
+  a.na = c->na;
+  a.nb = c->nb;
+  a.nta = (c->na + c->rk2 - 1) / c->rk2;
+  a.ntb = c->ntb;
+  a.dt_scale = dt_scale;
+  a.dxf = (float)c->cfg.grid_spacing;
+  return a;
+}
+
+template <int TA, bool HEUN>
+void launch_rk2_t(const amx_fv_ctx* c, const Rk2Args& a, int nspan, hipStream_t st) {
+  const dim3 grid((unsigned)(a.nta * a.ntb), nspan), block(1024);
+  const bool hllc = c->cfg.riemann == AMX_HLLC;
+  if (c->cfg.limiter == AMX_MINMOD) {
+    if (hllc)
+      hipLaunchKernelGGL((k_rk2<TA, AMX_HLLC, LX_MINMOD, HEUN>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_rk2<TA, AMX_HLL, LX_MINMOD, HEUN>), grid, block, 0, st, a);
+  } else if constexpr (HEUN) {  // the reverse mode covers minmod only
+    if (hllc)
+      hipLaunchKernelGGL((k_rk2<TA, AMX_HLLC, LX_VAN_ALBADA, HEUN>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_rk2<TA, AMX_HLL, LX_VAN_ALBADA, HEUN>), grid, block, 0, st, a);
+  }
+}
+
+template <bool HEUN>
+hipError_t launch_rk2(amx_fv_ctx* c, const Rk2Args& a, int nspan, hipStream_t st) {
+  const int e = time_begin(c, st);
+  if (c->rk2 == 8)
+    launch_rk2_t<8, HEUN>(c, a, nspan, st);
+  else
+    launch_rk2_t<4, HEUN>(c, a, nspan, st);
+  const hipError_t err = hipGetLastError();
+  time_end(c, st, e, CLS_STAGE, 0);
+  return err;
+}
+
+// the rows that k_rk2 wrote, home into the state's
+hipError_t rk2_home(const amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, int gate) {
+  const long n = (long)c->NV * c->ncell;
+  const long blocks = (n + 1023) / 1024;
+  hipLaunchKernelGGL(k_rows_home, dim3(blocks < 2048 ? blocks : 2048, nspan), dim3(256), 0, st, c->ctl, b.gas[0],
+                     b.G1, n, c->sstride, gate);
+  return hipGetLastError();
+}
+
 // Launches the fixed-point pair (L, L+1): input = launch L-1's output (the
 // state's B and gas velocity for L = 0); the kernel picks the iterate sets
 // from ctl->bset (iterate_set).
@@ -2678,10 +3003,10 @@ hipError_t launch_mag_pair(amx_fv_ctx* c, const Bufs& b, int L, int nspan, hipSt
   m.regen = regen;
   m.skip_mask = c->skip_mask;
   for (int k = 0; k < 3; ++k) m.B0[k] = b.B[k];
-  m.v0[0] = b.gas[1];
-  m.v0[1] = b.gas[2];
-  m.v0[2] = dim == 3 ? b.gas[3] : nullptr;
-  m.rho = b.gas[0];
+  m.v0[0] = b.mid[1];
+  m.v0[1] = b.mid[2];
+  m.v0[2] = dim == 3 ? b.mid[3] : nullptr;
+  m.rho = b.mid[0];
   for (int j = 0; j < 4; ++j)
     for (int k = 0; k < 6; ++k) m.PS[j][k] = b.P[j][k];
   m.L = L;
@@ -2705,6 +3030,19 @@ unsigned skip_mask_for(int upto) {
 // Phase 1: S_A(dt/2) and the speculative batch of fixed-point launches.
 amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, int want_cfl, int* klast) {
   const int NV = c->NV;
+  if (!c->cfg.mhd && c->rk2) {
+    Rk2Args a = rk2_base(c, 1.0f);
+    for (int v = 0; v < NV; ++v) {
+      a.src[v] = b.gas[v];
+      a.out[v] = b.G1 + (long)v * c->ncell;
+    }
+    a.want_cfl = want_cfl;
+    a.swap = c->rk2_swap;
+    HIPCHK((launch_rk2<true>(c, a, nspan, st)));
+    if (!c->rk2_swap) HIPCHK(rk2_home(c, b, nspan, st, 1));
+    *klast = 0;
+    return AMX_OK;
+  }
   if (!c->cfg.mhd) {
     // SSP-RK2 on the whole state: W1 = E(W0); W = prim(0.5 (U0 + cons(E(W1)))) in place
     StageArgs a1 = stage_base(c, 1.0f);
@@ -2729,24 +3067,33 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
     return AMX_OK;
   }
   const int dim = c->cfg.dim;
-  // ---- S_A(dt/2): RK2 with the result in place in the gas rows
-  StageArgs a1 = stage_base(c, 0.5f);
-  for (int v = 0; v < NV; ++v) {
-    a1.src[v] = b.gas[v];
-    a1.out[v] = b.G1 + (long)v * c->ncell;
+  // ---- S_A(dt/2): RK2 with the result in b.mid: in place, or (k_rk2) in rows of its own
+  if (c->rk2) {
+    Rk2Args a = rk2_base(c, 0.5f);
+    for (int v = 0; v < NV; ++v) {
+      a.src[v] = b.gas[v];
+      a.out[v] = b.mid[v];
+    }
+    HIPCHK((launch_rk2<true>(c, a, nspan, st)));
+  } else {
+    StageArgs a1 = stage_base(c, 0.5f);
+    for (int v = 0; v < NV; ++v) {
+      a1.src[v] = b.gas[v];
+      a1.out[v] = b.G1 + (long)v * c->ncell;
+    }
+    int e = time_begin(c, st);
+    HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a1, nspan, st)));
+    time_end(c, st, e, CLS_STAGE, 0);
+    StageArgs a2 = stage_base(c, 0.5f);
+    for (int v = 0; v < NV; ++v) {
+      a2.src[v] = b.G1 + (long)v * c->ncell;
+      a2.w0[v] = b.gas[v];
+      a2.out[v] = b.gas[v];
+    }
+    e = time_begin(c, st);
+    HIPCHK((launch_stage<SRC_PLAIN, true, SRC_PLAIN>(c, a2, nspan, st)));
+    time_end(c, st, e, CLS_STAGE, 0);
   }
-  int e = time_begin(c, st);
-  HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a1, nspan, st)));
-  time_end(c, st, e, CLS_STAGE, 0);
-  StageArgs a2 = stage_base(c, 0.5f);
-  for (int v = 0; v < NV; ++v) {
-    a2.src[v] = b.G1 + (long)v * c->ncell;
-    a2.w0[v] = b.gas[v];
-    a2.out[v] = b.gas[v];
-  }
-  e = time_begin(c, st);
-  HIPCHK((launch_stage<SRC_PLAIN, true, SRC_PLAIN>(c, a2, nspan, st)));
-  time_end(c, st, e, CLS_STAGE, 0);
   // ---- S_B(dt): fixed point on (B, v) with rho from the gas, in pairs of
   // launches; the speculative batch covers the last step's launch count
   const int maxit = c->cfg.max_fixed_point_iterations;
@@ -2831,7 +3178,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   HIPCHK(hipGetLastError());
   StageArgs b1 = stage_base(c, 0.5f);
   for (int v = 0; v < NV; ++v) {
-    b1.src[v] = b.gas[v];
+    b1.src[v] = b.mid[v];
     b1.out[v] = b.G1 + (long)v * c->ncell;
   }
   b1.pfix = b.PF;
@@ -2847,7 +3194,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   StageArgs b2 = stage_base(c, 0.5f);
   for (int v = 0; v < NV; ++v) {
     b2.src[v] = b.G1 + (long)v * c->ncell;
-    b2.w0[v] = b.gas[v];
+    b2.w0[v] = b.mid[v];
     b2.out[v] = b.gas[v];
   }
   for (int j = 0; j < 4; ++j)
@@ -3177,14 +3524,16 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // next step's B0) and is copied into the state once, after the loop.
   struct KeepB {
     amx_fv_ctx* c;
-    ~KeepB() { c->keep_b = 0; }
+    ~KeepB() { c->keep_b = c->rk2_swap = 0; }
   } keep_guard{c};
   // (a record takes the whole state of every step)
   c->keep_b = c->cfg.mhd && !snp && !c->hook && !rec ? 1 : 0;
   auto record = [&]() -> hipError_t {
     if (!rec) return hipSuccess;
+    RecordArgs ra = *rec;
+    ra.odd = c->rk2_swap ? c->mem : nullptr;
     const long blocks = rec->max_inputs > 0 ? (rec->n + 1023) / 1024 : 1;
-    hipLaunchKernelGGL(k_record, dim3(blocks < 4096 ? blocks : 4096), dim3(256), 0, st, c->ctl, *rec);
+    hipLaunchKernelGGL(k_record, dim3(blocks < 4096 ? blocks : 4096), dim3(256), 0, st, c->ctl, ra);
     return hipGetLastError();
   };
   const Bufs bl = bufs(c, state);
@@ -3205,6 +3554,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // between steps: they are queued in batches and t is read once per batch
   // (k_step_begin clears ctl.run past the end, so surplus steps do nothing).
   const bool batch = !c->cfg.mhd && !snp && !c->hook;
+  c->rk2_swap = batch && c->rk2;
   // MHD steps of such loops are queued in batches too, each with its
   // speculative fixed-point launches and its second half behind them; the
   // device decides whether each step's launches settled the fixed point. A
@@ -3364,6 +3714,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   if (c->keep_b && !b_home) {
     HIPCHK(copy_b_home(c, bl, st, 0));
   }
+  if (c->rk2_swap && (steps & 1)) HIPCHK(rk2_home(c, bl, 1, st, 0));
   if (!b_home) {
     HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cflp), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
@@ -3397,7 +3748,7 @@ extern "C" amx_status amx_fv_time_integration_recorded(amx_fv_ctx* c, float* sta
     return fail(AMX_ERR_INVALID, "record arrays missing%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   if (run->fixed_timestep && run->num_timesteps <= 0) return fail(AMX_ERR_INVALID, "num_timesteps must be positive%s");
-  const RecordArgs rec = {state, inputs, dts, (long)c->NS * c->ncell, max_inputs, max_dts};
+  const RecordArgs rec = {state, nullptr, inputs, dts, (long)c->NS * c->ncell, max_inputs, max_dts};
   return fv_loop(c, state, run, nullptr, stats, (hipStream_t)stream, &rec);
 }
 
@@ -3488,6 +3839,15 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
   float* L1 = NU + (long)NV * n;       // lam of W1
   float* CON = L1 + (long)NV * n;      // DIM x 4 x NV interface contributions
   // recompute the two stage states with the forward kernel (dt in ctl[0])
+  if (DIM == 2 && c->rk2) {
+    Rk2Args a = rk2_base(c, dt_scale);
+    for (int v = 0; v < NV; ++v) {
+      a.src[v] = w0 + (long)v * n;
+      a.out[v] = G1 + (long)v * n;
+      a.out2[v] = G2 + (long)v * n;
+    }
+    HIPCHK((launch_rk2<false>(c, a, 1, st)));
+  } else {
   StageArgs a1 = stage_base(c, dt_scale);
   for (int v = 0; v < NV; ++v) {
     a1.src[v] = w0 + (long)v * n;
@@ -3500,6 +3860,7 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
     a2.out[v] = G2 + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a2, 1, st)));
+  }
   const Phys ph = c->hph[0];  // the interface kernels read dt from ctl[0]
   // AMX_ADJ_DUAL=1: the flux Jacobians by dual numbers (a cross-check of the reverse sweep)
   const bool duals = env_int("AMX_ADJ_DUAL", 0) != 0;
@@ -3596,6 +3957,14 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
   if (r != AMX_OK) return r;
   // ---- forward: S_A(dt/2) of the state's gas rows into W_A
   float* G1 = c->mem;
+  if (c->rk2) {
+    Rk2Args a = rk2_base(c, 0.5f);
+    for (int v = 0; v < NV; ++v) {
+      a.src[v] = state + (long)v * n;
+      a.out[v] = c->adjm + (long)v * n;
+    }
+    HIPCHK((launch_rk2<true>(c, a, 1, st)));
+  } else {
   StageArgs a1 = stage_base(c, 0.5f);
   for (int v = 0; v < NV; ++v) {
     a1.src[v] = state + (long)v * n;
@@ -3609,6 +3978,7 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
     a2.out[v] = c->adjm + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, true, SRC_PLAIN>(c, a2, 1, st)));
+  }
   // ---- forward: the fixed point, launch k's output to iterate slot k. The
   // pairs of the last step's count are queued before the residuals are read.
   c->skip_mask = 0u;
@@ -3622,7 +3992,7 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
     if (r != AMX_OK) return r;
     Bufs b;
     memset(&b, 0, sizeof(b));
-    for (int v = 0; v < NV; ++v) b.gas[v] = c->adjm + (long)v * n;
+    for (int v = 0; v < NV; ++v) b.mid[v] = c->adjm + (long)v * n;
     for (int k = 0; k < 3; ++k) b.B[k] = const_cast<float*>(state) + (long)(NV + k) * n;
     float* IT = c->adjm + adjm_fixed_fields(c) * n;
     for (; L <= upto; L += 2) {
