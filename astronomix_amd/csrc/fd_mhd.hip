@@ -24,6 +24,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -88,6 +89,15 @@ __device__ __forceinline__ unsigned nb(const Grid& g, const Pos& p, int axis, in
   return p.o + (out ? wrapped : in);
 }
 
+// step control of the FD loop: dt, t and the slotted CFL partial maxima
+struct Ctl {
+  float dt;
+  float t;
+  int steps;
+  int run;  // the current step is taken (a step queued past the loop's end is not)
+  unsigned cflp[3][NSLOT];
+};
+
 __device__ __forceinline__ float dss(float x) { return fsqrt(fmaxf(x, 1e-12f)); }
 
 // Rows of a direction's frame in the state's numbering (the reference's swaps
@@ -131,6 +141,44 @@ __device__ __forceinline__ void cell_speeds(const float* q, float* sp, const Phy
   sp[1] = dss(fmaxf(0.f, 0.5f * (s + droot)));
   sp[2] = dss(fmaxf(0.f, (Bx * Bx) * rinv));
   sp[3] = dss(fmaxf(0.f, 0.5f * (s - droot)));
+}
+
+// _cfl_time_step_fd (_timestep_estimator.py(FD):25-87): mx[d] = max of itself and
+// |lambda| of the 7 modes along d of the conserved state of the primitive row values w
+__device__ __forceinline__ void cfl_speeds(const float* w, const Phys& ph, float* mx) {
+  const float rho = w[0];
+  const float vx = w[1], vy = w[2], vz = w[3];
+  const float Bx = w[5], By = w[6], Bz = w[7];
+  const float u2 = (vx * vx + vy * vy) + vz * vz;
+  const float b2 = (Bx * Bx + By * By) + Bz * Bz;
+  const float u[8] = {rho, rho * vx, rho * vy, rho * vz, (w[4] * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2, Bx, By, Bz};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    float r[8], sp[4];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) r[v] = u[perm(d, v)];
+    cell_speeds(r, sp, ph);
+    const float l[7] = {sp[0] - sp[1], sp[0] - sp[2], sp[0] - sp[3], sp[0], sp[0] + sp[3], sp[0] + sp[2], sp[0] + sp[1]};
+#pragma unroll
+    for (int s = 0; s < 7; ++s) {
+      const float m = fabsf(l[s]);
+      mx[d] = (m != m || m > mx[d]) ? m : mx[d];
+    }
+  }
+}
+
+// A block's maxima into its slot: an atomic only where the slot is still
+// below (an L2 round trip each; at one block per 256 cells of a 256^3 grid the
+// unconditional ones took longer than the pass over the state).
+__device__ __forceinline__ void cfl_reduce(const float* mx, Ctl* ctl, unsigned (*sred)[4]) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const unsigned m = block_max_u<4>(canon_bits(mx[d]), sred[d]);
+    if (threadIdx.x == 0) {
+      unsigned* slot = &ctl->cflp[d][blockIdx.x & (NSLOT - 1)];
+      if (m > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(slot, m);
+    }
+  }
 }
 
 // LDS fields of a staged cell, in the direction's frame.
@@ -324,6 +372,7 @@ struct WenoDir {
 };
 
 struct WenoArgs {
+  const Ctl* ctl;
   WenoDir d[3];
   unsigned first[4];  // first block of each direction, and the number of blocks
   int zin;            // interfaces of a z block
@@ -448,6 +497,7 @@ __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, 
 // 32 -> 12 us, three launches in one.
 __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_weno(const WenoArgs a) {
   __shared__ float s[NFIELD][NCELL];
+  if (!a.ctl->run) return;
   const Grid g = a.g;
   const Phys ph = a.ph;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
@@ -546,11 +596,16 @@ __device__ __forceinline__ float c2f(const Grid& g, const float* a, const Pos& p
   return (((-ld(a, nb(g, p, ax, -1)) + 9.f * ld(a, p.o)) + 9.f * ld(a, nb(g, p, ax, 1))) - ld(a, nb(g, p, ax, 2))) * (1.f / 16.f);
 }
 
+// of the faces at offsets -3 .. 2
+__device__ __forceinline__ float f2c_of(const float* f) {
+  return (((((3.f * f[0] - 25.f * f[1]) + 150.f * f[2]) + 150.f * f[3]) - 25.f * f[4]) + 3.f * f[5]) * (1.f / 256.f);
+}
+
 __device__ __forceinline__ float f2c(const Grid& g, const float* f, const Pos& p, int ax) {
-  return (((((3.f * ld(f, nb(g, p, ax, -3)) - 25.f * ld(f, nb(g, p, ax, -2))) + 150.f * ld(f, nb(g, p, ax, -1))) + 150.f * ld(f, p.o)) -
-           25.f * ld(f, nb(g, p, ax, 1))) +
-          3.f * ld(f, nb(g, p, ax, 2))) *
-         (1.f / 256.f);
+  float v[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) v[k] = ld(f, k == 3 ? p.o : nb(g, p, ax, k - 3));
+  return f2c_of(v);
 }
 
 __device__ __forceinline__ float d6(const Grid& g, const float* f, const Pos& p, int ax) {
@@ -569,21 +624,15 @@ __device__ __forceinline__ float p2a(const Grid& g, const float* q, const Pos& p
   for (unsigned c = blockIdx.x * blockDim.x + threadIdx.x; c < (unsigned)(g).nc; \
        c += gridDim.x * blockDim.x)
 
-// Conserved rows of a primitive state (_equations.py:65-101).
-__device__ __forceinline__ void conserved(const float* const* w, unsigned o, const Phys& ph, float* q) {
-  const float rho = ld(w[0], o);
-  const float vx = ld(w[1], o), vy = ld(w[2], o), vz = ld(w[3], o);
-  const float Bx = ld(w[5], o), By = ld(w[6], o), Bz = ld(w[7], o);
+// Conserved rows of the primitive ones (rho, v, p, B), in place (_equations.py:65-101).
+__device__ __forceinline__ void conserved(float* q, const Phys& ph) {
+  const float rho = q[0], vx = q[1], vy = q[2], vz = q[3];
   const float u2 = (vx * vx + vy * vy) + vz * vz;
-  const float b2 = (Bx * Bx + By * By) + Bz * Bz;
-  q[0] = rho;
+  const float b2 = (q[5] * q[5] + q[6] * q[6]) + q[7] * q[7];
   q[1] = rho * vx;
   q[2] = rho * vy;
   q[3] = rho * vz;
-  q[4] = (ld(w[4], o) * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2;
-  q[5] = Bx;
-  q[6] = By;
-  q[7] = Bz;
+  q[4] = (q[4] * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2;
 }
 
 // _enforce_positivity of conserved rows with the field energy b2/2 (_enforce_positivity.py:21-59)
@@ -609,6 +658,7 @@ __device__ __forceinline__ void centre_field(const Grid& g, const float* const* 
 // (R11 W8): with the copies of q0 in three buffers and a pass of its own for
 // the floors it moved 49 fields.
 struct FirstArgs {
+  const Ctl* ctl;
   const float* w[11];
   float* q[4];
   float* qt[4];
@@ -617,12 +667,15 @@ struct FirstArgs {
 };
 
 __global__ void k_first(const FirstArgs a) {
+  if (!a.ctl->run) return;
   const Grid g = a.g;
   const Phys ph = a.ph;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
     float q[8], B[3];
-    conserved(a.w, P.o, ph, q);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) q[v] = ld(a.w[v], P.o);
+    conserved(q, ph);
     const float b2 = (q[5] * q[5] + q[6] * q[6]) + q[7] * q[7];
     if (ph.positivity) floor_state(q[0], q[4], q + 1, b2, ph);
     centre_field(g, a.w + 8, P, B);
@@ -637,6 +690,7 @@ __global__ void k_first(const FirstArgs a) {
 
 // edge EMFs (_constrained_transport.py:104-131)
 struct EdgeArgs {
+  const Ctl* ctl;
   const float* fyx;  // B_y flux at x-faces (modified)
   const float* fzx;  // B_z flux at x-faces
   const float* fxy;  // B_x flux at y-faces
@@ -648,28 +702,35 @@ struct EdgeArgs {
 };
 
 __global__ void k_ct_edge(const EdgeArgs a) {
+  if (!a.ctl->run) return;
   const Grid g = a.g;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    st(a.O[2], P.o, c2f(g, a.fxy, P, 0) - c2f(g, a.fyx, P, 1));
-    st(a.O[0], P.o, c2f(g, a.fyz, P, 1) - c2f(g, a.fzy, P, 2));
-    st(a.O[1], P.o, c2f(g, a.fzx, P, 2) - c2f(g, a.fxz, P, 0));
+    const float oz = c2f(g, a.fxy, P, 0) - c2f(g, a.fyx, P, 1);
+    const float ox = c2f(g, a.fyz, P, 1) - c2f(g, a.fzy, P, 2);
+    const float oy = c2f(g, a.fzx, P, 2) - c2f(g, a.fxz, P, 0);
+    st(a.O[2], P.o, oz);
+    st(a.O[0], P.o, ox);
+    st(a.O[1], P.o, oy);
   }
 }
 
 struct AvgArgs {
+  const Ctl* ctl;
   const float* O[3];
   float* Ob[3];
   Grid g;
 };
 
 __global__ void k_ct_avg(const AvgArgs a) {
+  if (!a.ctl->run) return;
   const Grid g = a.g;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
-    st(a.Ob[2], P.o, p2a(g, a.O[2], P, 0, 1));
-    st(a.Ob[0], P.o, p2a(g, a.O[0], P, 1, 2));
-    st(a.Ob[1], P.o, p2a(g, a.O[1], P, 0, 2));
+    const float oz = p2a(g, a.O[2], P, 0, 1), ox = p2a(g, a.O[0], P, 1, 2), oy = p2a(g, a.O[1], P, 0, 2);
+    st(a.Ob[2], P.o, oz);
+    st(a.Ob[0], P.o, ox);
+    st(a.Ob[1], P.o, oy);
   }
 }
 
@@ -688,7 +749,7 @@ struct FaceArgs {
   const float* b0[3];
   float* bc[3];
   float* bf[3];
-  const float* dtp;
+  const Ctl* ctl;
   float inv_dx, ff0;
   Coef k;
   Grid g;
@@ -697,8 +758,9 @@ struct FaceArgs {
 // 6th-order curl of the averaged EMFs and the stage combine of the faces
 template <int ST>
 __global__ void k_face(const FaceArgs a) {
+  if (!a.ctl->run) return;
   const Grid g = a.g;
-  const float dtdx = (a.k.k2 * (*a.dtp)) * a.inv_dx;
+  const float dtdx = (a.k.k2 * a.ctl->dt) * a.inv_dx;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
     const float r[3] = {(-dtdx) * d6(g, a.Ob[2], P, 1) + dtdx * d6(g, a.Ob[1], P, 2),
@@ -733,8 +795,9 @@ struct CombineArgs {
   float* qf[8];
   const float* b[3];     // the stage's new faces
   float* qt[4];
-  const float* dtp;
+  Ctl* ctl;
   float inv_dx, ff0;
+  int want_cfl;          // last stage: the CFL maxima of the new state
   int floors;            // of the next stage's input
   Coef k;
   Grid g;
@@ -751,31 +814,54 @@ struct CombineArgs {
 // of 302.
 template <int ST>
 __global__ void k_combine(const CombineArgs a) {
+  __shared__ unsigned sred[3][4];
+  if (!a.ctl->run) return;
+  float mx[3] = {0.f, 0.f, 0.f};
   const Grid g = a.g;
   const Phys ph = a.ph;
-  const float dtdx = (a.k.k2 * (*a.dtp)) * a.inv_dx;
+  const float dtdx = (a.k.k2 * a.ctl->dt) * a.inv_dx;
   FD_LOOP(g) {
     const Pos P = pos_of(g, c);
     const unsigned xm = nb(g, P, 0, -1), ym = nb(g, P, 1, -1), zm = nb(g, P, 2, -1);
-    // every load before the first store, which the compiler may not move them past
-    float q0[8], q[8], qf[8], B[3];
-    if (ST != ST_LAST) conserved(a.w, P.o, ph, q0);
+    // Every load first, and kept there by the scheduling barrier: left to
+    // itself the compiler paired them with their uses, two in flight at a time
+    // (1119 instead of 860 us in the stages that carry all rows).
+    float q0[8], q[8], qf[8], qc[8], B[3], f0[3][8], f1[3][8], bf[3][6];
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      float div = v == 5 ? 0.f : ld(a.F[0][v], P.o) - ld(a.F[0][v], xm);
-      if (v != 6) div += ld(a.F[1][v], P.o) - ld(a.F[1][v], ym);
-      if (v != 7) div += ld(a.F[2][v], P.o) - ld(a.F[2][v], zm);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        if (v == 5 + d) continue;
+        f0[d][v] = ld(a.F[d][v], P.o);
+        f1[d][v] = ld(a.F[d][v], d == 0 ? xm : (d == 1 ? ym : zm));
+      }
+      if (ST != ST_LAST) q0[v] = ld(a.w[v], P.o);
+      if (ST >= ST_MID) qf[v] = ld(a.qf[v], P.o);
+      if (ST == ST_SECOND || ST == ST_MID) qc[v] = ld(a.qc[v], P.o);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) bf[i][k] = ld(a.b[i], k == 3 ? P.o : nb(g, P, i, k - 3));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (ST != ST_LAST) conserved(q0, ph);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      float div = v == 5 ? 0.f : f0[0][v] - f1[0][v];
+      if (v != 6) div += f0[1][v] - f1[1][v];
+      if (v != 7) div += f0[2][v] - f1[2][v];
       const float rhs = (-dtdx) * div;
-      qf[v] = ST >= ST_MID ? ld(a.qf[v], P.o) : 0.f;
       if (ST == ST_LAST) {
         q[v] = qf[v] + rhs;
         continue;
       }
-      q[v] = ST == ST_FIRST ? __fmul_rn(a.k.k1, q0[v]) + rhs : (a.k.k1 * q0[v] + a.k.k3 * ld(a.qc[v], P.o)) + rhs;
+      q[v] = ST == ST_FIRST ? __fmul_rn(a.k.k1, q0[v]) + rhs : (a.k.k1 * q0[v] + a.k.k3 * qc[v]) + rhs;
       if (ST == ST_SECOND) qf[v] = __fmul_rn(a.ff0, q0[v]);
-      qf[v] = qf[v] + q[v] * a.k.ff;
+      if (ST != ST_FIRST) qf[v] = qf[v] + q[v] * a.k.ff;
     }
-    centre_field(g, a.b, P, B);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) B[i] = f2c_of(bf[i]);
     const float ob2 = (q[5] * q[5] + q[6] * q[6]) + q[7] * q[7];
     const float nb2 = (B[0] * B[0] + B[1] * B[1]) + B[2] * B[2];
     if (ST != ST_LAST) {
@@ -799,9 +885,6 @@ __global__ void k_combine(const CombineArgs a) {
         rho = fmaxf(rho, ph.rhomin);
         p = fmaxf(p, ph.pgmin);
       }
-      float bf[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) bf[i] = ld(a.b[i], P.o);
       st(a.w[0], P.o, rho);
       st(a.w[1], P.o, ux);
       st(a.w[2], P.o, uy);
@@ -810,66 +893,89 @@ __global__ void k_combine(const CombineArgs a) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         st(a.w[5 + i], P.o, B[i]);
-        st(a.w[8 + i], P.o, bf[i]);
+        st(a.w[8 + i], P.o, bf[i][3]);
+      }
+      if (a.want_cfl) {
+        const float wn[8] = {rho, ux, uy, uz, p, B[0], B[1], B[2]};
+        cfl_speeds(wn, ph, mx);
       }
     }
   }
+  if (ST == ST_LAST && a.want_cfl) cfl_reduce(mx, a.ctl, sred);
 }
-
-// step control of the FD loop: dt, t and the slotted CFL partial maxima
-struct Ctl {
-  float dt;
-  float t;
-  int steps;
-  int pad;
-  unsigned cflp[3][NSLOT];
-};
 
 struct StepParams {
   float t_end, C, dx, dt_max;
-  int fixed, num_timesteps, exact_end, use_cfl;
+  int fixed, num_timesteps, exact_end;
+  int any_time;      // no loop: the step size of a state by itself
   int clamp_tp = 0;  // clamp dt to tp - t (snapshot time points, time_integration.py:671-674)
   float tp = 0.f;
 };
 
-// One wavefront, a lane per partial slot; the scalars are the same in every lane.
-// dt = min(C dx / (lx + ly + lz), dt_max) (_timestep_estimator.py(FD):89-90),
-// or t_end / num_timesteps; clamp to t_end - t (time_integration.py:667-678)
-__global__ void k_step_begin(Ctl* c, StepParams p) {
+// One wavefront, a lane per partial slot; the scalars are the same in every
+// lane, and everything read is loaded before the first store.
+//
+// END: the end of a step. BEGIN: the next step's dt = min(C dx / (lx + ly + lz),
+// dt_max) (_timestep_estimator.py(FD):89-90), or t_end / num_timesteps; clamp to
+// t_end - t (time_integration.py:667-678); and whether there is one.
+template <bool END, bool BEGIN>
+__device__ __forceinline__ void step_control(Ctl* c, const StepParams& p) {
+  const int run = c->run;
+  const float dt0 = c->dt;
+  float t = c->t;
+  int steps = c->steps;
+  unsigned m[3] = {0u, 0u, 0u};
+  if (BEGIN) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) m[d] = c->cflp[d][threadIdx.x];
+  }
+  if (END && run) {
+    t = t + dt0;
+    steps += 1;
+    c->t = t;
+    c->steps = steps;
+  }
+  if (!BEGIN) return;
+  const int go = p.fixed ? steps < p.num_timesteps : (p.any_time || t < p.t_end);
+  c->run = go;
+  if (!go) return;
   float dt;
   if (p.fixed) {
     dt = p.t_end / (float)p.num_timesteps;
-  } else if (p.use_cfl) {
+  } else {
     float l[3];
-    for (int d = 0; d < 3; ++d) l[d] = __uint_as_float(slots_max(c->cflp[d]));
+#pragma unroll
+    for (int d = 0; d < 3; ++d) l[d] = __uint_as_float(wave_max_u(m[d]));
     dt = (p.C * p.dx) / ((l[0] + l[1]) + l[2]);
     dt = p.dt_max < dt ? p.dt_max : dt;
-  } else {
-    dt = c->dt;
   }
   if (p.clamp_tp) {
-    const float rem = p.tp - c->t;
+    const float rem = p.tp - t;
     dt = rem < dt ? rem : dt;
   }
   if (p.exact_end) {
-    const float rem = p.t_end - c->t;
+    const float rem = p.t_end - t;
     dt = rem < dt ? rem : dt;
   }
   c->dt = dt;
+#pragma unroll
   for (int d = 0; d < 3; ++d) c->cflp[d][threadIdx.x] = 0u;
 }
 
-__global__ void k_set_dt(Ctl* c, const float* dtp) { c->dt = *dtp; }
+__global__ void k_step_begin(Ctl* c, StepParams p) { step_control<false, true>(c, p); }
+__global__ void k_step_end(Ctl* c) { step_control<true, false>(c, StepParams()); }
+__global__ void k_step_end_begin(Ctl* c, StepParams p) { step_control<true, true>(c, p); }
 
-__global__ void k_step_end(Ctl* c) {
-  c->t = c->t + c->dt;
-  c->steps += 1;
+__global__ void k_set_dt(Ctl* c, const float* dtp) {
+  c->dt = *dtp;
+  c->run = 1;
 }
 
 __global__ void k_reset(Ctl* c) {
   c->dt = 0.f;
   c->t = 0.f;
   c->steps = 0;
+  c->run = 0;
   for (int d = 0; d < 3; ++d) c->cflp[d][threadIdx.x] = 0u;
 }
 
@@ -921,7 +1027,6 @@ amx_status fd_validate(const amx_fd_config* c) {
 
 dim3 fd_grid(const amx_fd_ctx* c) {
   long b = (c->g.nc + 255) / 256;
-  if (b > 256L * 64) b = 256L * 64;
   return dim3((unsigned)b);
 }
 
@@ -962,6 +1067,7 @@ void fd_tresolve(amx_fd_ctx* c) {
 hipError_t launch_weno(amx_fd_ctx* c, hipStream_t st) {
   const Grid& g = c->g;
   WenoArgs a;
+  a.ctl = c->ctl;
   for (int d = 0; d < 3; ++d) {
     for (int v = 0; v < 8; ++v) {
       const int r = FRAME[d][v];
@@ -997,12 +1103,13 @@ const float K3[5] = {0.0f, 0.55562950593266f, 0.37989814861460f, 0.8219200458922
 const float FF[5] = {-2.081261929715610e-02f, 0.0f, 0.51723167208978f, -6.518979800418380e-12f, 5.03580947213895e-01f};
 
 // one _evolve_state_fd on the (11, nx, ny, nz) state with dt in ctl->dt
-amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
+amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st, int want_cfl) {
   const long nc = c->g.nc;
   float* w[11];
   for (int v = 0; v < 11; ++v) w[v] = state + (long)v * nc;
   const dim3 grid = fd_grid(c), blk(256);
   FirstArgs ia;
+  ia.ctl = c->ctl;
   for (int v = 0; v < 11; ++v) ia.w[v] = w[v];
   for (int v = 0; v < 4; ++v) {
     ia.q[v] = c->QC[v];
@@ -1012,7 +1119,6 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
   ia.ph = c->ph;
   hipLaunchKernelGGL(k_first, grid, blk, 0, st, ia);
   AMX_HIPCHK(hipGetLastError());
-  const float* dtp = &c->ctl->dt;
   for (int s = 0; s < 5; ++s) {
     Coef k;
     k.k1 = K1[s];
@@ -1021,6 +1127,7 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     k.ff = s < 4 ? FF[s + 1] : 0.f;
     AMX_HIPCHK(launch_weno(c, st));
     EdgeArgs ea;
+    ea.ctl = c->ctl;
     ea.fyx = c->MOD[0];
     ea.fzx = c->MOD[1];
     ea.fxy = c->MOD[2];
@@ -1032,6 +1139,7 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     hipLaunchKernelGGL(k_ct_edge, grid, blk, 0, st, ea);
     AMX_HIPCHK(hipGetLastError());
     AvgArgs av;
+    av.ctl = c->ctl;
     for (int i = 0; i < 3; ++i) {
       av.O[i] = c->OM[i];
       av.Ob[i] = c->OMB[i];
@@ -1046,7 +1154,7 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
       fa.bc[i] = c->BC[i];
       fa.bf[i] = c->BF[i];
     }
-    fa.dtp = dtp;
+    fa.ctl = c->ctl;
     fa.inv_dx = c->inv_dx;
     fa.ff0 = FF[0];
     fa.k = k;
@@ -1063,7 +1171,8 @@ amx_status fd_step(amx_fd_ctx* c, float* state, hipStream_t st) {
     for (int v = 0; v < 11; ++v) qa.w[v] = w[v];
     for (int v = 0; v < 4; ++v) qa.qt[v] = c->QT[v];
     for (int i = 0; i < 3; ++i) qa.b[i] = s == 4 ? c->BF[i] : c->BC[i];
-    qa.dtp = dtp;
+    qa.ctl = c->ctl;
+    qa.want_cfl = want_cfl;
     qa.inv_dx = c->inv_dx;
     qa.ff0 = FF[0];
     qa.floors = s + 1 < 4 && c->ph.positivity;  // the last stage's input has none (_ssprk.py:333-335)
@@ -1169,39 +1278,18 @@ struct CflArgs {
   Ctl* ctl;
 };
 
-// _cfl_time_step_fd maxima: per direction, max over cells and the 7 modes of
-// |lambda| of the conserved state of w (_timestep_estimator.py(FD):25-87)
+// the CFL maxima of a state (the step loop takes them in its last k_combine)
 __global__ void k_cfl(const CflArgs a) {
   __shared__ unsigned sred[3][4];
   const Grid g = a.g;
-  const Phys ph = a.ph;
   float mx[3] = {0.f, 0.f, 0.f};
   FD_LOOP(g) {
-    const float rho = ld(a.w[0], 4u * c);
-    const float vx = ld(a.w[1], 4u * c), vy = ld(a.w[2], 4u * c), vz = ld(a.w[3], 4u * c);
-    const float Bx = ld(a.w[5], 4u * c), By = ld(a.w[6], 4u * c), Bz = ld(a.w[7], 4u * c);
-    const float u2 = (vx * vx + vy * vy) + vz * vz;
-    const float b2 = (Bx * Bx + By * By) + Bz * Bz;
-    const float u[8] = {rho, rho * vx, rho * vy, rho * vz, (ld(a.w[4], 4u * c) * ph.inv_gm1 + (0.5f * rho) * u2) + 0.5f * b2, Bx, By, Bz};
+    float w[8];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      float r[8], sp[4];
-#pragma unroll
-      for (int v = 0; v < 8; ++v) r[v] = u[perm(d, v)];
-      cell_speeds(r, sp, ph);
-      const float l[7] = {sp[0] - sp[1], sp[0] - sp[2], sp[0] - sp[3], sp[0], sp[0] + sp[3], sp[0] + sp[2], sp[0] + sp[1]};
-#pragma unroll
-      for (int s = 0; s < 7; ++s) {
-        const float m = fabsf(l[s]);
-        mx[d] = (m != m || m > mx[d]) ? m : mx[d];
-      }
-    }
+    for (int v = 0; v < 8; ++v) w[v] = ld(a.w[v], 4u * c);
+    cfl_speeds(w, a.ph, mx);
   }
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const unsigned m = block_max_u<4>(canon_bits(mx[d]), sred[d]);
-    if (threadIdx.x == 0 && m) atomicMax(&a.ctl->cflp[d][blockIdx.x & (NSLOT - 1)], m);
-  }
+  cfl_reduce(mx, a.ctl, sred);
 }
 
 }  // namespace fd
@@ -1215,11 +1303,12 @@ hipError_t fd_cfl(amx_fd_ctx* c, const float* state, hipStream_t st) {
   a.g = c->g;
   a.ph = c->ph;
   a.ctl = c->ctl;
-  hipLaunchKernelGGL(k_cfl, fd_grid(c), dim3(256), 0, st, a);
+  const dim3 grid = fd_grid(c);  // fewer blocks, each with one atomic per direction
+  hipLaunchKernelGGL(k_cfl, dim3(grid.x < 4096 ? grid.x : 4096), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
-StepParams fd_params(const amx_fd_ctx* c, const amx_fv_run* run, int use_cfl) {
+StepParams fd_params(const amx_fd_ctx* c, const amx_fv_run* run) {
   StepParams p;
   p.t_end = run ? run->t_end : 0.f;
   p.C = c->cfg.C_cfl;
@@ -1228,7 +1317,7 @@ StepParams fd_params(const amx_fd_ctx* c, const amx_fv_run* run, int use_cfl) {
   p.fixed = run ? run->fixed_timestep : 0;
   p.num_timesteps = run ? run->num_timesteps : 1;
   p.exact_end = run ? run->exact_end_time : 0;
-  p.use_cfl = use_cfl;
+  p.any_time = !run;
   return p;
 }
 
@@ -1240,7 +1329,7 @@ extern "C" amx_status amx_fd_cfl_dt(amx_fd_ctx* c, const float* state, float* d_
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl);
   AMX_HIPCHK(hipGetLastError());
   AMX_HIPCHK(fd_cfl(c, state, st));
-  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, fd_params(c, nullptr, 1));
+  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, fd_params(c, nullptr));
   hipLaunchKernelGGL(k_dt_out, dim3(1), dim3(1), 0, st, (const Ctl*)c->ctl, d_dt);
   AMX_HIPCHK(hipGetLastError());
   return AMX_OK;
@@ -1251,7 +1340,7 @@ extern "C" amx_status amx_fd_evolve_state(amx_fd_ctx* c, float* state, const flo
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(1), 0, st, c->ctl, d_dt);
   AMX_HIPCHK(hipGetLastError());
-  return fd_step(c, state, st);
+  return fd_step(c, state, st, 0);
 }
 
 namespace {
@@ -1282,11 +1371,18 @@ amx_status fd_loop(amx_fd_ctx* c, float* state, const amx_fv_run* run, amx::snap
                    hipStream_t st) {
   hipLaunchKernelGGL(k_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl);
   AMX_HIPCHK(hipGetLastError());
-  StepParams sp = fd_params(c, run, 1);
+  StepParams sp = fd_params(c, run);
   // the end-time clamp is off with snapshot time points (time_integration.py:677)
   if (snp && snp->spec->use_timepoints) sp.exact_end = 0;
   long steps = 0;
-  float t = 0.f;
+  float t = 0.f, dt = 0.f;
+  // Without snapshot rows or a hook nothing is needed from the host between
+  // steps: they are queued in batches, one readback each, as many as the last
+  // dt says are left (16 at most; one at first). Steps queued past the end do
+  // nothing (ctl.run). The CFL maxima of a new state come from its last stage.
+  const bool batch = !snp && !c->hook;
+  const int want_cfl = !run->fixed_timestep;
+  if (want_cfl) AMX_HIPCHK(fd_cfl(c, state, st));
   for (;;) {
     if (run->fixed_timestep) {
       if (steps >= run->num_timesteps) break;
@@ -1300,22 +1396,37 @@ amx_status fd_loop(amx_fd_ctx* c, float* state, const amx_fv_run* run, amx::snap
       sp.clamp_tp = snp->clamp();
       if (sp.clamp_tp) sp.tp = snp->clamp_target();
     }
-    if (!run->fixed_timestep) AMX_HIPCHK(fd_cfl(c, state, st));
+    long n = 1;
+    if (batch) {
+      long left = run->fixed_timestep ? run->num_timesteps - steps : 1;
+      if (!run->fixed_timestep && dt > 0.f) {
+        const float rest = (run->t_end - t) / dt;
+        left = rest < 16.f ? (long)ceilf(rest) : 16;
+      }
+      if (run->max_steps >= 0 && run->max_steps - steps < left) left = run->max_steps - steps;
+      n = left < 1 ? 1 : (left > 16 ? 16 : left);
+    }
     hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
     AMX_HIPCHK(hipGetLastError());
     if (c->hook && c->hook(c->hook_user, state, &c->ctl->dt, steps, st) != 0)
       return amx_fail(AMX_ERR_INVALID, "the step hook stopped the run%s");
-    amx_status s = fd_step(c, state, st);
-    if (s != AMX_OK) return s;
-    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, st, c->ctl);
-    AMX_HIPCHK(hipGetLastError());
+    for (long i = 0; i < n; ++i) {
+      amx_status s = fd_step(c, state, st, want_cfl);
+      if (s != AMX_OK) return s;
+      if (i + 1 < n)
+        hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
+      else
+        hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl);
+      AMX_HIPCHK(hipGetLastError());
+    }
     AMX_HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cflp), hipMemcpyDeviceToHost, st));
     AMX_HIPCHK(hipStreamSynchronize(st));
     fd_tresolve(c);
     t = c->hctl->t;
-    ++steps;
+    dt = c->hctl->dt;
+    steps = c->hctl->steps;
     if (snp) {
-      s = snp->end(t, state, st);
+      amx_status s = snp->end(t, state, st);
       if (s != AMX_OK) return s;
     }
   }
