@@ -1414,7 +1414,8 @@ struct MagArgs {
   int L;               // first launch index of the pair (even)
   int write_first;     // store the pair's first iterate (0: only where L is the slot's kprev)
   int regen;           // regeneration launch: see k_mag
-  unsigned skip_mask;  // regeneration: speculative pairs (bit L / 2), whose first iterate depends on kprev
+  unsigned skip_mask;  // speculative pairs (bit L / 2), whose first iterate depends on kprev
+  unsigned half_mask;  // pairs that make their first iterate only where it is the slot's kprev (pair_half)
   int max_iter;
   float tol;
   int euler;           // IMPLICIT_EULER: average = iterate
@@ -1433,6 +1434,20 @@ __host__ __device__ inline int pair_final(int L, float r0, float r1, float tol, 
   if (!(r0 > tol) || L >= max_iter) return L;
   if (!(r1 > tol) || L + 1 >= max_iter) return L + 1;
   return -1;
+}
+
+// Pair (L, L+1) of the running speculative batch made iterate L only: its slot's
+// previous step ended on L, so this one is expected to, and iterate L+1 (its
+// curls and 6 of the launch's 25 fields) would be thrown away. Where residual
+// L says that the fixed point goes on, the regeneration launch makes iterate
+// L+1 and its residual, and the pair counts as a whole one from there on.
+__host__ __device__ inline bool pair_half(unsigned half_mask, int L, int kprev) {
+  return L >= 0 && L <= 62 && ((half_mask >> (L >> 1)) & 1u) && L == kprev;
+}
+
+// pair_final of such a pair before its second iterate is made
+__host__ __device__ inline int half_final(int L, float r0, float tol, int max_iter) {
+  return !(r0 > tol) || L >= max_iter ? L : -1;
 }
 
 // Raw iterate and fixed-point inputs of one cell.
@@ -1599,29 +1614,45 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   }
   if (!c_run) return;
   int L = a.L;
-  bool one = a.regen;  // the launch computes its first iterate only
+  bool one = a.regen || pair_half(a.half_mask, L, c_kprev);  // the launch computes its first iterate only
+  bool fill = false;  // regeneration: the second iterate of a half pair, with its residual
   if (a.regen) {
     // Regeneration: the fixed point's final launch is read from the residuals
     // of the last executed pair; if it is that pair's first launch and the
     // pair did not store its iterate (a speculative pair not starting at the
     // previous step's final index), the launch is computed again (the same
     // arithmetic on the same inputs, so bit-identical) and only that iterate
-    // is stored. Residuals, counters and flags are left as they are.
+    // is stored. Residuals, counters and flags are left as they are. Of a
+    // half pair whose fixed point goes on, the second iterate is made from
+    // the first, and its residual recorded (run again, the launch finds and
+    // leaves the same values).
     const int Ll = c_iters - 1;
     if (Ll < 0 || Ll > 62) return;
     const float r0 = __uint_as_float(wave_max_u(C->resp[Ll % NRES][tid & 63]));
-    const float r1 = __uint_as_float(wave_max_u(C->resp[(Ll + 1) % NRES][tid & 63]));
-    if (pair_final(Ll, r0, r1, a.tol, a.max_iter) != Ll || !((a.skip_mask >> (Ll >> 1)) & 1u) || Ll == c_kprev)
-      return;
-    L = Ll;
+    if (pair_half(a.half_mask, Ll, c_kprev)) {
+      if (half_final(Ll, r0, a.tol, a.max_iter) == Ll) return;
+      fill = true;
+      L = Ll + 1;
+    } else {
+      const float r1 = __uint_as_float(wave_max_u(C->resp[(Ll + 1) % NRES][tid & 63]));
+      if (pair_final(Ll, r0, r1, a.tol, a.max_iter) != Ll || !((a.skip_mask >> (Ll >> 1)) & 1u) || Ll == c_kprev)
+        return;
+      L = Ll;
+    }
   } else if (L > 0) {
     if (c_done) return;
+    // only behind the pair before it, which a half pair can have kept from
+    // running (L + 1: this launch's own block 0, or the same launch before)
+    if (c_iters != L - 1 && c_iters != L + 1) return;
     const float r0 = __uint_as_float(wave_max_u(prev0));
     const float r1 = __uint_as_float(wave_max_u(prev1));
-    if (pair_final(L - 2, r0, r1, a.tol, a.max_iter) >= 0) {
+    const bool half = pair_half(a.half_mask, L - 2, c_kprev);
+    const int f = half ? half_final(L - 2, r0, a.tol, a.max_iter) : pair_final(L - 2, r0, r1, a.tol, a.max_iter);
+    if (f >= 0) {
       if (blockIdx.x == 0 && tid == 0) C->done = 1;
       return;
     }
+    if (half) return;  // the second iterate comes first
   }
   __shared__ float sK[2][6][NC];
   __shared__ float sK1[2][6][NC1];
@@ -1794,7 +1825,9 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
     for (int i = 0; i < 6; ++i) e1m[i] = e1c[i] = 0.f;
 #pragma unroll
     for (int i = 0; i < 3; ++i) Bp[i] = vp[i] = B0p[i] = v0p[i] = 0.f;
-    for (int x = x0 - 1; x <= x1; ++x) {
+    // (the planes beside the chunk matter to the second iterate only)
+    const int xe = one ? x1 - 1 : x1;
+    for (int x = x0 - 1; x <= xe; ++x) {
       const int bx = x & 1;
       // prefetch x + 2
       MagRaw rnn;
@@ -1910,7 +1943,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   }
   const unsigned m0 = block_max_u<NW>(canon_bits(res0), sred[0]);
   const unsigned m1 = block_max_u<NW>(canon_bits(res1), sred[1]);
-  if (tid == 0 && !a.regen) {
+  if (tid == 0 && (!a.regen || fill)) {
     if (m0) atomicMax(&C->resp[L % NRES][blockIdx.x & (NSLOT - 1)], m0);
     if (m1) atomicMax(&C->resp[(L + 1) % NRES][blockIdx.x & (NSLOT - 1)], m1);
   }
@@ -1928,7 +1961,12 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
 // regeneration launch queued before this one; a speculative call without
 // one queued (regen_queued = 0) holds the step instead, and the host
 // queues the regeneration when it finishes the step.
-__global__ void k_mag_final(Ctl* ctl, float tol, int max_iter, int spec, unsigned skip_mask, int regen_queued) {
+//
+// half_mask: a half pair (pair_half) whose fixed point goes on holds the step
+// like one that ended on an unstored first iterate, unless the regeneration
+// launch has made its second iterate.
+__global__ void k_mag_final(Ctl* ctl, float tol, int max_iter, int spec, unsigned skip_mask, unsigned half_mask,
+                            int regen_queued) {
   Ctl* const c = ctl + blockIdx.x;
   // everything read is loaded first (as in step_control)
   const int run = c->run, L = c->iters - 1, kprev = c->kprev, regen_ev = c->regen_ev;
@@ -1944,9 +1982,11 @@ __global__ void k_mag_final(Ctl* ctl, float tol, int max_iter, int spec, unsigne
     m1 = k == i1 ? res[k] : m1;
   }
   const float r0 = __uint_as_float(wave_max_u(m0)), r1 = __uint_as_float(wave_max_u(m1));
-  const int f = pair_final(L, r0, r1, tol, max_iter);
+  const bool open = pair_half(half_mask, L, kprev) && half_final(L, r0, tol, max_iter) < 0;
+  const bool half = pair_half(half_mask, L, kprev) && !(open && regen_queued);
+  const int f = half ? half_final(L, r0, tol, max_iter) : pair_final(L, r0, r1, tol, max_iter);
   const bool unstored = f >= 0 && f == L && L <= 62 && ((skip_mask >> (L >> 1)) & 1u) && L != kprev;
-  if (spec && unstored && kprev >= 0) c->regen_ev = regen_ev + 1;
+  if (spec && ((unstored && kprev >= 0) || open)) c->regen_ev = regen_ev + 1;
   if ((f < 0 || (unstored && !regen_queued)) && spec) {
     c->held = 1;
     c->stall = 1;
@@ -2332,6 +2372,7 @@ struct amx_fv_ctx {
   int rk2_swap;     // the running loop leaves each hydro step's result where k_rk2 wrote it
   int use_graphs;   // pool: replay captured HIP graphs of the step halves
   unsigned skip_mask;  // pairs of the current step queued without storing their first iterate
+  int half;            // queued batches of steps: half pairs (pair_half); the host reads one status per batch
   int batch;        // pool: steps queued by one step_launch (1: a step in two halves)
   int batching;     // pool: the launched step is a queued batch
   std::map<std::tuple<int, int, int>, hipGraphExec_t> g_batch;  // (span, last count, steps)
@@ -2863,6 +2904,7 @@ MagArgs mag_base(const amx_fv_ctx* c) {
   m.write_first = 1;
   m.regen = 0;
   m.skip_mask = 0u;
+  m.half_mask = 0u;
   m.tol = c->cfg.fixed_point_tol;
   m.euler = c->cfg.magnetic_integrator == AMX_IMPLICIT_EULER;
   m.nx = c->nxm;
@@ -2994,7 +3036,9 @@ hipError_t rk2_home(const amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t s
 
 // Launches the fixed-point pair (L, L+1): input = launch L-1's output (the
 // state's B and gas velocity for L = 0); the kernel picks the iterate sets
-// from ctl->bset (iterate_set).
+// from ctl->bset (iterate_set). A speculative launch (write_first = 0) and a
+// regeneration know the half pairs; one that the host queues later, behind
+// the regeneration, takes every pair as whole.
 hipError_t launch_mag_pair(amx_fv_ctx* c, const Bufs& b, int L, int nspan, hipStream_t st, int write_first = 1,
                            int regen = 0) {
   const int dim = c->cfg.dim;
@@ -3002,6 +3046,7 @@ hipError_t launch_mag_pair(amx_fv_ctx* c, const Bufs& b, int L, int nspan, hipSt
   m.write_first = write_first;
   m.regen = regen;
   m.skip_mask = c->skip_mask;
+  m.half_mask = c->half && (regen || !write_first) ? c->skip_mask : 0u;
   for (int k = 0; k < 3; ++k) m.B0[k] = b.B[k];
   m.v0[0] = b.mid[1];
   m.v0[1] = b.mid[2];
@@ -3113,8 +3158,9 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
 }
 
 // Final launch index of a running slot's fixed point from a readback of its
-// control block, or -1 if the reference's loop would still run.
-int slot_final(const amx_fv_ctx* c, const Ctl& h) {
+// control block, or -1 if the reference's loop would still run. half: the
+// speculative batch's half pairs have not been completed.
+int slot_final(const amx_fv_ctx* c, const Ctl& h, int half = 0) {
   const int L = h.iters - 1;  // last executed pair
   unsigned r0 = 0, r1 = 0;
   for (int i = 0; i < NSLOT; ++i) {
@@ -3124,6 +3170,8 @@ int slot_final(const amx_fv_ctx* c, const Ctl& h) {
   float f0, f1;
   memcpy(&f0, &r0, sizeof(float));
   memcpy(&f1, &r1, sizeof(float));
+  if (half && pair_half(c->skip_mask, L, h.kprev))
+    return half_final(L, f0, c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations);
   return pair_final(L, f0, f1, c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations);
 }
 
@@ -3146,10 +3194,27 @@ int fixed_point_settled(const amx_fv_ctx* c, int nspan, int* kmax) {
 }
 
 // Launches further pairs after klast (two pairs per round) with a readback
-// after each round until every running slot has settled.
+// after each round until every running slot has settled. The speculative
+// batch's half pairs are completed first; a slot that one kept from the rest
+// of the batch goes on from there (the pair kernel leaves slots that are
+// further on alone).
 amx_status fixed_point_more(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, int* klast) {
   const int maxit = c->cfg.max_fixed_point_iterations;
   int kmax = 0;
+  int open = 0;
+  for (int s = 0; s < nspan && c->half; ++s) {
+    const Ctl& h = c->hctl[s];
+    if (h.run && slot_final(c, h, 1) < 0 && pair_half(c->skip_mask, h.iters - 1, h.kprev)) open = 1;
+  }
+  if (open) {
+    HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
+    HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl) * nspan, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    for (int s = 0; s < nspan; ++s) {
+      const Ctl& h = c->hctl[s];
+      if (h.run && slot_final(c, h) < 0 && h.iters < *klast) *klast = h.iters;
+    }
+  }
   while (!fixed_point_settled(c, nspan, &kmax) && *klast < maxit) {
     for (int r = 0; r < 2 && *klast < maxit; ++r) {
       const int L = *klast + 1;
@@ -3174,7 +3239,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   const int rq = c->skip_mask && (regen || !spec);
   if (rq) HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
   hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(NSLOT), 0, st, c->ctl, c->cfg.fixed_point_tol,
-                     c->cfg.max_fixed_point_iterations, spec, c->skip_mask, rq);
+                     c->cfg.max_fixed_point_iterations, spec, c->skip_mask, c->half ? c->skip_mask : 0u, rq);
   HIPCHK(hipGetLastError());
   StageArgs b1 = stage_base(c, 0.5f);
   for (int v = 0; v < NV; ++v) {
@@ -3524,7 +3589,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // next step's B0) and is copied into the state once, after the loop.
   struct KeepB {
     amx_fv_ctx* c;
-    ~KeepB() { c->keep_b = c->rk2_swap = 0; }
+    ~KeepB() { c->keep_b = c->rk2_swap = c->half = 0; }
   } keep_guard{c};
   // (a record takes the whole state of every step)
   c->keep_b = c->cfg.mhd && !snp && !c->hook && !rec ? 1 : 0;
@@ -3563,6 +3628,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // stalled step with the further launches and goes on. Event timing keeps
   // the step-by-step path, which sorts out early-exited launches per step.
   const bool mbatch = c->cfg.mhd && (c->keep_b || (rec && !c->hook)) && c->timing == 0;
+  c->half = mbatch;
   // A loop with an end time takes about (t_end - t) / dt more steps, from the
   // last step's dt; the first batch, before any dt is known, has 4. (Sixteen
   // steps a batch whatever was left: a 20-step run of a 256^2 grid queued 32,
@@ -4412,6 +4478,7 @@ extern "C" amx_status amx_fv_pool_set_batch(amx_fv_pool* p, int steps) {
   if (p->c->stepping) return fail(AMX_ERR_INVALID, "a step is in flight%s");
   if (steps < 1 || steps > 256) return fail(AMX_ERR_INVALID, "steps per launch must be in 1..256%s");
   p->c->batch = steps;
+  p->c->half = steps > 1;
   return AMX_OK;
 }
 
