@@ -37,8 +37,8 @@
 namespace amx {
 namespace fd {
 
-constexpr int TBZ = 64;  // lanes along the contiguous axis
-constexpr int TP = 8;    // waves per WENO block
+constexpr int TBZ = 32;  // columns of a WENO block of the x and y directions
+constexpr int TP = 16;   // its interfaces along the direction
 constexpr int NTH = TP * TBZ;
 
 struct Phys {
@@ -329,39 +329,36 @@ __device__ __forceinline__ void project(const EB& e, const float* u, float* m) {
   m[5] = A1 - e.al * A2;
 }
 
-// 6 times the WENO interpolant with Jiang-Shu weights (_weno.py:185-205). The
+// 3 times the WENO interpolant with Jiang-Shu weights (_weno.py:185-205). The
 // indicators are taken over 13 (the weights do not change, the floor of their
 // sum does by 169). SAFE: one reciprocal per weight, for any finite indicator.
-// Otherwise the weights share one reciprocal of their common denominator,
-// whose products hold for indicators up to PHI_MAX; `top` collects the largest
-// indicator, and the caller repeats the interface the SAFE way above it.
-constexpr float PHI_MAX = 1e8f;
+// Otherwise the weights share one reciprocal of their common denominator: a sum
+// of products, all positive, that overflow together with it; `sum` returns it,
+// and the caller repeats the interface the SAFE way above PHI_MAX, where the
+// reciprocal would lose digits.
+constexpr float PHI_MAX = 1e37f;
 
 template <bool SAFE>
-__device__ __forceinline__ float weno_phi6(float a, float b, float c, float d, float& top) {
+__device__ __forceinline__ float weno_phi3(float a, float b, float c, float d, float& sum) {
   const float eps = 1e-8f / 13.f, r3 = 3.f / 13.f, lim = 169e-14f;
   const float x = a - b, y = b - c, z = c - d;
   const float t0 = x - 2.f * b, t1 = b + c, t2 = 2.f * c + z;
   const float e0 = x * x + ((r3 * t0) * t0 + eps);
   const float e1 = y * y + ((r3 * t1) * t1 + eps);
   const float e2 = z * z + ((r3 * t2) * t2 + eps);
-  float w0, w2;
   if (SAFE) {
     const float a0 = frcp(e0 * e0) * (1.f / 169.f), a1 = frcp(e1 * e1) * (6.f / 169.f), a2 = frcp(e2 * e2) * (3.f / 169.f);
     const float rs = frcp(fmaxf((a0 + a1) + a2, 1e-14f));
-    w0 = a0 * rs;
-    w2 = a2 * rs;
+    sum = 0.f;
+    return (a0 * rs) * (x - y) + (0.5f * (a2 * rs) - 0.25f) * (y - z);
   } else {
-    top = fmaxf(fmaxf(top, e0), fmaxf(e1, e2));
     const float s0 = e0 * e0, s1 = e1 * e1, s2 = e2 * e2;
-    const float n0 = s1 * s2, q = 3.f * s0;
-    const float n2 = q * s1, n1 = q * s2;  // n1: half of it
-    const float sum = 2.f * n1 + (n0 + n2);
+    const float n0 = s1 * s2, q = 1.5f * s0;
+    const float n2 = q * s1, n1 = q * s2;  // half and a quarter of them
+    sum = 4.f * n1 + (2.f * n2 + n0);
     const float r = frcp(fmaxf(sum, (lim * s0) * n0));
-    w0 = n0 * r;
-    w2 = n2 * r;
+    return (n0 * r) * (x - y) + (n2 * r - 0.25f) * (y - z);
   }
-  return (2.f * w0) * (x - y) + (w2 - 0.5f) * (y - z);
 }
 
 struct WenoDir {
@@ -382,23 +379,30 @@ struct WenoArgs {
   Phys ph;
 };
 
-constexpr int NCELL = (TP + 5) * TBZ;  // staged cells of a block
+constexpr int NSTAGE = (TP + 5) * TBZ;           // staged cells of a block
+constexpr int NCELL = (NSTAGE + 63) / 64 * 64;  // an LDS field: whole units of ds_read2st64
 
 __device__ __forceinline__ unsigned small_div(unsigned x, unsigned m) { return (x * m) >> 20; }
 
 // The 7 characteristic WENO-5 fluxes of one interface added to the linear part
 // (_weno.py:134-235). s: the staged cells, c: LDS index of cell i-2, ws: index
-// step between window cells. Returns the largest smoothness indicator.
-template <bool SAFE>
+// step between window cells (known to the compiler: WS, else 0). Returns the
+// largest sum of weno_phi3.
+template <bool SAFE, int WS>
 __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, int ws, const Phys& ph, float* out) {
+  // Field v of window cell k. Single reads: the compiler would pair reads, whose
+  // offsets have 8 bits, and sum up addresses for them (71 to 85 of 1312
+  // instructions); a single read has 16 bits, enough for every field.
+  auto rd = [&](int v, int k) -> float {
+    return __hip_atomic_load(&s[v][c + k * (WS ? WS : ws)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  };
   float A[8], B[8];
   {
-    const int i = c + 2 * ws, j = c + 3 * ws;
     constexpr int f[8] = {C_Q, C_VX, C_VY, C_VZ, C_H, C_Q + 5, C_Q + 6, C_Q + 7};
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      A[v] = s[f[v]][i];
-      B[v] = s[f[v]][j];
+      A[v] = rd(f[v], 2);
+      B[v] = rd(f[v], 3);
     }
   }
   const EB e = interface_blocks(A, B, ph);
@@ -409,7 +413,7 @@ __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, 
     for (int v = 0; v < 7; ++v) {
       float w[6];
 #pragma unroll
-      for (int k = 0; k < 6; ++k) w[k] = s[C_F + v][c + k * ws];
+      for (int k = 0; k < 6; ++k) w[k] = rd(C_F + v, k);
 #pragma unroll
       for (int k = 0; k < 5; ++k) t[k][v] = w[k + 1] - w[k];
       out[v] = (1.0f / 12.0f) * (((-w[1] + 7.f * w[2]) + 7.f * w[3]) - w[4]);
@@ -421,7 +425,7 @@ __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, 
       float w[6];
       const int row = v < 5 ? v : v + 1;
 #pragma unroll
-      for (int k = 0; k < 6; ++k) w[k] = s[C_Q + row][c + k * ws];
+      for (int k = 0; k < 6; ++k) w[k] = rd(C_Q + row, k);
 #pragma unroll
       for (int k = 0; k < 5; ++k) t[k][v] = w[k + 1] - w[k];
     }
@@ -434,12 +438,11 @@ __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, 
   for (int m = 0; m < 7; ++m) am[m] = 0.f;
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
-    const int i = c + k * ws;
-    const float vx = s[C_VX][i];
+    const float vx = rd(C_VX, k);
     am[3] = fmaxf(am[3], fabsf(vx));
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-      const float sp = s[C_CF + m][i];
+      const float sp = rd(C_CF + m, k);
       am[m] = fmaxf(am[m], fabsf(vx - sp));
       am[6 - m] = fmaxf(am[6 - m], fabsf(vx + sp));
     }
@@ -449,11 +452,13 @@ __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, 
 #pragma unroll
   for (int m = 0; m < 7; ++m) {
     const float x = am[m];
-    const float up = weno_phi6<SAFE>(df[0][m] + x * dq[0][m], df[1][m] + x * dq[1][m], df[2][m] + x * dq[2][m],
-                                     df[3][m] + x * dq[3][m], top);
-    const float dn = weno_phi6<SAFE>(df[4][m] - x * dq[4][m], df[3][m] - x * dq[3][m], df[2][m] - x * dq[2][m],
-                                     df[1][m] - x * dq[1][m], top);
-    fs[m] = (dn - up) * (1.f / 6.f);
+    float su, sd;
+    const float up = weno_phi3<SAFE>(df[0][m] + x * dq[0][m], df[1][m] + x * dq[1][m], df[2][m] + x * dq[2][m],
+                                     df[3][m] + x * dq[3][m], su);
+    const float dn = weno_phi3<SAFE>(df[4][m] - x * dq[4][m], df[3][m] - x * dq[3][m], df[2][m] - x * dq[2][m],
+                                     df[1][m] - x * dq[1][m], sd);
+    top = fmaxf(fmaxf(top, su), sd);
+    fs[m] = (dn - up) * (1.f / 3.f);
   }
   // the columns (_eigen_R_col, _eigen.py:340-622) on the shared combinations
   const float p = fs[0] + fs[6], q = fs[6] - fs[0], ps = fs[2] + fs[4], qs = fs[4] - fs[2];
@@ -478,29 +483,31 @@ __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, 
 // interface per thread. A block stages the cells of its window in LDS with
 // their flux, speeds and enthalpy (each thread's own work), then every thread
 // computes one interface from 6 staged cells.
-//   x, y: TP positions along the direction (+ 5 halo cells) times 64 lanes that
+//   x, y: 16 positions along the direction (+ 5 halo cells) times 32 lanes that
 //         run along the flattened plane of the other two axes, so that no lane
-//         is idle whatever nz is;
+//         is idle whatever nz is (8 times 64 stages 13 cells for 8 interfaces
+//         instead of 21 for 16);
 //   z:    a range of `zin` interfaces in linear order; each row piece in it is
 //         staged with its own 5 halo cells (wrapped in its row).
 //
-// Bound by VALU issue: about 1300 instructions an interface, 14 WENO functions
-// of 38 among them. What keeps them few: differences of the window are
-// projected rather than its cells (10 vectors, not 12, and the flux's
-// cancellation happens before the products); the rows and columns of the seven
-// fields share their sums (34 operations a vector instead of 45, and no row is
-// ever formed); the three weights of a WENO function share one quarter-rate
-// reciprocal. LDS holds 22 fields of a cell (73 KB a block, two blocks of 8
-// waves on a CU), each read once per interface; 119 VGPRs, 4 waves a SIMD.
-// 256^3, three directions: 3554 -> 1923 us; 101^3: 305 -> 137 us, where 64
+// Bound by VALU issue: 1190 instructions an interface, 14 WENO functions of 36
+// among them. What keeps them few: differences of the window are projected
+// rather than its cells (10 vectors, not 12, and the flux's cancellation happens
+// before the products); the rows and columns of the seven fields share their
+// sums (34 operations a vector instead of 45, and no row is ever formed); the
+// three weights of a WENO function share one quarter-rate reciprocal; LDS
+// offsets are immediates. LDS holds 22 fields of a cell (62 KB a block, two
+// blocks of 8 waves on a CU), each read once per interface; 119 VGPRs, 4 waves a
+// SIMD.
+// 256^3, three directions: 3554 -> 1794 us; 101^3: 305 -> 128 us, where 64
 // lanes along z of 101 cells had also left a fifth of the lanes idle; 32^3:
-// 32 -> 12 us, three launches in one.
+// 32 -> 10.7 us, three launches in one.
 __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_weno(const WenoArgs a) {
   __shared__ float s[NFIELD][NCELL];
   if (!a.ctl->run) return;
   const Grid g = a.g;
   const Phys ph = a.ph;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const int tid = threadIdx.x, w = tid / TBZ, l = tid % TBZ;
   unsigned bid = blockIdx.x;
   const int dir = bid < a.first[1] ? 0 : (bid < a.first[2] ? 1 : 2);
   bid -= a.first[dir];
@@ -566,12 +573,21 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   __syncthreads();
   if (!live) return;
   float out[7];
-  const float top = interface_flux<false>(s, c0, ws, ph, out);
+  float top;
+  if (dir < 2) {
+    top = interface_flux<false, TBZ>(s, c0, ws, ph, out);
+    // the two forms kept apart: joined at their weights (as the compiler would,
+    // the code being the same) they spill 31 registers, 1.9 times the time
+    asm volatile("; x, y" : "+v"(top), "+v"(out[0]), "+v"(out[1]), "+v"(out[2]), "+v"(out[3]), "+v"(out[4]), "+v"(out[5]), "+v"(out[6]));
+  } else {
+    top = interface_flux<false, 1>(s, c0, ws, ph, out);
+    asm volatile("; z" : "+v"(top), "+v"(out[0]), "+v"(out[1]), "+v"(out[2]), "+v"(out[3]), "+v"(out[4]), "+v"(out[5]), "+v"(out[6]));
+  }
   if (!(top < PHI_MAX)) {
     // opaque to the compiler, which otherwise keeps the first pass's 70
     // projections in registers for this one
     asm volatile("" : "+v"(c0));
-    interface_flux<true>(s, c0, ws, ph, out);
+    interface_flux<true, 0>(s, c0, ws, ph, out);
   }
 #pragma unroll
   for (int v = 0; v < 7; ++v) st(D.F[v], 4u * gc, out[v]);
@@ -825,7 +841,7 @@ __global__ void k_combine(const CombineArgs a) {
     const unsigned xm = nb(g, P, 0, -1), ym = nb(g, P, 1, -1), zm = nb(g, P, 2, -1);
     // Every load first, and kept there by the scheduling barrier: left to
     // itself the compiler paired them with their uses, two in flight at a time
-    // (1119 instead of 860 us in the stages that carry all rows).
+    // (1119 instead of 882 us in the stages that carry all rows).
     float q0[8], q[8], qf[8], qc[8], B[3], f0[3][8], f1[3][8], bf[3][6];
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
@@ -1081,7 +1097,10 @@ hipError_t launch_weno(amx_fd_ctx* c, hipStream_t st) {
   a.ntx = up(g.nx, TP);
   a.nty = up(g.ny, TP);
   // short rows: fewer interfaces per z block, so that their halo cells fit
-  a.zin = g.nz >= 12 ? NTH : NTH / 2;
+  // (512 interfaces meet up to 1 + ceil(511 / nz) rows, 5 halo cells each)
+  static_assert(NTH + 5 * (1 + (NTH - 1 + 16) / 17) <= NCELL && NTH / 2 + 5 * (1 + (NTH / 2 - 1 + 5) / 6) <= NCELL,
+                "z blocks do not fit");
+  a.zin = g.nz >= 17 ? NTH : NTH / 2;
   a.mz = up(1 << 20, g.nz);
   a.mzp = up(1 << 20, g.nz + 5);
   a.first[0] = 0;
