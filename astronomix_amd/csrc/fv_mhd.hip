@@ -82,6 +82,11 @@ struct Ctl {
   int iters_sum;
   int iters_max;
   int iters_bmax;  // largest count of the current batch
+  // chained steps (Front): t and the step count after the last step, in one of
+  // two places, and the final launch index of the step's fixed point
+  float tq[2];
+  int sq[2];
+  int fin;
   unsigned cfl[4];              // reduced CFL maxima per axis
   unsigned cflp[3][NSLOT];      // CFL partial maxima
   unsigned resp[NRES][NSLOT];   // fixed-point residual partials, by launch index % NRES
@@ -92,6 +97,7 @@ struct Ctl {
                                 // pair starting there stores its first iterate, the others leave it out
   int regen_ev;                 // steps of the current batch that ended on a first iterate their pair did not
                                 // store (previous final index known): the next batch queues regeneration launches
+  unsigned cflx[2][3][NSLOT];   // further CFL partial maxima of chained gas steps (cfl_slots)
 };
 
 // Iterate set of fixed-point launch k: the three sets other than bset
@@ -475,6 +481,229 @@ __device__ __forceinline__ void load_w(const float* const* s, unsigned c, float*
   derive_w<DIM, MODE>(r, w);
 }
 
+// The fixed point's stopping rule on an executed pair (L, L+1) with residual
+// maxima r0 = res_L, r1 = res_{L+1} (res_k = max(max|B_k - B_{k-1}|,
+// max|v_k - v_{k-1}|), launch k making iterate k+1): launch k runs while
+// res_{k-1} > tol and k-1 < max_iter (_magnetic_field_update.py:127-141).
+// Returns the last launch that the reference would run (L or L+1), or -1 when
+// launch L+2 would still run.
+__host__ __device__ inline int pair_final(int L, float r0, float r1, float tol, int max_iter) {
+  if (!(r0 > tol) || L >= max_iter) return L;
+  if (!(r1 > tol) || L + 1 >= max_iter) return L + 1;
+  return -1;
+}
+
+// Pair (L, L+1) of the running speculative batch made iterate L only: its slot's
+// previous step ended on L, so this one is expected to, and iterate L+1 (its
+// curls and 6 of the launch's 25 fields) would be thrown away. Where residual
+// L says that the fixed point goes on, the regeneration launch makes iterate
+// L+1 and its residual, and the pair counts as a whole one from there on.
+__host__ __device__ inline bool pair_half(unsigned half_mask, int L, int kprev) {
+  return L >= 0 && L <= 62 && ((half_mask >> (L >> 1)) & 1u) && L == kprev;
+}
+
+// pair_final of such a pair before its second iterate is made
+__host__ __device__ inline int half_final(int L, float r0, float tol, int max_iter) {
+  return !(r0 > tol) || L >= max_iter ? L : -1;
+}
+
+struct StepParams {
+  int fixed;
+  int num_timesteps;
+  int exact_end;
+  float C;
+  float dx;
+  int dim;
+  int clamp_tp = 0;  // clamp dt to tp - t (snapshot time points, time_integration.py:671-674)
+  float tp = 0.f;
+  int batch_first = 0;  // first step of a queued batch: restarts the batch's iteration maximum
+};
+
+// dt = C / sum_a(max_a / dx) (_timestep_estimator.py:128), or t_end/num_timesteps
+// (time_integration.py:667-668); clamp to t_end - t (time_integration.py:677-678).
+__device__ __forceinline__ float cfl_dt_from(const unsigned* cfl, float C, float dx, int dim) {
+  float s = __uint_as_float(cfl[0]) / dx + __uint_as_float(cfl[1]) / dx;
+  if (dim == 3) s = s + __uint_as_float(cfl[2]) / dx;
+  return (C * 1.0f) / s;
+}
+
+// Chained steps: the kernels of a queued step do its control work themselves,
+// and the one-wavefront launches between them (3-4 us and a gap each, two of
+// the eight launches of a 2D MHD step, one of the two of a hydro step) go away.
+//
+//   step_front, in the first kernel of a step: whether the step runs and its
+//     dt, by every wavefront for itself from the last step's partial maxima (a
+//     load and a wave reduction, behind the block's other first loads);
+//   mag_front, in the stage kernel after the fixed point: its final launch index
+//     and whether the step is held.
+//
+// The first wavefront of block 0 writes the results for the kernels behind, and
+// no kernel writes what other blocks of the same launch read: t and the step
+// count after a step (tq, sq), fin and held are written by mag_front and read by
+// step_front, dt, run and the rest the other way round. A gas step, which
+// need not have a second kernel, reads and writes places that alternate from
+// launch to launch (qi, qo of tq and sq; ci, co of the CFL maxima, while cz is
+// cleared for the launch behind).
+// Before and after: 2D MHD 256^2, 20 steps, 899 -> 797 us; hydro 512^2, 40 steps,
+// 785 -> 716; blast at 64^3, 20 steps, 1924 -> 1868; 256^3 unchanged.
+enum { CHAIN_MHD = 1, CHAIN_GAS = 2 };
+
+struct Front {
+  int mode;        // 0: dt and run are in the control block; CHAIN_*
+  int qi, qo, ci, co, cz;
+  int keep_b;
+  StepParams sp;
+};
+
+// partial CFL maxima, place i
+__device__ __forceinline__ unsigned (*cfl_slots(Ctl* c, int i))[NSLOT] { return i == 0 ? c->cflp : c->cflx[i - 1]; }
+
+__device__ __forceinline__ unsigned wave_max_uniform(unsigned v) {
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)wave_max_u(v));
+}
+
+struct FrontStep {
+  int go, steps;
+  float dt;
+};
+
+__device__ __forceinline__ FrontStep step_front(Ctl* c, const Front& f) {
+  const int lane = threadIdx.x & 63;
+  const int live = c->live, held = c->held, steps = c->sq[f.qi];
+  const float t_end = c->t_end, t = c->tq[f.qi];
+  unsigned mx[3] = {0u, 0u, 0u};
+  unsigned(*const p)[NSLOT] = cfl_slots(c, f.ci);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) mx[k] = p[k][lane];
+  const bool writer = blockIdx.x == 0 && threadIdx.x < 64;
+  // the last step's end, of which the writer alone reads what it writes
+  int run = 0, fin = 0, bset = 0, isum = 0, imax = 0, ibmax = 0;
+  if (writer) {
+    run = c->run;
+    fin = c->fin;
+    bset = c->bset;
+    isum = c->iters_sum;
+    imax = c->iters_max;
+    ibmax = c->iters_bmax;
+  }
+  FrontStep o;
+  o.steps = steps;
+  o.go = live && !held && (f.sp.fixed ? steps < f.sp.num_timesteps : t < t_end);
+  float dt;
+  if (f.sp.fixed) {
+    dt = t_end / (float)f.sp.num_timesteps;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) mx[k] = wave_max_uniform(mx[k]);
+    dt = cfl_dt_from(mx, f.sp.C, f.sp.dx, f.sp.dim);
+  }
+  if (f.sp.exact_end) {
+    const float rem = t_end - t;
+    dt = rem < dt ? rem : dt;
+  }
+  o.dt = dt;
+  if (writer) {
+    if (f.mode == CHAIN_MHD && run) {
+      if (held) {
+        c->stall = 1;
+      } else {
+        c->iters = fin;
+        c->kprev = fin;
+        c->iters_sum = isum + fin;
+        c->iters_max = fin > imax ? fin : imax;
+        c->iters_bmax = fin > ibmax ? fin : ibmax;
+        if (f.keep_b) c->bset = iterate_set(bset, fin);
+      }
+    }
+    if (!held) {
+      c->t = t;
+      c->steps = steps;
+    }
+    c->run = o.go;
+    if (f.mode == CHAIN_GAS) {
+      c->tq[f.qo] = o.go ? t + dt : t;
+      c->sq[f.qo] = steps + o.go;
+      unsigned(*const z)[NSLOT] = cfl_slots(c, f.cz);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) z[k][lane] = 0u;
+    }
+    if (o.go) {
+      c->dt = dt;
+      if (!f.sp.fixed) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          if (k < f.sp.dim) c->cfl[k] = mx[k];
+      }
+      if (f.mode == CHAIN_MHD) {
+        c->resp[0][lane] = c->resp[1][lane] = 0u;
+        c->iters = 0;
+        c->done = 0;
+      }
+    }
+  }
+  return o;
+}
+
+// What ends the fixed point of a queued step (see k_mag_final)
+struct FinalRule {
+  float tol;
+  int max_iter, spec, regen_queued;
+  unsigned skip_mask, half_mask;
+};
+
+struct FinalIter {
+  int f;        // final launch index; -1: none yet
+  int held;     // the step waits for further launches
+  int counted;  // the next batch queues regeneration launches
+};
+
+__device__ __forceinline__ FinalIter final_iter(const FinalRule& q, int L, int kprev, float r0, float r1) {
+  FinalIter o;
+  const bool hp = pair_half(q.half_mask, L, kprev);
+  const bool open = hp && half_final(L, r0, q.tol, q.max_iter) < 0;
+  const bool half = hp && !(open && q.regen_queued);
+  o.f = half ? half_final(L, r0, q.tol, q.max_iter) : pair_final(L, r0, r1, q.tol, q.max_iter);
+  const bool unstored = o.f >= 0 && o.f == L && L <= 62 && ((q.skip_mask >> (L >> 1)) & 1u) && L != kprev;
+  o.counted = q.spec && ((unstored && kprev >= 0) || open);
+  o.held = (o.f < 0 || (unstored && !q.regen_queued)) && q.spec;
+  return o;
+}
+
+// residual maxima of the last executed pair, its launches L and L + 1
+__device__ __forceinline__ void pair_residuals(const Ctl* c, int L, float& r0, float& r1) {
+  unsigned res[NRES], m0 = 0u, m1 = 0u;
+#pragma unroll
+  for (int k = 0; k < NRES; ++k) res[k] = c->resp[k][threadIdx.x & 63];
+  const int i0 = L % NRES, i1 = (L + 1) % NRES;
+#pragma unroll
+  for (int k = 0; k < NRES; ++k) {
+    m0 = k == i0 ? res[k] : m0;
+    m1 = k == i1 ? res[k] : m1;
+  }
+  r0 = __uint_as_float(wave_max_uniform(m0));
+  r1 = __uint_as_float(wave_max_uniform(m1));
+}
+
+// The final launch index, or -1 where the slot's step does not go on now.
+__device__ __forceinline__ int mag_front(Ctl* c, const FinalRule& q) {
+  const int run = c->run, L = c->iters - 1, kprev = c->kprev, steps = c->steps;
+  const float t = c->t, dt = c->dt;
+  float r0, r1;
+  pair_residuals(c, L, r0, r1);
+  if (!run) return -1;
+  const FinalIter o = final_iter(q, L, kprev, r0, r1);
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    if (o.counted) c->regen_ev = c->regen_ev + 1;
+    c->fin = o.f;
+    c->held = o.held;
+    c->tq[0] = o.held ? t : t + dt;
+    c->sq[0] = o.held ? steps : steps + 1;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) c->cflp[k][threadIdx.x] = 0u;
+  }
+  return o.held ? -1 : o.f;
+}
+
 // Buffers are given for slot 0; slot s (blockIdx.y + slot0) adds s * sstride
 // floats to every pointer and uses ctl[s] and phs[s]. A single simulation is
 // slot 0 with sstride 0.
@@ -513,6 +742,12 @@ struct StageArgs {
   // energy-fixed pressure of the magnetic sub-step's output: written by the
   // SRC_MAGFIX stage (when set), read by the W0M == SRC_PFIX Heun centre
   float* pfix;
+  // chained steps: the first stage of a step (SRC_PLAIN, no Heun) takes `front`,
+  // the SRC_MAGFIX stage `fr`; chained: the final launch index is in ctl.fin.
+  // co: the place of the CFL maxima (cfl_slots)
+  Front front;
+  FinalRule fr;
+  int chained, co;
 };
 
 // One unsplit forward-Euler stage (evolve_state.py:338-414), optionally with
@@ -557,9 +792,21 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   // all that the block needs of the control block and the physics in one
   // batch of scalar loads, before the branches that would order them one
   // after another (at 256^2 a stage launch is a few memory latencies long)
-  const int c_run = C->run, c_held = C->held, c_bset = C->bset, c_iters = C->iters;
-  const float c_dt = C->dt;
+  int c_run = C->run, c_held = C->held, c_iters = C->iters;
+  const int c_bset = C->bset, c_fin = C->fin;
+  float c_dt = C->dt;
   const Phys ph = a.phs[slot];
+  if (SRC == SRC_PLAIN && !HEUN && a.front.mode) {
+    const FrontStep fs = step_front(C, a.front);
+    c_run = fs.go;
+    c_dt = fs.dt;
+  }
+  if (SRC == SRC_MAGFIX && a.chained) {
+    c_iters = mag_front(C, a.fr);
+    c_held = c_iters < 0;
+  } else if (W0M == SRC_PFIX && a.chained) {
+    c_iters = c_fin;
+  }
   if (!c_run) return;  // block-uniform: empty or finished slot
   if (a.gated && c_held) return;  // queued behind a fixed point that needs more launches
   const long so = slot * a.sstride;
@@ -958,7 +1205,7 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
 #pragma unroll
     for (int k = 0; k < DIM; ++k) {
       const unsigned m = block_max_u<TA + 1>(canon_bits(mx[k]), sred[k]);
-      if (tid == 0 && m) atomicMax(&C->cflp[k][blockIdx.x & (NSLOT - 1)], m);
+      if (tid == 0 && m) atomicMax(&cfl_slots(C, a.co)[k][blockIdx.x & (NSLOT - 1)], m);
     }
   }
 }
@@ -995,6 +1242,7 @@ struct Rk2Args {
   int swap;
   int na, nb, nta, ntb;
   float dt_scale, dxf;
+  Front front;  // chained steps: see step_front
 };
 
 template <int TA, int RS, int LIMX, bool HEUN>
@@ -1016,9 +1264,15 @@ __global__ __launch_bounds__(1024) void k_rk2(const Rk2Args a) {
   __shared__ unsigned sred[2][16];
   const int tid = threadIdx.x, slot = a.slot0 + blockIdx.y;
   Ctl* const C = a.ctl + slot;
-  const int c_run = C->run, c_steps = C->steps;
-  const float c_dt = C->dt;
+  int c_run = C->run, c_steps = C->steps;
+  float c_dt = C->dt;
   const Phys ph = a.phs[slot];
+  if (HEUN && a.front.mode) {
+    const FrontStep fs = step_front(C, a.front);
+    c_run = fs.go;
+    c_dt = fs.dt;
+    c_steps = fs.steps;
+  }
   if (!c_run) return;
   const long so = slot * a.sstride;
   const bool swap = a.swap && (c_steps & 1);
@@ -1181,7 +1435,7 @@ __global__ __launch_bounds__(1024) void k_rk2(const Rk2Args a) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const unsigned m = block_max_u<16>(canon_bits(mx[k]), sred[k]);
-      if (tid == 0 && m) atomicMax(&C->cflp[k][blockIdx.x & (NSLOT - 1)], m);
+      if (tid == 0 && m) atomicMax(&cfl_slots(C, a.front.co)[k][blockIdx.x & (NSLOT - 1)], m);
     }
   }
 }
@@ -1423,32 +1677,6 @@ struct MagArgs {
   float inv_dx;
   AxisBc bx, ba, bb;    // boundaries of the kernel axes x (3D), A and B (kernels with BCX)
 };
-
-// The fixed point's stopping rule on an executed pair (L, L+1) with residual
-// maxima r0 = res_L, r1 = res_{L+1} (res_k = max(max|B_k - B_{k-1}|,
-// max|v_k - v_{k-1}|), launch k making iterate k+1): launch k runs while
-// res_{k-1} > tol and k-1 < max_iter (_magnetic_field_update.py:127-141).
-// Returns the last launch that the reference would run (L or L+1), or -1 when
-// launch L+2 would still run.
-__host__ __device__ inline int pair_final(int L, float r0, float r1, float tol, int max_iter) {
-  if (!(r0 > tol) || L >= max_iter) return L;
-  if (!(r1 > tol) || L + 1 >= max_iter) return L + 1;
-  return -1;
-}
-
-// Pair (L, L+1) of the running speculative batch made iterate L only: its slot's
-// previous step ended on L, so this one is expected to, and iterate L+1 (its
-// curls and 6 of the launch's 25 fields) would be thrown away. Where residual
-// L says that the fixed point goes on, the regeneration launch makes iterate
-// L+1 and its residual, and the pair counts as a whole one from there on.
-__host__ __device__ inline bool pair_half(unsigned half_mask, int L, int kprev) {
-  return L >= 0 && L <= 62 && ((half_mask >> (L >> 1)) & 1u) && L == kprev;
-}
-
-// pair_final of such a pair before its second iterate is made
-__host__ __device__ inline int half_final(int L, float r0, float tol, int max_iter) {
-  return !(r0 > tol) || L >= max_iter ? L : -1;
-}
 
 // Raw iterate and fixed-point inputs of one cell.
 struct MagRaw {
@@ -1965,35 +2193,22 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
 // half_mask: a half pair (pair_half) whose fixed point goes on holds the step
 // like one that ended on an unstored first iterate, unless the regeneration
 // launch has made its second iterate.
-__global__ void k_mag_final(Ctl* ctl, float tol, int max_iter, int spec, unsigned skip_mask, unsigned half_mask,
-                            int regen_queued) {
+__global__ void k_mag_final(Ctl* ctl, FinalRule q) {
   Ctl* const c = ctl + blockIdx.x;
   // everything read is loaded first (as in step_control)
   const int run = c->run, L = c->iters - 1, kprev = c->kprev, regen_ev = c->regen_ev;
-  unsigned res[NRES];
-#pragma unroll
-  for (int k = 0; k < NRES; ++k) res[k] = c->resp[k][threadIdx.x];
+  float r0, r1;
+  pair_residuals(c, L, r0, r1);
   if (!run) return;
-  const int i0 = L % NRES, i1 = (L + 1) % NRES;
-  unsigned m0 = 0u, m1 = 0u;
-#pragma unroll
-  for (int k = 0; k < NRES; ++k) {
-    m0 = k == i0 ? res[k] : m0;
-    m1 = k == i1 ? res[k] : m1;
-  }
-  const float r0 = __uint_as_float(wave_max_u(m0)), r1 = __uint_as_float(wave_max_u(m1));
-  const bool open = pair_half(half_mask, L, kprev) && half_final(L, r0, tol, max_iter) < 0;
-  const bool half = pair_half(half_mask, L, kprev) && !(open && regen_queued);
-  const int f = half ? half_final(L, r0, tol, max_iter) : pair_final(L, r0, r1, tol, max_iter);
-  const bool unstored = f >= 0 && f == L && L <= 62 && ((skip_mask >> (L >> 1)) & 1u) && L != kprev;
-  if (spec && ((unstored && kprev >= 0) || open)) c->regen_ev = regen_ev + 1;
-  if ((f < 0 || (unstored && !regen_queued)) && spec) {
+  const FinalIter o = final_iter(q, L, kprev, r0, r1);
+  if (o.counted) c->regen_ev = regen_ev + 1;
+  if (o.held) {
     c->held = 1;
     c->stall = 1;
     return;
   }
-  c->iters = f >= 0 ? f : L + 1;
-  if (f >= 0) c->kprev = f;
+  c->iters = o.f >= 0 ? o.f : L + 1;
+  if (o.f >= 0) c->kprev = o.f;
   c->held = 0;
   c->stall = 0;
 }
@@ -2057,26 +2272,6 @@ __global__ void k_cfl(const CflArgs a) {
   }
 }
 
-struct StepParams {
-  int fixed;
-  int num_timesteps;
-  int exact_end;
-  float C;
-  float dx;
-  int dim;
-  int clamp_tp = 0;  // clamp dt to tp - t (snapshot time points, time_integration.py:671-674)
-  float tp = 0.f;
-  int batch_first = 0;  // first step of a queued batch: restarts the batch's iteration maximum
-};
-
-// dt = C / sum_a(max_a / dx) (_timestep_estimator.py:128), or t_end/num_timesteps
-// (time_integration.py:667-668); clamp to t_end - t (time_integration.py:677-678).
-__device__ __forceinline__ float cfl_dt_from(const unsigned* cfl, float C, float dx, int dim) {
-  float s = __uint_as_float(cfl[0]) / dx + __uint_as_float(cfl[1]) / dx;
-  if (dim == 3) s = s + __uint_as_float(cfl[2]) / dx;
-  return (C * 1.0f) / s;
-}
-
 __device__ __forceinline__ void fixed_point_reset(Ctl* c) {
   c->resp[0][threadIdx.x] = c->resp[1][threadIdx.x] = 0u;
   c->iters = 0;
@@ -2094,12 +2289,14 @@ __device__ __forceinline__ void zero_cflp(Ctl* c) {
 //
 // END: the end of a step. keep_b: the final B of the step stays in its iterate
 // set, which holds B0 of the next step (the state's B rows are written once, by
-// k_copy_bset). BEGIN: the next step's dt, and whether the slot runs it (live
+// k_copy_bset). chained: mag_front left the final launch index in fin, and a
+// held step has yet to stall the steps behind it. BEGIN: the next step's dt, and whether the slot runs it (live
 // and not yet at t_end / num_timesteps).
 template <bool END, bool BEGIN>
-__device__ __forceinline__ void step_control(Ctl* c, int keep_b, const StepParams& p) {
+__device__ __forceinline__ void step_control(Ctl* c, int keep_b, int chained, const StepParams& p) {
   const int lane = threadIdx.x;
-  const int run = c->run, held = c->held, live = c->live, stall = c->stall, iters = c->iters, bset = c->bset;
+  const int run = c->run, held = c->held, live = c->live, stall = c->stall, bset = c->bset;
+  const int iters = chained ? c->fin : c->iters;
   const int isum = c->iters_sum, imax = c->iters_max, ibmax = c->iters_bmax;
   const float dt0 = c->dt, t_end = c->t_end;
   int steps = c->steps;
@@ -2118,8 +2315,12 @@ __device__ __forceinline__ void step_control(Ctl* c, int keep_b, const StepParam
     c->iters_max = iters > imax ? iters : imax;
     c->iters_bmax = iters > ibmax ? iters : ibmax;
     if (keep_b) c->bset = iterate_set(bset, iters);
+    if (chained) c->iters = c->kprev = iters;
   }
+  if (END && chained && run && held) c->stall = 1;
   if (!BEGIN) return;
+  c->tq[0] = t;
+  c->sq[0] = steps;
   if (p.batch_first) {
     c->iters_bmax = 0;
     c->regen_ev = 0;
@@ -2152,7 +2353,7 @@ __device__ __forceinline__ void step_control(Ctl* c, int keep_b, const StepParam
   fixed_point_reset(c);
 }
 
-__global__ void k_step_begin(Ctl* ctl, StepParams p) { step_control<false, true>(ctl + blockIdx.x, 0, p); }
+__global__ void k_step_begin(Ctl* ctl, StepParams p) { step_control<false, true>(ctl + blockIdx.x, 0, 0, p); }
 
 // dt given by the caller (one step of _evolve_state_fv)
 __global__ void k_set_dt(Ctl* c, const float* dtp) {
@@ -2165,11 +2366,13 @@ __global__ void k_set_dt(Ctl* c, const float* dtp) {
   fixed_point_reset(c);
 }
 
-__global__ void k_step_end(Ctl* ctl, int keep_b) { step_control<true, false>(ctl + blockIdx.x, keep_b, StepParams()); }
+__global__ void k_step_end(Ctl* ctl, int keep_b, int chained) {
+  step_control<true, false>(ctl + blockIdx.x, keep_b, chained, StepParams());
+}
 
 // the end of one queued step and the beginning of the next, in one launch
 __global__ void k_step_end_begin(Ctl* ctl, int keep_b, StepParams p) {
-  step_control<true, true>(ctl + blockIdx.x, keep_b, p);
+  step_control<true, true>(ctl + blockIdx.x, keep_b, 0, p);
 }
 
 // n floats from src to dst for every slot that took part in the step (gate), or for all.
@@ -2258,6 +2461,12 @@ __global__ void k_slot_reset(Ctl* ctl, int slot0, float t_end, int live, int fre
   c->dt = 0.f;
   c->t = 0.f;
   c->steps = 0;
+  for (int i = 0; i < 2; ++i) {
+    c->tq[i] = 0.f;
+    c->sq[i] = 0;
+    for (int k = 0; k < 3; ++k) c->cflx[i][k][threadIdx.x] = 0u;
+  }
+  c->fin = 0;
   for (int i = 0; i < 4; ++i) c->cfl[i] = 0u;
   zero_cflp(c);
   for (int k = 0; k < NRES; ++k) c->resp[k][threadIdx.x] = 0u;
@@ -2368,6 +2577,8 @@ struct amx_fv_ctx {
   void* snapwork;   // snapshot diagnostics partials (allocated on first use)
   int klast;        // pool: last fixed-point launch of the step in flight
   int keep_b;       // the running loop keeps B in the iterate sets (no per-step copy)
+  int chain;        // CHAIN_*: the queued steps do their control work in their own kernels
+  Front front;      // that of the next step to be queued (mode 0: k_step_begin has run)
   int rk2;          // gas steps by k_rk2: its tile rows, or 0 (two stage launches)
   int rk2_swap;     // the running loop leaves each hydro step's result where k_rk2 wrote it
   int use_graphs;   // pool: replay captured HIP graphs of the step halves
@@ -3083,6 +3294,7 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
     }
     a.want_cfl = want_cfl;
     a.swap = c->rk2_swap;
+    a.front = c->front;
     HIPCHK((launch_rk2<true>(c, a, nspan, st)));
     if (!c->rk2_swap) HIPCHK(rk2_home(c, b, nspan, st, 1));
     *klast = 0;
@@ -3091,6 +3303,7 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   if (!c->cfg.mhd) {
     // SSP-RK2 on the whole state: W1 = E(W0); W = prim(0.5 (U0 + cons(E(W1)))) in place
     StageArgs a1 = stage_base(c, 1.0f);
+    a1.front = c->front;
     for (int v = 0; v < NV; ++v) {
       a1.src[v] = b.gas[v];
       a1.out[v] = b.G1 + (long)v * c->ncell;
@@ -3105,6 +3318,7 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
       a2.out[v] = b.gas[v];
     }
     a2.want_cfl = want_cfl;
+    a2.co = c->front.co;
     e = time_begin(c, st);
     HIPCHK((launch_stage<SRC_PLAIN, true, SRC_PLAIN>(c, a2, nspan, st)));
     time_end(c, st, e, CLS_STAGE, 0);
@@ -3119,9 +3333,11 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
       a.src[v] = b.gas[v];
       a.out[v] = b.mid[v];
     }
+    a.front = c->front;
     HIPCHK((launch_rk2<true>(c, a, nspan, st)));
   } else {
     StageArgs a1 = stage_base(c, 0.5f);
+    a1.front = c->front;
     for (int v = 0; v < NV; ++v) {
       a1.src[v] = b.gas[v];
       a1.out[v] = b.G1 + (long)v * c->ncell;
@@ -3227,6 +3443,22 @@ amx_status fixed_point_more(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t
   return AMX_OK;
 }
 
+// Queued steps of these schemes chain. The others reduce over the stage's input
+// in launches of their own before it, which read what a chained step's
+// first kernel and the stage after the fixed point have yet to decide.
+bool chains(const amx_fv_ctx* c) {
+  const int r = c->cfg.riemann;
+  return (r == AMX_HLL || r == AMX_HLLC || r == AMX_HLLC_LM) && c->cfg.limiter != AMX_VAN_ALBADA_PP;
+}
+
+Front mhd_front(const amx_fv_ctx* c, const StepParams& sp) {
+  Front f = Front();
+  f.mode = CHAIN_MHD;
+  f.keep_b = c->keep_b;
+  f.sp = sp;
+  return f;
+}
+
 // Phase 3: S_A(dt/2) on the magnetically updated gas (v <- v_K, energy fix on
 // the fly); the final iterate of every slot is picked on the device.
 // regen: queue the regeneration launch (a speculative call without it holds
@@ -3238,10 +3470,16 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   // the final iterate, where it is the first of a pair that did not store it
   const int rq = c->skip_mask && (regen || !spec);
   if (rq) HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
-  hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(NSLOT), 0, st, c->ctl, c->cfg.fixed_point_tol,
-                     c->cfg.max_fixed_point_iterations, spec, c->skip_mask, c->half ? c->skip_mask : 0u, rq);
-  HIPCHK(hipGetLastError());
+  const FinalRule fr = {c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations, spec, rq, c->skip_mask,
+                        c->half ? c->skip_mask : 0u};
+  const int chained = c->chain == CHAIN_MHD && spec;
+  if (!chained) {
+    hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(NSLOT), 0, st, c->ctl, fr);
+    HIPCHK(hipGetLastError());
+  }
   StageArgs b1 = stage_base(c, 0.5f);
+  b1.fr = fr;
+  b1.chained = chained;
   for (int v = 0; v < NV; ++v) {
     b1.src[v] = b.mid[v];
     b1.out[v] = b.G1 + (long)v * c->ncell;
@@ -3257,6 +3495,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   HIPCHK((launch_stage<SRC_MAGFIX, false, SRC_PLAIN>(c, b1, nspan, st)));
   time_end(c, st, e, CLS_STAGE, spec);
   StageArgs b2 = stage_base(c, 0.5f);
+  b2.chained = chained;
   for (int v = 0; v < NV; ++v) {
     b2.src[v] = b.G1 + (long)v * c->ncell;
     b2.w0[v] = b.mid[v];
@@ -3589,7 +3828,10 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // next step's B0) and is copied into the state once, after the loop.
   struct KeepB {
     amx_fv_ctx* c;
-    ~KeepB() { c->keep_b = c->rk2_swap = c->half = 0; }
+    ~KeepB() {
+      c->keep_b = c->rk2_swap = c->half = c->chain = 0;
+      c->front = Front();
+    }
   } keep_guard{c};
   // (a record takes the whole state of every step)
   c->keep_b = c->cfg.mhd && !snp && !c->hook && !rec ? 1 : 0;
@@ -3629,6 +3871,10 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // the step-by-step path, which sorts out early-exited launches per step.
   const bool mbatch = c->cfg.mhd && (c->keep_b || (rec && !c->hook)) && c->timing == 0;
   c->half = mbatch;
+  // A record is taken behind a step's first kernels, which must have left the input whole.
+  if (batch && (!rec || c->rk2_swap) && chains(c)) c->chain = CHAIN_GAS;
+  if (mbatch && (!rec || c->rk2) && chains(c)) c->chain = CHAIN_MHD;
+  long queued = 0;  // chained gas steps so far
   // A loop with an end time takes about (t_end - t) / dt more steps, from the
   // last step's dt; the first batch, before any dt is known, has 4. (Sixteen
   // steps a batch whatever was left: a 20-step run of a 256^2 grid queued 32,
@@ -3658,9 +3904,18 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       long left = run->fixed_timestep ? run->num_timesteps - steps : -1;
       long n = batch_steps(last_dt, left);
       if (run->max_steps >= 0 && run->max_steps - steps < n) n = run->max_steps - steps;
-      hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
-      HIPCHK(hipGetLastError());
-      for (long i = 0; i < n; ++i) {
+      for (long i = 0; c->chain && i < n; ++i, ++queued) {
+        const int q = (int)(queued & 1), r = (int)(queued % 3);
+        c->front = Front{CHAIN_GAS, q, q ^ 1, r, (r + 1) % 3, (r + 2) % 3, 0, sp};
+        amx_status s = do_step(c, state, st, !run->fixed_timestep, nullptr);
+        if (s != AMX_OK) return s;
+        HIPCHK(record());
+      }
+      if (!c->chain) {
+        hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, sp);
+        HIPCHK(hipGetLastError());
+      }
+      for (long i = 0; !c->chain && i < n; ++i) {
         HIPCHK(record());
         amx_status s = do_step(c, state, st, !run->fixed_timestep, nullptr);
         if (s != AMX_OK) return s;
@@ -3668,12 +3923,16 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
         if (i + 1 < n)
           hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, sp);
         else
-          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0);
+          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, 0);
         HIPCHK(hipGetLastError());
       }
       HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cflp), hipMemcpyDeviceToHost, st));
       HIPCHK(hipStreamSynchronize(st));
       time_resolve(c);
+      if (c->chain) {
+        c->hctl[0].t = c->hctl[0].tq[queued & 1];
+        c->hctl[0].steps = c->hctl[0].sq[queued & 1];
+      }
       t = c->hctl[0].t;
       steps = c->hctl[0].steps;
       last_dt = c->hctl[0].dt;
@@ -3693,16 +3952,18 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
       for (long i = 0; i < n; ++i) {
-        HIPCHK(record());
+        if (!c->chain) HIPCHK(record());
+        c->front = c->chain && i > 0 ? mhd_front(c, spi) : Front();
         amx_status s = step_phase1(c, bl, 1, st, !run->fixed_timestep, &klast);
         if (s != AMX_OK) return s;
+        if (c->chain) HIPCHK(record());
         s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 1, c->regen_q);
         if (s != AMX_OK) return s;
         // this step's end and the next one's beginning
-        if (i + 1 < n)
+        if (i + 1 == n)
+          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b, c->chain != 0);
+        else if (!c->chain)
           hipLaunchKernelGGL(k_step_end_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b, spi);
-        else
-          hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
         HIPCHK(hipGetLastError());
       }
       // the loop's last batch (by its step bound, or as the last dt has it): B
@@ -3729,7 +3990,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
         fixed_point_settled(c, 1, &K);
         s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 0);
         if (s != AMX_OK) return s;
-        hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
+        hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b, 0);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cfl), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
@@ -3757,7 +4018,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
     int K = 0;
     amx_status s = do_step(c, state, st, !run->fixed_timestep, &K);
     if (s != AMX_OK) return s;
-    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
+    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b, 0);
     HIPCHK(hipGetLastError());
     if (!c->cfg.mhd) {
       // hydro steps have no fixed-point readback: read dt here
@@ -3782,8 +4043,10 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   }
   if (c->rk2_swap && (steps & 1)) HIPCHK(rk2_home(c, bl, 1, st, 0));
   if (!b_home) {
+    const float tg = c->hctl[0].t;  // of chained gas steps: in one of two places of the control block
     HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, offsetof(Ctl, cflp), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    if (c->chain == CHAIN_GAS && queued) c->hctl[0].t = tg;
   }
   time_resolve(c);
   if (snp) snp->finish(steps);
@@ -4351,17 +4614,28 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
       hipLaunchKernelGGL(k_step_begin, dim3(span), dim3(NSLOT), 0, st, c->ctl, spi);
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
+      // (a pool of gas steps keeps the control launches: its graphs are
+      // replayed, and the places of its chain alternate from launch to launch)
+      const struct Unchain {
+        amx_fv_ctx* c;
+        ~Unchain() {
+          c->chain = 0;
+          c->front = Front();
+        }
+      } guard{c};
+      c->chain = c->cfg.mhd && chains(c) ? CHAIN_MHD : 0;
       for (int i = 0; i < nb; ++i) {
+        c->front = c->chain && i > 0 ? mhd_front(c, spi) : Front();
         int kl = 0;
         amx_status r = step_phase1(c, b, span, st, !c->sp.fixed, &kl);
         if (r != AMX_OK) return r;
         r = step_phase3(c, b, span, st, !c->sp.fixed, 1);
         if (r != AMX_OK) return r;
         // this step's end and the next one's beginning
-        if (i + 1 < nb)
+        if (i + 1 == nb)
+          hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b, c->chain != 0);
+        else if (!c->chain)
           hipLaunchKernelGGL(k_step_end_begin, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b, spi);
-        else
-          hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
         HIPCHK(hipGetLastError());
       }
       return AMX_OK;
@@ -4432,7 +4706,7 @@ extern "C" amx_status amx_fv_pool_step_finish(amx_fv_pool* p, void* stream) {
       bmax = km > bmax ? km : bmax;
       s = step_phase3(c, b, span, st, !c->sp.fixed, 0);
       if (s != AMX_OK) return s;
-      hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
+      hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b, 0);
       HIPCHK(hipGetLastError());
     }
     if (c->cfg.mhd && bmax > 0) c->last_k = bmax;
@@ -4454,7 +4728,7 @@ extern "C" amx_status amx_fv_pool_step_finish(amx_fv_pool* p, void* stream) {
   amx_status s = replay_or_capture(c, st, &x, x != nullptr, [&]() -> amx_status {
     amx_status r = step_phase3(c, b, span, st, !c->sp.fixed, 0);
     if (r != AMX_OK) return r;
-    hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b);
+    hipLaunchKernelGGL(k_step_end, dim3(span), dim3(NSLOT), 0, st, c->ctl, c->keep_b, 0);
     HIPCHK(hipGetLastError());
     return AMX_OK;
   });
