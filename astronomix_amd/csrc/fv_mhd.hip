@@ -546,13 +546,15 @@ __device__ __forceinline__ float cfl_dt_from(const unsigned* cfl, float C, float
 // cleared for the launch behind).
 // Before and after: 2D MHD 256^2, 20 steps, 899 -> 797 us; hydro 512^2, 40 steps,
 // 785 -> 716; blast at 64^3, 20 steps, 1924 -> 1868; 256^3 unchanged.
-enum { CHAIN_MHD = 1, CHAIN_GAS = 2 };
+// CHAIN_GIVEN: a single step of a caller's state and dt (k_set_dt's work).
+enum { CHAIN_MHD = 1, CHAIN_GAS = 2, CHAIN_GIVEN = 3 };
 
 struct Front {
   int mode;        // 0: dt and run are in the control block; CHAIN_*
   int qi, qo, ci, co, cz;
   int keep_b;
   StepParams sp;
+  const float* dtp;  // CHAIN_GIVEN
 };
 
 // partial CFL maxima, place i
@@ -569,6 +571,20 @@ struct FrontStep {
 
 __device__ __forceinline__ FrontStep step_front(Ctl* c, const Front& f) {
   const int lane = threadIdx.x & 63;
+  if (f.mode == CHAIN_GIVEN) {
+    const float dt = *f.dtp;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+      c->dt = dt;
+      c->run = 1;
+      c->held = 0;
+      c->stall = 0;
+      c->bset = -1;  // B0 is the state's B rows
+      c->resp[0][lane] = c->resp[1][lane] = 0u;
+      c->iters = 0;
+      c->done = 0;
+    }
+    return FrontStep{1, 0, dt};
+  }
   const int live = c->live, held = c->held, steps = c->sq[f.qi];
   const float t_end = c->t_end, t = c->tq[f.qi];
   unsigned mx[3] = {0u, 0u, 0u};
@@ -747,7 +763,7 @@ struct StageArgs {
   // co: the place of the CFL maxima (cfl_slots)
   Front front;
   FinalRule fr;
-  int chained, co;
+  int chained, co;  // chained 2: and the step ends with the Heun stage (no front behind it)
 };
 
 // One unsplit forward-Euler stage (evolve_state.py:338-414), optionally with
@@ -806,6 +822,7 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
     c_held = c_iters < 0;
   } else if (W0M == SRC_PFIX && a.chained) {
     c_iters = c_fin;
+    if (a.chained == 2 && blockIdx.x == 0 && threadIdx.x == 0 && c_run && !c_held) C->iters = C->kprev = c_fin;
   }
   if (!c_run) return;  // block-uniform: empty or finished slot
   if (a.gated && c_held) return;  // queued behind a fixed point that needs more launches
@@ -2579,6 +2596,8 @@ struct amx_fv_ctx {
   int keep_b;       // the running loop keeps B in the iterate sets (no per-step copy)
   int chain;        // CHAIN_*: the queued steps do their control work in their own kernels
   Front front;      // that of the next step to be queued (mode 0: k_step_begin has run)
+  int store_all;    // every pair of the step stores both iterates (no regeneration launch)
+  int cfl_clean;    // the CFL partial maxima are zero between calls
   int rk2;          // gas steps by k_rk2: its tile rows, or 0 (two stage launches)
   int rk2_swap;     // the running loop leaves each hydro step's result where k_rk2 wrote it
   int use_graphs;   // pool: replay captured HIP graphs of the step halves
@@ -3365,7 +3384,7 @@ amx_status step_phase1(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   // pair reads the second): each slot's pairs store it only where its
   // previous step ended (ctl.kprev), and step_phase3 regenerates it in the
   // steps where it is final after all (skip_mask: the speculative pairs)
-  c->skip_mask = skip_mask_for(upto);
+  c->skip_mask = c->store_all ? 0u : skip_mask_for(upto);
   for (int L = 0; L <= upto; L += 2) {
     HIPCHK(launch_mag_pair(c, b, L, nspan, st, L > 62 || !((c->skip_mask >> (L >> 1)) & 1u)));
     *klast = L + 1;
@@ -3495,7 +3514,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   HIPCHK((launch_stage<SRC_MAGFIX, false, SRC_PLAIN>(c, b1, nspan, st)));
   time_end(c, st, e, CLS_STAGE, spec);
   StageArgs b2 = stage_base(c, 0.5f);
-  b2.chained = chained;
+  b2.chained = chained && c->front.mode == CHAIN_GIVEN ? 2 : chained;
   for (int v = 0; v < NV; ++v) {
     b2.src[v] = b.G1 + (long)v * c->ncell;
     b2.w0[v] = b.mid[v];
@@ -3623,11 +3642,15 @@ extern "C" amx_status amx_fv_cfl_dt(amx_fv_ctx* c, const float* state, float* d_
   if (!c || !state || !d_dt) return fail(AMX_ERR_INVALID, "null argument%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_zero_cfl, dim3(1), dim3(NSLOT), 0, st, c->ctl);
-  HIPCHK(hipGetLastError());
+  if (!c->cfl_clean) {
+    hipLaunchKernelGGL(k_zero_cfl, dim3(1), dim3(NSLOT), 0, st, c->ctl);
+    HIPCHK(hipGetLastError());
+  }
+  c->cfl_clean = 0;
   HIPCHK(launch_cfl(c, state, 0, 1, st));
   hipLaunchKernelGGL(k_cfl_out, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->cfg.C_cfl, c->dx, c->cfg.dim, d_dt);
   HIPCHK(hipGetLastError());
+  c->cfl_clean = 1;  // k_cfl_out clears them; a step of evolve_state or the reverse mode takes none
   return AMX_OK;
 }
 
@@ -3636,8 +3659,28 @@ extern "C" amx_status amx_fv_evolve_state(amx_fv_ctx* c, float* state, const flo
   if (!c || !state || !d_dt) return fail(AMX_ERR_INVALID, "null argument%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(NSLOT), 0, st, c->ctl, d_dt);
-  HIPCHK(hipGetLastError());
+  // A caller's own loop pays each launch on the host (4 us) and, on a small grid,
+  // on the device: the step takes its dt and ends its fixed point in its own
+  // kernels (step_front, mag_front), and up to STORE_ALL cells its pairs store
+  // both iterates (a microsecond or two there, 0.1 ms a pair at 256^3) so that no
+  // regeneration launch has to stand by: 13 launches of CFL operator and step become 9.
+  constexpr long STORE_ALL = 1L << 18;
+  struct Given {
+    amx_fv_ctx* c;
+    ~Given() {
+      c->chain = c->store_all = 0;
+      c->front = Front();
+    }
+  } guard{c};
+  if (chains(c)) {
+    c->chain = c->cfg.mhd ? CHAIN_MHD : 0;
+    c->front.mode = CHAIN_GIVEN;
+    c->front.dtp = d_dt;
+    c->store_all = c->ncell <= STORE_ALL;
+  } else {
+    hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(NSLOT), 0, st, c->ctl, d_dt);
+    HIPCHK(hipGetLastError());
+  }
   int K = 0;
   amx_status s = do_step(c, state, st, 0, &K);
   if (s != AMX_OK) return s;
@@ -3821,6 +3864,7 @@ hipError_t copy_b_home(amx_fv_ctx* c, const Bufs& bl, hipStream_t st, int gate) 
 // snapshot driver, rows are taken as in time_integration.py:539-610, 736-745.
 amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Driver* snp, amx_fv_stats* stats,
                    hipStream_t st, const RecordArgs* rec = nullptr) {
+  c->cfl_clean = 0;
   hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, run->t_end, 1, 0);
   HIPCHK(hipGetLastError());
   // Without snapshot rows or a step hook nothing reads the state's B rows
