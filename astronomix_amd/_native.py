@@ -161,9 +161,10 @@ SIGNATURES = {
     "amx_fv_set_timing": (ctypes.c_int, [_P, ctypes.c_int]),
     "amx_fv_get_timing": (ctypes.c_int, [_P, ctypes.POINTER(AmxFvTiming)]),
     "amx_fv_set_physics": (ctypes.c_int, [_P, ctypes.c_float, ctypes.c_float]),
-    "amx_fv_time_integration_recorded": (ctypes.c_int, [_P, _P, ctypes.POINTER(AmxFvRun), _P, ctypes.c_long, _P,
+    "amx_fv_time_integration_recorded": (ctypes.c_int, [_P, _P, ctypes.POINTER(AmxFvRun), _P, ctypes.c_long, _P, _P,
                                                         ctypes.c_long, ctypes.POINTER(AmxFvStats), _P]),
     "amx_fv_adjoint_step": (ctypes.c_int, [_P, _P, _P, _P, _P, _P]),
+    "amx_fv_adjoint_step_counted": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int, _P]),
     "amx_fv_pool_slot_bytes": (ctypes.c_int, [ctypes.POINTER(AmxFvConfig), ctypes.POINTER(ctypes.c_size_t)]),
     "amx_fv_pool_create": (ctypes.c_int, [ctypes.POINTER(AmxFvConfig), ctypes.POINTER(AmxFvRun), ctypes.c_int,
                                           ctypes.POINTER(_P)]),
@@ -295,10 +296,12 @@ class FvContext:
         check(self.lib.amx_fv_get_timing(self.handle, ctypes.byref(t)), "amx_fv_get_timing")
         return t
 
-    def adjoint_step(self, state, dt, lam_out, lam_in, stream=None):
-        check(self.lib.amx_fv_adjoint_step(self.handle, ctypes.c_void_p(state.data_ptr()), ctypes.c_void_p(dt.data_ptr()),
-                                           ctypes.c_void_p(lam_out.data_ptr()), ctypes.c_void_p(lam_in.data_ptr()),
-                                           self._stream(stream)), "amx_fv_adjoint_step")
+    def adjoint_step(self, state, dt, lam_out, lam_in, stream=None, count=-1):
+        """count: the forward step's fixed-point iterations, where known."""
+        check(self.lib.amx_fv_adjoint_step_counted(
+            self.handle, ctypes.c_void_p(state.data_ptr()), ctypes.c_void_p(dt.data_ptr()),
+            ctypes.c_void_p(lam_out.data_ptr()), ctypes.c_void_p(lam_in.data_ptr()), int(count),
+            self._stream(stream)), "amx_fv_adjoint_step")
 
     def set_physics(self, gamma: float, C_cfl: float):
         check(self.lib.amx_fv_set_physics(self.handle, float(gamma), float(C_cfl)), "amx_fv_set_physics")
@@ -311,14 +314,18 @@ class FvContext:
                                                ctypes.byref(st), self._stream(stream)), "amx_fv_time_integration")
         return st
 
-    def time_integration_recorded(self, state, run: AmxFvRun, inputs, dts, stream=None) -> AmxFvStats:
-        """time_integration that records the step sizes into `dts` and the
-        first steps' input states into `inputs` (a stack of states)."""
+    def time_integration_recorded(self, state, run: AmxFvRun, inputs, dts, stream=None, counts=None) -> AmxFvStats:
+        """time_integration that records the step sizes into `dts`, the first
+        steps' input states into `inputs` (a stack of states) and the steps'
+        fixed-point iterations into `counts` (int32, as long as `dts`)."""
+        if counts is not None and counts.shape[0] < dts.shape[0]:
+            raise ValueError("counts must be as long as dts")
         st = AmxFvStats()
         check(self.lib.amx_fv_time_integration_recorded(
             self.handle, ctypes.c_void_p(state.data_ptr()), ctypes.byref(run),
             ctypes.c_void_p(inputs.data_ptr()) if inputs.shape[0] else None, int(inputs.shape[0]),
-            ctypes.c_void_p(dts.data_ptr()), int(dts.shape[0]), ctypes.byref(st), self._stream(stream)),
+            ctypes.c_void_p(dts.data_ptr()), ctypes.c_void_p(counts.data_ptr()) if counts is not None else None,
+            int(dts.shape[0]), ctypes.byref(st), self._stream(stream)),
             "amx_fv_time_integration_recorded")
         return st
 

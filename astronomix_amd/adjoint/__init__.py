@@ -43,32 +43,39 @@ def _function():
     import torch
 
     def record(state, ctx, run, every):
-        """(final state, dts, the inputs of the steps) of a loop that fits the
-        record; (None, dts, None) of one that does not."""
+        """(final state, dts, the inputs of the steps, their fixed-point
+        counts) of a loop that fits the record; (None, dts, None, None) of
+        one that does not."""
         n = int(run.num_timesteps) if run.fixed_timestep else None
         most = RECORD_BYTES // (state.numel() * 4)
         if n is not None:
             if n < 1 or n > most or n > -(-n // every) + every:
-                return None, step_sizes(state, ctx, run.t_end, max(n, 0), bool(run.exact_end_time)), None
+                return None, step_sizes(state, ctx, run.t_end, max(n, 0), bool(run.exact_end_time)), None, None
             most = n
         else:
             most = min(most, every)
         inputs = state.new_empty((most,) + tuple(state.shape))
         cap = n or 1 << 16
+        # in host memory, as the loop's end has waited for the GPU already
+        counts = torch.empty((cap,), dtype=torch.int32, pin_memory=True) if ctx.cfg.mhd else None
         while True:
             s = state.clone()
             dts = state.new_empty((cap,))
-            steps = ctx.time_integration_recorded(s, run, inputs, dts).steps
+            steps = ctx.time_integration_recorded(s, run, inputs, dts, counts=counts).steps
             if steps <= cap:
                 break
             cap = 2 * steps
-        return (s if steps <= most else None), list(dts[:steps].unbind()), (inputs if steps <= most else None)
+            counts = torch.empty((cap,), dtype=torch.int32, pin_memory=True) if ctx.cfg.mhd else None
+        known = list(dts[:steps].unbind())
+        if steps > most:
+            return None, known, None, None
+        return s, known, inputs, counts[:steps].tolist() if counts is not None else [-1] * steps
 
     class Rollout(torch.autograd.Function):
         @staticmethod
         def forward(fctx, state, ctx, run, every):
             first = state.detach().contiguous()
-            s, dts, inputs = record(first, ctx, run, every)
+            s, dts, inputs, counts = record(first, ctx, run, every)
             ckpts = None
             if inputs is None:
                 # not recorded: step by step, with a checkpoint every `every` steps
@@ -81,6 +88,7 @@ def _function():
             if inputs is not None:
                 every = max(1, len(dts))  # one segment
             fctx.ctx, fctx.dts, fctx.every, fctx.ckpts, fctx.inputs = ctx, dts, every, ckpts, inputs
+            fctx.counts = counts
             return s
 
         @staticmethod
@@ -93,15 +101,15 @@ def _function():
             for j in reversed(range(nseg)):
                 lo, hi = j * every, min((j + 1) * every, len(dts))
                 if fctx.inputs is not None:
-                    inputs = fctx.inputs
+                    inputs, counts = fctx.inputs, fctx.counts
                 else:
                     s = fctx.ckpts[j].clone()
-                    inputs = []
+                    inputs, counts = [], []
                     for k in range(lo, hi):
                         inputs.append(s.clone())
-                        ctx.evolve_state(s, dts[k])
+                        counts.append(ctx.evolve_state(s, dts[k]))
                 for k in reversed(range(lo, hi)):
-                    ctx.adjoint_step(inputs[k - lo], dts[k], lam, lam_in)
+                    ctx.adjoint_step(inputs[k - lo], dts[k], lam, lam_in, count=counts[k - lo])
                     lam, lam_in = lam_in, lam
             fctx.ckpts = fctx.inputs = None
             return lam, None, None, None

@@ -665,6 +665,8 @@ struct FinalRule {
   float tol;
   int max_iter, spec, regen_queued;
   unsigned skip_mask, half_mask;
+  int* counts;  // record of the final launch index of each step, or null
+  long max_counts;
 };
 
 struct FinalIter {
@@ -712,6 +714,7 @@ __device__ __forceinline__ int mag_front(Ctl* c, const FinalRule& q) {
     if (o.counted) c->regen_ev = c->regen_ev + 1;
     c->fin = o.f;
     c->held = o.held;
+    if (!o.held && q.counts && steps < q.max_counts && threadIdx.x == 0) q.counts[steps] = o.f;
     c->tq[0] = o.held ? t : t + dt;
     c->sq[0] = o.held ? steps : steps + 1;
 #pragma unroll
@@ -1284,7 +1287,7 @@ __global__ __launch_bounds__(1024) void k_rk2(const Rk2Args a) {
   int c_run = C->run, c_steps = C->steps;
   float c_dt = C->dt;
   const Phys ph = a.phs[slot];
-  if (HEUN && a.front.mode) {
+  if (a.front.mode) {
     const FrontStep fs = step_front(C, a.front);
     c_run = fs.go;
     c_dt = fs.dt;
@@ -2213,7 +2216,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
 __global__ void k_mag_final(Ctl* ctl, FinalRule q) {
   Ctl* const c = ctl + blockIdx.x;
   // everything read is loaded first (as in step_control)
-  const int run = c->run, L = c->iters - 1, kprev = c->kprev, regen_ev = c->regen_ev;
+  const int run = c->run, L = c->iters - 1, kprev = c->kprev, regen_ev = c->regen_ev, steps = c->steps;
   float r0, r1;
   pair_residuals(c, L, r0, r1);
   if (!run) return;
@@ -2226,6 +2229,7 @@ __global__ void k_mag_final(Ctl* ctl, FinalRule q) {
   }
   c->iters = o.f >= 0 ? o.f : L + 1;
   if (o.f >= 0) c->kprev = o.f;
+  if (q.counts && steps < q.max_counts && threadIdx.x == 0) q.counts[steps] = c->iters;
   c->held = 0;
   c->stall = 0;
 }
@@ -2408,6 +2412,7 @@ struct RecordArgs {
   float* inputs;
   float* dts;
   long n, max_inputs, max_dts;
+  int* counts;  // up to max_dts of them (FinalRule), or null
 };
 
 __global__ void k_record(const Ctl* c, RecordArgs a) {
@@ -2596,6 +2601,8 @@ struct amx_fv_ctx {
   int keep_b;       // the running loop keeps B in the iterate sets (no per-step copy)
   int chain;        // CHAIN_*: the queued steps do their control work in their own kernels
   Front front;      // that of the next step to be queued (mode 0: k_step_begin has run)
+  int* counts;      // recording loop: its steps' final launch indices
+  long max_counts;
   int store_all;    // every pair of the step stores both iterates (no regeneration launch)
   int cfl_clean;    // the CFL partial maxima are zero between calls
   int rk2;          // gas steps by k_rk2: its tile rows, or 0 (two stage launches)
@@ -3490,7 +3497,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   const int rq = c->skip_mask && (regen || !spec);
   if (rq) HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
   const FinalRule fr = {c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations, spec, rq, c->skip_mask,
-                        c->half ? c->skip_mask : 0u};
+                        c->half ? c->skip_mask : 0u, c->counts, c->max_counts};
   const int chained = c->chain == CHAIN_MHD && spec;
   if (!chained) {
     hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(NSLOT), 0, st, c->ctl, fr);
@@ -3874,10 +3881,13 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
     amx_fv_ctx* c;
     ~KeepB() {
       c->keep_b = c->rk2_swap = c->half = c->chain = 0;
+      c->counts = nullptr;
       c->front = Front();
     }
   } keep_guard{c};
   // (a record takes the whole state of every step)
+  c->counts = rec ? rec->counts : nullptr;
+  c->max_counts = rec ? rec->max_dts : 0;
   c->keep_b = c->cfg.mhd && !snp && !c->hook && !rec ? 1 : 0;
   auto record = [&]() -> hipError_t {
     if (!rec) return hipSuccess;
@@ -4114,14 +4124,14 @@ extern "C" amx_status amx_fv_time_integration(amx_fv_ctx* c, float* state, const
 }
 
 extern "C" amx_status amx_fv_time_integration_recorded(amx_fv_ctx* c, float* state, const amx_fv_run* run,
-                                                       float* inputs, long max_inputs, float* dts, long max_dts,
-                                                       amx_fv_stats* stats, void* stream) {
+                                                       float* inputs, long max_inputs, float* dts, int* counts,
+                                                       long max_dts, amx_fv_stats* stats, void* stream) {
   if (!c || !state || !run) return fail(AMX_ERR_INVALID, "null argument%s");
   if (max_inputs < 0 || max_dts < 0 || (max_inputs && !inputs) || (max_dts && !dts))
     return fail(AMX_ERR_INVALID, "record arrays missing%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   if (run->fixed_timestep && run->num_timesteps <= 0) return fail(AMX_ERR_INVALID, "num_timesteps must be positive%s");
-  const RecordArgs rec = {state, nullptr, inputs, dts, (long)c->NS * c->ncell, max_inputs, max_dts};
+  const RecordArgs rec = {state, nullptr, inputs, dts, (long)c->NS * c->ncell, max_inputs, max_dts, counts};
   return fv_loop(c, state, run, nullptr, stats, (hipStream_t)stream, &rec);
 }
 
@@ -4198,6 +4208,13 @@ hipError_t launch_adj_tile(const amx_fv_ctx* c, const adj::AdjTileArgs& a, hipSt
   return hipGetLastError();
 }
 
+// The front of the step's first kernel, which alone takes it.
+Front take_front(amx_fv_ctx* c) {
+  const Front f = c->front;
+  c->front = Front();
+  return f;
+}
+
 // Reverse mode of one SSP-RK2 gas step of dt_scale times the step size in ctl.
 template <int DIM>
 amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, float* lam_in, float dt_scale,
@@ -4214,6 +4231,7 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
   // recompute the two stage states with the forward kernel (dt in ctl[0])
   if (DIM == 2 && c->rk2) {
     Rk2Args a = rk2_base(c, dt_scale);
+    a.front = take_front(c);
     for (int v = 0; v < NV; ++v) {
       a.src[v] = w0 + (long)v * n;
       a.out[v] = G1 + (long)v * n;
@@ -4222,6 +4240,7 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
     HIPCHK((launch_rk2<false>(c, a, 1, st)));
   } else {
   StageArgs a1 = stage_base(c, dt_scale);
+  a1.front = take_front(c);
   for (int v = 0; v < NV; ++v) {
     a1.src[v] = w0 + (long)v * n;
     a1.out[v] = G1 + (long)v * n;
@@ -4321,8 +4340,12 @@ amx_status adjm_reserve(amx_fv_ctx* c, int iters, hipStream_t st) {
 // the forward's own), every iterate written to a place of its own; then the
 // second gas half, the magnetic sub-step and the first gas half are reversed
 // (adjoint_step_t at dt/2, adj::k_adjm_back).
+//
+// count: the forward step's final launch index where the caller has it (the
+// recording loop and evolve_state give it). Without it the residuals are read
+// back in the middle of the step, 25-40 us in which the GPU is idle.
 template <int DIM>
-amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_out, float* lam_in,
+amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_out, float* lam_in, int count,
                             hipStream_t st) {
   constexpr int NV = DIM + 2;
   const long n = c->ncell;
@@ -4332,6 +4355,7 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
   float* G1 = c->mem;
   if (c->rk2) {
     Rk2Args a = rk2_base(c, 0.5f);
+    a.front = take_front(c);
     for (int v = 0; v < NV; ++v) {
       a.src[v] = state + (long)v * n;
       a.out[v] = c->adjm + (long)v * n;
@@ -4339,6 +4363,7 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
     HIPCHK((launch_rk2<true>(c, a, 1, st)));
   } else {
   StageArgs a1 = stage_base(c, 0.5f);
+  a1.front = take_front(c);
   for (int v = 0; v < NV; ++v) {
     a1.src[v] = state + (long)v * n;
     a1.out[v] = G1 + (long)v * n;
@@ -4358,7 +4383,7 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
   int F = -1;
   for (int L = 0; F < 0;) {
     const int maxit = c->cfg.max_fixed_point_iterations;
-    int upto = L == 0 ? (c->last_k < 1 ? 1 : c->last_k) : L;
+    int upto = L == 0 ? (count >= 0 ? count : c->last_k < 1 ? 1 : c->last_k) : L;
     if (upto > maxit) upto = maxit;
     if (upto < L) upto = L;
     r = adjm_reserve(c, upto + 2, st);  // may move the workspace: the buffers are taken again
@@ -4374,6 +4399,10 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
       for (int k = L > 0 ? L - 1 : 0; k <= L + 1; ++k)
         for (int f = 0; f < 6; ++f) b.P[iterate_set(-1, k)][f] = IT + (long)(6 * k + f) * n;
       HIPCHK(launch_mag_pair(c, b, L, 1, st, 1, 0));
+    }
+    if (count >= 0) {
+      F = count;
+      break;
     }
     HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
@@ -4434,14 +4463,16 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
   return adjoint_step_t<DIM>(c, state, LWA, lam_in, 0.5f, st);
 }
 
-extern "C" amx_status amx_fv_adjoint_step(amx_fv_ctx* c, const float* state, const float* d_dt, const float* lam_out,
-                                          float* lam_in, void* stream) {
+extern "C" amx_status amx_fv_adjoint_step_counted(amx_fv_ctx* c, const float* state, const float* d_dt,
+                                                  const float* lam_out, float* lam_in, int count, void* stream) {
   if (!c || !state || !d_dt || !lam_out || !lam_in) return fail(AMX_ERR_INVALID, "null argument%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context has no reverse mode%s");
   if ((c->cfg.riemann != AMX_HLL && c->cfg.riemann != AMX_HLLC) || c->cfg.limiter != AMX_MINMOD)
     return fail(AMX_ERR_UNSUPPORTED, "reverse mode covers the HLL / HLLC fluxes with the minmod limiter%s");
   if (c->bcx) return fail(AMX_ERR_UNSUPPORTED, "reverse mode covers periodic boundaries only%s");
   if (lam_in == lam_out || lam_in == state) return fail(AMX_ERR_INVALID, "lam_in must not alias its inputs%s");
+  if (count < -1 || (c->cfg.mhd && count > c->cfg.max_fixed_point_iterations))
+    return fail(AMX_ERR_INVALID, "count must be a fixed-point iteration count or -1%s");
   const int NV = c->NV, dim = c->cfg.dim;
   if (!c->adj) {
     const size_t fields = (size_t)4 * NV + (size_t)dim * 4 * NV;
@@ -4451,12 +4482,21 @@ extern "C" amx_status amx_fv_adjoint_step(amx_fv_ctx* c, const float* state, con
     }
   }
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_set_dt, dim3(1), dim3(NSLOT), 0, st, c->ctl, d_dt);
-  HIPCHK(hipGetLastError());
+  struct Given {
+    amx_fv_ctx* c;
+    ~Given() { c->front = Front(); }
+  } guard{c};
+  c->front.mode = CHAIN_GIVEN;  // the first kernel takes the dt
+  c->front.dtp = d_dt;
   if (c->cfg.mhd)
-    return dim == 3 ? adjoint_step_mhd<3>(c, state, lam_out, lam_in, st) : adjoint_step_mhd<2>(c, state, lam_out, lam_in, st);
+    return dim == 3 ? adjoint_step_mhd<3>(c, state, lam_out, lam_in, count, st) : adjoint_step_mhd<2>(c, state, lam_out, lam_in, count, st);
   return dim == 3 ? adjoint_step_t<3>(c, state, lam_out, lam_in, 1.0f, st)
                   : adjoint_step_t<2>(c, state, lam_out, lam_in, 1.0f, st);
+}
+
+extern "C" amx_status amx_fv_adjoint_step(amx_fv_ctx* c, const float* state, const float* d_dt, const float* lam_out,
+                                          float* lam_in, void* stream) {
+  return amx_fv_adjoint_step_counted(c, state, d_dt, lam_out, lam_in, -1, stream);
 }
 
 // ============================================================================

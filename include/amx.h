@@ -163,12 +163,14 @@ amx_status amx_fv_time_integration(amx_fv_ctx* ctx, float* state, const amx_fv_r
 
 /* The same loop with a record for the reverse mode: dts[k] receives the size
  * of step k (k < max_dts) and inputs[k] the state it starts from (whole states,
- * k < max_inputs). Steps past the arrays run unrecorded; stats->steps tells how
- * many there were. Device arrays; may be NULL with a maximum of 0. The state and
- * the steps are those of amx_fv_time_integration, bit for bit. */
+ * k < max_inputs). counts, which may be NULL, receives the fixed-point iterations
+ * of each MHD step (k < max_dts). Steps past the arrays run unrecorded; stats->steps
+ * tells how many there were. Device arrays (counts: or pinned host memory); may be
+ * NULL with a maximum of 0. The state and the steps are those of
+ * amx_fv_time_integration, bit for bit. */
 amx_status amx_fv_time_integration_recorded(amx_fv_ctx* ctx, float* state, const amx_fv_run* run, float* inputs,
-                                            long max_inputs, float* dts, long max_dts, amx_fv_stats* stats,
-                                            void* stream);
+                                            long max_inputs, float* dts, int* counts, long max_dts,
+                                            amx_fv_stats* stats, void* stream);
 
 /* Reverse mode of one step: lam_in = (dW_out/dW)^T lam_out where W_out is
  * the state amx_fv_evolve_state makes from `state` with the step size in
@@ -186,6 +188,12 @@ amx_status amx_fv_time_integration_recorded(amx_fv_ctx* ctx, float* state, const
  * HLLC with minmod, periodic boundaries. */
 amx_status amx_fv_adjoint_step(amx_fv_ctx* ctx, const float* state, const float* d_dt, const float* lam_out,
                                float* lam_in, void* stream);
+
+/* The same with the fixed-point iterations of the forward step, as
+ * amx_fv_evolve_state or the recording loop gave them for this state and step
+ * size (mhd = 1; -1: not known): the call then only queues work. */
+amx_status amx_fv_adjoint_step_counted(amx_fv_ctx* ctx, const float* state, const float* d_dt, const float* lam_out,
+                                       float* lam_in, int count, void* stream);
 
 /* Per-kernel-class device time of the launches made while timing is on,
  * measured with HIP events on the launch stream. Fixed-point launches that
