@@ -332,14 +332,18 @@ __device__ __forceinline__ void project(const EB& e, const float* u, float* m) {
 // 3 times the WENO interpolant with Jiang-Shu weights (_weno.py:185-205). The
 // indicators are taken over 13 (the weights do not change, the floor of their
 // sum does by 169). SAFE: one reciprocal per weight, for any finite indicator.
-// Otherwise the weights share one reciprocal of their common denominator: a sum
-// of products, all positive, that overflow together with it; `sum` returns it,
-// and the caller repeats the interface the SAFE way above PHI_MAX, where the
-// reciprocal would lose digits.
+// Otherwise the weights share one reciprocal of their common denominator: the
+// sum of products of two squared indicators, or its floor, a product of three,
+// which grows faster and is the larger from differences of about 1e3 on. `den`
+// returns the value that is inverted, and the caller repeats the interface the
+// SAFE way above PHI_MAX, where the reciprocal would lose digits. (Looking at
+// the sum alone let the floor overflow below it: weights of 0, an interpolant off
+// by up to a tenth of the differences where these are 3e3 to 1e5; now within 6e-7
+// of float64 from 1 to 1e8, as the SAFE form.)
 constexpr float PHI_MAX = 1e37f;
 
 template <bool SAFE>
-__device__ __forceinline__ float weno_phi3(float a, float b, float c, float d, float& sum) {
+__device__ __forceinline__ float weno_phi3(float a, float b, float c, float d, float& den) {
   const float eps = 1e-8f / 13.f, r3 = 3.f / 13.f, lim = 169e-14f;
   const float x = a - b, y = b - c, z = c - d;
   const float t0 = x - 2.f * b, t1 = b + c, t2 = 2.f * c + z;
@@ -349,14 +353,14 @@ __device__ __forceinline__ float weno_phi3(float a, float b, float c, float d, f
   if (SAFE) {
     const float a0 = frcp(e0 * e0) * (1.f / 169.f), a1 = frcp(e1 * e1) * (6.f / 169.f), a2 = frcp(e2 * e2) * (3.f / 169.f);
     const float rs = frcp(fmaxf((a0 + a1) + a2, 1e-14f));
-    sum = 0.f;
+    den = 0.f;
     return (a0 * rs) * (x - y) + (0.5f * (a2 * rs) - 0.25f) * (y - z);
   } else {
     const float s0 = e0 * e0, s1 = e1 * e1, s2 = e2 * e2;
     const float n0 = s1 * s2, q = 1.5f * s0;
     const float n2 = q * s1, n1 = q * s2;  // half and a quarter of them
-    sum = 4.f * n1 + (2.f * n2 + n0);
-    const float r = frcp(fmaxf(sum, (lim * s0) * n0));
+    den = fmaxf(4.f * n1 + (2.f * n2 + n0), (lim * s0) * n0);
+    const float r = frcp(den);
     return (n0 * r) * (x - y) + (n2 * r - 0.25f) * (y - z);
   }
 }
@@ -387,7 +391,7 @@ __device__ __forceinline__ unsigned small_div(unsigned x, unsigned m) { return (
 // The 7 characteristic WENO-5 fluxes of one interface added to the linear part
 // (_weno.py:134-235). s: the staged cells, c: LDS index of cell i-2, ws: index
 // step between window cells (known to the compiler: WS, else 0). Returns the
-// largest sum of weno_phi3.
+// largest denominator of weno_phi3.
 template <bool SAFE, int WS>
 __device__ __forceinline__ float interface_flux(const float (*s)[NCELL], int c, int ws, const Phys& ph, float* out) {
   // Field v of window cell k. Single reads: the compiler would pair reads, whose
