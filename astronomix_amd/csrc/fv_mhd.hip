@@ -97,7 +97,8 @@ struct Ctl {
                                 // pair starting there stores its first iterate, the others leave it out
   int regen_ev;                 // steps of the current batch that ended on a first iterate their pair did not
                                 // store (previous final index known): the next batch queues regeneration launches
-  unsigned cflx[2][3][NSLOT];   // further CFL partial maxima of chained gas steps (cfl_slots)
+  unsigned cflx[3][3][NSLOT];   // further CFL partial maxima (cfl_slots): two places of chained gas steps, and
+                                // the CFL operator's own, which are zero between its calls whatever a loop leaves
 };
 
 // Iterate set of fixed-point launch k: the three sets other than bset
@@ -557,7 +558,8 @@ struct Front {
   const float* dtp;  // CHAIN_GIVEN
 };
 
-// partial CFL maxima, place i
+// partial CFL maxima, place i (CFL_OP: those of amx_fv_cfl_dt)
+constexpr int CFL_OP = 3;
 __device__ __forceinline__ unsigned (*cfl_slots(Ctl* c, int i))[NSLOT] { return i == 0 ? c->cflp : c->cflx[i - 1]; }
 
 __device__ __forceinline__ unsigned wave_max_uniform(unsigned v) {
@@ -2244,6 +2246,7 @@ struct CflArgs {
   long sstride;
   long n;
   int slot0;
+  int place;  // of the maxima (cfl_slots)
 };
 
 // V4: the rows are 16-byte aligned and n is a multiple of 4; each thread
@@ -2289,7 +2292,7 @@ __global__ void k_cfl(const CflArgs a) {
 #pragma unroll
   for (int k = 0; k < DIM; ++k) {
     const unsigned m = block_max_u<4>(canon_bits(mx[k]), sred[k]);
-    if (threadIdx.x == 0 && m) atomicMax(&C->cflp[k][blockIdx.x & (NSLOT - 1)], m);
+    if (threadIdx.x == 0 && m) atomicMax(&cfl_slots(C, a.place)[k][blockIdx.x & (NSLOT - 1)], m);
   }
 }
 
@@ -2460,20 +2463,19 @@ __global__ void k_resume(Ctl* ctl) {
 }
 
 __global__ void k_cfl_out(Ctl* c, float C, float dx, int dim, float* out) {
+  unsigned(*const p)[NSLOT] = cfl_slots(c, CFL_OP);
   unsigned m[3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) m[k] = c->cflp[k][threadIdx.x];
+  for (int k = 0; k < 3; ++k) m[k] = p[k][threadIdx.x];
 #pragma unroll
   for (int k = 0; k < 3; ++k) m[k] = wave_max_u(m[k]);
   *out = cfl_dt_from(m, C, dx, dim);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     c->cfl[k] = m[k];
-    c->cflp[k][threadIdx.x] = 0u;
+    p[k][threadIdx.x] = 0u;
   }
 }
-
-__global__ void k_zero_cfl(Ctl* c) { zero_cflp(c); }
 
 // (Re)start slot blockIdx.x + slot0 at t = 0 (live = 1), or empty it (live = 0).
 // fresh: a new simulation in the slot (a loop restarting on the same
@@ -2486,8 +2488,9 @@ __global__ void k_slot_reset(Ctl* ctl, int slot0, float t_end, int live, int fre
   for (int i = 0; i < 2; ++i) {
     c->tq[i] = 0.f;
     c->sq[i] = 0;
-    for (int k = 0; k < 3; ++k) c->cflx[i][k][threadIdx.x] = 0u;
   }
+  for (int i = 0; i < 3; ++i)
+    for (int k = 0; k < 3; ++k) c->cflx[i][k][threadIdx.x] = 0u;
   c->fin = 0;
   for (int i = 0; i < 4; ++i) c->cfl[i] = 0u;
   zero_cflp(c);
@@ -2604,7 +2607,6 @@ struct amx_fv_ctx {
   int* counts;      // recording loop: its steps' final launch indices
   long max_counts;
   int store_all;    // every pair of the step stores both iterates (no regeneration launch)
-  int cfl_clean;    // the CFL partial maxima are zero between calls
   int rk2;          // gas steps by k_rk2: its tile rows, or 0 (two stage launches)
   int rk2_swap;     // the running loop leaves each hydro step's result where k_rk2 wrote it
   int use_graphs;   // pool: replay captured HIP graphs of the step halves
@@ -3188,7 +3190,7 @@ hipError_t launch_mag(const amx_fv_ctx* c, const MagArgs& m, int nspan, hipStrea
 }
 
 // CFL maxima of slots [slot0, slot0 + nspan) of the state whose slot-0 rows start at `state`
-hipError_t launch_cfl(const amx_fv_ctx* c, const float* state, int slot0, int nspan, hipStream_t st) {
+hipError_t launch_cfl(const amx_fv_ctx* c, const float* state, int slot0, int nspan, hipStream_t st, int place = 0) {
   const long n = c->ncell;
   CflArgs a;
   memset(&a, 0, sizeof(a));
@@ -3199,6 +3201,7 @@ hipError_t launch_cfl(const amx_fv_ctx* c, const float* state, int slot0, int ns
   a.sstride = c->sstride;
   a.n = n;
   a.slot0 = slot0;
+  a.place = place;
   bool v4 = (n & 3) == 0 && (a.sstride & 3) == 0;
   for (int v = 0; v <= c->cfg.dim; ++v) v4 = v4 && ((uintptr_t)a.w[v] & 15) == 0;
   v4 = v4 && ((uintptr_t)a.p & 15) == 0;
@@ -3649,15 +3652,9 @@ extern "C" amx_status amx_fv_cfl_dt(amx_fv_ctx* c, const float* state, float* d_
   if (!c || !state || !d_dt) return fail(AMX_ERR_INVALID, "null argument%s");
   if (c->own_state) return fail(AMX_ERR_INVALID, "a pool context is stepped with amx_fv_pool_*%s");
   hipStream_t st = (hipStream_t)stream;
-  if (!c->cfl_clean) {
-    hipLaunchKernelGGL(k_zero_cfl, dim3(1), dim3(NSLOT), 0, st, c->ctl);
-    HIPCHK(hipGetLastError());
-  }
-  c->cfl_clean = 0;
-  HIPCHK(launch_cfl(c, state, 0, 1, st));
+  HIPCHK(launch_cfl(c, state, 0, 1, st, CFL_OP));
   hipLaunchKernelGGL(k_cfl_out, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->cfg.C_cfl, c->dx, c->cfg.dim, d_dt);
   HIPCHK(hipGetLastError());
-  c->cfl_clean = 1;  // k_cfl_out clears them; a step of evolve_state or the reverse mode takes none
   return AMX_OK;
 }
 
@@ -3871,7 +3868,6 @@ hipError_t copy_b_home(amx_fv_ctx* c, const Bufs& bl, hipStream_t st, int gate) 
 // snapshot driver, rows are taken as in time_integration.py:539-610, 736-745.
 amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Driver* snp, amx_fv_stats* stats,
                    hipStream_t st, const RecordArgs* rec = nullptr) {
-  c->cfl_clean = 0;
   hipLaunchKernelGGL(k_slot_reset, dim3(1), dim3(NSLOT), 0, st, c->ctl, 0, run->t_end, 1, 0);
   HIPCHK(hipGetLastError());
   // Without snapshot rows or a step hook nothing reads the state's B rows
