@@ -1690,6 +1690,7 @@ struct MagArgs {
   int L;               // first launch index of the pair (even)
   int write_first;     // store the pair's first iterate (0: only where L is the slot's kprev)
   int regen;           // regeneration launch: see k_mag
+  int counted;         // the caller knows the final launch: the pair is made whatever the residuals
   unsigned skip_mask;  // speculative pairs (bit L / 2), whose first iterate depends on kprev
   unsigned half_mask;  // pairs that make their first iterate only where it is the slot's kprev (pair_half)
   int max_iter;
@@ -1858,7 +1859,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   const int c_run = C->run, c_done = C->done, c_kprev = C->kprev, c_bset = C->bset, c_iters = C->iters;
   const float c_dt = C->dt;
   unsigned prev0 = 0u, prev1 = 0u;
-  if (!a.regen && a.L > 0) {
+  if (!a.regen && !a.counted && a.L > 0) {
     prev0 = C->resp[(a.L - 2) % NRES][tid & 63];
     prev1 = C->resp[(a.L - 1) % NRES][tid & 63];
   }
@@ -1889,7 +1890,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
         return;
       L = Ll;
     }
-  } else if (L > 0) {
+  } else if (L > 0 && !a.counted) {
     if (c_done) return;
     // only behind the pair before it, which a half pair can have kept from
     // running (L + 1: this launch's own block 0, or the same launch before)
@@ -3142,6 +3143,7 @@ MagArgs mag_base(const amx_fv_ctx* c) {
   m.max_iter = c->cfg.max_fixed_point_iterations;
   m.write_first = 1;
   m.regen = 0;
+  m.counted = 0;
   m.skip_mask = 0u;
   m.half_mask = 0u;
   m.tol = c->cfg.fixed_point_tol;
@@ -3280,11 +3282,12 @@ hipError_t rk2_home(const amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t s
 // regeneration know the half pairs; one that the host queues later, behind
 // the regeneration, takes every pair as whole.
 hipError_t launch_mag_pair(amx_fv_ctx* c, const Bufs& b, int L, int nspan, hipStream_t st, int write_first = 1,
-                           int regen = 0) {
+                           int regen = 0, int counted = 0) {
   const int dim = c->cfg.dim;
   MagArgs m = mag_base(c);
   m.write_first = write_first;
   m.regen = regen;
+  m.counted = counted;
   m.skip_mask = c->skip_mask;
   m.half_mask = c->half && (regen || !write_first) ? c->skip_mask : 0u;
   for (int k = 0; k < 3; ++k) m.B0[k] = b.B[k];
@@ -4338,8 +4341,10 @@ amx_status adjm_reserve(amx_fv_ctx* c, int iters, hipStream_t st) {
 // (adjoint_step_t at dt/2, adj::k_adjm_back).
 //
 // count: the forward step's final launch index where the caller has it (the
-// recording loop and evolve_state give it). Without it the residuals are read
-// back in the middle of the step, 25-40 us in which the GPU is idle.
+// recording loop and evolve_state give it): that many launches are made,
+// whatever their residuals, so that no iterate of another step is read where a
+// caller's count is larger. Without it the residuals are read back in the
+// middle of the step, 25-40 us in which the GPU is idle.
 template <int DIM>
 amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_out, float* lam_in, int count,
                             hipStream_t st) {
@@ -4394,7 +4399,7 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
         for (int f = 0; f < 6; ++f) b.P[j][f] = IT + (long)f * n;  // sets that the pair does not use
       for (int k = L > 0 ? L - 1 : 0; k <= L + 1; ++k)
         for (int f = 0; f < 6; ++f) b.P[iterate_set(-1, k)][f] = IT + (long)(6 * k + f) * n;
-      HIPCHK(launch_mag_pair(c, b, L, 1, st, 1, 0));
+      HIPCHK(launch_mag_pair(c, b, L, 1, st, 1, 0, count >= 0));
     }
     if (count >= 0) {
       F = count;

@@ -191,7 +191,9 @@ amx_status amx_fv_adjoint_step(amx_fv_ctx* ctx, const float* state, const float*
 
 /* The same with the fixed-point iterations of the forward step, as
  * amx_fv_evolve_state or the recording loop gave them for this state and step
- * size (mhd = 1; -1: not known): the call then only queues work. */
+ * size (mhd = 1; -1: not known): the call then only queues work. The reverse is
+ * that of a step of `count` iterations, whether or not the fixed point settles
+ * there. */
 amx_status amx_fv_adjoint_step_counted(amx_fv_ctx* ctx, const float* state, const float* d_dt, const float* lam_out,
                                        float* lam_in, int count, void* stream);
 
