@@ -88,13 +88,16 @@ def _function():
             if inputs is not None:
                 every = max(1, len(dts))  # one segment
             fctx.ctx, fctx.dts, fctx.every, fctx.ckpts, fctx.inputs = ctx, dts, every, ckpts, inputs
-            fctx.counts = counts
+            fctx.counts, fctx.physics = counts, (ctx.cfg.gamma, ctx.cfg.C_cfl)
             return s
 
         @staticmethod
         def backward(fctx, grad):
             import torch
             ctx, dts, every = fctx.ctx, fctx.dts, fctx.every
+            if (ctx.cfg.gamma, ctx.cfg.C_cfl) != fctx.physics:
+                # the context is shared: another run has set its own since
+                ctx.set_physics(*fctx.physics)
             lam = grad.contiguous().clone()
             lam_in = torch.empty_like(lam)
             nseg = (len(dts) + every - 1) // every
