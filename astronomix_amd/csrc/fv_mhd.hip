@@ -3923,7 +3923,16 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // stalled step with the further launches and goes on. Event timing keeps
   // the step-by-step path, which sorts out early-exited launches per step.
   const bool mbatch = c->cfg.mhd && (c->keep_b || (rec && !c->hook)) && c->timing == 0;
-  c->half = mbatch;
+  // Half pairs (pair_half) where the second iterate they leave out is worth the
+  // regeneration launch that then stands by in every step: in a batch without it
+  // the step whose count rises is held, and the rest of the batch runs empty
+  // (20 steps of 256^3 after 5: 1.668 ms a step without half pairs, 1.696 with
+  // them alone, 1.654 with the launch too). With / without, 3D: 48^3 1455 / 1470
+  // us, 64^3 1816 / 1826, 96^3 2017 / 2032; 8 steps of 128^3 269 / 286 a step, of
+  // 256^3 1664 / 1784. In 2D the launch costs what they save, at an even count
+  // 512^2 54.5 / 53.4 us a step, 1024^2 141.4 / 137.3, 1448^2 285.2 / 284.1.
+  constexpr long HALF_CELLS = 1L << 18;
+  c->half = mbatch && c->cfg.dim == 3 && c->ncell >= HALF_CELLS;
   // A record is taken behind a step's first kernels, which must have left the input whole.
   if (batch && (!rec || c->rk2_swap) && chains(c)) c->chain = CHAIN_GAS;
   if (mbatch && (!rec || c->rk2) && chains(c)) c->chain = CHAIN_MHD;
@@ -3945,6 +3954,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
     return n;
   };
   float last_dt = 0.f;
+  int kprev = 0;  // final launch index of the last step
   bool b_home = false;  // the final B is in the state's rows and hctl is current
   for (;;) {
     if (run->fixed_timestep) {
@@ -4004,13 +4014,17 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, spi);
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
+      // regeneration launches: after a batch that needed one, where half pairs
+      // may come (they start at even counts), and in a loop's first step, whose
+      // pairs go by the count of whatever this context ran last
+      const bool regen = c->regen_q || (c->half && (steps == 0 || !(kprev & 1)));
       for (long i = 0; i < n; ++i) {
         if (!c->chain) HIPCHK(record());
         c->front = c->chain && i > 0 ? mhd_front(c, spi) : Front();
         amx_status s = step_phase1(c, bl, 1, st, !run->fixed_timestep, &klast);
         if (s != AMX_OK) return s;
         if (c->chain) HIPCHK(record());
-        s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 1, c->regen_q);
+        s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 1, regen || steps + i == 0);
         if (s != AMX_OK) return s;
         // this step's end and the next one's beginning
         if (i + 1 == n)
@@ -4027,9 +4041,10 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       HIPCHK(hipMemcpyAsync(c->hctl, c->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, st));
       HIPCHK(hipStreamSynchronize(st));
       b_home = last && !c->hctl[0].stall;
-      // regeneration launches in the next batch only if a step of this one
-      // ended on an unstored first iterate (otherwise such a step stalls)
+      // a step of this batch ended on an unstored first iterate (without a
+      // regeneration launch behind it such a step stalls)
       c->regen_q = c->hctl[0].regen_ev > 0;
+      kprev = c->hctl[0].kprev;
       if (c->hctl[0].stall) {
         // the stalled step's launches up to klast have run (every launch
         // queued behind it exited at once): the further pairs, then its
@@ -4041,6 +4056,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
         amx_status s = fixed_point_more(c, bl, 1, st, &klast);
         if (s != AMX_OK) return s;
         fixed_point_settled(c, 1, &K);
+        kprev = K;
         s = step_phase3(c, bl, 1, st, !run->fixed_timestep, 0);
         if (s != AMX_OK) return s;
         hipLaunchKernelGGL(k_step_end, dim3(1), dim3(NSLOT), 0, st, c->ctl, c->keep_b, 0);

@@ -1,0 +1,55 @@
+"""Loops on both sides of the line from which on queued steps take half pairs
+(2^18 cells): a fixed point whose count rises from an even value, in a loop's
+first batch of steps and in a later one, gives the bits and counts of single
+steps."""
+
+import numpy as np
+import pytest
+
+from astronomix_amd import _native
+from astronomix_amd import workloads as W
+from astronomix_amd._finite_volume import native_config
+from astronomix_amd.option_classes.simulation_config import HLL
+
+pytestmark = pytest.mark.gpu
+
+
+def blast(shape):
+    """The blast's pressures and field on a grid of any shape."""
+    s = np.zeros((len(shape) + 5,) + shape, dtype=np.float32)
+    x = np.meshgrid(*[(np.arange(n) + 0.5) / n for n in shape], indexing="ij")
+    s[0] = 1.0
+    s[len(shape) + 1] = np.where(sum((a - 0.5) ** 2 for a in x) < 0.01, 10.0, 0.1)
+    s[len(shape) + 2:len(shape) + 4] = np.sqrt(0.5)
+    return s
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 64), (63, 65, 64), (512, 512)], ids=["line", "below", "2d"])
+@pytest.mark.parametrize("bound", ["time", "steps"])
+def test_rising_count(gpu, shape, bound):
+    import torch
+    print(f"[gpu] half pairs at their line {shape} {bound}", flush=True)
+    dim, steps = len(shape), 28
+    state = torch.from_numpy(blast(shape)).cuda()
+    cfg = native_config(tuple(state.shape), W.fv_config(dim, shape[-1], mhd=True, riemann=HLL), 5 / 3, 0.3,
+                        1.0 / shape[-1])
+    single = _native.FvContext(_native.AmxFvConfig.from_buffer_copy(cfg))
+    loop = _native.FvContext(_native.AmxFvConfig.from_buffer_copy(cfg))
+    one, dt, t, ks = state.clone(), torch.empty((), device="cuda"), np.float32(0), []
+    for _ in range(steps):
+        single.cfl_dt(one, dt)
+        before, t = t, np.float32(t + np.float32(dt.item()))
+        ks.append(single.evolve_state(one, dt))
+    print(ks, flush=True)
+    if bound == "time":  # batches of 4 and then up to 16 steps
+        run = dict(t_end=float(before + np.float32(0.5) * (t - before)), max_steps=-1)
+    else:                # 16 and the rest
+        run = dict(t_end=1.0, max_steps=steps)
+    run = _native.AmxFvRun(fixed_timestep=0, num_timesteps=0, exact_end_time=0, **run)
+    for _ in range(2):  # the second loop starts from the first one's last count
+        out = state.clone()
+        st = loop.time_integration(out, run)
+        assert st.steps == steps and st.fixed_point_iterations == sum(ks)
+        assert torch.equal(out, one)
+    if dim == 3:
+        assert any(a % 2 == 0 and b > a for a, b in zip(ks[4:], ks[5:])), ks
