@@ -93,6 +93,7 @@ struct Ctl {
   unsigned lfp[3][NSLOT];       // Lax-Friedrichs: partial maxima of |u| + c of the stage input
   int bset;                     // iterate set holding B0 of the magnetic sub-step; -1: the state's B rows
   int held;                     // the fixed point had not settled when k_mag_final ran: gated stage kernels return
+  int khalf, finh;              // kprev and fin where the next step may take half pairs, else -1 (pair_half)
   int kprev;                    // final launch index of the slot's previous step (k_mag_final): the speculative
                                 // pair starting there stores its first iterate, the others leave it out
   int regen_ev;                 // steps of the current batch that ended on a first iterate their pair did not
@@ -538,12 +539,12 @@ __host__ __device__ inline int pair_final(int L, float r0, float r1, float tol, 
 }
 
 // Pair (L, L+1) of the running speculative batch made iterate L only: its slot's
-// previous step ended on L, so this one is expected to, and iterate L+1 (its
-// curls and 6 of the launch's 25 fields) would be thrown away. Where residual
+// previous step ended on L, and so is this one expected to (khalf); iterate L+1
+// (its curls and 6 of the launch's 25 fields) would be thrown away. Where residual
 // L says that the fixed point goes on, the regeneration launch makes iterate
 // L+1 and its residual, and the pair counts as a whole one from there on.
-__host__ __device__ inline bool pair_half(unsigned half_mask, int L, int kprev) {
-  return L >= 0 && L <= 62 && ((half_mask >> (L >> 1)) & 1u) && L == kprev;
+__host__ __device__ inline bool pair_half(unsigned half_mask, int L, int khalf) {
+  return L >= 0 && L <= 62 && ((half_mask >> (L >> 1)) & 1u) && L == khalf;
 }
 
 // pair_final of such a pair before its second iterate is made
@@ -638,10 +639,11 @@ __device__ __forceinline__ FrontStep step_front(Ctl* c, const Front& f) {
   for (int k = 0; k < 3; ++k) mx[k] = p[k][lane];
   const bool writer = blockIdx.x == 0 && threadIdx.x < 64;
   // the last step's end, of which the writer alone reads what it writes
-  int run = 0, fin = 0, bset = 0, isum = 0, imax = 0, ibmax = 0;
+  int run = 0, fin = 0, finh = 0, bset = 0, isum = 0, imax = 0, ibmax = 0;
   if (writer) {
     run = c->run;
     fin = c->fin;
+    finh = c->finh;
     bset = c->bset;
     isum = c->iters_sum;
     imax = c->iters_max;
@@ -670,6 +672,7 @@ __device__ __forceinline__ FrontStep step_front(Ctl* c, const Front& f) {
       } else {
         c->iters = fin;
         c->kprev = fin;
+        c->khalf = finh;
         c->iters_sum = isum + fin;
         c->iters_max = fin > imax ? fin : imax;
         c->iters_bmax = fin > ibmax ? fin : ibmax;
@@ -710,25 +713,28 @@ struct FinalRule {
   float tol;
   int max_iter, spec, regen_queued;
   unsigned skip_mask, half_mask;
+  float half_tol;  // the next step may take half pairs if the final residual is not above
   int* counts;  // record of the final launch index of each step, or null
   long max_counts;
 };
 
 struct FinalIter {
   int f;        // final launch index; -1: none yet
+  int h;        // f where the next step may take half pairs, else -1
   int held;     // the step waits for further launches
   int counted;  // the next batch queues regeneration launches
 };
 
-__device__ __forceinline__ FinalIter final_iter(const FinalRule& q, int L, int kprev, float r0, float r1) {
+__device__ __forceinline__ FinalIter final_iter(const FinalRule& q, int L, int kprev, int khalf, float r0, float r1) {
   FinalIter o;
-  const bool hp = pair_half(q.half_mask, L, kprev);
+  const bool hp = pair_half(q.half_mask, L, khalf);
   const bool open = hp && half_final(L, r0, q.tol, q.max_iter) < 0;
   const bool half = hp && !(open && q.regen_queued);
   o.f = half ? half_final(L, r0, q.tol, q.max_iter) : pair_final(L, r0, r1, q.tol, q.max_iter);
   const bool unstored = o.f >= 0 && o.f == L && L <= 62 && ((q.skip_mask >> (L >> 1)) & 1u) && L != kprev;
   o.counted = q.spec && ((unstored && kprev >= 0) || open);
   o.held = (o.f < 0 || (unstored && !q.regen_queued)) && q.spec;
+  o.h = (o.f == L ? r0 : r1) <= q.half_tol ? o.f : -1;
   return o;
 }
 
@@ -749,15 +755,16 @@ __device__ __forceinline__ void pair_residuals(const Ctl* c, int L, float& r0, f
 
 // The final launch index, or -1 where the slot's step does not go on now.
 __device__ __forceinline__ int mag_front(Ctl* c, const FinalRule& q) {
-  const int run = c->run, L = c->iters - 1, kprev = c->kprev, steps = c->steps;
+  const int run = c->run, L = c->iters - 1, kprev = c->kprev, khalf = c->khalf, steps = c->steps;
   const float t = c->t, dt = c->dt;
   float r0, r1;
   pair_residuals(c, L, r0, r1);
   if (!run) return -1;
-  const FinalIter o = final_iter(q, L, kprev, r0, r1);
+  const FinalIter o = final_iter(q, L, kprev, khalf, r0, r1);
   if (blockIdx.x == 0 && threadIdx.x < 64) {
     if (o.counted) c->regen_ev = c->regen_ev + 1;
     c->fin = o.f;
+    c->finh = o.h;
     c->held = o.held;
     if (!o.held && q.counts && steps < q.max_counts && threadIdx.x == 0) q.counts[steps] = o.f;
     c->tq[0] = o.held ? t : t + dt;
@@ -857,7 +864,7 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
   // batch of scalar loads, before the branches that would order them one
   // after another (at 256^2 a stage launch is a few memory latencies long)
   int c_run = C->run, c_held = C->held, c_iters = C->iters;
-  const int c_bset = C->bset, c_fin = C->fin;
+  const int c_bset = C->bset, c_fin = C->fin, c_finh = C->finh;
   float c_dt = C->dt;
   const Phys ph = a.phs[slot];
   if (SRC == SRC_PLAIN && !HEUN && a.front.mode) {
@@ -870,7 +877,10 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
     c_held = c_iters < 0;
   } else if (W0M == SRC_PFIX && a.chained) {
     c_iters = c_fin;
-    if (a.chained == 2 && blockIdx.x == 0 && threadIdx.x == 0 && c_run && !c_held) C->iters = C->kprev = c_fin;
+    if (a.chained == 2 && blockIdx.x == 0 && threadIdx.x == 0 && c_run && !c_held) {
+      C->iters = C->kprev = c_fin;
+      C->khalf = c_finh;
+    }
   }
   if (!c_run) return;  // block-uniform: empty or finished slot
   if (a.gated && c_held) return;  // queued behind a fixed point that needs more launches
@@ -1746,7 +1756,7 @@ struct MagArgs {
   int regen;           // regeneration launch: see k_mag
   int counted;         // the caller knows the final launch: the pair is made whatever the residuals
   unsigned skip_mask;  // speculative pairs (bit L / 2), whose first iterate depends on kprev
-  unsigned half_mask;  // pairs that make their first iterate only where it is the slot's kprev (pair_half)
+  unsigned half_mask;  // pairs that make their first iterate only where it is the slot's khalf (pair_half)
   int max_iter;
   float tol;
   int euler;           // IMPLICIT_EULER: average = iterate
@@ -1910,7 +1920,8 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   Ctl* const C = a.ctl + slot;
   // the control block's scalars in one batch of loads (as in k_stage), and
   // with them the residuals that a launch after the first looks at
-  const int c_run = C->run, c_done = C->done, c_kprev = C->kprev, c_bset = C->bset, c_iters = C->iters;
+  const int c_run = C->run, c_done = C->done, c_kprev = C->kprev, c_khalf = C->khalf, c_bset = C->bset,
+            c_iters = C->iters;
   const float c_dt = C->dt;
   unsigned prev0 = 0u, prev1 = 0u;
   if (!a.regen && !a.counted && a.L > 0) {
@@ -1919,7 +1930,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
   }
   if (!c_run) return;
   int L = a.L;
-  bool one = a.regen || pair_half(a.half_mask, L, c_kprev);  // the launch computes its first iterate only
+  bool one = a.regen || pair_half(a.half_mask, L, c_khalf);  // the launch computes its first iterate only
   bool fill = false;  // regeneration: the second iterate of a half pair, with its residual
   if (a.regen) {
     // Regeneration: the fixed point's final launch is read from the residuals
@@ -1934,7 +1945,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
     const int Ll = c_iters - 1;
     if (Ll < 0 || Ll > 62) return;
     const float r0 = __uint_as_float(wave_max_u(C->resp[Ll % NRES][tid & 63]));
-    if (pair_half(a.half_mask, Ll, c_kprev)) {
+    if (pair_half(a.half_mask, Ll, c_khalf)) {
       if (half_final(Ll, r0, a.tol, a.max_iter) == Ll) return;
       fill = true;
       L = Ll + 1;
@@ -1951,7 +1962,7 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
     if (c_iters != L - 1 && c_iters != L + 1) return;
     const float r0 = __uint_as_float(wave_max_u(prev0));
     const float r1 = __uint_as_float(wave_max_u(prev1));
-    const bool half = pair_half(a.half_mask, L - 2, c_kprev);
+    const bool half = pair_half(a.half_mask, L - 2, c_khalf);
     const int f = half ? half_final(L - 2, r0, a.tol, a.max_iter) : pair_final(L - 2, r0, r1, a.tol, a.max_iter);
     if (f >= 0) {
       if (blockIdx.x == 0 && tid == 0) C->done = 1;
@@ -2273,11 +2284,11 @@ __global__ __launch_bounds__(((TA + 4) * (TBM + 4) + 255) / 256 * 256) void k_ma
 __global__ void k_mag_final(Ctl* ctl, FinalRule q) {
   Ctl* const c = ctl + blockIdx.x;
   // everything read is loaded first (as in step_control)
-  const int run = c->run, L = c->iters - 1, kprev = c->kprev, regen_ev = c->regen_ev, steps = c->steps;
+  const int run = c->run, L = c->iters - 1, kprev = c->kprev, khalf = c->khalf, regen_ev = c->regen_ev, steps = c->steps;
   float r0, r1;
   pair_residuals(c, L, r0, r1);
   if (!run) return;
-  const FinalIter o = final_iter(q, L, kprev, r0, r1);
+  const FinalIter o = final_iter(q, L, kprev, khalf, r0, r1);
   if (o.counted) c->regen_ev = regen_ev + 1;
   if (o.held) {
     c->held = 1;
@@ -2285,7 +2296,10 @@ __global__ void k_mag_final(Ctl* ctl, FinalRule q) {
     return;
   }
   c->iters = o.f >= 0 ? o.f : L + 1;
-  if (o.f >= 0) c->kprev = o.f;
+  if (o.f >= 0) {
+    c->kprev = o.f;
+    c->khalf = o.h;
+  }
   if (q.counts && steps < q.max_counts && threadIdx.x == 0) q.counts[steps] = c->iters;
   c->held = 0;
   c->stall = 0;
@@ -2374,7 +2388,7 @@ __device__ __forceinline__ void zero_cflp(Ctl* c) {
 template <bool END, bool BEGIN>
 __device__ __forceinline__ void step_control(Ctl* c, int keep_b, int chained, const StepParams& p) {
   const int lane = threadIdx.x;
-  const int run = c->run, held = c->held, live = c->live, stall = c->stall, bset = c->bset;
+  const int run = c->run, held = c->held, live = c->live, stall = c->stall, bset = c->bset, finh = c->finh;
   const int iters = chained ? c->fin : c->iters;
   const int isum = c->iters_sum, imax = c->iters_max, ibmax = c->iters_bmax;
   const float dt0 = c->dt, t_end = c->t_end;
@@ -2394,7 +2408,10 @@ __device__ __forceinline__ void step_control(Ctl* c, int keep_b, int chained, co
     c->iters_max = iters > imax ? iters : imax;
     c->iters_bmax = iters > ibmax ? iters : ibmax;
     if (keep_b) c->bset = iterate_set(bset, iters);
-    if (chained) c->iters = c->kprev = iters;
+    if (chained) {
+      c->iters = c->kprev = iters;
+      c->khalf = finh;
+    }
   }
   if (END && chained && run && held) c->stall = 1;
   if (!BEGIN) return;
@@ -2559,7 +2576,7 @@ __global__ void k_slot_reset(Ctl* ctl, int slot0, float t_end, int live, int fre
   c->held = 0;
   c->stall = 0;
   c->regen_ev = 0;
-  if (fresh) c->kprev = -1;
+  if (fresh) c->kprev = c->khalf = -1;
   c->iters_sum = 0;
   c->iters_max = 0;
   c->iters_bmax = 0;
@@ -2667,6 +2684,7 @@ struct amx_fv_ctx {
   int use_graphs;   // pool: replay captured HIP graphs of the step halves
   unsigned skip_mask;  // pairs of the current step queued without storing their first iterate
   int half;            // queued batches of steps: half pairs (pair_half); the host reads one status per batch
+  float half_tol;      // behind a final residual up to this
   int batch;        // pool: steps queued by one step_launch (1: a step in two halves)
   int batching;     // pool: the launched step is a queued batch
   std::map<std::tuple<int, int, int>, hipGraphExec_t> g_batch;  // (span, last count, steps)
@@ -3472,7 +3490,7 @@ int slot_final(const amx_fv_ctx* c, const Ctl& h, int half = 0) {
   float f0, f1;
   memcpy(&f0, &r0, sizeof(float));
   memcpy(&f1, &r1, sizeof(float));
-  if (half && pair_half(c->skip_mask, L, h.kprev))
+  if (half && pair_half(c->skip_mask, L, h.khalf))
     return half_final(L, f0, c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations);
   return pair_final(L, f0, f1, c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations);
 }
@@ -3506,7 +3524,7 @@ amx_status fixed_point_more(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t
   int open = 0;
   for (int s = 0; s < nspan && c->half; ++s) {
     const Ctl& h = c->hctl[s];
-    if (h.run && slot_final(c, h, 1) < 0 && pair_half(c->skip_mask, h.iters - 1, h.kprev)) open = 1;
+    if (h.run && slot_final(c, h, 1) < 0 && pair_half(c->skip_mask, h.iters - 1, h.khalf)) open = 1;
   }
   if (open) {
     HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
@@ -3537,6 +3555,10 @@ bool chains(const amx_fv_ctx* c) {
   return (r == AMX_HLL || r == AMX_HLLC || r == AMX_HLLC_LM) && c->cfg.limiter != AMX_VAN_ALBADA_PP;
 }
 
+// Grids up to this store both iterates of a pair (a microsecond or two there, 0.1
+// ms at 256^3) where a regeneration launch would have to stand by otherwise.
+constexpr long STORE_ALL = 1L << 18;
+
 Front mhd_front(const amx_fv_ctx* c, const StepParams& sp) {
   Front f = Front();
   f.mode = CHAIN_MHD;
@@ -3557,7 +3579,7 @@ amx_status step_phase3(amx_fv_ctx* c, const Bufs& b, int nspan, hipStream_t st, 
   const int rq = c->skip_mask && (regen || !spec);
   if (rq) HIPCHK(launch_mag_pair(c, b, 0, nspan, st, 1, 1));
   const FinalRule fr = {c->cfg.fixed_point_tol, c->cfg.max_fixed_point_iterations, spec, rq, c->skip_mask,
-                        c->half ? c->skip_mask : 0u, c->counts, c->max_counts};
+                        c->half ? c->skip_mask : 0u, c->half_tol, c->counts, c->max_counts};
   const int chained = c->chain == CHAIN_MHD && spec;
   if (!chained) {
     hipLaunchKernelGGL(k_mag_final, dim3(nspan), dim3(NSLOT), 0, st, c->ctl, fr);
@@ -3723,9 +3745,7 @@ extern "C" amx_status amx_fv_evolve_state(amx_fv_ctx* c, float* state, const flo
   // A caller's own loop pays each launch on the host (4 us) and, on a small grid,
   // on the device: the step takes its dt and ends its fixed point in its own
   // kernels (step_front, mag_front), and up to STORE_ALL cells its pairs store
-  // both iterates (a microsecond or two there, 0.1 ms a pair at 256^3) so that no
-  // regeneration launch has to stand by: 13 launches of CFL operator and step become 9.
-  constexpr long STORE_ALL = 1L << 18;
+  // both iterates: 13 launches of CFL operator and step become 9.
   struct Given {
     amx_fv_ctx* c;
     ~Given() {
@@ -3826,7 +3846,7 @@ __global__ void k_noalloc_begin(Ctl* c, Phys* ph, Phys v, const float* dtp) {
   c->dt = *dtp;
   c->run = 1;
   c->bset = -1;
-  c->kprev = -1;
+  c->kprev = c->khalf = -1;
   c->regen_ev = 0;
   for (int i = 0; i < 4; ++i) c->cfl[i] = 0u;
   zero_cflp(c);
@@ -3933,7 +3953,7 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   struct KeepB {
     amx_fv_ctx* c;
     ~KeepB() {
-      c->keep_b = c->rk2_swap = c->half = c->chain = 0;
+      c->keep_b = c->rk2_swap = c->half = c->chain = c->store_all = 0;
       c->counts = nullptr;
       c->front = Front();
     }
@@ -3977,16 +3997,19 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
   // stalled step with the further launches and goes on. Event timing keeps
   // the step-by-step path, which sorts out early-exited launches per step.
   const bool mbatch = c->cfg.mhd && (c->keep_b || (rec && !c->hook)) && c->timing == 0;
-  // Half pairs (pair_half) where the second iterate they leave out is worth the
-  // regeneration launch that then stands by in every step: in a batch without it
-  // the step whose count rises is held, and the rest of the batch runs empty
-  // (20 steps of 256^3 after 5: 1.668 ms a step without half pairs, 1.696 with
-  // them alone, 1.654 with the launch too). With / without, 3D: 48^3 1455 / 1470
-  // us, 64^3 1816 / 1826, 96^3 2017 / 2032; 8 steps of 128^3 269 / 286 a step, of
-  // 256^3 1664 / 1784. In 2D the launch costs what they save, at an even count
-  // 512^2 54.5 / 53.4 us a step, 1024^2 141.4 / 137.3, 1448^2 285.2 / 284.1.
-  constexpr long HALF_CELLS = 1L << 18;
-  c->half = mbatch && c->cfg.dim == 3 && c->ncell >= HALF_CELLS;
+  // Half pairs (pair_half). A step whose count rises from one's is held, and the
+  // rest of its batch runs empty, unless the regeneration launch stands by: 20
+  // steps of 256^3 after 5 took 1.696 ms each with half pairs alone, 1.668 without,
+  // 1.649 with both. The launch costs 3-4 us a step in 3D, so smaller grids, where
+  // that is most of what a half pair saves, and 2D do without: they take half pairs
+  // only behind a final residual up to HALF_MARGIN of the tolerance. Ahead of a
+  // rise it grows by 5-25 % a step (blasts of 32^3-256^3, Orszag-Tang), so that the
+  // steps about the rise make whole pairs and none is held.
+  constexpr long STANDBY_CELLS = 1L << 20;
+  constexpr float HALF_MARGIN = 0.75f;
+  const bool standby = c->cfg.dim == 3 && c->ncell >= STANDBY_CELLS;
+  c->half = mbatch;
+  c->half_tol = standby ? INFINITY : HALF_MARGIN * c->cfg.fixed_point_tol;
   // A record is taken behind a step's first kernels, which must have left the input whole.
   if (batch && (!rec || c->rk2_swap) && chains(c)) c->chain = CHAIN_GAS;
   if (mbatch && (!rec || c->rk2) && chains(c)) c->chain = CHAIN_MHD;
@@ -4068,13 +4091,15 @@ amx_status fv_loop(amx_fv_ctx* c, float* state, const amx_fv_run* run, snap::Dri
       hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(NSLOT), 0, st, c->ctl, spi);
       HIPCHK(hipGetLastError());
       spi.batch_first = 0;
-      // regeneration launches: after a batch that needed one, where half pairs
-      // may come (they start at even counts), and in a loop's first step, whose
-      // pairs go by the count of whatever this context ran last
-      const bool regen = c->regen_q || (c->half && (steps == 0 || !(kprev & 1)));
+      // regeneration launches: after a batch that needed one, and where they stand
+      // by for half pairs (which start at even counts). A loop's first step, whose
+      // pairs go by the count of whatever this context ran last, has one, or on
+      // small grids stores every iterate.
+      const bool regen = c->regen_q || (standby && (steps == 0 || !(kprev & 1)));
       for (long i = 0; i < n; ++i) {
         if (!c->chain) HIPCHK(record());
         c->front = c->chain && i > 0 ? mhd_front(c, spi) : Front();
+        c->store_all = steps + i == 0 && c->ncell <= STORE_ALL;
         amx_status s = step_phase1(c, bl, 1, st, !run->fixed_timestep, &klast);
         if (s != AMX_OK) return s;
         if (c->chain) HIPCHK(record());
@@ -4908,6 +4933,7 @@ extern "C" amx_status amx_fv_pool_set_batch(amx_fv_pool* p, int steps) {
   if (steps < 1 || steps > 256) return fail(AMX_ERR_INVALID, "steps per launch must be in 1..256%s");
   p->c->batch = steps;
   p->c->half = steps > 1;
+  p->c->half_tol = INFINITY;  // its batches queue the regeneration launch
   return AMX_OK;
 }
 
