@@ -127,11 +127,6 @@ constexpr float G53M1 = 1.6666666f - 1.0f;
 // i.e. the median of {a, b, 0}: one v_med3_f32.
 __device__ __forceinline__ float minmod(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.f); }
 
-// limited gradient times dx/2 (limited_gradients.py:50-60, reconstruction.py:409-412)
-__device__ __forceinline__ float half_slope(float wm, float w0, float wp) {
-  return 0.5f * minmod(w0 - wm, wp - w0);
-}
-
 // Limiter ids (simulation_config.py:29-34 values).
 enum { LIM_MINMOD = 0, LIM_OSHER = 1, LIM_DOUBLE_MINMOD = 2, LIM_SUPERBEE = 3, LIM_VAN_ALBADA = 4, LIM_VAN_ALBADA_PP = 5 };
 
@@ -180,19 +175,22 @@ __device__ __forceinline__ float limited_gradient(float wm, float w0, float wp, 
 // instruction cache, and without the factors' LDS it takes the lagged update.
 enum { LX_MINMOD = 0, LX_VAN_ALBADA = 1, LX_ANY = 2 };
 
-// Limited slope: minmod's in its exact difference form, halved, or another limiter's gradient.
-template <int LIMX>
+// Limited slope: with minmod the limited difference, limited gradient times dx
+// (limited_gradients.py:50-60), in 2D halved already; or another limiter's gradient.
+template <int DIM, int LIMX>
 __device__ __forceinline__ float slope(float wm, float w0, float wp, int lim, const GradScale& gs) {
-  if (LIMX == LX_MINMOD) return half_slope(wm, w0, wp);
+  if (LIMX == LX_MINMOD) return DIM == 3 ? minmod(w0 - wm, wp - w0) : 0.5f * minmod(w0 - wm, wp - w0);
   return limited_gradient(wm, w0, wp, LIMX == LX_VAN_ALBADA ? (int)LIM_VAN_ALBADA : lim, gs);
 }
 
 // A cell's value at its upper (SIDE = 1) or lower (-1) interface from its slope
-// (reconstruction.py:409-412).
-template <int LIMX, int SIDE>
+// (reconstruction.py:409-412). In 3D the half is in the FMA at every place: halved
+// beforehand here and in the sum there, subnormal differences would round apart.
+template <int DIM, int LIMX, int SIDE>
 __device__ __forceinline__ float edge(float w, float s, const GradScale& gs) {
-  if (LIMX == LX_MINMOD) return SIDE > 0 ? w + s : w - s;
-  return __builtin_fmaf(SIDE > 0 ? gs.half_dx : -gs.half_dx, s, w);
+  if (LIMX == LX_MINMOD && DIM != 3) return SIDE > 0 ? w + s : w - s;
+  const float half = LIMX == LX_MINMOD ? 0.5f : gs.half_dx;
+  return __builtin_fmaf(SIDE > 0 ? half : -half, s, w);
 }
 
 // Boundary codes (AMX_BC_*) of the two sides of one axis.
@@ -1019,14 +1017,14 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
       }
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        da[v] = slope<LIMX>(qm1[v], qa[v], qb[v], lim, ldx);
-        float sm = slope<LIMX>(qm2[v], qm1[v], qa[v], lim, ldx);
+        da[v] = slope<DIM, LIMX>(qm1[v], qa[v], qb[v], lim, ldx);
+        float sm = slope<DIM, LIMX>(qm2[v], qm1[v], qa[v], lim, ldx);
         if (pp) {
           da[v] = da[v] * fsel(fa0, fk0, fb0, v);
           sm = sm * fsel(fam, fkm, fbm, v);
         }
-        wl[v] = edge<LIMX, 1>(qm1[v], sm, ldx);
-        wr[v] = edge<LIMX, -1>(qa[v], da[v], ldx);
+        wl[v] = edge<DIM, LIMX, 1>(qm1[v], sm, ldx);
+        wr[v] = edge<DIM, LIMX, -1>(qa[v], da[v], ldx);
       }
       riemann<DIM, 1, RS>(wl, wr, Fa, ph, alf[0], AMS && gsw[(unsigned)x0 * sx + col]);
     } else {
@@ -1163,10 +1161,10 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
         if (pp) ppx(x + 1, fa1, fk1, fb1);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-          d1[v] = slope<LIMX>(q0[v], q1[v], q2[v], lim, ldx);
+          d1[v] = slope<DIM, LIMX>(q0[v], q1[v], q2[v], lim, ldx);
           if (pp) d1[v] = d1[v] * fsel(fa1, fk1, fb1, v);
-          wl[v] = edge<LIMX, 1>(q0[v], d0[v], ldx);
-          wr[v] = edge<LIMX, -1>(q1[v], d1[v], ldx);
+          wl[v] = edge<DIM, LIMX, 1>(q0[v], d0[v], ldx);
+          wr[v] = edge<DIM, LIMX, -1>(q1[v], d1[v], ldx);
         }
         riemann<DIM, 1, RS>(wl, wr, Fn, ph, alf[0],
                             AMS && gsw[(unsigned)wrapi(x + 1, a.nx) * sx + col]);
@@ -1207,13 +1205,13 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         const float w0 = W[v][o - 2 * WW], w1 = W[v][o - WW], w2 = W[v][o], w3 = W[v][o + WW];
-        float s1 = slope<LIMX>(w0, w1, w2, lim, ldx), s2 = slope<LIMX>(w1, w2, w3, lim, ldx);
+        float s1 = slope<DIM, LIMX>(w0, w1, w2, lim, ldx), s2 = slope<DIM, LIMX>(w1, w2, w3, lim, ldx);
         if (pp) {
           s1 = s1 * fsel(sPF[0][o - WW], sPF[1][o - WW], sPF[4][o - WW], v);
           s2 = s2 * fsel(sPF[0][o], sPF[1][o], sPF[4][o], v);
         }
-        wl[v] = edge<LIMX, 1>(w1, s1, ldx);
-        wr[v] = edge<LIMX, -1>(w2, s2, ldx);
+        wl[v] = edge<DIM, LIMX, 1>(w1, s1, ldx);
+        wr[v] = edge<DIM, LIMX, -1>(w2, s2, ldx);
       }
       riemann<DIM, AXA, RS>(wl, wr, f, ph, alf[AXA - 1], AMS && G[o]);
 #pragma unroll
@@ -1226,13 +1224,13 @@ __global__ __launch_bounds__((TA + 1) * TB) __attribute__((amdgpu_waves_per_eu(A
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         const float w0 = W[v][o - 2], w1 = W[v][o - 1], w2 = W[v][o], w3 = W[v][o + 1];
-        float s1 = slope<LIMX>(w0, w1, w2, lim, ldx), s2 = slope<LIMX>(w1, w2, w3, lim, ldx);
+        float s1 = slope<DIM, LIMX>(w0, w1, w2, lim, ldx), s2 = slope<DIM, LIMX>(w1, w2, w3, lim, ldx);
         if (pp) {
           s1 = s1 * fsel(sPF[2][o - 1], sPF[3][o - 1], sPF[4][o - 1], v);
           s2 = s2 * fsel(sPF[2][o], sPF[3][o], sPF[4][o], v);
         }
-        wl[v] = edge<LIMX, 1>(w1, s1, ldx);
-        wr[v] = edge<LIMX, -1>(w2, s2, ldx);
+        wl[v] = edge<DIM, LIMX, 1>(w1, s1, ldx);
+        wr[v] = edge<DIM, LIMX, -1>(w2, s2, ldx);
       }
       riemann<DIM, AXB, RS>(wl, wr, f, ph, alf[AXB - 1], AMS && G[o]);
 #pragma unroll
@@ -1396,8 +1394,8 @@ __global__ __launch_bounds__(1024) void k_rk2(const Rk2Args a) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const float q0 = s[v * st + o - 2 * d], q1 = s[v * st + o - d], q2 = s[v * st + o], q3 = s[v * st + o + d];
-      wl[v] = edge<LIMX, 1>(q1, slope<LIMX>(q0, q1, q2, LIM_VAN_ALBADA, gs), gs);
-      wr[v] = edge<LIMX, -1>(q2, slope<LIMX>(q1, q2, q3, LIM_VAN_ALBADA, gs), gs);
+      wl[v] = edge<2, LIMX, 1>(q1, slope<2, LIMX>(q0, q1, q2, LIM_VAN_ALBADA, gs), gs);
+      wr[v] = edge<2, LIMX, -1>(q2, slope<2, LIMX>(q1, q2, q3, LIM_VAN_ALBADA, gs), gs);
     }
     riemann<2, AX, RS>(wl, wr, fl, ph, 0.f, false);
 #pragma unroll
