@@ -2648,6 +2648,7 @@ struct amx_fv_ctx {
   int bcx;          // some axis has open / reflective boundaries
   AxisBc bx, ba, bb;  // boundaries of the kernel axes x, A, B
   int ntb, nta, ntb_mag, nta_mag, ncx, lx, ncx_mag, lx_mag;
+  int lx1;          // lx of one simulation (a pool's lx goes by its span)
   int cap;
   long sstride;     // floats per slot (0 for a single simulation)
   float* mem;       // pool: cap x [state NS | G1 NV | P0 6 | P1 6]; single: [G1 | P0 | P1]
@@ -2963,6 +2964,16 @@ int pick_stage_chunk(long tiles, int nx) {
   return best;
 }
 
+// Planes per block along x of the 3D stage kernels on grids that fill the chip:
+// about 1900 blocks, the chunk the multiple of 4 planes (the kernels' x-march
+// unroll) nearest to that (the kernels reload 4 planes at each chunk start, so
+// longer chunks save traffic). Measured at 256^3 (148 tiles): 20 planes 1.718 ms
+// per step, 16: 1.753, 24 and 30: 1.73, 28: 1.80, 36: 1.85.
+int full_stage_chunk(long tiles, int nx) {
+  const long target = (tiles * nx + 950) / 1900;
+  return (int)(((target + 2) / 4) * 4);
+}
+
 // Geometry and launch shapes of a context of cap slots (no allocation).
 void init_geometry(amx_fv_ctx* c, const amx_fv_config* cfg, int cap, int own_state) {
   c->cfg = *cfg;
@@ -2995,18 +3006,12 @@ void init_geometry(amx_fv_ctx* c, const amx_fv_config* cfg, int cap, int own_sta
   c->nta_mag = (c->na + TA_MAG - 1) / TA_MAG;
   c->ntb_mag = (c->nb + TB_MAG - 1) / TB_MAG;
   if (cfg->dim == 3) {
-    // planes per block along x for the stage kernels: about 1900 blocks, the
-    // chunk the multiple of 4 planes (the kernels' x-march unroll) nearest to
-    // that (the kernels reload 4 planes at each chunk start, so longer chunks
-    // save traffic). Measured at 256^3 (148 tiles): 20 planes 1.718 ms per
-    // step, 16: 1.753, 24 and 30: 1.73, 28: 1.80, 36: 1.85. Grids whose chunk
-    // would be 8 planes or less (up to about 190^3) are short of blocks
-    // instead: pick_stage_chunk.
+    // grids whose chunk would be 8 planes or less (up to about 190^3) are short
+    // of blocks instead: pick_stage_chunk
     const long tiles = (long)c->ntb * c->nta;
     c->lx = env_int("AMX_LX", 0);
     if (c->lx <= 0) {
-      const long target = (tiles * cfg->nx + 950) / 1900;
-      c->lx = (int)(((target + 2) / 4) * 4);
+      c->lx = full_stage_chunk(tiles, cfg->nx);
       if (c->lx <= 8) c->lx = pick_stage_chunk(tiles, cfg->nx);
     }
     if (c->lx > cfg->nx) c->lx = cfg->nx;
@@ -3017,6 +3022,7 @@ void init_geometry(amx_fv_ctx* c, const amx_fv_config* cfg, int cap, int own_sta
   } else {
     c->lx = c->lx_mag = 1;
   }
+  c->lx1 = c->lx;
   c->ncx = (c->nxm + c->lx - 1) / c->lx;
   c->ncx_mag = (c->nxm + c->lx_mag - 1) / c->lx_mag;
   c->rk2 = rk2_rows(cfg);
@@ -4737,6 +4743,32 @@ extern "C" amx_status amx_fv_pool_read(amx_fv_pool* p, int slot, float* dst, voi
   return AMX_OK;
 }
 
+namespace {
+
+// Planes per block along x of a pool's stage launches: of a full chip where the
+// slots' tiles together fill it, else of one simulation. (A slot's bits do not
+// depend on it.) Stream of 32 requests, slots of up to 128^3, solves/s: chunks of
+// one simulation 8.25, these 8.37, pick_stage_chunk for the span's tiles 8.32;
+// six small requests: 3.92 ms with each.
+void pool_chunk(amx_fv_ctx* c, int span) {
+  if (c->cfg.dim != 3 || env_int("AMX_LX", 0) > 0) return;
+  const int full = full_stage_chunk((long)c->ntb * c->nta * span, c->cfg.nx);
+  c->lx = full > 8 ? full : c->lx1;
+  if (c->lx > c->cfg.nx) c->lx = c->cfg.nx;
+  c->ncx = (c->nxm + c->lx - 1) / c->lx;
+}
+
+// A pool's queued steps chain where a stage launch is one round of blocks, two a
+// CU: what a chained step's blocks do each for themselves (step_front, mag_front)
+// costs a microsecond or two a round, as much as the launches that it saves where
+// there are several. The stream above with every step chained / up to one round /
+// none: 8.25 / 8.28 / 8.29 solves/s; the six requests: 3.97 / 3.97 / 4.09 ms.
+bool pool_chains(const amx_fv_ctx* c, int span) {
+  return c->cfg.mhd && chains(c) && (long)span * c->ntb * c->nta * c->ncx <= 2L * device_cus();
+}
+
+}  // namespace
+
 extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
   if (!p || !p->c) return fail(AMX_ERR_INVALID, "null pool%s");
   amx_fv_ctx* c = p->c;
@@ -4746,6 +4778,7 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
     if (c->live[s]) span = s + 1;
   c->span = span;
   if (span == 0) return AMX_OK;
+  pool_chunk(c, span);
   hipStream_t st = (hipStream_t)stream;
   const Bufs b = bufs(c, nullptr);
   int klast = 0;
@@ -4801,7 +4834,7 @@ extern "C" amx_status amx_fv_pool_step_launch(amx_fv_pool* p, void* stream) {
           c->front = Front();
         }
       } guard{c};
-      c->chain = c->cfg.mhd && chains(c) ? CHAIN_MHD : 0;
+      c->chain = pool_chains(c, span) ? CHAIN_MHD : 0;
       for (int i = 0; i < nb; ++i) {
         c->front = c->chain && i > 0 ? mhd_front(c, spi) : Front();
         int kl = 0;
