@@ -69,6 +69,10 @@ def _function():
         known = list(dts[:steps].unbind())
         if steps > most:
             return None, known, None, None
+        if 2 * steps <= most:
+            # the record was made before the number of steps was known, and
+            # the graph holds it until the backward sweep
+            inputs = inputs[:steps].clone()
         return s, known, inputs, counts[:steps].tolist() if counts is not None else [-1] * steps
 
     class Rollout(torch.autograd.Function):
