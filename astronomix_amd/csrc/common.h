@@ -56,11 +56,9 @@ __device__ __forceinline__ unsigned block_max_u(unsigned v, unsigned* sred) {
   return m;
 }
 
-// Max over the slots, one slot a lane: called by a whole wavefront. (The
-// control kernels run one wavefront per simulation; a single thread walking
-// the slots took 3.5-6 us a launch, most of it one load after another.)
+// The control kernels run one wavefront per simulation, a lane per slot (a single
+// thread walking the slots took 3.5-6 us a launch, one load after another).
 static_assert(NSLOT == 64, "one slot a lane");
-__device__ __forceinline__ unsigned slots_max(const unsigned* p) { return wave_max_u(p[threadIdx.x & 63]); }
 
 }  // namespace amx
 

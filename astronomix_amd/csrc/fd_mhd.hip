@@ -52,8 +52,6 @@ struct Grid {
   long nc;
 };
 
-__device__ __forceinline__ long cell(const Grid& g, int x, int y, int z) { return (long)x * g.sx + (long)y * g.sy + z; }
-
 // Byte offset of a cell in a field, with its coordinates: one division per
 // cell in 32-bit arithmetic (grids have < 2^30 cells), none for its stencil
 // neighbours, and loads with a scalar base and a 32-bit offset.
@@ -214,9 +212,8 @@ __device__ __forceinline__ void stage_cell(const float* u, const Phys& ph, float
   o[C_F + 6] = Bz * vx - Bx * vz;
   // the eigen-system's own floors (_eigen.py:62-74, 148-160)
   const bool low = rho < ph.rhomin;
-  const float ra = low ? ph.rhomin : rho, rinv = low ? ph.inv_rhomin : ri;
+  const float rinv = low ? ph.inv_rhomin : ri;
   const float pe = pc < ph.pgmin ? ph.pgmin : pc;
-  (void)ra;
   const float cs2 = fmaxf(0.f, ph.gamma * fabsf(pe * rinv));
   const float s = b2 * rinv + cs2;
   const float bx2 = (Bx * Bx) * rinv;

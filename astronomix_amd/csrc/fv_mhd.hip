@@ -2817,9 +2817,6 @@ amx_status validate(const amx_fv_config* c) {
   return AMX_OK;
 }
 
-// G1 (gas rows) | P0 | P1 | P2 (B, v iterates of the fixed point)
-// G1 (gas rows) | P0 | P1 | P2 (B, v iterate sets) | PF (fixed pressure) | P3
-// (the fourth set: step loops and pools keep B in the sets)
 // Rows of the tiles in which k_rk2 takes this configuration's gas steps, or 0:
 // two stage launches. It covers 2D, the solvers and limiters that need no pass
 // or ghost cells between the stages, and grids that latency bounds. The lines by
@@ -2839,7 +2836,9 @@ int rk2_rows(const amx_fv_config* cfg) {
   return tiles <= 160 ? 4 : 8;
 }
 
-// (with k_rk2 the gas rows between the halves of an MHD step have rows of their own)
+// Workspace rows: G1 (gas rows) | P0 | P1 | P2 (B, v iterate sets) | PF (fixed
+// pressure) | P3 (the fourth set: step loops and pools keep B in the sets) | with
+// k_rk2 the gas rows between the halves of an MHD step
 long ws_fields(const amx_fv_config* cfg, int /*own_state*/) {
   return (cfg->dim + 2) + (cfg->mhd ? 25 + (rk2_rows(cfg) ? cfg->dim + 2 : 0) : 0);
 }
@@ -4337,11 +4336,11 @@ amx_status adjoint_step_t(amx_fv_ctx* c, const float* w0, const float* lam_out, 
     }
     HIPCHK((launch_rk2<false>(c, a, 1, st)));
   } else {
-  StageArgs a1 = stage_base(c, dt_scale);
-  a1.front = take_front(c);
-  for (int v = 0; v < NV; ++v) {
-    a1.src[v] = w0 + (long)v * n;
-    a1.out[v] = G1 + (long)v * n;
+    StageArgs a1 = stage_base(c, dt_scale);
+    a1.front = take_front(c);
+    for (int v = 0; v < NV; ++v) {
+      a1.src[v] = w0 + (long)v * n;
+      a1.out[v] = G1 + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a1, 1, st)));
   StageArgs a2 = stage_base(c, dt_scale);
@@ -4462,11 +4461,11 @@ amx_status adjoint_step_mhd(amx_fv_ctx* c, const float* state, const float* lam_
     }
     HIPCHK((launch_rk2<true>(c, a, 1, st)));
   } else {
-  StageArgs a1 = stage_base(c, 0.5f);
-  a1.front = take_front(c);
-  for (int v = 0; v < NV; ++v) {
-    a1.src[v] = state + (long)v * n;
-    a1.out[v] = G1 + (long)v * n;
+    StageArgs a1 = stage_base(c, 0.5f);
+    a1.front = take_front(c);
+    for (int v = 0; v < NV; ++v) {
+      a1.src[v] = state + (long)v * n;
+      a1.out[v] = G1 + (long)v * n;
   }
   HIPCHK((launch_stage<SRC_PLAIN, false, SRC_PLAIN>(c, a1, 1, st)));
   StageArgs a2 = stage_base(c, 0.5f);
