@@ -3558,9 +3558,11 @@ bool chains(const amx_fv_ctx* c) {
   return (r == AMX_HLL || r == AMX_HLLC || r == AMX_HLLC_LM) && c->cfg.limiter != AMX_VAN_ALBADA_PP;
 }
 
-// Grids up to this store both iterates of a pair (a microsecond or two there, 0.1
-// ms at 256^3) where a regeneration launch would have to stand by otherwise.
-constexpr long STORE_ALL = 1L << 18;
+// Grids up to this store both iterates of a pair where a regeneration launch would
+// have to stand by otherwise. Operators (CFL step and step), with the launch /
+// storing both, us: 64^3 145.5 / 139.0, 80^3 183.0 / 179.5, 96^3 224.2 / 224.7, 128^3
+// 350.6 / 356.8; 2D 512^2 104.5 / 105.0, 724^2 134.5 / 129.3, 1024^2 170.9 / 165.7.
+constexpr long STORE_ALL = 1L << 19;
 
 Front mhd_front(const amx_fv_ctx* c, const StepParams& sp) {
   Front f = Front();

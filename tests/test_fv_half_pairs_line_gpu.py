@@ -1,5 +1,5 @@
 """Loops on both sides of the lines between the ways of queued steps around half
-pairs (every iterate of the first step stored up to 2^18 cells, regeneration
+pairs (every iterate of the first step stored up to 2^19 cells, regeneration
 launches standing by in 3D from 2^20): a fixed point whose count rises from an
 even value, in a loop's first batch of steps and in a later one, gives the bits
 and counts of single steps."""
@@ -25,7 +25,7 @@ def blast(shape):
     return s
 
 
-@pytest.mark.parametrize("shape", [(64, 64, 64), (63, 65, 65), (104, 100, 102), (512, 512)],
+@pytest.mark.parametrize("shape", [(64, 128, 64), (64, 65, 128), (104, 100, 102), (512, 512)],
                          ids=["stored", "first", "standby", "2d"])
 @pytest.mark.parametrize("bound", ["time", "steps"])
 def test_rising_count(gpu, shape, bound):
