@@ -3784,9 +3784,13 @@ extern "C" amx_status amx_fv_evolve_state(amx_fv_ctx* c, float* state, const flo
 // block, constants; the stage and iterate buffers are written before read).
 namespace {
 constexpr size_t NOALLOC_SCRATCH_BYTES = AMX_NOALLOC_SCRATCH_BYTES;
+// The bound counts this much for the control block, whatever it has grown to, so
+// that it refuses the same grids; the rest of the block has room behind it.
+constexpr size_t NOALLOC_CTL_BYTES = 3328, NOALLOC_CTL_ROOM = 4096;
+static_assert(sizeof(Ctl) <= NOALLOC_CTL_BYTES + NOALLOC_CTL_ROOM, "the scratch has no room for the control block");
 }  // namespace
 
-static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES + NOALLOC_CTL_ROOM];
 
 namespace {
 
@@ -3864,10 +3868,11 @@ extern "C" amx_status amx_fv_evolve_state_noalloc(const amx_fv_config* cfg, floa
   if (s != AMX_OK) return s;
   if (!state || !d_dt) return fail(AMX_ERR_INVALID, "null argument%s");
   const ScratchLayout L = scratch_layout(cfg);
-  if (L.total > NOALLOC_SCRATCH_BYTES) {
+  const size_t need = L.total - L.phys + NOALLOC_CTL_BYTES;
+  if (need > NOALLOC_SCRATCH_BYTES) {
     char msg[160];
     snprintf(msg, sizeof(msg), "this grid needs %zu bytes of scratch, the allocation-free step has %zu",
-             L.total, NOALLOC_SCRATCH_BYTES);
+             need, NOALLOC_SCRATCH_BYTES);
     return fail(AMX_ERR_INVALID, "%s", msg);
   }
   unsigned char* base = nullptr;
